@@ -423,11 +423,18 @@ struct EpaWork {
     int edges[EPA_MAXF * 3][2];
 };
 
+// A face without area has no plane: it is given a distance no other face exceeds, so that it
+// is never the closest one (the work area holds an earlier pair's faces otherwise).
+constexpr float EPA_NO_FACE = 3.0e38f;
 AXM_D bool epa_make_face(EpaWork& W, int f) {
     const f3 a = W.vt[W.fv[f][0]].w, b = W.vt[W.fv[f][1]].w, c = W.vt[W.fv[f][2]].w;
     f3 nn = cross(b - a, c - a);
     const float l = sqrtf(dot(nn, nn));
-    if (!(l > 1e-12f)) return false;
+    if (!(l > 1e-12f)) {
+        W.fn[f] = {0.0f, 0.0f, 0.0f};
+        W.fd[f] = EPA_NO_FACE;
+        return false;
+    }
     nn = nn * (1.0f / l);
     W.fn[f] = nn;
     W.fd[f] = dot(nn, a);
@@ -535,9 +542,11 @@ AXM_D EpaOut epa(const Shp& Aw, const Shp& Bw, const GjkOut& g, EpaWork& W, int 
         }
         if (bad || nf == 0) break;
     }
+    if (nf == 0) return o;
     best = 0;
     for (int f = 1; f < nf; ++f)
         if (W.fd[f] < W.fd[best]) best = f;
+    if (!(W.fd[best] < EPA_NO_FACE)) return o;
     const f3 pr = W.fn[best] * W.fd[best];
     const f3 a = W.vt[W.fv[best][0]].w, b = W.vt[W.fv[best][1]].w, c = W.vt[W.fv[best][2]].w;
     const f3 e0 = b - a, e1 = c - a, e2 = pr - a;

@@ -454,7 +454,12 @@ template <class T> inline EpaOut<T> epa(const Shape<T>& Aw, const Shape<T>& Bw, 
         const V3<T> a = vt[fv[f][0]].w, b = vt[fv[f][1]].w, c = vt[fv[f][2]].w;
         V3<T> nn = cross(b - a, c - a);
         const T l = std::sqrt(dot(nn, nn));
-        if (!(l > T(1e-12))) return false;
+        if (!(l > T(1e-12))) {
+            // no plane: never the closest face
+            fn[f] = {T(0), T(0), T(0)};
+            fd[f] = T(3.0e38);
+            return false;
+        }
         nn = nn * (T(1) / l);
         fn[f] = nn;
         fd[f] = dot(nn, a);
@@ -520,9 +525,11 @@ template <class T> inline EpaOut<T> epa(const Shape<T>& Aw, const Shape<T>& Bw, 
         if (bad || nf == 0) break;
     }
     o.iters = it;
+    if (nf == 0) return o;
     best = 0;
     for (int f = 1; f < nf; ++f)
         if (fd[f] < fd[best]) best = f;
+    if (!(fd[best] < T(3.0e38))) return o;
     // barycentric weights of the origin's projection onto the closest face
     const V3<T> pr = fn[best] * fd[best];
     const V3<T> a = vt[fv[best][0]].w, b = vt[fv[best][1]].w, c = vt[fv[best][2]].w;
