@@ -1137,16 +1137,27 @@ __global__ void __launch_bounds__(256) k_col_sort_input(Bodies B, const uint2* _
         val[m] = m;
     }
 }
-// The work list of the islands solved by one workgroup each, from the sorted keys: (first
-// slot, manifolds) of every small island of more than ISLAND_LANE_MAX manifolds; the smaller
-// ones are only counted (the bundle kernel finds them by their slots).
+// Size classes of the islands of more than ISLAND_LANE_MAX manifolds (k_pgs_islands solves
+// the largest first): 0 above 256 manifolds, 1 above 64, 2 above 32, 3 above 16, 4 the rest.
+// Their work list entries (first slot, manifolds) lie in one region per class, each as long as
+// the manifold capacity allows islands of its class.
+__device__ __forceinline__ uint32_t isl_class(uint32_t n) {
+    return n > 256u ? 0u : (n > 64u ? 1u : (n > 32u ? 2u : (n > 16u ? 3u : 4u)));
+}
+__device__ __forceinline__ uint32_t isl_region(uint32_t c, uint32_t cap) {
+    uint32_t o = 0;
+    if (c > 0u) o += cap / 257u;
+    if (c > 1u) o += cap / 65u;
+    if (c > 2u) o += cap / 33u;
+    if (c > 3u) o += cap / 17u;
+    return o;
+}
 // One pass over the sorted keys skey (thread gid of gsz, both whole waves; every lane of a
 // wave takes part in each round): with off, the colour offsets off[c] = first position whose
 // key has colour >= c (c = 0..K, a small island's key counting as colour K, since those
 // keys sort above every colour) and m_glob = off[K]; with list, the work list of the small
-// islands solved by one workgroup each (first slot, manifolds), the one-lane islands only
-// counted (per wave).  An island starts where its key differs from the one before it above
-// the colour bits.
+// islands of more than ISLAND_LANE_MAX manifolds (the smaller ones are found by their slots).
+// An island starts where its key differs from the one before it above the colour bits.
 __device__ __forceinline__ void sorted_keys_part(const Bodies& B, const uint32_t* __restrict__ skey,
                                                  uint32_t* __restrict__ off, uint2* __restrict__ list, uint32_t cap,
                                                  Counters* cnt, uint32_t gid, uint32_t gsz) {
@@ -1172,9 +1183,21 @@ __device__ __forceinline__ void sorted_keys_part(const Bodies& B, const uint32_t
             }
         }
         if (list) {
-            const uint64_t one = __ballot(start && size <= ISLAND_LANE_MAX);
-            if (lane == 0u && one) atomicAdd(&cnt->isl_lane_n, (uint32_t)__popcll(one));
-            if (start && size > ISLAND_LANE_MAX) list[atomicAdd(&cnt->isl_group_n, 1u)] = make_uint2(s, size);
+            const bool big = start && size > ISLAND_LANE_MAX;
+            if (__ballot(big) != 0ull) {
+                // one atomic per class of the wave's islands
+                const uint32_t cls = isl_class(size);
+                for (uint32_t c = 0; c < ISLAND_CLASSES; ++c) {
+                    const uint64_t in = __ballot(big && cls == c);
+                    if (in == 0ull) continue;
+                    uint32_t at = 0;
+                    if (lane == 0u) at = atomicAdd(&cnt->isl_n[c], (uint32_t)__popcll(in));
+                    at = (uint32_t)__shfl((int)at, 0, 64);
+                    if (big && cls == c)
+                        list[isl_region(c, cap) + at + (uint32_t)__popcll(in & ((1ull << lane) - 1ull))] =
+                            make_uint2(s, size);
+                }
+            }
         }
     }
 }
@@ -1692,9 +1715,14 @@ __device__ __forceinline__ void solve_slot(const Bodies& B, const StepParams& sp
     load_vel<false>(B, a, A);
     if (plane) zero_sb(Bd); else load_vel<false>(B, b, Bd);
     float4 L[4];
-    for (uint32_t k = 0; k < np; ++k) L[k] = R.lam[(size_t)k * cap + s];
+    // over a fixed 4 so that L stays in registers
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k)
+        if (k < np) L[k] = R.lam[(size_t)k * cap + s];
     solve_core(R, s, cap, np, plane, sp.keep, first, A, Bd, L);
-    for (uint32_t k = 0; k < np; ++k) R.lam[(size_t)k * cap + s] = make_float4(L[k].x, L[k].y, L[k].z, 0.0f);
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k)
+        if (k < np) R.lam[(size_t)k * cap + s] = make_float4(L[k].x, L[k].y, L[k].z, 0.0f);
     if (A.dyn) {
         B.sv[a] = f4(A.v, A.im);
         B.sw[a] = f4(A.w, 0.0f);
@@ -1827,8 +1855,8 @@ __device__ __forceinline__ uint32_t next_colour(unsigned long long mk, uint32_t 
 // Before a launch, per slot: the next visit of each dynamic body, and the inbox
 // words: a body's first visit (rank 0) gets the body's solver velocity with
 // version 0, every other inbox a version no visit waits for.
-// (Thread gid of gsz; also run by the small islands' workgroup kernel, k_pgs_group, whose
-// bodies and slots are disjoint from the large islands'.)
+// (Thread gid of gsz; also run by the small islands' kernel, k_pgs_islands, whose bodies and
+// slots are disjoint from the large islands'.)
 __device__ __forceinline__ void flow_init_part(const Bodies& B, const SolverRows& R, const uint64_t* __restrict__ bmask,
                                                const Counters* __restrict__ cnt, uint32_t gid, uint32_t gsz) {
     // the rows exist only when this step's preparation ran
@@ -2454,210 +2482,47 @@ __device__ __forceinline__ float slot_residual(const Bodies& B, float keep, cons
     }
     return res;
 }
-// One island's result: sweeps run, final residual (bits), whether it missed the tolerance,
-// contact points; folded into the counters.
-__device__ __forceinline__ void local_done(Counters* cnt, uint32_t sweeps, float res, bool miss, uint32_t pts,
-                                           bool bundle) {
-    atomicMax(&cnt->loc_sweeps, sweeps);
-    atomicMax(&cnt->loc_res_bits, __float_as_uint(res));
-    if (miss) atomicOr(&cnt->loc_miss, 1u);
-    atomicAdd(&cnt->loc_points, pts);
-    atomicAdd(&cnt->loc_point_sweeps, (unsigned long long)pts * sweeps);
-    if (bundle) atomicAdd(&cnt->bundle_point_sweeps, (unsigned long long)pts * sweeps);
-}
-// Islands of at most ISLAND_LANE_MAX manifolds, bundled: the islands whose first slot lies
-// in window w (BUNDLE_SLOTS slots from the first small-island slot on) are solved by
-// workgroup w, one wave, one lane per slot (at most BUNDLE_SLOTS + ISLAND_LANE_MAX - 1 lanes).
-// Each sweep runs phases: in phase p every island visits the slots of its p-th colour, all
-// at once (within an island a colour's slots share no dynamic body, and islands share none
-// at all), with a barrier between phases; then each island's residual is the maximum over
-// its lanes, and an island that is done stops while the others go on.
-//
-// Everything a sweep touches stays on chip for the whole solve: each lane's Jacobian rows
-// and impulses in its registers (a lane visits the same slot in every sweep; with one wave
-// per SIMD the rows fit the register file, accumulation registers included), and each
-// body's solver velocity in LDS, in one home slot: the first (lane, side) of its island
-// that names it (dynamic bodies appear in one island only; a static partner keeps its own
-// slot).  The visits are the arithmetic of solve_slot on those copies; velocities and
-// impulses go back to memory once, at the end.
-constexpr uint32_t BUNDLE_SLOTS = 56;
-static_assert(BUNDLE_SLOTS + ISLAND_LANE_MAX - 1u <= 64u, "a bundle fits one wave");
-constexpr uint32_t BUNDLE_BODY0 = 0u;  // first body slot (float4 units)
-constexpr uint32_t BUNDLE_LDS_BYTES = (BUNDLE_BODY0 + 4u * 64u) * 16u;
-__device__ __forceinline__ void home_load(const float4* lds, uint32_t h, SB& X) {
-    const float4 v = lds[BUNDLE_BODY0 + h], w = lds[BUNDLE_BODY0 + 128u + h];
-    X.v = xyz(v);
-    X.im = v.w;
-    X.w = xyz(w);
-    X.dyn = v.w > 0.0f;
-}
-__device__ __forceinline__ void home_store(float4* lds, uint32_t h, const SB& X) {
-    lds[BUNDLE_BODY0 + h] = f4(X.v, X.im);
-    lds[BUNDLE_BODY0 + 128u + h] = f4(X.w, 0.0f);
-}
-__global__ void __launch_bounds__(64) k_pgs_bundle(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap,
-                                                   const uint32_t* __restrict__ skey, float tol,
-                                                   uint32_t max_sweeps) {
-    extern __shared__ float4 bl[];
-    __shared__ uint32_t isl_res[2][64];  // per island (first slot - window start): residual bits, two sweeps
-    __shared__ uint32_t isl_pts[64];
-    __shared__ uint2 ab[64];
-    __shared__ uint32_t colr[64];
-    __shared__ uint32_t kmax_w;
-    if (cnt->sticky != 0u) return;
-    const uint32_t M = min(cap, cnt->m_eff), M0 = cnt->m_glob, lane = threadIdx.x;
-    const uint32_t nwin = M > M0 ? (M - M0 + BUNDLE_SLOTS - 1u) / BUNDLE_SLOTS : 0u;
-    const bool tol_mode = tol > 0.0f;
-    const float keep = sp.keep;
-    for (uint32_t win = blockIdx.x; win < nwin; win += gridDim.x) {
-        const uint32_t w0 = M0 + win * BUNDLE_SLOTS, s = w0 + lane;
-        // this lane's slot belongs to the bundle when its island is a one-lane island whose
-        // first slot lies in the window
-        bool mine = false;
-        uint32_t li = 0, colour = 0;
-        if (s < M) {
-            const uint32_t k = skey[s];
-            if (B.icnt[(k & ~LOCAL_KEY) >> 8] <= ISLAND_LANE_MAX) {
-                uint32_t st = s;
-                while (st > M0 && ((skey[st - 1u] ^ k) >> 8) == 0u) --st;  // at most ISLAND_LANE_MAX - 1 steps
-                mine = st >= w0 && st < w0 + BUNDLE_SLOTS;
-                li = mine ? st - w0 : 0u;
-                colour = k & 0xFFu;
-            }
-        }
-        const uint4 h = mine ? R.hdr[s] : make_uint4(UNSET, UNSET, 0u, 0u);
-        const uint32_t np = min(h.z, 4u);
-        const bool plane = (h.y & PLANE_BIT) != 0u;
-        ab[lane] = make_uint2(h.x, h.y);
-        colr[lane] = mine ? colour : UNSET;
-        isl_res[0][lane] = 0u;
-        isl_res[1][lane] = 0u;
-        isl_pts[lane] = 0u;
-        if (lane == 0u) kmax_w = 0u;
-        // the slot's rows and impulses in registers
-        float4 Jr[4][JROWS];
-        float4 L[4];
-#pragma unroll
-        for (uint32_t k = 0; k < 4; ++k) L[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (mine) {
-            // own copies of both bodies' velocities
-            const float4 va = B.sv[h.x], wa = B.sw[h.x];
-            bl[BUNDLE_BODY0 + lane] = va;
-            bl[BUNDLE_BODY0 + 128u + lane] = make_float4(wa.x, wa.y, wa.z, 0.0f);
-            // a plane's side holds zeros (velocity, inverse mass): it loads as a static body
-            float4 vb = make_float4(0.0f, 0.0f, 0.0f, 0.0f), wb = vb;
-            if (!plane) {
-                vb = B.sv[h.y];
-                wb = B.sw[h.y];
-            }
-            bl[BUNDLE_BODY0 + 64u + lane] = vb;
-            bl[BUNDLE_BODY0 + 192u + lane] = make_float4(wb.x, wb.y, wb.z, 0.0f);
-            load_rows(R, s, cap, np, plane, Jr);
-#pragma unroll
-            for (uint32_t k = 0; k < 4; ++k)
-                if (k < np) L[k] = R.lam[(size_t)k * cap + s];
-        }
-        __syncthreads();
-        // home slot of each side: the first (lane, side) of the island naming the body; the
-        // lane's phase: the colours of its island below its own (an island's slots ascend by
-        // colour), so each island visits its own colours in turn, lanes of one phase at once
-        uint32_t home_a = lane, home_b = 64u + lane, phase = 0;
-        if (mine) {
-            for (uint32_t j = li + 1u; j <= lane; ++j) phase += colr[j] != colr[j - 1u] ? 1u : 0u;
-            atomicMax(&kmax_w, phase);
-            atomicAdd(&isl_pts[li], np);
-            auto home_of = [&](uint32_t body, uint32_t own) {
-                for (uint32_t j = li; j <= lane; ++j) {
-                    const uint2 o = ab[j];
-                    if (o.x == body) return j;
-                    if (o.y == body) return 64u + j;
-                }
-                return own;
-            };
-            home_a = home_of(h.x, lane);
-            if (!plane) home_b = home_of(h.y, 64u + lane);
-        }
-        __syncthreads();
-        const uint32_t kmax = kmax_w;
-        bool active = mine;
-        uint32_t sweeps = 0;
-        float res = 0.0f;
-        for (uint32_t it = 0; it < max_sweeps; ++it) {
-            if (!__syncthreads_or(active)) break;
-            for (uint32_t c = 0; c <= kmax; ++c) {
-                if (active && phase == c) {
-                    SB A, Bd;
-                    home_load(bl, home_a, A);
-                    home_load(bl, home_b, Bd);
-                    solve_regs(Jr, np, keep, it == 0u, A, Bd, L);
-#pragma unroll
-                    for (uint32_t k = 0; k < 4; ++k) L[k].w = 0.0f;
-                    if (A.dyn) home_store(bl, home_a, A);
-                    if (Bd.dyn) home_store(bl, home_b, Bd);
-                }
-                __syncthreads();
-            }
-            if (tol_mode || it + 1u == max_sweeps) {
-                uint32_t* cur = isl_res[it & 1u];
-                isl_res[(it + 1u) & 1u][lane] = 0u;  // the next sweep's words (not read in this one)
-                if (active) {
-                    SB A, Bd;
-                    home_load(bl, home_a, A);
-                    home_load(bl, home_b, Bd);
-                    float r = 0.0f;
-#pragma unroll
-                    for (uint32_t k = 0; k < 4; ++k) {
-                        if (k >= np) break;
-                        const float e = point_residual_regs(Jr[k], keep, A, Bd, L[k]);
-                        if (e > r) r = e;
-                    }
-                    atomicMax(&cur[li], __float_as_uint(r));
-                }
-                __syncthreads();
-                if (active) {
-                    res = __uint_as_float(cur[li]);
-                    if (tol_mode && res <= tol) {
-                        sweeps = it + 1u;
-                        active = false;
-                    }
-                }
-            }
-            if (active && it + 1u == max_sweeps) {
-                sweeps = max_sweeps;
-                active = false;
-            }
-        }
-        __syncthreads();
-        if (mine) {
-            // impulses and the velocities of the bodies whose home this lane holds back to memory
-#pragma unroll
-            for (uint32_t k = 0; k < 4; ++k)
-                if (k < np) R.lam[(size_t)k * cap + s] = L[k];
-            SB A;
-            home_load(bl, lane, A);
-            if (home_a == lane && A.dyn) {
-                B.sv[h.x] = f4(A.v, A.im);
-                B.sw[h.x] = f4(A.w, 0.0f);
-            }
-            if (!plane && home_b == 64u + lane) {
-                SB Bd;
-                home_load(bl, 64u + lane, Bd);
-                if (Bd.dyn) {
-                    B.sv[h.y] = f4(Bd.v, Bd.im);
-                    B.sw[h.y] = f4(Bd.w, 0.0f);
-                }
-            }
-            // one lane per island (its first slot) reports it
-            if (s == w0 + li) local_done(cnt, sweeps, res, tol_mode && !(res <= tol), isl_pts[li], true);
-        }
-        __syncthreads();
+// Results of the islands a thread reports: the most sweeps, the largest final residual
+// (bits), whether one missed the tolerance, contact points and contact points x sweeps.
+struct IslandAcc {
+    uint32_t sweeps, res_bits, miss, pts;
+    unsigned long long point_sweeps;
+    __device__ void add(uint32_t sw, float res, bool missed, uint32_t p) {
+        sweeps = max(sweeps, sw);
+        res_bits = max(res_bits, __float_as_uint(res));
+        miss |= missed ? 1u : 0u;
+        pts += p;
+        point_sweeps += (unsigned long long)p * sw;
     }
+};
+// Folds a wave's results into the counters: once per wave and launch, since every atomic
+// here is on a word all waves share.
+__device__ __forceinline__ void island_flush(Counters* cnt, IslandAcc a) {
+    for (int o = 32; o >= 1; o >>= 1) {
+        a.sweeps = max(a.sweeps, (uint32_t)__shfl_xor((int)a.sweeps, o, 64));
+        a.res_bits = max(a.res_bits, (uint32_t)__shfl_xor((int)a.res_bits, o, 64));
+        a.miss |= (uint32_t)__shfl_xor((int)a.miss, o, 64);
+        a.pts += (uint32_t)__shfl_xor((int)a.pts, o, 64);
+        a.point_sweeps += __shfl_xor(a.point_sweeps, o, 64);
+    }
+    if ((threadIdx.x & 63u) != 0u || a.pts == 0u) return;
+    atomicMax(&cnt->loc_sweeps, a.sweeps);
+    atomicMax(&cnt->loc_res_bits, a.res_bits);
+    if (a.miss) atomicOr(&cnt->loc_miss, 1u);
+    atomicAdd(&cnt->loc_points, a.pts);
+    atomicAdd(&cnt->loc_point_sweeps, a.point_sweeps);
+    atomicAdd(&cnt->bundle_point_sweeps, a.point_sweeps);
 }
-int pgs_bundle_setup() {
-    return hipFuncSetAttribute((const void*)k_pgs_bundle, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)BUNDLE_LDS_BYTES) == hipSuccess ? 1 : 0;
+// Orders a wave's LDS accesses before and after this point (a wave's LDS operations execute
+// in order, so no wait is needed, only that the compiler moves none across).
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-// Block-wide maximum and sum of 256 threads (red: 8 words of LDS); every thread gets both.
+constexpr uint32_t ISL_THREADS = 512, ISL_WAVES = ISL_THREADS / 64u;
+// Block-wide maximum and sum over the workgroup's waves (red: two words of LDS per wave);
+// every thread gets both.
 __device__ __forceinline__ void block_max_sum(uint32_t& mx, uint32_t& sum, uint32_t* red) {
     for (int o = 32; o >= 1; o >>= 1) {
         const uint32_t om = __shfl_xor(mx, o, 64), os = __shfl_xor(sum, o, 64);
@@ -2665,70 +2530,908 @@ __device__ __forceinline__ void block_max_sum(uint32_t& mx, uint32_t& sum, uint3
         sum += os;
     }
     if ((threadIdx.x & 63u) == 0u) {
-        red[threadIdx.x >> 6] = mx;
-        red[4 + (threadIdx.x >> 6)] = sum;
+        red[2u * (threadIdx.x >> 6)] = mx;
+        red[2u * (threadIdx.x >> 6) + 1u] = sum;
     }
     __syncthreads();
-    mx = max(max(red[0], red[1]), max(red[2], red[3]));
-    sum = red[4] + red[5] + red[6] + red[7];
+    mx = sum = 0u;
+#pragma unroll
+    for (uint32_t w = 0; w < ISL_WAVES; ++w) {
+        mx = max(mx, red[2u * w]);
+        sum += red[2u * w + 1u];
+    }
     __syncthreads();
 }
-// Larger islands: one workgroup each.  A colour's slots share no dynamic body, so the
-// workgroup visits them together and meets at a barrier before the next colour (the
-// velocities move through global memory, visible within the workgroup after the barrier).
-__global__ void __launch_bounds__(256) k_pgs_group(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap,
-                                                   const uint2* __restrict__ list, const uint32_t* __restrict__ skey,
-                                                   float tol, uint32_t max_sweeps,
-                                                   const uint64_t* __restrict__ flow_bmask) {
-    __shared__ uint32_t red[8];
-    // with flow_bmask, the large islands' sweep launch is prepared here (as k_flow_init)
-    if (flow_bmask) flow_init_part(B, R, flow_bmask, cnt, blockIdx.x * blockDim.x + threadIdx.x,
-                                   gridDim.x * blockDim.x);
-    if (cnt->sticky != 0u) return;
-    const uint32_t n = cnt->isl_group_n, t = threadIdx.x;
+// The small islands' kernel: one workgroup of eight waves per CU, two waves per SIMD.  A sweep
+// of an island is a chain of dependent visits, colour after colour, and each visit a chain of
+// three row updates per contact point.  What binds is that chain, so what a sweep touches
+// stays on chip: rows and impulses in registers (a lane visits the same slot in every sweep),
+// body velocities in LDS.  Velocities and impulses go back to memory once per island.  Above
+// 256 manifolds a CU no longer holds the rows (240 B per point); they are read at each visit.
+//
+// Work is taken largest first, so that the long solves start early and the short ones fill
+// the tail.  The workgroups first share the islands of more than 64 manifolds, one island at
+// a time; then each wave on its own takes islands of the smaller classes, several to a wave
+// in blocks of 64, 32 or 16 lanes, and last the windows of the islands of at most
+// ISLAND_LANE_MAX manifolds: those whose first slot lies in one run of BUNDLE_SLOTS slots, one
+// lane per slot (at most BUNDLE_SLOTS + ISLAND_LANE_MAX - 1 lanes).
+//
+// Each sweep runs phases: in phase p every island of the wave (or the workgroup's island)
+// visits the slots of its p-th colour, all at once (within an island a colour's slots share no
+// dynamic body, and islands share none at all); then each island's residual is the maximum
+// over its lanes, and an island that is done stops while the others go on.  The visits are the
+// arithmetic of solve_slot.  A body's velocity has one home in LDS, that of its first visit in
+// a sweep (the lowest colour of its mask, whose slot the row preparation recorded in vslot).
+//
+// Per step, before (a workgroup of 256 threads per island of 9 to 4096 manifolds, rows and
+// velocities in memory; a kernel of its own for the smaller ones) and now: 1000 bodies at
+// residual 1e-4 (76 sweeps, largest island 154 manifolds) 1.55 -> 0.47 ms; 256 worlds at 1e-4
+// (159k manifolds, 119 sweeps) 7.2 -> 2.8 ms; 4096 worlds at ten sweeps (1.7M manifolds)
+// 11.3 -> 1.1 ms; an island of 1880 manifolds, 73 sweeps, 4.9 -> 3.2 ms.
+constexpr uint32_t BUNDLE_SLOTS = 56;
+static_assert(BUNDLE_SLOTS + ISLAND_LANE_MAX - 1u <= 64u, "a bundle fits one wave");
+// LDS of a wave's own work
+constexpr uint32_t LAST_ROWS = JROWS - 1u;
+struct WaveLds {
+    float4 vel[256];              // v of the homes (64 * side + lane), then w
+    float4 last[LAST_ROWS * 64];  // rows of every lane's fourth point (the last row in spare .w)
+    uint32_t res[2][64];          // per island (its first lane): residual bits, two sweeps
+    uint32_t pts[64];             // per island: contact points
+    uint2 ab[64];
+};
+// LDS of a workgroup's island: this, then the tables, the velocities and the pool of rows
+struct GroupLds {
+    uint32_t off[66];  // first slot (island-relative) of colour >= c
+    uint32_t red[2 * ISL_WAVES];
+    unsigned long long mask;  // the island's colours
+    uint32_t bodies, next;
+};
+constexpr uint32_t ISL_LDS_BYTES = 160u * 1024u;
+constexpr uint32_t ISL_HEAD = (sizeof(GroupLds) + 15u) / 16u * 16u;
+constexpr uint32_t ISL_TABLE_BYTES = 5u * ISLAND_LOCAL_MAX;  // 16-bit homes of both sides, points of every slot
+static_assert(ISL_HEAD + ISL_TABLE_BYTES + 32u * (ISLAND_LOCAL_MAX + 1u) <= ISL_LDS_BYTES,
+              "the velocities of any island's dynamic bodies fit");
+static_assert(ISL_WAVES * sizeof(WaveLds) <= ISL_LDS_BYTES, "the waves' parts fit");
+// homes of a side without a dynamic body: a plane, a static body
+constexpr uint32_t PLANE_HOME = 0xFFFEu, NO_HOME = 0xFFFFu;
+
+__device__ __forceinline__ void vel_load(const float4* v, const float4* w, uint32_t h, SB& X) {
+    const float4 a = v[h], b = w[h];
+    X.v = xyz(a);
+    X.im = a.w;
+    X.w = xyz(b);
+    X.dyn = a.w > 0.0f;
+}
+__device__ __forceinline__ void vel_store(float4* v, float4* w, uint32_t h, const SB& X) {
+    v[h] = f4(X.v, X.im);
+    w[h] = f4(X.w, 0.0f);
+}
+__device__ __forceinline__ void vel_out(const Bodies& B, uint32_t body, const SB& X) {
+    B.sv[body] = f4(X.v, X.im);
+    B.sw[body] = f4(X.w, 0.0f);
+}
+// The first visit of a dynamic body in a sweep: slot << 1 | side.
+__device__ __forceinline__ uint32_t first_visit(const Bodies& B, const uint64_t* __restrict__ bmask, uint32_t body) {
+    return B.vslot[(size_t)body * 64u + (uint32_t)__ffsll((unsigned long long)bmask[body]) - 1u];
+}
+// Row updates of a point: relative velocity, projection, impulse.
+__device__ __forceinline__ void friction_row(const Dir& D, float m, float maxf, float keep, float& l, SB& A, SB& Bd) {
+    float nl = fmaf(-m, jvel(D, A, Bd), keep * l);
+    nl = clamp_sym(nl, maxf);
+    const float d = nl - l;
+    l = nl;
+    japply_both(D, d, A, Bd);
+}
+__device__ __forceinline__ void normal_row(const Dir& D, float m, float tg, float keep, float& l, SB& A, SB& Bd) {
+    float nl = fmaf(m, tg - jvel(D, A, Bd), keep * l);
+    nl = fmaxf(nl, 0.0f);
+    const float d = nl - l;
+    l = nl;
+    japply_both(D, d, A, Bd);
+}
+__device__ __forceinline__ void friction_regs(const float4 (&J)[JROWS], float keep, float4& L, SB& A, SB& Bd) {
+    float m1, m2, maxf, w3;
+    const Dir D1 = dir_regs(J, 1, m1, maxf);
+    friction_row(D1, m1, maxf, keep, L.y, A, Bd);
+    const Dir D2 = dir_regs(J, 2, m2, w3);
+    friction_row(D2, m2, maxf, keep, L.z, A, Bd);
+}
+__device__ __forceinline__ void normal_regs(const float4 (&J)[JROWS], float keep, float4& L, SB& A, SB& Bd) {
+    float m, tg;
+    const Dir D = dir_regs(J, 0, m, tg);
+    normal_row(D, m, tg, keep, L.x, A, Bd);
+}
+__device__ __forceinline__ void start_regs(const float4 (&J)[JROWS], const float4& L, SB& A, SB& Bd) {
+    float w0, w3;
+    japply_both(dir_regs(J, 0, w0, w3), L.x, A, Bd);
+    japply_both(dir_regs(J, 1, w0, w3), L.y, A, Bd);
+    japply_both(dir_regs(J, 2, w0, w3), L.z, A, Bd);
+}
+// The fourth point's rows in LDS: row r of a lane at last[r * 64]; the last row rides in the
+// unused .w of rows 2, 4 and 7.
+__device__ __forceinline__ void last_put(float4* last, const float4 (&J)[JROWS]) {
+#pragma unroll
+    for (uint32_t r = 0; r < LAST_ROWS; ++r) {
+        float4 x = J[r];
+        if (r == 2u) x.w = J[LAST_ROWS].x;
+        if (r == 4u) x.w = J[LAST_ROWS].y;
+        if (r == 7u) x.w = J[LAST_ROWS].z;
+        last[r * 64u] = x;
+    }
+}
+__device__ __forceinline__ void last_get(const float4* last, float4 (&J)[JROWS]) {
+    // an opaque zero: each use reads the rows it needs, none is kept in registers for the next
+    uint32_t zero = 0u;
+    asm volatile("" : "+v"(zero));
+    last += zero;
+#pragma unroll
+    for (uint32_t r = 0; r < LAST_ROWS; ++r) J[r] = last[r * 64u];
+    J[LAST_ROWS] = make_float4(J[2].w, J[4].w, J[7].w, 0.0f);
+}
+// The rows of point k of slot s (zeros for the b side of a plane contact).
+__device__ __forceinline__ void point_rows(const SolverRows& R, uint32_t s, uint32_t cap, uint32_t k, bool plane,
+                                           float4 (&J)[JROWS]) {
+#pragma unroll
+    for (uint32_t r = 0; r < JROWS; ++r) {
+        const bool bside = (r % 5u) == 2u || (r % 5u) == 4u;
+        J[r] = bside && plane ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : R.J[((size_t)k * JROWS + r) * cap + s];
+    }
+}
+
+// Islands of one wave, one lane per slot: the lane's slot s (when mine), its island's first
+// lane li and its colour.  search: the homes are found among the island's lanes instead of by
+// the bodies' first visits (few lanes, or more colours than a mask holds).
+__device__ __forceinline__ void wave_islands(const Bodies& B, float keep, const SolverRows& R, uint32_t cap, float tol,
+                                             uint32_t max_sweeps, const uint64_t* __restrict__ bmask, WaveLds& W,
+                                             bool mine, uint32_t s, uint32_t li, uint32_t colour, bool search,
+                                             IslandAcc& acc) {
+    const uint32_t lane = threadIdx.x & 63u;
     const bool tol_mode = tol > 0.0f;
-    for (uint32_t g = blockIdx.x; g < n; g += gridDim.x) {
-        const uint2 e = list[g];
-        const uint32_t s0 = e.x, s1 = e.x + e.y;
-        const uint32_t k0 = skey[s0], k1 = skey[s1 - 1u];
-        uint32_t it = 0;
-        float res = 0.0f;
-        for (; it < max_sweeps; ++it) {
-            uint32_t a = s0;
-            for (uint32_t c = k0 & 0xFFu; c <= (k1 & 0xFFu); ++c) {
-                // [a, b): the island's slots of colour c (the keys ascend, equal above the colour)
-                const uint32_t kc = (k0 & ~0xFFu) | c;
-                uint32_t lo = a, hi = s1;
-                while (lo < hi) {
-                    const uint32_t mid = (lo + hi) >> 1;
-                    if (skey[mid] <= kc) lo = mid + 1u; else hi = mid;
+    float4 *vv = W.vel, *vw = W.vel + 128, *last = W.last + lane;
+    const uint4 h = mine ? R.hdr[s] : make_uint4(UNSET, UNSET, 0u, 0u);
+    const uint32_t np = min(h.z, 4u);
+    const bool plane = (h.y & PLANE_BIT) != 0u;
+    W.ab[lane] = make_uint2(h.x, h.y);
+    W.res[0][lane] = 0u;
+    W.res[1][lane] = 0u;
+    W.pts[lane] = 0u;
+    // the slot's impulses and the rows of its first three points in registers
+    float4 Jr[3][JROWS];
+    float4 L[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) L[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    // a plane's side holds zeros (velocity, inverse mass): it loads as a static body
+    float4 va = make_float4(0.0f, 0.0f, 0.0f, 0.0f), wa = va, vb = va, wb = va;
+    if (mine) {
+        va = B.sv[h.x];
+        wa = B.sw[h.x];
+        if (!plane) {
+            vb = B.sv[h.y];
+            wb = B.sw[h.y];
+        }
+        if (np > 3u) {
+            float4 J[JROWS];
+            point_rows(R, s, cap, 3u, plane, J);
+            last_put(last, J);
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 3; ++k)
+            if (k < np) point_rows(R, s, cap, k, plane, Jr[k]);
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k)
+            if (k < np) L[k] = R.lam[(size_t)k * cap + s];
+    }
+    const bool dyn_a = va.w > 0.0f, dyn_b = vb.w > 0.0f;
+    wave_sync();
+    // home of each side; the lane's phase: the colours of its island below its own (an
+    // island's slots ascend by colour)
+    uint32_t home_a = lane, home_b = 64u + lane;
+    const uint32_t before = (uint32_t)__shfl_up((int)colour, 1, 64);
+    const uint64_t heads = __ballot(mine && lane != li && before != colour);
+    const uint64_t upto = (2ull << lane) - 1ull, from = ~((2ull << li) - 1ull);
+    const uint32_t phase = (uint32_t)__popcll(heads & upto & from);
+    if (mine) {
+        if (search) {
+            auto home_of = [&](uint32_t body, uint32_t own) {
+                for (uint32_t j = li; j <= lane; ++j) {
+                    const uint2 o = W.ab[j];
+                    if (o.x == body) return j;
+                    if (o.y == body) return 64u + j;
                 }
-                if (lo > a) {
-                    for (uint32_t s = a + t; s < lo; s += blockDim.x) solve_slot(B, sp, R, R.hdr[s], s, cap, it == 0u);
-                    __syncthreads();
-                }
-                a = lo;
+                return own;
+            };
+            home_a = home_of(h.x, lane);
+            if (!plane) home_b = home_of(h.y, 64u + lane);
+        } else {
+            const uint32_t s0 = s - (lane - li);
+            if (dyn_a) {
+                const uint32_t f = first_visit(B, bmask, h.x);
+                home_a = (f & 1u) * 64u + (((f >> 1) - s0 + li) & 63u);
             }
-            if (tol_mode || it + 1u == max_sweeps) {
-                float r = 0.0f;
-                for (uint32_t s = s0 + t; s < s1; s += blockDim.x) {
-                    const float q = slot_residual(B, sp.keep, R, s, cap);
-                    if (q > r) r = q;
+            if (dyn_b) {
+                const uint32_t f = first_visit(B, bmask, h.y);
+                home_b = (f & 1u) * 64u + (((f >> 1) - s0 + li) & 63u);
+            }
+        }
+        vv[lane] = va;
+        vw[lane] = make_float4(wa.x, wa.y, wa.z, 0.0f);
+        vv[64u + lane] = vb;
+        vw[64u + lane] = make_float4(wb.x, wb.y, wb.z, 0.0f);
+        atomicAdd(&W.pts[li], np);
+    }
+    uint32_t phases = mine ? phase + 1u : 0u;
+    for (int o = 32; o >= 1; o >>= 1) phases = max(phases, (uint32_t)__shfl_xor((int)phases, o, 64));
+    wave_sync();
+    bool active = mine;
+    uint32_t sweeps = 0;
+    float res = 0.0f;
+    for (uint32_t it = 0; it < max_sweeps; ++it) {
+        if (__ballot(active) == 0ull) break;
+        for (uint32_t c = 0; c < phases; ++c) {
+            if (active && phase == c) {
+                SB A, Bd;
+                vel_load(vv, vw, home_a, A);
+                vel_load(vv, vw, home_b, Bd);
+                if (it == 0u) {
+#pragma unroll
+                    for (uint32_t k = 0; k < 3; ++k) {
+                        if (k >= np) break;
+                        start_regs(Jr[k], L[k], A, Bd);
+                    }
+                    if (np > 3u) {
+                        float4 J[JROWS];
+                        last_get(last, J);
+                        start_regs(J, L[3], A, Bd);
+                    }
                 }
-                uint32_t mx = __float_as_uint(r), unused = 0u;
-                block_max_sum(mx, unused, red);
-                res = __uint_as_float(mx);
-                if (tol_mode && res <= tol) {
-                    ++it;
-                    break;
+#pragma unroll
+                for (uint32_t k = 0; k < 3; ++k) {
+                    if (k >= np) break;
+                    friction_regs(Jr[k], keep, L[k], A, Bd);
+                }
+                if (np > 3u) {
+                    float4 J[JROWS];
+                    last_get(last, J);
+                    friction_regs(J, keep, L[3], A, Bd);
+                }
+#pragma unroll
+                for (uint32_t k = 0; k < 3; ++k) {
+                    if (k >= np) break;
+                    normal_regs(Jr[k], keep, L[k], A, Bd);
+                }
+                if (np > 3u) {
+                    float4 J[JROWS];
+                    last_get(last, J);
+                    normal_regs(J, keep, L[3], A, Bd);
+                }
+                if (A.dyn) vel_store(vv, vw, home_a, A);
+                if (Bd.dyn) vel_store(vv, vw, home_b, Bd);
+            }
+            wave_sync();
+        }
+        if (tol_mode || it + 1u == max_sweeps) {
+            uint32_t* cur = W.res[it & 1u];
+            W.res[(it + 1u) & 1u][lane] = 0u;  // the next sweep's words (not read in this one)
+            if (active) {
+                SB A, Bd;
+                vel_load(vv, vw, home_a, A);
+                vel_load(vv, vw, home_b, Bd);
+                float r = 0.0f;
+#pragma unroll
+                for (uint32_t k = 0; k < 3; ++k) {
+                    if (k >= np) break;
+                    const float e = point_residual_regs(Jr[k], keep, A, Bd, L[k]);
+                    if (e > r) r = e;
+                }
+                if (np > 3u) {
+                    float4 J[JROWS];
+                    last_get(last, J);
+                    const float e = point_residual_regs(J, keep, A, Bd, L[3]);
+                    if (e > r) r = e;
+                }
+                atomicMax(&cur[li], __float_as_uint(r));
+            }
+            wave_sync();
+            if (active) {
+                res = __uint_as_float(cur[li]);
+                if ((tol_mode && res <= tol) || it + 1u == max_sweeps) {
+                    sweeps = it + 1u;
+                    active = false;
                 }
             }
         }
-        uint32_t pts = 0, mx = 0u;
-        for (uint32_t s = s0 + t; s < s1; s += blockDim.x) pts += min(R.hdr[s].z, 4u);
-        block_max_sum(mx, pts, red);
-        if (t == 0u) local_done(cnt, it, res, tol_mode && !(res <= tol), pts, false);
     }
+    wave_sync();
+    if (mine) {
+        // impulses and the velocities of the bodies whose home this lane holds back to memory
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k)
+            if (k < np) R.lam[(size_t)k * cap + s] = make_float4(L[k].x, L[k].y, L[k].z, 0.0f);
+        SB X;
+        if (dyn_a && home_a == lane) {
+            vel_load(vv, vw, lane, X);
+            vel_out(B, h.x, X);
+        }
+        if (dyn_b && home_b == 64u + lane) {
+            vel_load(vv, vw, 64u + lane, X);
+            vel_out(B, h.y, X);
+        }
+        if (lane == li) acc.add(sweeps, res, tol_mode && !(res <= tol), W.pts[li]);
+    }
+    wave_sync();
+}
+
+// ---- an island of 65 to 256 manifolds: two lanes of the workgroup per slot, one per body
+// A visit is a chain of row updates, each 32 instructions with both bodies in one lane.  Two
+// neighbouring lanes share them: the even lane holds body a's velocity and rows, the odd lane
+// body b's, and the relative velocity is put together by DPP exchanges inside the adds.  That is
+// 22 instructions per row, and half the registers, so every row of four points stays in them.
+// The odd lane keeps -d, the even lane -a and -IA a: with these signs both lanes run the same
+// instructions, and every product, sum and rounding is that of solve_rows (zeros may differ in
+// sign).
+template <int CTRL> __device__ __forceinline__ float dpp(float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, true));
+}
+constexpr int DPP_SWAP = 0xB1, DPP_EVEN = 0xA0, DPP_ODD = 0xF5;  // quad_perm [1,0,3,2], [0,0,2,2], [1,1,3,3]
+struct HalfDir {
+    f3 d, a, ia;
+};
+struct HalfPoint {
+    HalfDir n, t1, t2;
+    float mN, kN, tg, mT1, kT1, maxf, mT2, kT2;
+};
+struct HalfBody {
+    f3 v, w;
+    float im;
+};
+__device__ __forceinline__ float half_jvel(const HalfDir& D, const HalfBody& X) {
+    const f3 dv = f3{dpp<DPP_SWAP>(X.v.x) - X.v.x, dpp<DPP_SWAP>(X.v.y) - X.v.y, dpp<DPP_SWAP>(X.v.z) - X.v.z};
+    const float ang = fdot(D.a, X.w);
+    const float r = fdot(D.d, dv) + dpp<DPP_ODD>(ang);
+    return r + dpp<DPP_EVEN>(ang);
+}
+__device__ __forceinline__ void half_apply(const HalfDir& D, float lam, HalfBody& X) {
+    const float s = -(lam * X.im);
+    X.v = f3{fmaf(s, D.d.x, X.v.x), fmaf(s, D.d.y, X.v.y), fmaf(s, D.d.z, X.v.z)};
+    X.w = f3{fmaf(lam, D.ia.x, X.w.x), fmaf(lam, D.ia.y, X.w.y), fmaf(lam, D.ia.z, X.w.z)};
+}
+__device__ __forceinline__ void half_friction(const HalfDir& D, float m, float maxf, float keep, float& l, HalfBody& X) {
+    float nl = fmaf(-m, half_jvel(D, X), keep * l);
+    nl = clamp_sym(nl, maxf);
+    const float d = nl - l;
+    l = nl;
+    half_apply(D, d, X);
+}
+__device__ __forceinline__ void half_normal(const HalfDir& D, float m, float tg, float keep, float& l, HalfBody& X) {
+    float nl = fmaf(m, tg - half_jvel(D, X), keep * l);
+    nl = fmaxf(nl, 0.0f);
+    const float d = nl - l;
+    l = nl;
+    half_apply(D, d, X);
+}
+// point_residual_regs of the pair (both lanes get it).
+__device__ __forceinline__ float half_residual(const HalfPoint& P, float keep, const HalfBody& X, float ln, float l1,
+                                               float l2) {
+    float nl = fmaf(P.mN, P.tg - half_jvel(P.n, X), keep * ln);
+    nl = fmaxf(nl, 0.0f);
+    float e = fabsf(nl - ln) * P.kN;
+    float q1 = fmaf(-P.mT1, half_jvel(P.t1, X), keep * l1);
+    q1 = clamp_sym(q1, P.maxf);
+    const float e1 = fabsf(q1 - l1) * P.kT1;
+    float q2 = fmaf(-P.mT2, half_jvel(P.t2, X), keep * l2);
+    q2 = clamp_sym(q2, P.maxf);
+    const float e2 = fabsf(q2 - l2) * P.kT2;
+    if (e1 > e) e = e1;
+    if (e2 > e) e = e2;
+    return e;
+}
+__device__ __forceinline__ void half_rows(const SolverRows& R, uint32_t s, uint32_t cap, uint32_t k, bool odd, bool plane,
+                                          HalfPoint& P) {
+    const float4* J = R.J + (size_t)k * JROWS * cap + s;
+    auto dir = [&](uint32_t r0, HalfDir& D, float& m, float& kk, float& w3) {
+        const float4 d = J[(size_t)r0 * cap], ra = J[(size_t)(r0 + 1u) * cap], ria = J[(size_t)(r0 + 3u) * cap];
+        m = d.w;
+        kk = ra.w;
+        w3 = ria.w;
+        // the b-side rows of a plane contact are not there: zeros
+        float4 rb = make_float4(0.0f, 0.0f, 0.0f, 0.0f), rib = rb;
+        if (odd && !plane) {
+            rb = J[(size_t)(r0 + 2u) * cap];
+            rib = J[(size_t)(r0 + 4u) * cap];
+        }
+        D.d = odd ? f3{-d.x, -d.y, -d.z} : xyz(d);
+        D.a = odd ? xyz(rb) : f3{-ra.x, -ra.y, -ra.z};
+        D.ia = odd ? xyz(rib) : f3{-ria.x, -ria.y, -ria.z};
+    };
+    float w3;
+    dir(0u, P.n, P.mN, P.kN, P.tg);
+    dir(5u, P.t1, P.mT1, P.kT1, P.maxf);
+    dir(10u, P.t2, P.mT2, P.kT2, w3);
+}
+constexpr uint32_t PAIR_SLOTS = ISL_THREADS / 2u;
+__device__ __forceinline__ void pair_island(const Bodies& B, float keep, const SolverRows& R, uint32_t cap, float tol,
+                                            uint32_t max_sweeps, const uint64_t* __restrict__ bmask,
+                                            const uint32_t* __restrict__ skey, unsigned char* lds, uint2 e,
+                                            IslandAcc& acc) {
+    GroupLds& G = *reinterpret_cast<GroupLds*>(lds);
+    float4* vv = reinterpret_cast<float4*>(lds + ISL_HEAD);  // home of (slot, side): 2 * slot + side
+    float4* vw = vv + 2u * PAIR_SLOTS;
+    const uint32_t t = threadIdx.x, u = t >> 1, s0 = e.x, s = s0 + u;
+    const bool odd = (t & 1u) != 0u, mine = u < e.y, tol_mode = tol > 0.0f;
+    const uint32_t colour = mine ? skey[s] & 63u : 0u;
+    if (t == 0u) G.mask = 0ull;
+    const uint4 h = mine ? R.hdr[s] : make_uint4(UNSET, UNSET, 0u, 0u);
+    const uint32_t np = min(h.z, 4u);
+    const bool plane = (h.y & PLANE_BIT) != 0u;
+    const uint32_t body = odd ? h.y : h.x;
+    HalfPoint P[4];
+    float ln[4], l1[4], l2[4];
+    float4 v4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), w4 = v4;
+    uint32_t home = t;
+    if (mine) {
+        if (!(odd && plane)) {
+            v4 = B.sv[body];
+            w4 = B.sw[body];
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k)
+            if (k < np) {
+                half_rows(R, s, cap, k, odd, plane, P[k]);
+                const float4 L = R.lam[(size_t)k * cap + s];
+                ln[k] = L.x;
+                l1[k] = L.y;
+                l2[k] = L.z;
+            }
+        if (v4.w > 0.0f) home = min(first_visit(B, bmask, body) - 2u * s0, 2u * PAIR_SLOTS - 1u);
+        vv[t] = v4;
+        vw[t] = make_float4(w4.x, w4.y, w4.z, 0.0f);
+    }
+    const bool dyn = v4.w > 0.0f;
+    HalfBody X;
+    X.im = v4.w;
+    auto get = [&]() {
+        const float4 a = vv[home], b = vw[home];
+        X.v = xyz(a);
+        X.w = xyz(b);
+    };
+    __syncthreads();
+    if (mine && !odd) atomicOr(&G.mask, 1ull << colour);
+    __syncthreads();
+    const uint64_t mask = G.mask;
+    const uint32_t phases = (uint32_t)__popcll(mask);
+    const uint32_t phase = mine ? (uint32_t)__popcll(mask & ((1ull << colour) - 1ull)) : UNSET;
+    uint32_t it = 0;
+    float res = 0.0f;
+    for (; it < max_sweeps; ++it) {
+        for (uint32_t c = 0; c < phases; ++c) {
+            if (phase == c) {
+                get();
+                if (it == 0u) {
+#pragma unroll
+                    for (uint32_t k = 0; k < 4; ++k) {
+                        if (k >= np) break;
+                        half_apply(P[k].n, ln[k], X);
+                        half_apply(P[k].t1, l1[k], X);
+                        half_apply(P[k].t2, l2[k], X);
+                    }
+                }
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k) {
+                    if (k >= np) break;
+                    half_friction(P[k].t1, P[k].mT1, P[k].maxf, keep, l1[k], X);
+                    half_friction(P[k].t2, P[k].mT2, P[k].maxf, keep, l2[k], X);
+                }
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k) {
+                    if (k >= np) break;
+                    half_normal(P[k].n, P[k].mN, P[k].tg, keep, ln[k], X);
+                }
+                if (dyn) {
+                    vv[home] = f4(X.v, X.im);
+                    vw[home] = f4(X.w, 0.0f);
+                }
+            }
+            __syncthreads();
+        }
+        if (tol_mode || it + 1u == max_sweeps) {
+            float r = 0.0f;
+            if (mine) {
+                get();
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k) {
+                    if (k >= np) break;
+                    const float q = half_residual(P[k], keep, X, ln[k], l1[k], l2[k]);
+                    if (q > r) r = q;
+                }
+            }
+            uint32_t mx = __float_as_uint(r), unused = 0u;
+            block_max_sum(mx, unused, G.red);
+            res = __uint_as_float(mx);
+            if (tol_mode && res <= tol) {
+                ++it;
+                break;
+            }
+        }
+    }
+    if (mine) {
+        if (!odd) {
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k)
+                if (k < np) R.lam[(size_t)k * cap + s] = make_float4(ln[k], l1[k], l2[k], 0.0f);
+        }
+        if (dyn && home == t) {
+            get();
+            B.sv[body] = f4(X.v, X.im);
+            B.sw[body] = f4(X.w, 0.0f);
+        }
+    }
+    uint32_t mx = 0u, pts = odd ? 0u : np;
+    block_max_sum(mx, pts, G.red);
+    if (t == 0u) acc.add(it, res, tol_mode && !(res <= tol), pts);
+}
+
+// ---- an island of more than 256 manifolds, one workgroup
+// The dynamic bodies' velocities are packed in LDS, their homes numbered as their first visits
+// claim them (at most one more than the manifolds); the rows, more than a CU holds, are read
+// from the row arrays at each visit.  A lane asks for the rows of its next visit's first point
+// before it waits at the barrier, and within a visit for the next point's rows before it works
+// on this one's, so that most of their latency passes behind other work.
+struct PointT {  // the friction rows of a point
+    float4 r[10];
+};
+struct PointN {  // its normal rows
+    float4 r[5];
+};
+__device__ __forceinline__ void rows_t(const SolverRows& R, uint32_t s, uint32_t cap, uint32_t k, bool plane, PointT& T) {
+    const float4* J = R.J + ((size_t)k * JROWS + 5u) * cap + s;
+#pragma unroll
+    for (uint32_t r = 0; r < 10u; ++r) {
+        const bool bside = r % 5u == 2u || r % 5u == 4u;
+        T.r[r] = bside && plane ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : J[(size_t)r * cap];
+    }
+}
+__device__ __forceinline__ void rows_n(const SolverRows& R, uint32_t s, uint32_t cap, uint32_t k, bool plane, PointN& N) {
+    const float4* J = R.J + (size_t)k * JROWS * cap + s;
+#pragma unroll
+    for (uint32_t r = 0; r < 5u; ++r) {
+        const bool bside = r == 2u || r == 4u;
+        N.r[r] = bside && plane ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : J[(size_t)r * cap];
+    }
+}
+__device__ __forceinline__ Dir dir_of(const float4* r) {
+    return Dir{xyz(r[0]), xyz(r[1]), xyz(r[2]), xyz(r[3]), xyz(r[4])};
+}
+__device__ __forceinline__ void friction_t(const PointT& T, float keep, float4& L, SB& A, SB& Bd) {
+    const float maxf = T.r[3].w;
+    friction_row(dir_of(T.r), T.r[0].w, maxf, keep, L.y, A, Bd);
+    friction_row(dir_of(T.r + 5), T.r[5].w, maxf, keep, L.z, A, Bd);
+}
+__device__ __forceinline__ void normal_n(const PointN& N, float keep, float4& L, SB& A, SB& Bd) {
+    normal_row(dir_of(N.r), N.r[0].w, N.r[3].w, keep, L.x, A, Bd);
+}
+__device__ __forceinline__ void stream_island(const Bodies& B, float keep, const SolverRows& R, uint32_t cap, float tol,
+                                              uint32_t max_sweeps, const uint64_t* __restrict__ bmask,
+                                              const uint32_t* __restrict__ skey, unsigned char* lds, uint2 e,
+                                              IslandAcc& acc) {
+    GroupLds& G = *reinterpret_cast<GroupLds*>(lds);
+    const uint32_t t = threadIdx.x, s0 = e.x, n = e.y;
+    uint16_t* home = reinterpret_cast<uint16_t*>(lds + ISL_HEAD);
+    uint8_t* pts_of = reinterpret_cast<uint8_t*>(home + 2u * ISLAND_LOCAL_MAX);
+    float4* const vv = reinterpret_cast<float4*>(lds + ISL_HEAD + ISL_TABLE_BYTES);
+    float4* const vw = vv + (ISLAND_LOCAL_MAX + 1u);
+    const bool tol_mode = tol > 0.0f;
+    if (t == 0u) G.bodies = 0u;
+    const uint32_t c_end = (skey[s0 + n - 1u] & 0xFFu) + 1u;  // the island's colours lie below c_end (<= 64)
+    __syncthreads();
+    // colour offsets; points; homes of the bodies whose first visit is here, with their velocities
+    for (uint32_t i = t; i < n; i += ISL_THREADS) {
+        const uint32_t c = skey[s0 + i] & 0xFFu;
+        for (uint32_t q = i ? (skey[s0 + i - 1u] & 0xFFu) + 1u : 0u; q <= c; ++q) G.off[q] = i;
+        if (i == n - 1u) G.off[c_end] = n;
+        const uint4 h = R.hdr[s0 + i];
+        pts_of[i] = (uint8_t)min(h.z, 4u);
+        auto claim = [&](uint32_t body, uint32_t at) {
+            uint32_t id = (body & PLANE_BIT) ? PLANE_HOME : NO_HOME;
+            if (id == NO_HOME) {
+                const float4 v = B.sv[body];
+                if (v.w > 0.0f && first_visit(B, bmask, body) == 2u * s0 + at) {
+                    id = min(atomicAdd(&G.bodies, 1u), ISLAND_LOCAL_MAX);
+                    const float4 w = B.sw[body];
+                    vv[id] = v;
+                    vw[id] = make_float4(w.x, w.y, w.z, 0.0f);
+                }
+            }
+            home[at] = (uint16_t)id;
+        };
+        claim(h.x, 2u * i);
+        claim(h.y, 2u * i + 1u);
+    }
+    __syncthreads();
+    // the other visits' homes (a claimed entry is only read here)
+    for (uint32_t i = t; i < n; i += ISL_THREADS) {
+        const uint4 h = R.hdr[s0 + i];
+        auto side = [&](uint32_t body, uint32_t at) {
+            if (home[at] == NO_HOME && B.sv[body].w > 0.0f)
+                home[at] = home[min(first_visit(B, bmask, body) - 2u * s0, 2u * n - 1u)];
+        };
+        side(h.x, 2u * i);
+        side(h.y, 2u * i + 1u);
+    }
+    __syncthreads();
+    // static partners are read from memory (planes: zeros)
+    auto load_side = [&](uint32_t id, uint32_t i, uint32_t side, SB& X) {
+        if (id < PLANE_HOME) {
+            vel_load(vv, vw, id, X);
+        } else {
+            zero_sb(X);
+            if (id == NO_HOME) load_vel<false>(B, side ? R.hdr[s0 + i].y : R.hdr[s0 + i].x, X);
+        }
+    };
+    // this lane's visits in order: in colour c the slots off[c] + t, off[c] + t + 512, ...
+    PointT T0;
+    PointN N0;
+    float4 L0;
+    auto ask = [&](uint32_t c, uint32_t i) {
+        // the first point of the visit after slot i of colour c (i UNSET: of the first one from
+        // colour c on)
+        uint32_t nx = UNSET;
+        if (i != UNSET && i + ISL_THREADS < G.off[c + 1u]) {
+            nx = i + ISL_THREADS;
+        } else {
+            for (uint32_t q = i == UNSET ? c : c + 1u; q < c_end; ++q)
+                if (G.off[q] + t < G.off[q + 1u]) {
+                    nx = G.off[q] + t;
+                    break;
+                }
+        }
+        if (nx != UNSET) {
+            const bool plane = home[2u * nx + 1u] == PLANE_HOME;
+            rows_t(R, s0 + nx, cap, 0u, plane, T0);
+            rows_n(R, s0 + nx, cap, 0u, plane, N0);
+            L0 = R.lam[s0 + nx];
+        }
+    };
+    uint32_t it = 0;
+    float res = 0.0f;
+    for (; it < max_sweeps; ++it) {
+        ask(0u, UNSET);
+        for (uint32_t c = 0; c < c_end; ++c) {
+            const uint32_t a = G.off[c], b = G.off[c + 1u];
+            if (a == b) continue;
+            for (uint32_t i = a + t; i < b; i += ISL_THREADS) {
+                const uint32_t s = s0 + i, ia = home[2u * i], ib = home[2u * i + 1u], np = pts_of[i];
+                const bool plane = ib == PLANE_HOME;
+                SB A, Bd;
+                load_side(ia, i, 0u, A);
+                load_side(ib, i, 1u, Bd);
+                float4 L[4];
+                L[0] = L0;
+                PointT Ta, Tb;
+                PointN Na, Nb;
+                if (np > 1u) {
+                    rows_t(R, s, cap, 1u, plane, Ta);
+#pragma unroll
+                    for (uint32_t k = 1; k < 4; ++k)
+                        if (k < np) L[k] = R.lam[(size_t)k * cap + s];
+                }
+                if (it == 0u) {
+                    // the warm start (rows read again below)
+                    japply_both(dir_of(N0.r), L[0].x, A, Bd);
+                    japply_both(dir_of(T0.r), L[0].y, A, Bd);
+                    japply_both(dir_of(T0.r + 5), L[0].z, A, Bd);
+#pragma unroll
+                    for (uint32_t k = 1; k < 4; ++k) {
+                        if (k >= np) break;
+                        rows_t(R, s, cap, k, plane, Tb);
+                        rows_n(R, s, cap, k, plane, Nb);
+                        japply_both(dir_of(Nb.r), L[k].x, A, Bd);
+                        japply_both(dir_of(Tb.r), L[k].y, A, Bd);
+                        japply_both(dir_of(Tb.r + 5), L[k].z, A, Bd);
+                    }
+                }
+                friction_t(T0, keep, L[0], A, Bd);
+                if (np > 1u) {
+                    if (np > 2u) rows_t(R, s, cap, 2u, plane, Tb);
+                    else rows_n(R, s, cap, 1u, plane, Na);
+                    friction_t(Ta, keep, L[1], A, Bd);
+                }
+                if (np > 2u) {
+                    if (np > 3u) rows_t(R, s, cap, 3u, plane, Ta);
+                    rows_n(R, s, cap, 1u, plane, Na);
+                    friction_t(Tb, keep, L[2], A, Bd);
+                }
+                if (np > 3u) friction_t(Ta, keep, L[3], A, Bd);
+                if (np > 2u) rows_n(R, s, cap, 2u, plane, Nb);
+                normal_n(N0, keep, L[0], A, Bd);
+                if (np > 1u) normal_n(Na, keep, L[1], A, Bd);
+                if (np > 3u) rows_n(R, s, cap, 3u, plane, Na);
+                if (np > 2u) normal_n(Nb, keep, L[2], A, Bd);
+                if (np > 3u) normal_n(Na, keep, L[3], A, Bd);
+                if (ia < PLANE_HOME) vel_store(vv, vw, ia, A);
+                if (ib < PLANE_HOME) vel_store(vv, vw, ib, Bd);
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k)
+                    if (k < np) R.lam[(size_t)k * cap + s] = make_float4(L[k].x, L[k].y, L[k].z, 0.0f);
+                ask(c, i);
+            }
+            __syncthreads();
+        }
+        if (tol_mode || it + 1u == max_sweeps) {
+            float r = 0.0f;
+            for (uint32_t i = t; i < n; i += ISL_THREADS) {
+                SB A, Bd;
+                load_side(home[2u * i], i, 0u, A);
+                load_side(home[2u * i + 1u], i, 1u, Bd);
+                const bool plane = home[2u * i + 1u] == PLANE_HOME;
+                const uint32_t np = pts_of[i];
+                for (uint32_t k = 0; k < np; ++k) {
+                    const float q = point_residual(R.J + (size_t)k * JROWS * cap + s0 + i, cap, plane, keep, A, Bd,
+                                                   R.lam[(size_t)k * cap + s0 + i]);
+                    if (q > r) r = q;
+                }
+            }
+            uint32_t mx = __float_as_uint(r), unused = 0u;
+            block_max_sum(mx, unused, G.red);
+            res = __uint_as_float(mx);
+            if (tol_mode && res <= tol) {
+                ++it;
+                break;
+            }
+        }
+    }
+    uint32_t pts = 0;
+    for (uint32_t i = t; i < n; i += ISL_THREADS) {
+        pts += pts_of[i];
+        const uint4 h = R.hdr[s0 + i];
+        auto out = [&](uint32_t body, uint32_t at) {
+            const uint32_t id = home[at];
+            if (id >= PLANE_HOME || first_visit(B, bmask, body) != 2u * s0 + at) return;
+            SB X;
+            vel_load(vv, vw, id, X);
+            vel_out(B, body, X);
+        };
+        out(h.x, 2u * i);
+        out(h.y, 2u * i + 1u);
+    }
+    uint32_t mx = 0u;
+    block_max_sum(mx, pts, G.red);
+    if (t == 0u) acc.add(it, res, tol_mode && !(res <= tol), pts);
+}
+
+// An island with rows and velocities in memory (more colours than a body's colour mask holds).
+// A colour's slots share no dynamic body, so the workgroup visits them together and meets at a
+// barrier before the next colour (the velocities are visible within the workgroup after it).
+__device__ __forceinline__ void memory_island(const Bodies& B, const StepParams& sp, const SolverRows& R, uint32_t cap,
+                                              float tol, uint32_t max_sweeps, const uint32_t* __restrict__ skey,
+                                              uint32_t* red, uint2 e, IslandAcc& acc) {
+    const uint32_t s0 = e.x, s1 = e.x + e.y, t = threadIdx.x;
+    const uint32_t k0 = skey[s0], k1 = skey[s1 - 1u];
+    const bool tol_mode = tol > 0.0f;
+    uint32_t it = 0;
+    float res = 0.0f;
+    for (; it < max_sweeps; ++it) {
+        uint32_t a = s0;
+        for (uint32_t c = k0 & 0xFFu; c <= (k1 & 0xFFu); ++c) {
+            // [a, b): the island's slots of colour c (the keys ascend, equal above the colour)
+            const uint32_t kc = (k0 & ~0xFFu) | c;
+            uint32_t lo = a, hi = s1;
+            while (lo < hi) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (skey[mid] <= kc) lo = mid + 1u; else hi = mid;
+            }
+            if (lo > a) {
+                for (uint32_t s = a + t; s < lo; s += blockDim.x) solve_slot(B, sp, R, R.hdr[s], s, cap, it == 0u);
+                __syncthreads();
+            }
+            a = lo;
+        }
+        if (tol_mode || it + 1u == max_sweeps) {
+            float r = 0.0f;
+            for (uint32_t s = s0 + t; s < s1; s += blockDim.x) {
+                const float q = slot_residual(B, sp.keep, R, s, cap);
+                if (q > r) r = q;
+            }
+            uint32_t mx = __float_as_uint(r), unused = 0u;
+            block_max_sum(mx, unused, red);
+            res = __uint_as_float(mx);
+            if (tol_mode && res <= tol) {
+                ++it;
+                break;
+            }
+        }
+    }
+    uint32_t pts = 0, mx = 0u;
+    for (uint32_t s = s0 + t; s < s1; s += blockDim.x) pts += min(R.hdr[s].z, 4u);
+    block_max_sum(mx, pts, red);
+    if (t == 0u) acc.add(it, res, tol_mode && !(res <= tol), pts);
+}
+
+__global__ void __launch_bounds__(ISL_THREADS, 2)
+k_pgs_islands(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap, const uint2* __restrict__ list,
+              const uint32_t* __restrict__ skey, float tol, uint32_t max_sweeps, const uint64_t* __restrict__ bmask,
+              uint32_t flow_init) {
+    extern __shared__ __align__(16) unsigned char isl_lds[];
+    // with flow_init, the large islands' sweep launch is prepared here (as k_flow_init)
+    if (flow_init)
+        flow_init_part(B, R, bmask, cnt, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
+    if (cnt->sticky != 0u) return;
+    const uint32_t t = threadIdx.x, lane = t & 63u;
+    // the row preparation records no first visits when there are more colours than mask bits
+    const bool masks = cnt->max_colour <= 64u;
+    IslandAcc acc = {0u, 0u, 0u, 0u, 0ull};
+    GroupLds& G = *reinterpret_cast<GroupLds*>(isl_lds);
+    const uint32_t n0 = cnt->isl_n[0], n1 = cnt->isl_n[1], n2 = cnt->isl_n[2], n3 = cnt->isl_n[3], n4 = cnt->isl_n[4];
+
+    // ---- islands of one workgroup each (without masks: every island of the list)
+    const uint32_t n_wg = masks ? n0 + n1 : n0 + n1 + n2 + n3 + n4;
+    for (uint32_t w = blockIdx.x; w < n_wg;) {
+        uint32_t c = 0, i = w;
+        if (i >= n0) c = 1u, i -= n0;
+        if (c == 1u && i >= n1) c = 2u, i -= n1;
+        if (c == 2u && i >= n2) c = 3u, i -= n2;
+        if (c == 3u && i >= n3) c = 4u, i -= n3;
+        const uint2 e = list[isl_region(c, cap) + i];
+        if (!masks) memory_island(B, sp, R, cap, tol, max_sweeps, skey, G.red, e, acc);
+        else if (c == 0u) stream_island(B, sp.keep, R, cap, tol, max_sweeps, bmask, skey, isl_lds, e, acc);
+        else pair_island(B, sp.keep, R, cap, tol, max_sweeps, bmask, skey, isl_lds, e, acc);
+        if (t == 0u) G.next = gridDim.x + atomicAdd(&cnt->isl_wg_next, 1u);
+        __syncthreads();
+        w = G.next;
+        __syncthreads();
+    }
+    __syncthreads();
+
+    // ---- the rest, by waves
+    WaveLds& W = reinterpret_cast<WaveLds*>(isl_lds)[t >> 6];
+    const uint32_t M = min(cap, cnt->m_eff), M0 = cnt->m_glob;
+    const uint32_t n64 = masks ? n2 : 0u, n32 = masks ? (n3 + 1u) / 2u : 0u, n16 = masks ? (n4 + 3u) / 4u : 0u;
+    const uint32_t n_win = M > M0 ? (M - M0 + BUNDLE_SLOTS - 1u) / BUNDLE_SLOTS : 0u;
+    const uint32_t n_wave = n64 + n32 + n16 + n_win;
+    const uint32_t waves = gridDim.x * ISL_WAVES;
+    for (uint32_t w = blockIdx.x + gridDim.x * (t >> 6); w < n_wave;) {
+        // the next piece is asked for before this one is worked on
+        uint32_t nx = 0;
+        if (lane == 0u) nx = atomicAdd(&cnt->isl_wave_next, 1u);
+        bool mine = false, search = false;
+        uint32_t s = 0, li = 0, colour = 0;
+        if (w < n64 + n32 + n16) {
+            const uint32_t c = w < n64 ? 2u : (w < n64 + n32 ? 3u : 4u);
+            const uint32_t T = 64u >> (c - 2u);  // lanes per island
+            const uint32_t unit = c == 2u ? w : (c == 3u ? w - n64 : w - n64 - n32);
+            const uint32_t i = unit * (64u / T) + lane / T, u = lane % T;
+            if (i < (c == 2u ? n2 : (c == 3u ? n3 : n4))) {
+                const uint2 e = list[isl_region(c, cap) + i];
+                mine = u < e.y;
+                s = e.x + u;
+                li = lane - u;
+                if (mine) colour = skey[s] & 0xFFu;
+            }
+        } else {
+            // a lane's slot belongs to the window when its island is small and its first slot
+            // lies in it
+            const uint32_t w0 = M0 + (w - n64 - n32 - n16) * BUNDLE_SLOTS;
+            s = w0 + lane;
+            search = true;
+            if (s < M) {
+                const uint32_t k = skey[s];
+                if (B.icnt[(k & ~LOCAL_KEY) >> 8] <= ISLAND_LANE_MAX) {
+                    uint32_t st = s;
+                    while (st > M0 && ((skey[st - 1u] ^ k) >> 8) == 0u) --st;  // at most ISLAND_LANE_MAX - 1 steps
+                    mine = st >= w0 && st < w0 + BUNDLE_SLOTS;
+                    li = mine ? st - w0 : 0u;
+                    colour = k & 0xFFu;
+                }
+            }
+        }
+        if (__ballot(mine) != 0ull)
+            wave_islands(B, sp.keep, R, cap, tol, max_sweeps, bmask, W, mine, s, li, colour, search, acc);
+        w = waves + (uint32_t)__shfl((int)nx, 0, 64);
+    }
+    island_flush(cnt, acc);
+}
+int pgs_islands_setup() {
+    return hipFuncSetAttribute((const void*)k_pgs_islands, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)ISL_LDS_BYTES) == hipSuccess ? 1 : 0;
 }
 
 // Previous-step lookup table for the warm start: (a, b) -> slot.
@@ -3064,14 +3767,11 @@ void launch_col_sort_input(const Bodies& B, const uint2* m_ab, const uint32_t* c
 }
 void launch_pgs_local(const Bodies& B, const StepParams& sp, const SolverRows& R, Counters* cnt, uint32_t cap,
                       const uint32_t* skey, uint2* list, float tol, uint32_t max_sweeps, uint32_t groups,
-                      hipStream_t s, hipEvent_t ev0, hipEvent_t ev1, const uint64_t* flow_bmask) {
+                      hipStream_t s, const uint64_t* bmask, bool flow_init, hipEvent_t ev0, hipEvent_t ev1) {
     if (max_sweeps == 0u) return;
-    hipLaunchKernelGGL(k_pgs_group, dim3(groups), dim3(256), 0, s, B, sp, R, cnt, cap, list, skey, tol, max_sweeps,
-                       flow_bmask);
-    const uint32_t windows = (cap + BUNDLE_SLOTS - 1u) / BUNDLE_SLOTS;
     if (ev0) (void)hipEventRecord(ev0, s);
-    hipLaunchKernelGGL(k_pgs_bundle, dim3(std::max(1u, std::min(windows, 16384u))), dim3(64), BUNDLE_LDS_BYTES, s, B,
-                       sp, R, cnt, cap, skey, tol, max_sweeps);
+    hipLaunchKernelGGL(k_pgs_islands, dim3(groups), dim3(ISL_THREADS), ISL_LDS_BYTES, s, B, sp, R, cnt, cap, list, skey,
+                       tol, max_sweeps, bmask, flow_init ? 1u : 0u);
     if (ev1) (void)hipEventRecord(ev1, s);
 }
 void launch_prep(const Bodies& B, const StepParams& sp, const uint32_t* order, uint32_t cap, const uint2* m_ab,

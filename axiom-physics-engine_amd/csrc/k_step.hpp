@@ -107,14 +107,15 @@ void launch_colour(const Bodies& B, const uint2* m_ab, uint32_t cap_man, uint32_
 void launch_col_sort_input(const Bodies& B, const uint2* m_ab, const uint32_t* col, uint32_t cap, uint32_t* key,
                            uint32_t* val, const Counters* cnt, uint32_t split,
                            hipStream_t s);
-// The islands solved on their own (after the row preparation, which built their work
-// list): one lane or one workgroup per island; tol > 0 stops each at its own residual.
-// With flow_bmask (the colouring's per-body colour masks), its first launch also sets up
-// the large islands' sweep (as launch_pgs_flow does unless told it is inited).
+// The islands solved on their own (after the row preparation, which built their work list),
+// in `groups` workgroups (one per CU): tol > 0 stops each at its own residual.  bmask holds
+// the colouring's per-body colour masks.  With flow_init, the same launch also sets up the
+// large islands' sweep (as launch_pgs_flow does unless told it is inited).  Events ev0 / ev1,
+// when given, are recorded around it.
 void launch_pgs_local(const Bodies& B, const StepParams& sp, const SolverRows& R, Counters* cnt, uint32_t cap,
                       const uint32_t* skey, uint2* list, float tol, uint32_t max_sweeps, uint32_t groups,
-                      hipStream_t s, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr,
-                      const uint64_t* flow_bmask = nullptr);
+                      hipStream_t s, const uint64_t* bmask, bool flow_init, hipEvent_t ev0 = nullptr,
+                      hipEvent_t ev1 = nullptr);
 // Work the row preparation launch also does for the launches after it, each in a loop of
 // its own over the grid: the colour offsets of the sorted keys skey (col_off[c] = first
 // position whose key has colour >= c, c = 0..K, and m_glob = col_off[K], when col_off is
@@ -162,8 +163,7 @@ struct SweepStop {
 // Persistent sweep: `groups` workgroups of one wave, each with `lds_bytes` of LDS for
 // its staged rows; all of them must be resident at once (see pgs_own_setup).  Events
 // ev0 / ev1, when given, are recorded around the sweep kernel itself.  With inited, the
-// inboxes and next visits were already set up by this step's launch_pgs_local (given
-// bmask as flow_bmask).
+// inboxes and next visits were already set up by this step's launch_pgs_local.
 void launch_pgs_flow(const Bodies& B, const StepParams& sp, const SolverRows& R, uint32_t cap, const uint64_t* bmask,
                      uint32_t sweep0, uint32_t nsweeps, Counters* cnt,
                      uint32_t spin_limit, uint32_t groups, uint32_t lds_bytes, uint32_t tune, hipStream_t s,
@@ -172,8 +172,8 @@ void launch_pgs_flow(const Bodies& B, const StepParams& sp, const SolverRows& R,
 // Raises the sweep kernel's dynamic-LDS limit to max_lds_bytes and returns how many of
 // its workgroups with lds_bytes each fit on one CU (0 on error).
 int pgs_own_setup(uint32_t max_lds_bytes, uint32_t lds_bytes);
-// Allows the bundle kernel of the small islands its LDS (once per process); 0 on failure.
-int pgs_bundle_setup();
+// Allows the small islands' kernel its LDS (once per process); 0 on failure.
+int pgs_islands_setup();
 void launch_pgs(const Bodies& B, const StepParams& sp, const SolverRows& R, uint32_t s0, uint32_t s1, uint32_t cap,
                 uint32_t first, hipStream_t s);
 void launch_residual(const Bodies& B, const StepParams& sp, const SolverRows& R, const Counters* cnt, uint32_t cap,

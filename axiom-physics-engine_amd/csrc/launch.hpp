@@ -65,10 +65,11 @@ struct Bodies {
     uint32_t* wake;
     uint32_t* icnt;  // per step, per island root: the island's manifolds
 };
-// Islands of at most ISLAND_LOCAL_MAX manifolds are solved on their own (one lane each up
-// to ISLAND_LANE_MAX manifolds, else one workgroup), each to its own residual; their
-// solve slots follow those of the large islands, keyed LOCAL_KEY | root << 8 | colour.
-constexpr uint32_t ISLAND_LOCAL_MAX = 4096u, ISLAND_LANE_MAX = 8u;
+// Islands of at most ISLAND_LOCAL_MAX manifolds are solved on their own, each to its own
+// residual; their solve slots follow those of the large islands, keyed
+// LOCAL_KEY | root << 8 | colour.  Those of at most ISLAND_LANE_MAX manifolds are found by
+// their slots, the others through a work list in ISLAND_CLASSES size classes.
+constexpr uint32_t ISLAND_LOCAL_MAX = 4096u, ISLAND_LANE_MAX = 8u, ISLAND_CLASSES = 5u;
 constexpr uint32_t LOCAL_KEY = 0x80000000u, ISLAND_ROOT_LIMIT = 1u << 23;
 constexpr uint32_t ASLEEP_BIT = 0x80000000u, LABEL_MASK = 0x7FFFFFFFu, LABEL_NONE = 0x7FFFFFFFu;
 constexpr uint32_t BODY_KINEMATIC = 1u;
@@ -142,12 +143,12 @@ struct Counters {
     uint32_t tol_hit;      // 1: the step's sweeps stopped because the residual met the tolerance
     uint32_t loc_res_bits; // the largest residual an island solved on its own ended with
     uint32_t loc_miss;     // 1: an island solved on its own stopped at the sweep cap above the tolerance
-    uint32_t isl_lane_n;   // islands solved by one lane each
-    uint32_t isl_group_n;  // islands solved by one workgroup each
+    uint32_t isl_n[ISLAND_CLASSES];  // islands of the work list per size class
+    uint32_t isl_wg_next;    // work taken from the workgroups' and from the waves' part of it,
+    uint32_t isl_wave_next;  // beyond the first piece of each
     uint32_t loc_points;   // contact points of the islands solved on their own
-    uint32_t pad5;
     unsigned long long loc_point_sweeps;     // their contact points x the sweeps each island ran
-    unsigned long long bundle_point_sweeps;  // the same for the islands of the bundle kernel
+    unsigned long long bundle_point_sweeps;  // the same for the islands of k_pgs_islands
     // ---- kept across steps
     uint32_t sticky;       // STICKY_* bits; while set the integration is skipped (state untouched)
     uint32_t steps_done;   // steps whose integration ran
@@ -172,7 +173,7 @@ template <class T> inline T spread_total(const Counters& c, T SpreadRow::*f) {
     for (uint32_t k = 0; k < SPREAD; ++k) s += c.sp[k].*f;
     return s;
 }
-constexpr uint32_t COUNTERS_RESET_WORDS = 26;  // words of the first block (cleared per step)
+constexpr uint32_t COUNTERS_RESET_WORDS = 30;  // words of the first block (cleared per step)
 static_assert(offsetof(Counters, sticky) == 4 * COUNTERS_RESET_WORDS, "per-step block ends at sticky");
 enum : uint32_t {
     STICKY_PAIRS = 1u,        // pair capacity exceeded

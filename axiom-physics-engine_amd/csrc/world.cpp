@@ -170,7 +170,7 @@ struct axm_world_s {
     float graph_dt = 0.0f;
     uint32_t graph_iters = 0;
     hipEvent_t gprof_ev[4] = {nullptr, nullptr, nullptr, nullptr};  // sweep-kernel events per parity
-    hipEvent_t bprof_ev[4] = {nullptr, nullptr, nullptr, nullptr};  // bundle-kernel events (eager / per parity)
+    hipEvent_t bprof_ev[4] = {nullptr, nullptr, nullptr, nullptr};  // small islands' kernel events (eager / per parity)
     const uint32_t* solve_keys = nullptr;  // the sorted keys of the last step's solve order
 
     // last step
@@ -513,7 +513,7 @@ axm_status clear_sticky(axm_world_s* w) {
     return AXM_SUCCESS;
 }
 
-// The bundle kernel's profiling events of slot pair p (created on first use).
+// The small islands' kernel's profiling events of slot pair p (created on first use).
 axm_status bundle_events(axm_world_s* w, int p) {
     for (int k = 2 * p; k < 2 * p + 2; ++k)
         if (!w->bprof_ev[k]) AXM_HIP(hipEventCreate(&w->bprof_ev[k]));
@@ -721,7 +721,7 @@ axm_status enqueue_step(axm_world_s* w, float dt, const StepOpts& o) {
             b1 = w->bprof_ev[1];
         }
         launch_pgs_local(w->B, sp, R, w->cnt, rc, w->solve_keys, w->isl_list, w->desc.residual_tol, max_it,
-                         2u * (uint32_t)w->cu_count, s, b0, b1, flow_inited ? w->bmask : nullptr);
+                         (uint32_t)w->cu_count, s, w->bmask, flow_inited, b0, b1);
     }
     const bool want_res = (o.flags & AXM_STEP_RESIDUAL) || w->desc.record_residual || tol_mode;
     const uint32_t every = std::max<uint32_t>(w->desc.residual_every, 1u);
@@ -1041,7 +1041,7 @@ axm_status axm_world_create(const axm_world_desc* desc, axm_world* out) {
     w->max_lds = (uint32_t)std::min<size_t>(prop.sharedMemPerBlock, 160u * 1024u);
     w->sweep_lds = w->max_lds & ~16383u;
     const int own_per_cu = pgs_own_setup(w->max_lds, w->sweep_lds);
-    if (own_per_cu < 1 || !pgs_bundle_setup()) {
+    if (own_per_cu < 1 || !pgs_islands_setup()) {
         delete w;
         return AXM_GPU_OPERATION_FAILED;
     }
@@ -1367,8 +1367,8 @@ axm_status axm_world_run(axm_world w, float dt, uint32_t iters, uint32_t steps, 
                                                                  : iters;
                 if (split)
                     launch_pgs_local(w->B, sp, w->R[c], w->cnt, w->rcap[c], w->solve_keys, w->isl_list,
-                                     w->desc.residual_tol, nsw, 2u * (uint32_t)w->cu_count, w->stream,
-                                     w->bprof_ev[2 * c], w->bprof_ev[2 * c + 1], w->bmask);
+                                     w->desc.residual_tol, nsw, (uint32_t)w->cu_count, w->stream, w->bmask, true,
+                                     w->bprof_ev[2 * c], w->bprof_ev[2 * c + 1]);
                 launch_pgs_flow(w->B, sp, w->R[c], w->rcap[c], w->bmask, 0, nsw, w->cnt, SWEEP_SPIN_LIMIT_US,
                                 w->sweep_groups, w->sweep_lds, w->sweep_tune, w->stream, w->gprof_ev[2 * c],
                                 w->gprof_ev[2 * c + 1], checks ? stop : SweepStop{}, split);

@@ -239,13 +239,13 @@ def headline(args):
     value = bodies.n * args.steps / elapsed
     steps_done = max(int(tot.steps), 1)
     mean_sweeps = tot.sweeps / steps_done
-    # the sweep kernels, 240 B per contact point per sweep each: the bundle kernel of the small
+    # the sweep kernels, 240 B per contact point per sweep each: the kernel of the small
     # islands solved on their own (their points x the sweeps each island ran) and the persistent
     # sweep of the large islands (the rest); the roofline line is the one with more time
     kern = {"k_pgs_own": (B_SWEEP * float(tot.contact_sweeps - tot.local_contact_sweeps), prof.pgs_ms * 1e-3,
                           int(prof.pgs_launches))}
     if prof.bundle_launches:
-        kern["k_pgs_bundle"] = (B_SWEEP * float(prof.bundle_point_sweeps), prof.bundle_ms * 1e-3,
+        kern["k_pgs_islands"] = (B_SWEEP * float(prof.bundle_point_sweeps), prof.bundle_ms * 1e-3,
                                 int(prof.bundle_launches))
 
     def roof_of(name):

@@ -181,7 +181,7 @@ typedef struct axm_kernel_profile {
     double pgs_ms;        /* summed kernel durations */
     double pgs_bytes;     /* summed algorithmic bytes of those launches */
     uint64_t sweeps;
-    /* the bundle kernel of the islands solved on their own (island_solve) */
+    /* the kernel of the islands solved on their own (island_solve) */
     uint64_t bundle_launches;
     double bundle_ms;     /* summed kernel durations */
     uint64_t bundle_point_sweeps; /* contact points x sweeps of its islands (240 B each) */
