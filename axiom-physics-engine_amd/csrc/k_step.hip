@@ -1898,32 +1898,6 @@ __global__ void __launch_bounds__(256) k_flow_init(Bodies B, SolverRows R, const
                                                    const Counters* __restrict__ cnt) {
     flow_init_part(B, R, bmask, cnt, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
 }
-// After a launch: each dynamic body's final velocity is in the inbox of its first
-// visit (the last visit of the last sweep passed it on there).
-__global__ void __launch_bounds__(256) k_flow_finish(Bodies B, SolverRows R, const Counters* __restrict__ cnt) {
-    if (cnt->sticky != 0u) return;
-    const uint32_t M = cnt->m_glob;
-    for (uint32_t s = blockIdx.x * blockDim.x + threadIdx.x; s < M; s += gridDim.x * blockDim.x) {
-    const uint4 h = R.hdr[s];
-    const uint2 dp = R.dep[s];
-    const uint64_t* ib = R.inbox;
-    if (dp.x != UNSET && (dp.x & 0xFFu) == 0u) {
-        f3 v, w;
-        vunpack4(vsplit(ib[vin_word(s, 0, 0)]), vsplit(ib[vin_word(s, 0, 1)]), vsplit(ib[vin_word(s, 0, 2)]),
-                 vsplit(ib[vin_word(s, 0, 3)]), v, w);
-        B.sv[h.x] = f4(v, B.sv[h.x].w);
-        B.sw[h.x] = f4(w, 0.0f);
-    }
-    if (dp.y != UNSET && (dp.y & 0xFFu) == 0u) {
-        f3 v, w;
-        vunpack4(vsplit(ib[vin_word(s, 1, 0)]), vsplit(ib[vin_word(s, 1, 1)]), vsplit(ib[vin_word(s, 1, 2)]),
-                 vsplit(ib[vin_word(s, 1, 3)]), v, w);
-        B.sv[h.y] = f4(v, B.sv[h.y].w);
-        B.sw[h.y] = f4(w, 0.0f);
-    }
-    }
-}
-
 // Residual of one contact point: the largest velocity-space change (impulse change
 // times the row's effective mass inverse) that one more visit would make along the
 // normal or either friction direction, from the current velocities and impulses L.
@@ -2032,7 +2006,7 @@ constexpr uint32_t OWN_SLOTS = 16;  // slots per lane with a staged record
 // run in chunks of stop.every with a residual check after each chunk (every wave of
 // the grid meets at one arrival count per check).
 __global__ void __launch_bounds__(OWN_WAVE) k_pgs_own(Bodies B, StepParams sp, SolverRows R, Counters* cnt,
-                                                      uint32_t cap, uint32_t sweep0, uint32_t nsweeps,
+                                                      uint32_t cap, uint32_t nsweeps, uint32_t flow_slots,
                                                       uint32_t lds_f4, uint32_t spin_limit, uint32_t tune,
                                                       const uint64_t* __restrict__ bmask, SweepStop stop) {
     extern __shared__ float4 own_lds[];
@@ -2044,6 +2018,7 @@ __global__ void __launch_bounds__(OWN_WAVE) k_pgs_own(Bodies B, StepParams sp, S
         return;
     }
     if (cnt->sticky != 0u || nsweeps == 0u) return;
+    if (M > 0u && M <= flow_slots) return;  // k_pgs_flow ran them
     if (M == 0u && cnt->m_eff > 0u) {
         // every island was solved on its own: no sweep of the large ones runs
         if (blockIdx.x == 0 && lane == 0 && stop.bits) {
@@ -2243,8 +2218,8 @@ __global__ void __launch_bounds__(OWN_WAVE) k_pgs_own(Bodies B, StepParams sp, S
         return seen < CHECK_ABOVE ? 1 : 0;
     };
     const bool checks = stop.bits != nullptr;
+    uint32_t chunk_end = checks ? min(stop.every, nsweeps) : nsweeps;  // in the end the sweeps run
     auto sweep_loop = [&]<bool STAGED>() -> bool {
-        uint32_t chunk_end = checks ? min(stop.every, nsweeps) : nsweeps;
         uint32_t total = nv * chunk_end;
         uint32_t done = 0, sw = 0, j = 0, off = 0;
         Item it;
@@ -2327,7 +2302,7 @@ __global__ void __launch_bounds__(OWN_WAVE) k_pgs_own(Bodies B, StepParams sp, S
                 Bd.w = f3{tb ? bw.x : Bd.w.x, tb ? bw.y : Bd.w.y, tb ? bw.z : Bd.w.z};
             }
             if (ok) {
-                const bool first = sweep0 + sw == 0u;
+                const bool first = sw == 0u;
                 float4 L[4];
                 // the point loops run over a fixed 4 so that L stays in registers
                 const bool stg = STAGED || staged_slot(j);
@@ -2417,6 +2392,19 @@ __global__ void __launch_bounds__(OWN_WAVE) k_pgs_own(Bodies B, StepParams sp, S
                                                         : sweep_loop.template operator()<false>();
     if (!finished) return;
 
+    // each dynamic body's velocity after the last sweep, by the lane of its first visit
+    for (uint32_t j = 0; j < nv; ++j) {
+        const Item it = j < nrec ? item_get(recs + (size_t)j * 4u * OWN_WAVE) : item_global(B, R, slot_of(j));
+        SB X;
+        if (it.dp.x != UNSET && (it.dp.x & 0xFFu) == 0u && final_vel(it.h.x, it.dp.x, chunk_end, X)) {
+            B.sv[it.h.x] = f4(X.v, it.imA);
+            B.sw[it.h.x] = f4(X.w, 0.0f);
+        }
+        if (it.dp.y != UNSET && (it.dp.y & 0xFFu) == 0u && final_vel(it.h.y, it.dp.y, chunk_end, X)) {
+            B.sv[it.h.y] = f4(X.v, it.imB);
+            B.sw[it.h.y] = f4(X.w, 0.0f);
+        }
+    }
     // impulses of the staged points back to the rows
     uint32_t woff = 0;
     for (uint32_t jj = 0; jj < nv; ++jj) {
@@ -3434,6 +3422,316 @@ int pgs_islands_setup() {
                                (int)ISL_LDS_BYTES) == hipSuccess ? 1 : 0;
 }
 
+// ---------------------------------------------------------------- large islands in registers
+// The large islands' sweeps when every slot has two lanes of the GPU to itself (FLOW_SLOTS
+// slots at most; k_pgs_own takes more): the even lane of a pair holds body a's side of the
+// slot's rows, the odd lane body b's (half_jvel), with the impulses, in registers for the whole
+// solve.  Visits pass velocities on through the inboxes as in k_pgs_own; with one slot per pair
+// a wave's lanes wait for nothing but their own bodies, and a visit reads only the 32 bytes of
+// its inbox side from memory.  What binds is the chain of dependent visits: a handoff (store,
+// poll) of about 0.5 us and three row updates of 22 instructions per point.  Slots are dealt
+// out thinly (spw per wave, as few as M allows) so that a visit holds up few others.
+//
+// Residual checks run one sweep behind: after s sweeps (a check point) a slot's residual needs
+// its bodies' velocities after the sweep, which their first visits of the next sweep have in
+// their inboxes; the pair reads them there, stores its residual, and goes on with its next
+// visit while the other waves still arrive.  The visit keeps the impulses it replaces, so that
+// when the check says stop, the one visit run ahead is taken back.  A pair passes a check point
+// only after the check before it has been decided, so at most one visit is ever ahead, and an
+// inbox is never overwritten before every reader of its velocity has passed (the body's next
+// round of visits includes the reader's own).
+// A pile of 19.1k manifolds in 18 colours: 44.5 us per sweep in k_pgs_own -> 21.8 us; with a check
+// after every sweep 66 -> 28.9 us.  Fewer slots per wave (8 or 16, so that a visit holds up fewer
+// others) change the first by less than 2 % and cost up to 5 % in arrivals; polling harder (no
+// sleep, a tight loop, two polls in flight) gains nothing or loses.
+constexpr uint32_t FLOW_THREADS = 512, FLOW_WAVES = FLOW_THREADS / 64u;
+constexpr uint32_t FLOW_WAVE_SLOTS = 32;
+__device__ __forceinline__ u32x4_t flow_quad(const uint64_t* inbox, uint32_t byte) {
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint64_t*>(inbox), 0, 0x7FFFFFFF, 0x00020000);
+    // aux: sc0 | sc1, as vin_quad
+    return __builtin_amdgcn_raw_buffer_load_b128(rs, (int)byte, 0, 1 | 16);
+}
+template <bool CHECKS>
+__global__ void __launch_bounds__(FLOW_THREADS, 2)
+k_pgs_flow(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap, uint32_t nsweeps, uint32_t spin_limit,
+           const uint64_t* __restrict__ bmask, SweepStop stop) {
+    __shared__ uint32_t s_arrived, s_above, s_max;
+    const uint32_t M = cnt->m_glob, G = gridDim.x;
+    if (M == 0u || M > G * FLOW_WAVES * FLOW_WAVE_SLOTS || cnt->max_colour > 64u || cnt->sticky != 0u || nsweeps == 0u)
+        return;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t nw = (M + FLOW_WAVE_SLOTS - 1u) / FLOW_WAVE_SLOTS;
+    // wave w of the grid owns slots 32 w on; neighbouring waves (the same colour) lie on
+    // different CUs
+    const uint32_t wid = wave * G + blockIdx.x;
+    if (blockIdx.x >= nw) return;  // the whole workgroup has nothing
+    const uint32_t groups = min(G, nw);
+    const uint32_t wg_waves = (nw - blockIdx.x + G - 1u) / G;  // waves of this workgroup with slots
+    if (threadIdx.x == 0u) s_arrived = s_above = s_max = 0u;
+    __syncthreads();
+    if (wid >= nw) return;
+    const uint32_t pair = lane >> 1, s = wid * FLOW_WAVE_SLOTS + pair;
+    const bool odd = (lane & 1u) != 0u, active = s < M;
+    const uint32_t every = CHECKS ? max(stop.every, 1u) : nsweeps;
+    const float keep = sp.keep, tol = stop.tol;
+    uint32_t* err = &cnt->sticky;
+
+    // ---- the slot: rows, impulses, this side's body
+    HalfPoint P[4];
+    float ln[4], l1[4], l2[4], pn[4], p1[4], p2[4];  // impulses, and those before the last visit
+    HalfBody X;
+    X.v = X.w = f3{0.0f, 0.0f, 0.0f};
+    X.im = 0.0f;
+    HalfBody F = X;  // the body's velocity at the last check point (or after the last sweep)
+    uint32_t np = 0, body = 0, deg = 0, rank = 0, own = 0, from = 0, to = 0;
+    bool dyn = false;
+    if (active) {
+        const uint4 h = R.hdr[s];
+        const uint2 dp = R.dep[s], nx = R.next[s];
+        const bool plane = (h.y & PLANE_BIT) != 0u;
+        const uint32_t d = odd ? dp.y : dp.x;
+        np = min(h.z, 4u);
+        body = odd ? h.y : h.x;
+        dyn = d != UNSET;
+        if (!(odd && plane)) {
+            const float4 v = B.sv[body];
+            X.im = v.w;
+            if (!dyn) {
+                X.v = xyz(v);
+                X.w = xyz(B.sw[body]);
+            }
+        }
+        if (dyn) {
+            deg = d >> 8;
+            rank = d & 0xFFu;
+            own = (s << 1 | (odd ? 1u : 0u)) * 32u;  // bytes: four words per side
+            from = first_visit(B, bmask, body) * 32u;
+            to = (odd ? nx.y : nx.x) * 32u;
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k)
+            if (k < np) {
+                half_rows(R, s, cap, k, odd, plane, P[k]);
+                const float4 L = R.lam[(size_t)k * cap + s];
+                ln[k] = L.x;
+                l1[k] = L.y;
+                l2[k] = L.z;
+            }
+    }
+    F = X;
+    // a check's velocities are the next visit's inputs when both sides visit first
+    const bool first_both = (rank | (uint32_t)__shfl_xor((int)rank, 1, 64)) == 0u;
+    uint32_t k = 0;                        // this pair's sweeps done
+    uint32_t ver = 0;                      // its body's visits in them
+    uint32_t cp = min(every, nsweeps);     // its next check point (the end without checks)
+    uint32_t need = 0;                     // the check point before it, which must be decided first
+    bool fin = false;                      // it waits at check point cp (else for its inputs of visit k)
+    bool live = active;
+    float res = 0.0f;                      // its residual at the last check point
+    uint32_t arrived = 0;                  // the last check point this wave arrived at
+    uint32_t decided = 0;                  // the last check point known not to stop
+    uint32_t stop_at = UNSET;
+    uint32_t spins = 0;
+    const uint64_t t_start = wall_clock64(), t_limit = (uint64_t)spin_limit * 100ull;  // wall clock: 100 MHz
+    bool failed = false;
+    // whether every workgroup has arrived at check point c; then whether one is above the tolerance
+    auto arrivals = [&](uint32_t c, bool& above) -> bool {
+        uint32_t* arr = stop.arrive + (size_t)(c - 1u) * CHECK_ROWS * CHECK_ROW_WORDS;
+        uint32_t seen = 0;
+        if (lane < CHECK_ROWS)
+            seen = __hip_atomic_load(arr + lane * CHECK_ROW_WORDS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (uint32_t o = CHECK_ROWS / 2u; o >= 1u; o >>= 1) seen += (uint32_t)__shfl_xor((int)seen, (int)o, 64);
+        seen = (uint32_t)__builtin_amdgcn_readfirstlane((int)seen);
+        above = seen >= CHECK_ABOVE;
+        return (seen & (CHECK_ABOVE - 1u)) >= groups;
+    };
+    for (;;) {
+        bool ok = live && need <= decided;
+        if (ok && dyn) {
+            const uint32_t at = fin ? from : own, want = (fin ? ver : ver + rank) & 0xFFFFu;
+            const u32x4_t a = flow_quad(R.inbox, at), b = flow_quad(R.inbox, at + 16u);
+            ok = (((a[1] >> 16) ^ want) | ((a[3] >> 16) ^ want) | ((b[1] >> 16) ^ want) | ((b[3] >> 16) ^ want)) == 0u;
+            // X counts only in the pass in which every version matches
+            vunpack4(make_uint2(a[0], a[1]), make_uint2(a[2], a[3]), make_uint2(b[0], b[1]), make_uint2(b[2], b[3]), X.v,
+                     X.w);
+        }
+        const uint64_t oks = __ballot(ok);
+        const uint64_t got = oks & (((oks >> 1) & 0x5555555555555555ull) | ((oks << 1) & 0xAAAAAAAAAAAAAAAAull));
+        ok = ((got >> lane) & 1ull) != 0ull;
+        bool passed = false, ahead = false;
+        if (ok) {
+            passed = fin;
+            if (fin) {
+                F = X;
+                fin = false;
+                live = k < nsweeps;
+            }
+            if (live && (!passed || first_both)) {
+                ahead = true;
+                if (CHECKS) {
+#pragma unroll
+                    for (uint32_t q = 0; q < 4; ++q) {
+                        pn[q] = ln[q];
+                        p1[q] = l1[q];
+                        p2[q] = l2[q];
+                    }
+                }
+                if (k == 0u) {
+#pragma unroll
+                    for (uint32_t q = 0; q < 4; ++q) {
+                        if (q >= np) break;
+                        half_apply(P[q].n, ln[q], X);
+                        half_apply(P[q].t1, l1[q], X);
+                        half_apply(P[q].t2, l2[q], X);
+                    }
+                }
+#pragma unroll
+                for (uint32_t q = 0; q < 4; ++q) {
+                    if (q >= np) break;
+                    half_friction(P[q].t1, P[q].mT1, P[q].maxf, keep, l1[q], X);
+                    half_friction(P[q].t2, P[q].mT2, P[q].maxf, keep, l2[q], X);
+                }
+#pragma unroll
+                for (uint32_t q = 0; q < 4; ++q) {
+                    if (q >= np) break;
+                    half_normal(P[q].n, P[q].mN, P[q].tg, keep, ln[q], X);
+                }
+                if (dyn) {
+                    uint64_t o[4];
+                    vpack4(X.v, X.w, ver + rank + 1u, o);
+                    const __amdgpu_buffer_rsrc_t rs =
+                        __builtin_amdgcn_make_buffer_rsrc(R.inbox, 0, 0x7FFFFFFF, 0x00020000);
+                    const u32x4_t q0 = {(uint32_t)o[0], (uint32_t)(o[0] >> 32), (uint32_t)o[1], (uint32_t)(o[1] >> 32)};
+                    const u32x4_t q1 = {(uint32_t)o[2], (uint32_t)(o[2] >> 32), (uint32_t)o[3], (uint32_t)(o[3] >> 32)};
+                    // aux: sc1, as vin_store
+                    __builtin_amdgcn_raw_buffer_store_b128(q0, rs, (int)to, 0, 16);
+                    __builtin_amdgcn_raw_buffer_store_b128(q1, rs, (int)(to + 16u), 0, 16);
+                }
+                if (k == cp) {  // the visit goes past a check point
+                    need = cp;
+                    cp = min(cp + every, nsweeps);
+                }
+                ++k;
+                ver += deg;
+                fin = k == cp;
+            }
+            // the residual at the check point, after the visit that others wait for (its impulses
+            // are those before that visit)
+            if (CHECKS && passed) {
+                res = 0.0f;
+#pragma unroll
+                for (uint32_t q = 0; q < 4; ++q) {
+                    if (q >= np) break;
+                    const float e = half_residual(P[q], keep, F, ahead ? pn[q] : ln[q], ahead ? p1[q] : l1[q],
+                                                  ahead ? p2[q] : l2[q]);
+                    if (e > res) res = e;
+                }
+            }
+        }
+        // ---- the wave: arrival at a check point once all its pairs have passed it (no pair is
+        // further than the next one), decisions, the end
+        if (CHECKS) {
+            if (__ballot(passed) != 0ull) {
+                const uint32_t next = min(arrived + every, nsweeps);
+                // a pair short of the check point has yet to reach it or waits there
+                if (__ballot(active && (k < next || (k == next && fin))) == 0ull) {
+                    arrived = next;
+                    uint32_t bits = active ? __float_as_uint(res) : 0u;
+                    for (int o = 32; o >= 1; o >>= 1) bits = max(bits, (uint32_t)__shfl_xor((int)bits, o, 64));
+                    if (lane == 0u) {
+                        // the last wave of the workgroup to arrive sends all; the words are free again
+                        // before any wave can reach the next check point (it needs this one decided)
+                        atomicMax(&s_max, bits);
+                        if (__uint_as_float(bits) > tol) atomicOr(&s_above, 1u);
+                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+                        const uint32_t n = atomicAdd(&s_arrived, 1u);
+                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+                        if (n == wg_waves - 1u) {
+                            const uint32_t mx = s_max, ab = s_above;
+                            s_max = s_above = s_arrived = 0u;
+                            atomicMax(stop.bits + next - 1u, mx);
+                            __hip_atomic_fetch_add(
+                                stop.arrive + ((size_t)(next - 1u) * CHECK_ROWS + blockIdx.x % CHECK_ROWS) * CHECK_ROW_WORDS,
+                                1u + (ab ? CHECK_ABOVE : 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        }
+                    }
+                }
+            }
+            // the outstanding decision, when a pair waits for it or no pair got on (the inputs of a
+            // visit past the check point never come when the check stops the others)
+            if (decided < arrived && (got == 0ull || __ballot(live && need > decided) != 0ull)) {
+                bool above;
+                const uint32_t c = min(decided + every, nsweeps);
+                if (arrivals(c, above)) {
+                    if (!above) {
+                        stop_at = c;
+                        break;
+                    }
+                    decided = c;
+                }
+            }
+        }
+        if (got != 0ull) {
+            if (__ballot(live) == 0ull) break;
+            continue;
+        }
+        __builtin_amdgcn_s_sleep(1);
+        if ((++spins & 255u) == 0u) {
+            if (wall_clock64() - t_start > t_limit) {
+                if (lane == 0u) atomicOr(err, STICKY_TIMEOUT);
+                failed = true;
+                break;
+            }
+            if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) {
+                failed = true;  // another wave gave up
+                break;
+            }
+        }
+    }
+    if (failed) return;
+    // the step's sweeps and whether they met the tolerance
+    if (CHECKS && wid == 0u) {
+        bool hit = stop_at != UNSET;
+        if (!hit) {
+            bool above = true, all = false;
+            while (!(all = arrivals(nsweeps, above))) {
+                if (wall_clock64() - t_start > t_limit) break;
+                __builtin_amdgcn_s_sleep(1);
+            }
+            if (!all) {
+                if (lane == 0u) atomicOr(err, STICKY_TIMEOUT);
+                return;
+            }
+            hit = !above;
+        }
+        if (lane == 0u) {
+            __hip_atomic_store(&cnt->sweeps_run, stop_at != UNSET ? stop_at : nsweeps, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&cnt->tol_hit, hit ? 1u : 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    if (!active) return;
+    const bool back = CHECKS && stop_at != UNSET && k > stop_at;  // a visit ran ahead of the stop
+    if (!odd) {
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q)
+            if (q < np)
+                R.lam[(size_t)q * cap + s] =
+                    make_float4(back ? pn[q] : ln[q], back ? p1[q] : l1[q], back ? p2[q] : l2[q], 0.0f);
+    }
+    if (dyn && rank == 0u) {
+        B.sv[body] = f4(F.v, X.im);
+        B.sw[body] = f4(F.w, 0.0f);
+    }
+}
+int pgs_flow_setup() {
+    int nb = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_pgs_flow<true>, FLOW_THREADS, 0) != hipSuccess) return 0;
+    return nb;
+}
+
 // Previous-step lookup table for the warm start: (a, b) -> slot.
 // Each entry's table position goes to pos[slot], so that the next build of this table
 // clears only the entries it holds (cache_m of them) instead of the whole table.
@@ -3828,16 +4126,22 @@ int pgs_own_setup(uint32_t max_lds_bytes, uint32_t lds_bytes) {
     return nb;
 }
 void launch_pgs_flow(const Bodies& B, const StepParams& sp, const SolverRows& R, uint32_t cap, const uint64_t* bmask,
-                     uint32_t sweep0, uint32_t nsweeps, Counters* cnt,
-                     uint32_t spin_limit, uint32_t groups, uint32_t lds_bytes, uint32_t tune, hipStream_t s,
-                     hipEvent_t ev0, hipEvent_t ev1, const SweepStop& stop, bool inited) {
+                     uint32_t nsweeps, Counters* cnt, uint32_t spin_limit, uint32_t cus, uint32_t groups,
+                     uint32_t lds_bytes, uint32_t tune, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1,
+                     const SweepStop& stop, bool inited) {
     if (!nsweeps) return;
     if (!inited) hipLaunchKernelGGL(k_flow_init, grid_bounded(cap), dim3(256), 0, s, B, R, bmask, cnt);
     if (ev0) (void)hipEventRecord(ev0, s);
-    hipLaunchKernelGGL(k_pgs_own, dim3(groups ? groups : 1u), dim3(OWN_WAVE), lds_bytes, s, B, sp, R, cnt, cap, sweep0,
-                       nsweeps, lds_bytes / (uint32_t)sizeof(float4), spin_limit, tune, bmask, stop);
+    if (stop.bits)
+        hipLaunchKernelGGL(k_pgs_flow<true>, dim3(cus), dim3(FLOW_THREADS), 0, s, B, sp, R, cnt, cap, nsweeps,
+                           spin_limit, bmask, stop);
+    else
+        hipLaunchKernelGGL(k_pgs_flow<false>, dim3(cus), dim3(FLOW_THREADS), 0, s, B, sp, R, cnt, cap, nsweeps,
+                           spin_limit, bmask, stop);
+    hipLaunchKernelGGL(k_pgs_own, dim3(groups ? groups : 1u), dim3(OWN_WAVE), lds_bytes, s, B, sp, R, cnt, cap, nsweeps,
+                       cus * FLOW_WAVES * FLOW_WAVE_SLOTS, lds_bytes / (uint32_t)sizeof(float4), spin_limit, tune, bmask,
+                       stop);
     if (ev1) (void)hipEventRecord(ev1, s);
-    hipLaunchKernelGGL(k_flow_finish, grid_bounded(cap), dim3(256), 0, s, B, R, cnt);
 }
 void launch_pgs(const Bodies& B, const StepParams& sp, const SolverRows& R, uint32_t s0, uint32_t s1, uint32_t cap,
                 uint32_t first, hipStream_t s) {

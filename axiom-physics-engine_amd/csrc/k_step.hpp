@@ -160,15 +160,18 @@ struct SweepStop {
     float tol = -1.0f;
     uint32_t every = 1;
 };
-// Persistent sweep: `groups` workgroups of one wave, each with `lds_bytes` of LDS for
-// its staged rows; all of them must be resident at once (see pgs_own_setup).  Events
-// ev0 / ev1, when given, are recorded around the sweep kernel itself.  With inited, the
-// inboxes and next visits were already set up by this step's launch_pgs_local.
+// The large islands' sweeps.  Up to cus x 256 slots run with one slot per pair of lanes (`cus`
+// workgroups of 512 threads, all resident at once, see pgs_flow_setup); more in the staged
+// sweep: `groups` workgroups of one wave, each with `lds_bytes` of LDS for its staged rows; all
+// of them must be resident at once (see pgs_own_setup).  Events ev0 / ev1, when given, are
+// recorded around both.  With inited, the inboxes and next visits were already set up by this
+// step's launch_pgs_local.
 void launch_pgs_flow(const Bodies& B, const StepParams& sp, const SolverRows& R, uint32_t cap, const uint64_t* bmask,
-                     uint32_t sweep0, uint32_t nsweeps, Counters* cnt,
-                     uint32_t spin_limit, uint32_t groups, uint32_t lds_bytes, uint32_t tune, hipStream_t s,
-                     hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr, const SweepStop& stop = SweepStop{},
-                     bool inited = false);
+                     uint32_t nsweeps, Counters* cnt, uint32_t spin_limit, uint32_t cus, uint32_t groups,
+                     uint32_t lds_bytes, uint32_t tune, hipStream_t s, hipEvent_t ev0 = nullptr,
+                     hipEvent_t ev1 = nullptr, const SweepStop& stop = SweepStop{}, bool inited = false);
+// Workgroups of the register sweep that fit on one CU (0 on error).
+int pgs_flow_setup();
 // Raises the sweep kernel's dynamic-LDS limit to max_lds_bytes and returns how many of
 // its workgroups with lds_bytes each fit on one CU (0 on error).
 int pgs_own_setup(uint32_t max_lds_bytes, uint32_t lds_bytes);

@@ -741,8 +741,8 @@ axm_status enqueue_step(axm_world_s* w, float dt, const StepOpts& o) {
         hipEvent_t e0, e1;
         AXM_TRY(prof_event(w, nev, o.capture, e0));
         AXM_TRY(prof_event(w, nev, o.capture, e1));
-        launch_pgs_flow(w->B, sp, R, rc, w->bmask, 0, max_it, w->cnt, SWEEP_SPIN_LIMIT_US, w->sweep_groups,
-                        w->sweep_lds, w->sweep_tune, s, e0, e1, stop, flow_inited);
+        launch_pgs_flow(w->B, sp, R, rc, w->bmask, max_it, w->cnt, SWEEP_SPIN_LIMIT_US, (uint32_t)w->cu_count,
+                        w->sweep_groups, w->sweep_lds, w->sweep_tune, s, e0, e1, stop, flow_inited);
         it = max_it;  // at most; the count the launch ran is read back with the counters
     }
     bool all_local = false;
@@ -767,9 +767,9 @@ axm_status enqueue_step(axm_world_s* w, float dt, const StepOpts& o) {
             hipEvent_t e0, e1;
             AXM_TRY(prof_event(w, nev, o.capture, e0));
             AXM_TRY(prof_event(w, nev, o.capture, e1));
-            launch_pgs_flow(w->B, sp, R, rc, w->bmask, it, seg, w->cnt, SWEEP_SPIN_LIMIT_US,
-                            w->sweep_groups, w->sweep_lds, w->sweep_tune, s, e0, e1, SweepStop{},
-                            flow_inited && it == 0u);
+            // (one segment: the host checks a residual between segments in the per-colour launches only)
+            launch_pgs_flow(w->B, sp, R, rc, w->bmask, seg, w->cnt, SWEEP_SPIN_LIMIT_US, (uint32_t)w->cu_count,
+                            w->sweep_groups, w->sweep_lds, w->sweep_tune, s, e0, e1, SweepStop{}, flow_inited);
         }
         it += seg;
         const bool last = it == max_it;
@@ -1041,7 +1041,7 @@ axm_status axm_world_create(const axm_world_desc* desc, axm_world* out) {
     w->max_lds = (uint32_t)std::min<size_t>(prop.sharedMemPerBlock, 160u * 1024u);
     w->sweep_lds = w->max_lds & ~16383u;
     const int own_per_cu = pgs_own_setup(w->max_lds, w->sweep_lds);
-    if (own_per_cu < 1 || !pgs_islands_setup()) {
+    if (own_per_cu < 1 || pgs_flow_setup() < 1 || !pgs_islands_setup()) {
         delete w;
         return AXM_GPU_OPERATION_FAILED;
     }
@@ -1369,8 +1369,8 @@ axm_status axm_world_run(axm_world w, float dt, uint32_t iters, uint32_t steps, 
                     launch_pgs_local(w->B, sp, w->R[c], w->cnt, w->rcap[c], w->solve_keys, w->isl_list,
                                      w->desc.residual_tol, nsw, (uint32_t)w->cu_count, w->stream, w->bmask, true,
                                      w->bprof_ev[2 * c], w->bprof_ev[2 * c + 1]);
-                launch_pgs_flow(w->B, sp, w->R[c], w->rcap[c], w->bmask, 0, nsw, w->cnt, SWEEP_SPIN_LIMIT_US,
-                                w->sweep_groups, w->sweep_lds, w->sweep_tune, w->stream, w->gprof_ev[2 * c],
+                launch_pgs_flow(w->B, sp, w->R[c], w->rcap[c], w->bmask, nsw, w->cnt, SWEEP_SPIN_LIMIT_US,
+                                (uint32_t)w->cu_count, w->sweep_groups, w->sweep_lds, w->sweep_tune, w->stream, w->gprof_ev[2 * c],
                                 w->gprof_ev[2 * c + 1], checks ? stop : SweepStop{}, split);
                 AXM_HIP(hipGraphLaunch(w->gpost[c], w->stream));
             } else {
