@@ -1191,6 +1191,7 @@ __device__ __forceinline__ void sorted_keys_part(const Bodies& B, const uint32_t
                     const uint64_t in = __ballot(big && cls == c);
                     if (in == 0ull) continue;
                     uint32_t at = 0;
+                    if (c == 0u && big && cls == 0u) atomicAdd(&cnt->isl_wide, (size + 31u) / 32u);
                     if (lane == 0u) at = atomicAdd(&cnt->isl_n[c], (uint32_t)__popcll(in));
                     at = (uint32_t)__shfl((int)at, 0, 64);
                     if (big && cls == c)
@@ -1852,17 +1853,14 @@ __device__ __forceinline__ uint32_t next_colour(unsigned long long mk, uint32_t 
     return (uint32_t)__ffsll(above ? above : mk) - 1u;
 }
 
-// Before a launch, per slot: the next visit of each dynamic body, and the inbox
-// words: a body's first visit (rank 0) gets the body's solver velocity with
-// version 0, every other inbox a version no visit waits for.
-// (Thread gid of gsz; also run by the small islands' kernel, k_pgs_islands, whose bodies and
-// slots are disjoint from the large islands'.)
+// Before a launch, per slot of [s0, s1): the next visit of each dynamic body, and the inbox
+// words: a body's first visit (rank 0) gets the body's solver velocity with version 0, every
+// other inbox a version no visit waits for.  The rows exist only when this step's preparation
+// ran.  (Thread gid of gsz; also run by the small islands' kernel, k_pgs_islands, whose own
+// bodies and slots are disjoint from these.)
 __device__ __forceinline__ void flow_init_part(const Bodies& B, const SolverRows& R, const uint64_t* __restrict__ bmask,
-                                               const Counters* __restrict__ cnt, uint32_t gid, uint32_t gsz) {
-    // the rows exist only when this step's preparation ran
-    if (cnt->sticky != 0u) return;
-    const uint32_t M = cnt->m_glob;  // the large islands' slots
-    for (uint32_t s = gid; s < M; s += gsz) {
+                                               uint32_t s0, uint32_t s1, uint32_t gid, uint32_t gsz) {
+    for (uint32_t s = s0 + gid; s < s1; s += gsz) {
     const uint4 h = R.hdr[s];
     const uint2 dp = R.dep[s];
     const uint32_t c = R.colour[s];
@@ -1896,7 +1894,16 @@ __device__ __forceinline__ void flow_init_part(const Bodies& B, const SolverRows
 }
 __global__ void __launch_bounds__(256) k_flow_init(Bodies B, SolverRows R, const uint64_t* __restrict__ bmask,
                                                    const Counters* __restrict__ cnt) {
-    flow_init_part(B, R, bmask, cnt, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
+    if (cnt->sticky != 0u) return;
+    flow_init_part(B, R, bmask, 0u, cnt->m_glob, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
+}
+// Waves of the register sweep (k_pgs_flow, on G workgroups) that the islands of the largest class
+// take: all of them when they fit beside the large islands, else none (k_pgs_islands solves them).
+constexpr uint32_t FLOW_THREADS = 512, FLOW_WAVES = FLOW_THREADS / 64u;
+constexpr uint32_t FLOW_WAVE_SLOTS = 32;
+__device__ __forceinline__ uint32_t wide_waves(const Counters* cnt, uint32_t G) {
+    const uint32_t nl = (cnt->m_glob + FLOW_WAVE_SLOTS - 1u) / FLOW_WAVE_SLOTS;
+    return cnt->max_colour <= 64u && nl + cnt->isl_wide <= G * FLOW_WAVES ? cnt->isl_wide : 0u;
 }
 // Residual of one contact point: the largest velocity-space change (impulse change
 // times the row's effective mass inverse) that one more visit would make along the
@@ -2485,7 +2492,7 @@ struct IslandAcc {
 };
 // Folds a wave's results into the counters: once per wave and launch, since every atomic
 // here is on a word all waves share.
-__device__ __forceinline__ void island_flush(Counters* cnt, IslandAcc a) {
+__device__ __forceinline__ void island_flush(Counters* cnt, IslandAcc a, bool islands_kernel = true) {
     for (int o = 32; o >= 1; o >>= 1) {
         a.sweeps = max(a.sweeps, (uint32_t)__shfl_xor((int)a.sweeps, o, 64));
         a.res_bits = max(a.res_bits, (uint32_t)__shfl_xor((int)a.res_bits, o, 64));
@@ -2499,7 +2506,7 @@ __device__ __forceinline__ void island_flush(Counters* cnt, IslandAcc a) {
     if (a.miss) atomicOr(&cnt->loc_miss, 1u);
     atomicAdd(&cnt->loc_points, a.pts);
     atomicAdd(&cnt->loc_point_sweeps, a.point_sweeps);
-    atomicAdd(&cnt->bundle_point_sweeps, a.point_sweeps);
+    if (islands_kernel) atomicAdd(&cnt->bundle_point_sweeps, a.point_sweeps);
 }
 // Orders a wave's LDS accesses before and after this point (a wave's LDS operations execute
 // in order, so no wait is needed, only that the compiler moves none across).
@@ -3339,16 +3346,23 @@ k_pgs_islands(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap
               const uint32_t* __restrict__ skey, float tol, uint32_t max_sweeps, const uint64_t* __restrict__ bmask,
               uint32_t flow_init) {
     extern __shared__ __align__(16) unsigned char isl_lds[];
-    // with flow_init, the large islands' sweep launch is prepared here (as k_flow_init)
-    if (flow_init)
-        flow_init_part(B, R, bmask, cnt, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
     if (cnt->sticky != 0u) return;
     const uint32_t t = threadIdx.x, lane = t & 63u;
     // the row preparation records no first visits when there are more colours than mask bits
     const bool masks = cnt->max_colour <= 64u;
+    // with flow_init, the sweep launch that follows is prepared here: the large islands (as
+    // k_flow_init) and, when it takes them, the islands of the largest class
+    const bool wide = flow_init != 0u && wide_waves(cnt, gridDim.x) != 0u;
+    if (flow_init) {
+        const uint32_t gid = blockIdx.x * blockDim.x + t, gsz = gridDim.x * blockDim.x;
+        flow_init_part(B, R, bmask, 0u, cnt->m_glob, gid, gsz);
+        if (wide)
+            for (uint32_t i = blockIdx.x; i < cnt->isl_n[0]; i += gridDim.x)
+                flow_init_part(B, R, bmask, list[i].x, list[i].x + list[i].y, t, blockDim.x);
+    }
     IslandAcc acc = {0u, 0u, 0u, 0u, 0ull};
     GroupLds& G = *reinterpret_cast<GroupLds*>(isl_lds);
-    const uint32_t n0 = cnt->isl_n[0], n1 = cnt->isl_n[1], n2 = cnt->isl_n[2], n3 = cnt->isl_n[3], n4 = cnt->isl_n[4];
+    const uint32_t n0 = wide ? 0u : cnt->isl_n[0], n1 = cnt->isl_n[1], n2 = cnt->isl_n[2], n3 = cnt->isl_n[3], n4 = cnt->isl_n[4];
 
     // ---- islands of one workgroup each (without masks: every island of the list)
     const uint32_t n_wg = masks ? n0 + n1 : n0 + n1 + n2 + n3 + n4;
@@ -3440,12 +3454,15 @@ int pgs_islands_setup() {
 // only after the check before it has been decided, so at most one visit is ever ahead, and an
 // inbox is never overwritten before every reader of its velocity has passed (the body's next
 // round of visits includes the reader's own).
+//
+// Islands of more than 256 manifolds solved on their own run here too when all of them fit beside
+// the large ones (wide_waves): each checks and stops for itself after every sweep.  With the rows
+// read from memory by one workgroup (k_pgs_islands) an island of 1880 manifolds took 41 us per
+// sweep, here 14.9.
 // A pile of 19.1k manifolds in 18 colours: 44.5 us per sweep in k_pgs_own -> 21.8 us; with a check
 // after every sweep 66 -> 28.9 us.  Fewer slots per wave (8 or 16, so that a visit holds up fewer
 // others) change the first by less than 2 % and cost up to 5 % in arrivals; polling harder (no
 // sleep, a tight loop, two polls in flight) gains nothing or loses.
-constexpr uint32_t FLOW_THREADS = 512, FLOW_WAVES = FLOW_THREADS / 64u;
-constexpr uint32_t FLOW_WAVE_SLOTS = 32;
 __device__ __forceinline__ u32x4_t flow_quad(const uint64_t* inbox, uint32_t byte) {
     const __amdgpu_buffer_rsrc_t rs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint64_t*>(inbox), 0, 0x7FFFFFFF, 0x00020000);
@@ -3455,25 +3472,51 @@ __device__ __forceinline__ u32x4_t flow_quad(const uint64_t* inbox, uint32_t byt
 template <bool CHECKS>
 __global__ void __launch_bounds__(FLOW_THREADS, 2)
 k_pgs_flow(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap, uint32_t nsweeps, uint32_t spin_limit,
-           const uint64_t* __restrict__ bmask, SweepStop stop) {
+           const uint64_t* __restrict__ bmask, const uint2* __restrict__ list, SweepStop stop) {
     __shared__ uint32_t s_arrived, s_above, s_max;
     const uint32_t M = cnt->m_glob, G = gridDim.x;
-    if (M == 0u || M > G * FLOW_WAVES * FLOW_WAVE_SLOTS || cnt->max_colour > 64u || cnt->sticky != 0u || nsweeps == 0u)
-        return;
+    if (M > G * FLOW_WAVES * FLOW_WAVE_SLOTS || cnt->max_colour > 64u || cnt->sticky != 0u || nsweeps == 0u) return;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t nw = (M + FLOW_WAVE_SLOTS - 1u) / FLOW_WAVE_SLOTS;
-    // wave w of the grid owns slots 32 w on; neighbouring waves (the same colour) lie on
-    // different CUs
+    // wave w of the grid owns slots 32 w on of the large islands, or, from wave nl on, 32 slots of
+    // an island of the work list; neighbouring waves (the same colour) lie on different CUs
+    const uint32_t nl = (M + FLOW_WAVE_SLOTS - 1u) / FLOW_WAVE_SLOTS, nw = nl + (list ? wide_waves(cnt, G) : 0u);
     const uint32_t wid = wave * G + blockIdx.x;
     if (blockIdx.x >= nw) return;  // the whole workgroup has nothing
-    const uint32_t groups = min(G, nw);
-    const uint32_t wg_waves = (nw - blockIdx.x + G - 1u) / G;  // waves of this workgroup with slots
+    const uint32_t wg_waves = blockIdx.x < nl ? (nl - blockIdx.x + G - 1u) / G : 0u;  // with slots of the large islands
     if (threadIdx.x == 0u) s_arrived = s_above = s_max = 0u;
     __syncthreads();
     if (wid >= nw) return;
-    const uint32_t pair = lane >> 1, s = wid * FLOW_WAVE_SLOTS + pair;
-    const bool odd = (lane & 1u) != 0u, active = s < M;
-    const uint32_t every = CHECKS ? max(stop.every, 1u) : nsweeps;
+    const bool island = wid >= nl;
+    uint32_t groups = min(G, nl), s0 = wid * FLOW_WAVE_SLOTS, s1 = M;
+    unsigned long long* arrive = nullptr;  // an island's arrivals: two words, of the odd and the even check points
+    if (island) {
+        uint32_t j = wid - nl;
+        for (uint32_t i0 = 0; i0 < cnt->isl_n[0]; i0 += 64u) {
+            const uint2 e = i0 + lane < cnt->isl_n[0] ? list[i0 + lane] : make_uint2(0u, 0u);
+            const uint32_t w = (e.y + FLOW_WAVE_SLOTS - 1u) / FLOW_WAVE_SLOTS;
+            uint32_t inc = w;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const uint32_t x = (uint32_t)__shfl_up((int)inc, o, 64);
+                if (lane >= (uint32_t)o) inc += x;
+            }
+            const uint64_t past = __ballot(j < inc);
+            if (past != 0ull) {
+                const int l = __ffsll((unsigned long long)past) - 1;
+                groups = (uint32_t)__shfl((int)w, l, 64);
+                s0 = (uint32_t)__shfl((int)e.x, l, 64);
+                s1 = s0 + (uint32_t)__shfl((int)e.y, l, 64);
+                s0 += (j - ((uint32_t)__shfl((int)inc, l, 64) - groups)) * FLOW_WAVE_SLOTS;
+                arrive = stop.isl_arrive + (size_t)(i0 + (uint32_t)l) * ISL_ARRIVE_WORDS;
+                break;
+            }
+            j -= (uint32_t)__shfl((int)inc, 63, 64);
+        }
+    }
+    const uint32_t pair = lane >> 1, s = s0 + pair;
+    const bool odd = (lane & 1u) != 0u, active = s < s1;
+    // an island checks after every sweep
+    const uint32_t every = CHECKS ? (island ? 1u : max(stop.every, 1u)) : nsweeps;
     const float keep = sp.keep, tol = stop.tol;
     uint32_t* err = &cnt->sticky;
 
@@ -3535,8 +3578,22 @@ k_pgs_flow(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap, u
     uint32_t spins = 0;
     const uint64_t t_start = wall_clock64(), t_limit = (uint64_t)spin_limit * 100ull;  // wall clock: 100 MHz
     bool failed = false;
-    // whether every workgroup has arrived at check point c; then whether one is above the tolerance
+    // Whether all have arrived at check point c; then whether one is above the tolerance.  The
+    // large islands count in words of their own per check point, an island in two words for
+    // good (arrivals low, above the tolerance high): nobody reaches the check point after next
+    // before every wave has seen this one decided.
+    uint32_t above_seen[2] = {0u, 0u};
     auto arrivals = [&](uint32_t c, bool& above) -> bool {
+        if (island) {
+            const unsigned long long v =
+                __hip_atomic_load(arrive + (c & 1u) * (ISL_ARRIVE_WORDS / 2u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if ((uint32_t)v < ((c + 1u) / 2u) * groups) return false;
+            const uint32_t n = (uint32_t)(v >> 32), seen = (c & 1u) ? above_seen[1] : above_seen[0];
+            above = n != seen;
+            if (c & 1u) above_seen[1] = n;
+            else above_seen[0] = n;
+            return true;
+        }
         uint32_t* arr = stop.arrive + (size_t)(c - 1u) * CHECK_ROWS * CHECK_ROW_WORDS;
         uint32_t seen = 0;
         if (lane < CHECK_ROWS)
@@ -3619,7 +3676,7 @@ k_pgs_flow(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap, u
             }
             // the residual at the check point, after the visit that others wait for (its impulses
             // are those before that visit)
-            if (CHECKS && passed) {
+            if ((CHECKS || island) && passed) {
                 res = 0.0f;
 #pragma unroll
                 for (uint32_t q = 0; q < 4; ++q) {
@@ -3640,7 +3697,11 @@ k_pgs_flow(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap, u
                     arrived = next;
                     uint32_t bits = active ? __float_as_uint(res) : 0u;
                     for (int o = 32; o >= 1; o >>= 1) bits = max(bits, (uint32_t)__shfl_xor((int)bits, o, 64));
-                    if (lane == 0u) {
+                    if (lane == 0u && island) {
+                        const bool up = !(__uint_as_float(bits) <= tol);
+                        __hip_atomic_fetch_add(arrive + (next & 1u) * (ISL_ARRIVE_WORDS / 2u), up ? (1ull << 32) + 1ull : 1ull,
+                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    } else if (lane == 0u) {
                         // the last wave of the workgroup to arrive sends all; the words are free again
                         // before any wave can reach the next check point (it needs this one decided)
                         atomicMax(&s_max, bits);
@@ -3692,7 +3753,7 @@ k_pgs_flow(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap, u
     }
     if (failed) return;
     // the step's sweeps and whether they met the tolerance
-    if (CHECKS && wid == 0u) {
+    if (CHECKS && wid == 0u && !island) {
         bool hit = stop_at != UNSET;
         if (!hit) {
             bool above = true, all = false;
@@ -3711,6 +3772,11 @@ k_pgs_flow(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap, u
                                __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(&cnt->tol_hit, hit ? 1u : 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
+    }
+    if (island) {
+        IslandAcc acc = {0u, 0u, 0u, 0u, 0ull};
+        if (active && !odd) acc.add(stop_at != UNSET ? stop_at : nsweeps, res, CHECKS && !(res <= tol), np);
+        island_flush(cnt, acc, false);
     }
     if (!active) return;
     const bool back = CHECKS && stop_at != UNSET && k > stop_at;  // a visit ran ahead of the stop
@@ -4128,16 +4194,16 @@ int pgs_own_setup(uint32_t max_lds_bytes, uint32_t lds_bytes) {
 void launch_pgs_flow(const Bodies& B, const StepParams& sp, const SolverRows& R, uint32_t cap, const uint64_t* bmask,
                      uint32_t nsweeps, Counters* cnt, uint32_t spin_limit, uint32_t cus, uint32_t groups,
                      uint32_t lds_bytes, uint32_t tune, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1,
-                     const SweepStop& stop, bool inited) {
+                     const SweepStop& stop, const uint2* list) {
     if (!nsweeps) return;
-    if (!inited) hipLaunchKernelGGL(k_flow_init, grid_bounded(cap), dim3(256), 0, s, B, R, bmask, cnt);
+    if (!list) hipLaunchKernelGGL(k_flow_init, grid_bounded(cap), dim3(256), 0, s, B, R, bmask, cnt);
     if (ev0) (void)hipEventRecord(ev0, s);
     if (stop.bits)
         hipLaunchKernelGGL(k_pgs_flow<true>, dim3(cus), dim3(FLOW_THREADS), 0, s, B, sp, R, cnt, cap, nsweeps,
-                           spin_limit, bmask, stop);
+                           spin_limit, bmask, list, stop);
     else
         hipLaunchKernelGGL(k_pgs_flow<false>, dim3(cus), dim3(FLOW_THREADS), 0, s, B, sp, R, cnt, cap, nsweeps,
-                           spin_limit, bmask, stop);
+                           spin_limit, bmask, list, stop);
     hipLaunchKernelGGL(k_pgs_own, dim3(groups ? groups : 1u), dim3(OWN_WAVE), lds_bytes, s, B, sp, R, cnt, cap, nsweeps,
                        cus * FLOW_WAVES * FLOW_WAVE_SLOTS, lds_bytes / (uint32_t)sizeof(float4), spin_limit, tune, bmask,
                        stop);

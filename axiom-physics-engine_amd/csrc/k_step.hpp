@@ -151,12 +151,18 @@ void launch_mlp_apply(const SolverRows& R, const Counters* cnt, uint32_t cap, co
 // adds to row g mod CHECK_ROWS: atomics on one line queue one after another); both
 // arrays start the step at zero.  bits == nullptr means no checks.
 constexpr uint32_t CHECK_ROWS = 8, CHECK_ROW_WORDS = 32;
-// Words of a residual buffer for `cap` sweeps: the residual of each sweep, then the
-// arrival rows of a check after each sweep.
-inline uint32_t res_words(uint32_t cap) { return cap * (1u + CHECK_ROWS * CHECK_ROW_WORDS); }
+// The islands swept in the same launch count their arrivals in two 64-bit words each, 64 bytes
+// apart, ISL_ARRIVE_WORDS per island; at most ISL_ARRIVE_MAX islands (of at least nine waves
+// each on 8 waves per CU) fit, for up to 512 CUs.
+constexpr uint32_t ISL_ARRIVE_WORDS = 16, ISL_ARRIVE_MAX = 512u * 8u / 9u + 1u;
+// Words of a residual buffer for `cap` sweeps: the residual of each sweep, the arrival rows of
+// a check after each sweep, then the islands' arrival words.
+inline uint32_t res_arrive(uint32_t cap) { return (cap * (1u + CHECK_ROWS * CHECK_ROW_WORDS) + 31u) & ~31u; }
+inline uint32_t res_words(uint32_t cap) { return res_arrive(cap) + 2u * ISL_ARRIVE_WORDS * ISL_ARRIVE_MAX; }
 struct SweepStop {
     uint32_t* bits = nullptr;
     uint32_t* arrive = nullptr;
+    unsigned long long* isl_arrive = nullptr;
     float tol = -1.0f;
     uint32_t every = 1;
 };
@@ -164,12 +170,13 @@ struct SweepStop {
 // workgroups of 512 threads, all resident at once, see pgs_flow_setup); more in the staged
 // sweep: `groups` workgroups of one wave, each with `lds_bytes` of LDS for its staged rows; all
 // of them must be resident at once (see pgs_own_setup).  Events ev0 / ev1, when given, are
-// recorded around both.  With inited, the inboxes and next visits were already set up by this
-// step's launch_pgs_local.
+// recorded around both.  With the work list of the islands solved on their own, this step's
+// launch_pgs_local (with flow_init, in `cus` workgroups) has set up the inboxes and next visits
+// and left its largest islands to this launch when they fit.
 void launch_pgs_flow(const Bodies& B, const StepParams& sp, const SolverRows& R, uint32_t cap, const uint64_t* bmask,
                      uint32_t nsweeps, Counters* cnt, uint32_t spin_limit, uint32_t cus, uint32_t groups,
                      uint32_t lds_bytes, uint32_t tune, hipStream_t s, hipEvent_t ev0 = nullptr,
-                     hipEvent_t ev1 = nullptr, const SweepStop& stop = SweepStop{}, bool inited = false);
+                     hipEvent_t ev1 = nullptr, const SweepStop& stop = SweepStop{}, const uint2* list = nullptr);
 // Workgroups of the register sweep that fit on one CU (0 on error).
 int pgs_flow_setup();
 // Raises the sweep kernel's dynamic-LDS limit to max_lds_bytes and returns how many of

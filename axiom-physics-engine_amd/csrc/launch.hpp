@@ -144,9 +144,11 @@ struct Counters {
     uint32_t loc_res_bits; // the largest residual an island solved on its own ended with
     uint32_t loc_miss;     // 1: an island solved on its own stopped at the sweep cap above the tolerance
     uint32_t isl_n[ISLAND_CLASSES];  // islands of the work list per size class
+    uint32_t isl_wide;       // waves of 32 slots that the largest class would take in the register sweep
     uint32_t isl_wg_next;    // work taken from the workgroups' and from the waves' part of it,
     uint32_t isl_wave_next;  // beyond the first piece of each
     uint32_t loc_points;   // contact points of the islands solved on their own
+    uint32_t pad5;
     unsigned long long loc_point_sweeps;     // their contact points x the sweeps each island ran
     unsigned long long bundle_point_sweeps;  // the same for the islands of k_pgs_islands
     // ---- kept across steps
@@ -173,7 +175,7 @@ template <class T> inline T spread_total(const Counters& c, T SpreadRow::*f) {
     for (uint32_t k = 0; k < SPREAD; ++k) s += c.sp[k].*f;
     return s;
 }
-constexpr uint32_t COUNTERS_RESET_WORDS = 30;  // words of the first block (cleared per step)
+constexpr uint32_t COUNTERS_RESET_WORDS = 32;  // words of the first block (cleared per step)
 static_assert(offsetof(Counters, sticky) == 4 * COUNTERS_RESET_WORDS, "per-step block ends at sticky");
 enum : uint32_t {
     STICKY_PAIRS = 1u,        // pair capacity exceeded

@@ -682,6 +682,7 @@ bool sweep_checks(const axm_world_s* w, bool colour_launches, SweepStop& st) {
     if (colour_launches || !(w->desc.residual_tol > 0.0f || w->desc.record_residual)) return false;
     st.bits = w->res_bits;
     st.arrive = w->res_bits + w->res_cap;
+    st.isl_arrive = reinterpret_cast<unsigned long long*>(w->res_bits + res_arrive(w->res_cap));
     st.tol = w->desc.residual_tol > 0.0f ? w->desc.residual_tol : -1.0f;
     st.every = w->desc.record_residual ? 1u : std::max<uint32_t>(w->desc.residual_every, 1u);
     return true;
@@ -742,7 +743,8 @@ axm_status enqueue_step(axm_world_s* w, float dt, const StepOpts& o) {
         AXM_TRY(prof_event(w, nev, o.capture, e0));
         AXM_TRY(prof_event(w, nev, o.capture, e1));
         launch_pgs_flow(w->B, sp, R, rc, w->bmask, max_it, w->cnt, SWEEP_SPIN_LIMIT_US, (uint32_t)w->cu_count,
-                        w->sweep_groups, w->sweep_lds, w->sweep_tune, s, e0, e1, stop, flow_inited);
+                        w->sweep_groups, w->sweep_lds, w->sweep_tune, s, e0, e1, stop,
+                        flow_inited ? w->isl_list : nullptr);
         it = max_it;  // at most; the count the launch ran is read back with the counters
     }
     bool all_local = false;
@@ -769,7 +771,8 @@ axm_status enqueue_step(axm_world_s* w, float dt, const StepOpts& o) {
             AXM_TRY(prof_event(w, nev, o.capture, e1));
             // (one segment: the host checks a residual between segments in the per-colour launches only)
             launch_pgs_flow(w->B, sp, R, rc, w->bmask, seg, w->cnt, SWEEP_SPIN_LIMIT_US, (uint32_t)w->cu_count,
-                            w->sweep_groups, w->sweep_lds, w->sweep_tune, s, e0, e1, SweepStop{}, flow_inited);
+                            w->sweep_groups, w->sweep_lds, w->sweep_tune, s, e0, e1, SweepStop{},
+                            flow_inited ? w->isl_list : nullptr);
         }
         it += seg;
         const bool last = it == max_it;
@@ -1371,7 +1374,7 @@ axm_status axm_world_run(axm_world w, float dt, uint32_t iters, uint32_t steps, 
                                      w->bprof_ev[2 * c], w->bprof_ev[2 * c + 1]);
                 launch_pgs_flow(w->B, sp, w->R[c], w->rcap[c], w->bmask, nsw, w->cnt, SWEEP_SPIN_LIMIT_US,
                                 (uint32_t)w->cu_count, w->sweep_groups, w->sweep_lds, w->sweep_tune, w->stream, w->gprof_ev[2 * c],
-                                w->gprof_ev[2 * c + 1], checks ? stop : SweepStop{}, split);
+                                w->gprof_ev[2 * c + 1], checks ? stop : SweepStop{}, split ? w->isl_list : nullptr);
                 AXM_HIP(hipGraphLaunch(w->gpost[c], w->stream));
             } else {
                 AXM_HIP(hipGraphLaunch(w->gexec[c], w->stream));
