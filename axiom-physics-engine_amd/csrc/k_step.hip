@@ -1191,7 +1191,10 @@ __device__ __forceinline__ void sorted_keys_part(const Bodies& B, const uint32_t
                     const uint64_t in = __ballot(big && cls == c);
                     if (in == 0ull) continue;
                     uint32_t at = 0;
-                    if (c == 0u && big && cls == 0u) atomicAdd(&cnt->isl_wide, (size + 31u) / 32u);
+                    if (c == 0u && big && cls == 0u) {
+                        atomicAdd(&cnt->isl_wide, (size + 31u) / 32u);
+                        atomicMax(&cnt->isl_most, size);
+                    }
                     if (lane == 0u) at = atomicAdd(&cnt->isl_n[c], (uint32_t)__popcll(in));
                     at = (uint32_t)__shfl((int)at, 0, 64);
                     if (big && cls == c)
@@ -1897,13 +1900,20 @@ __global__ void __launch_bounds__(256) k_flow_init(Bodies B, SolverRows R, const
     if (cnt->sticky != 0u) return;
     flow_init_part(B, R, bmask, 0u, cnt->m_glob, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
 }
-// Waves of the register sweep (k_pgs_flow, on G workgroups) that the islands of the largest class
-// take: all of them when they fit beside the large islands, else none (k_pgs_islands solves them).
+// Launch shape of the register sweep (k_pgs_flow).
 constexpr uint32_t FLOW_THREADS = 512, FLOW_WAVES = FLOW_THREADS / 64u;
 constexpr uint32_t FLOW_WAVE_SLOTS = 32;
-__device__ __forceinline__ uint32_t wide_waves(const Counters* cnt, uint32_t G) {
-    const uint32_t nl = (cnt->m_glob + FLOW_WAVE_SLOTS - 1u) / FLOW_WAVE_SLOTS;
-    return cnt->max_colour <= 64u && nl + cnt->isl_wide <= G * FLOW_WAVES ? cnt->isl_wide : 0u;
+// Pieces of 32 slots of the islands of the largest class that the register sweep takes on G
+// workgroups: all of them, or none, when one workgroup per island (stream_island) is faster.
+// A sweep costs the register sweep its chain of visits (15 us at ten colours) while everything
+// fits its waves, and about 0.5 ns per slot beyond (160k slots: 80 us); one workgroup takes
+// about 25 ns per slot of its island, all islands at once on as many CUs (44 us for 1880 slots,
+// 100 us for 3950).
+__device__ __forceinline__ uint32_t wide_pieces(const Counters* cnt, uint32_t G) {
+    const uint32_t nl = (cnt->m_glob + FLOW_WAVE_SLOTS - 1u) / FLOW_WAVE_SLOTS, w = cnt->isl_wide;
+    if (cnt->max_colour > 64u) return 0u;
+    const bool fits = nl <= G * FLOW_WAVES && nl + w <= G * FLOW_WAVES;
+    return fits || (uint64_t)cnt->isl_most * 50u > (uint64_t)w * FLOW_WAVE_SLOTS ? w : 0u;
 }
 // Residual of one contact point: the largest velocity-space change (impulse change
 // times the row's effective mass inverse) that one more visit would make along the
@@ -2542,7 +2552,9 @@ __device__ __forceinline__ void block_max_sum(uint32_t& mx, uint32_t& sum, uint3
 // three row updates per contact point.  What binds is that chain, so what a sweep touches
 // stays on chip: rows and impulses in registers (a lane visits the same slot in every sweep),
 // body velocities in LDS.  Velocities and impulses go back to memory once per island.  Above
-// 256 manifolds a CU no longer holds the rows (240 B per point); they are read at each visit.
+// 256 manifolds a CU no longer holds the rows (240 B per point): those islands run across CUs in
+// the large islands' register sweep (k_pgs_flow), or, when there are too many (wide_pieces), here
+// with the rows read at each visit.
 //
 // Work is taken largest first, so that the long solves start early and the short ones fill
 // the tail.  The workgroups first share the islands of more than 64 manifolds, one island at
@@ -2562,7 +2574,7 @@ __device__ __forceinline__ void block_max_sum(uint32_t& mx, uint32_t& sum, uint3
 // velocities in memory; a kernel of its own for the smaller ones) and now: 1000 bodies at
 // residual 1e-4 (76 sweeps, largest island 154 manifolds) 1.55 -> 0.47 ms; 256 worlds at 1e-4
 // (159k manifolds, 119 sweeps) 7.2 -> 2.8 ms; 4096 worlds at ten sweeps (1.7M manifolds)
-// 11.3 -> 1.1 ms; an island of 1880 manifolds, 73 sweeps, 4.9 -> 3.2 ms.
+// 11.3 -> 1.1 ms.
 constexpr uint32_t BUNDLE_SLOTS = 56;
 static_assert(BUNDLE_SLOTS + ISLAND_LANE_MAX - 1u <= 64u, "a bundle fits one wave");
 // LDS of a wave's own work
@@ -2574,7 +2586,7 @@ struct WaveLds {
     uint32_t pts[64];             // per island: contact points
     uint2 ab[64];
 };
-// LDS of a workgroup's island: this, then the tables, the velocities and the pool of rows
+// LDS of a workgroup's island: this, then (above 256 manifolds) the tables, then the velocities
 struct GroupLds {
     uint32_t off[66];  // first slot (island-relative) of colour >= c
     uint32_t red[2 * ISL_WAVES];
@@ -3344,7 +3356,7 @@ __device__ __forceinline__ void memory_island(const Bodies& B, const StepParams&
 __global__ void __launch_bounds__(ISL_THREADS, 2)
 k_pgs_islands(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap, const uint2* __restrict__ list,
               const uint32_t* __restrict__ skey, float tol, uint32_t max_sweeps, const uint64_t* __restrict__ bmask,
-              uint32_t flow_init) {
+              uint32_t flow_init, unsigned long long* __restrict__ isl_arrive) {
     extern __shared__ __align__(16) unsigned char isl_lds[];
     if (cnt->sticky != 0u) return;
     const uint32_t t = threadIdx.x, lane = t & 63u;
@@ -3352,13 +3364,15 @@ k_pgs_islands(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap
     const bool masks = cnt->max_colour <= 64u;
     // with flow_init, the sweep launch that follows is prepared here: the large islands (as
     // k_flow_init) and, when it takes them, the islands of the largest class
-    const bool wide = flow_init != 0u && wide_waves(cnt, gridDim.x) != 0u;
+    const bool wide = flow_init != 0u && wide_pieces(cnt, gridDim.x) != 0u;
     if (flow_init) {
         const uint32_t gid = blockIdx.x * blockDim.x + t, gsz = gridDim.x * blockDim.x;
         flow_init_part(B, R, bmask, 0u, cnt->m_glob, gid, gsz);
         if (wide)
-            for (uint32_t i = blockIdx.x; i < cnt->isl_n[0]; i += gridDim.x)
+            for (uint32_t i = blockIdx.x; i < cnt->isl_n[0]; i += gridDim.x) {
                 flow_init_part(B, R, bmask, list[i].x, list[i].x + list[i].y, t, blockDim.x);
+                if (t < 2u) isl_arrive[(size_t)i * ISL_ARRIVE_WORDS + t * (ISL_ARRIVE_WORDS / 2u)] = 0ull;
+            }
     }
     IslandAcc acc = {0u, 0u, 0u, 0u, 0ull};
     GroupLds& G = *reinterpret_cast<GroupLds*>(isl_lds);
@@ -3455,10 +3469,9 @@ int pgs_islands_setup() {
 // inbox is never overwritten before every reader of its velocity has passed (the body's next
 // round of visits includes the reader's own).
 //
-// Islands of more than 256 manifolds solved on their own run here too when all of them fit beside
-// the large ones (wide_waves): each checks and stops for itself after every sweep.  With the rows
-// read from memory by one workgroup (k_pgs_islands) an island of 1880 manifolds took 41 us per
-// sweep, here 14.9.
+// Islands of more than 256 manifolds solved on their own run here too, in as many rounds as they
+// need (wide_pieces): each checks and stops for itself after every sweep.  With the rows read
+// from memory by one workgroup an island of 1880 manifolds took 41 us per sweep, here 14.9.
 // A pile of 19.1k manifolds in 18 colours: 44.5 us per sweep in k_pgs_own -> 21.8 us; with a check
 // after every sweep 66 -> 28.9 us.  Fewer slots per wave (8 or 16, so that a visit holds up fewer
 // others) change the first by less than 2 % and cost up to 5 % in arrivals; polling harder (no
@@ -3474,23 +3487,29 @@ __global__ void __launch_bounds__(FLOW_THREADS, 2)
 k_pgs_flow(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap, uint32_t nsweeps, uint32_t spin_limit,
            const uint64_t* __restrict__ bmask, const uint2* __restrict__ list, SweepStop stop) {
     __shared__ uint32_t s_arrived, s_above, s_max;
-    const uint32_t M = cnt->m_glob, G = gridDim.x;
-    if (M > G * FLOW_WAVES * FLOW_WAVE_SLOTS || cnt->max_colour > 64u || cnt->sticky != 0u || nsweeps == 0u) return;
+    const uint32_t G = gridDim.x, C = G * FLOW_WAVES;
+    if (cnt->max_colour > 64u || cnt->sticky != 0u || nsweeps == 0u) return;
+    const uint32_t M = cnt->m_glob <= C * FLOW_WAVE_SLOTS ? cnt->m_glob : 0u;  // more: k_pgs_own
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    // wave w of the grid owns slots 32 w on of the large islands, or, from wave nl on, 32 slots of
-    // an island of the work list; neighbouring waves (the same colour) lie on different CUs
-    const uint32_t nl = (M + FLOW_WAVE_SLOTS - 1u) / FLOW_WAVE_SLOTS, nw = nl + (list ? wide_waves(cnt, G) : 0u);
+    // Piece v is slots 32 v on of the large islands, or, from piece nl on, 32 slots of an island
+    // of the work list.  Wave w works on pieces w, w + C, ... in turn (C: the waves of the grid;
+    // the large islands are in the first round).  An island's pieces wait only for each other,
+    // and every wave comes to them through pieces of earlier islands, so none waits for ever.
+    // Neighbouring waves (the same colour) lie on different CUs.
+    const uint32_t nl = (M + FLOW_WAVE_SLOTS - 1u) / FLOW_WAVE_SLOTS, nw = nl + (list ? wide_pieces(cnt, G) : 0u);
     const uint32_t wid = wave * G + blockIdx.x;
     if (blockIdx.x >= nw) return;  // the whole workgroup has nothing
     const uint32_t wg_waves = blockIdx.x < nl ? (nl - blockIdx.x + G - 1u) / G : 0u;  // with slots of the large islands
     if (threadIdx.x == 0u) s_arrived = s_above = s_max = 0u;
     __syncthreads();
-    if (wid >= nw) return;
-    const bool island = wid >= nl;
-    uint32_t groups = min(G, nl), s0 = wid * FLOW_WAVE_SLOTS, s1 = M;
+    for (uint32_t v = wid; v < nw; v += C) {
+    // opaque per round, so that no row address is kept in registers through a solve for the next
+    asm volatile("" : "+s"(cap));
+    const bool island = v >= nl;
+    uint32_t groups = min(G, nl), s0 = v * FLOW_WAVE_SLOTS, s1 = M;
     unsigned long long* arrive = nullptr;  // an island's arrivals: two words, of the odd and the even check points
     if (island) {
-        uint32_t j = wid - nl;
+        uint32_t j = v - nl;
         for (uint32_t i0 = 0; i0 < cnt->isl_n[0]; i0 += 64u) {
             const uint2 e = i0 + lane < cnt->isl_n[0] ? list[i0 + lane] : make_uint2(0u, 0u);
             const uint32_t w = (e.y + FLOW_WAVE_SLOTS - 1u) / FLOW_WAVE_SLOTS;
@@ -3753,7 +3772,7 @@ k_pgs_flow(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap, u
     }
     if (failed) return;
     // the step's sweeps and whether they met the tolerance
-    if (CHECKS && wid == 0u && !island) {
+    if (CHECKS && v == 0u && !island) {
         bool hit = stop_at != UNSET;
         if (!hit) {
             bool above = true, all = false;
@@ -3778,7 +3797,7 @@ k_pgs_flow(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap, u
         if (active && !odd) acc.add(stop_at != UNSET ? stop_at : nsweeps, res, CHECKS && !(res <= tol), np);
         island_flush(cnt, acc, false);
     }
-    if (!active) return;
+    if (!active) continue;
     const bool back = CHECKS && stop_at != UNSET && k > stop_at;  // a visit ran ahead of the stop
     if (!odd) {
 #pragma unroll
@@ -3790,6 +3809,7 @@ k_pgs_flow(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap, u
     if (dyn && rank == 0u) {
         B.sv[body] = f4(F.v, X.im);
         B.sw[body] = f4(F.w, 0.0f);
+    }
     }
 }
 int pgs_flow_setup() {
@@ -4131,11 +4151,12 @@ void launch_col_sort_input(const Bodies& B, const uint2* m_ab, const uint32_t* c
 }
 void launch_pgs_local(const Bodies& B, const StepParams& sp, const SolverRows& R, Counters* cnt, uint32_t cap,
                       const uint32_t* skey, uint2* list, float tol, uint32_t max_sweeps, uint32_t groups,
-                      hipStream_t s, const uint64_t* bmask, bool flow_init, hipEvent_t ev0, hipEvent_t ev1) {
+                      hipStream_t s, const uint64_t* bmask, bool flow_init, unsigned long long* isl_arrive,
+                      hipEvent_t ev0, hipEvent_t ev1) {
     if (max_sweeps == 0u) return;
     if (ev0) (void)hipEventRecord(ev0, s);
     hipLaunchKernelGGL(k_pgs_islands, dim3(groups), dim3(ISL_THREADS), ISL_LDS_BYTES, s, B, sp, R, cnt, cap, list, skey,
-                       tol, max_sweeps, bmask, flow_init ? 1u : 0u);
+                       tol, max_sweeps, bmask, flow_init ? 1u : 0u, isl_arrive);
     if (ev1) (void)hipEventRecord(ev1, s);
 }
 void launch_prep(const Bodies& B, const StepParams& sp, const uint32_t* order, uint32_t cap, const uint2* m_ab,

@@ -110,12 +110,12 @@ void launch_col_sort_input(const Bodies& B, const uint2* m_ab, const uint32_t* c
 // The islands solved on their own (after the row preparation, which built their work list),
 // in `groups` workgroups (one per CU): tol > 0 stops each at its own residual.  bmask holds
 // the colouring's per-body colour masks.  With flow_init, the same launch also sets up the
-// large islands' sweep (as launch_pgs_flow does unless told it is inited).  Events ev0 / ev1,
-// when given, are recorded around it.
+// launch_pgs_flow that follows, which then solves the list's largest class too (isl_arrive: its
+// arrival words).  Events ev0 / ev1, when given, are recorded around it.
 void launch_pgs_local(const Bodies& B, const StepParams& sp, const SolverRows& R, Counters* cnt, uint32_t cap,
                       const uint32_t* skey, uint2* list, float tol, uint32_t max_sweeps, uint32_t groups,
-                      hipStream_t s, const uint64_t* bmask, bool flow_init, hipEvent_t ev0 = nullptr,
-                      hipEvent_t ev1 = nullptr);
+                      hipStream_t s, const uint64_t* bmask, bool flow_init, unsigned long long* isl_arrive,
+                      hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
 // Work the row preparation launch also does for the launches after it, each in a loop of
 // its own over the grid: the colour offsets of the sorted keys skey (col_off[c] = first
 // position whose key has colour >= c, c = 0..K, and m_glob = col_off[K], when col_off is
@@ -152,13 +152,13 @@ void launch_mlp_apply(const SolverRows& R, const Counters* cnt, uint32_t cap, co
 // arrays start the step at zero.  bits == nullptr means no checks.
 constexpr uint32_t CHECK_ROWS = 8, CHECK_ROW_WORDS = 32;
 // The islands swept in the same launch count their arrivals in two 64-bit words each, 64 bytes
-// apart, ISL_ARRIVE_WORDS per island; at most ISL_ARRIVE_MAX islands (of at least nine waves
-// each on 8 waves per CU) fit, for up to 512 CUs.
-constexpr uint32_t ISL_ARRIVE_WORDS = 16, ISL_ARRIVE_MAX = 512u * 8u / 9u + 1u;
-// Words of a residual buffer for `cap` sweeps: the residual of each sweep, the arrival rows of
-// a check after each sweep, then the islands' arrival words.
-inline uint32_t res_arrive(uint32_t cap) { return (cap * (1u + CHECK_ROWS * CHECK_ROW_WORDS) + 31u) & ~31u; }
-inline uint32_t res_words(uint32_t cap) { return res_arrive(cap) + 2u * ISL_ARRIVE_WORDS * ISL_ARRIVE_MAX; }
+// apart, ISL_ARRIVE_WORDS per island of the work list's largest class (launch_pgs_local clears
+// them): isl_arrive_words for a manifold capacity.
+constexpr uint32_t ISL_ARRIVE_WORDS = 16;
+inline size_t isl_arrive_words(uint32_t cap_man) { return (size_t)ISL_ARRIVE_WORDS * (cap_man / 257u + 1u); }
+// Words of a residual buffer for `cap` sweeps: the residual of each sweep, then the
+// arrival rows of a check after each sweep.
+inline uint32_t res_words(uint32_t cap) { return cap * (1u + CHECK_ROWS * CHECK_ROW_WORDS); }
 struct SweepStop {
     uint32_t* bits = nullptr;
     uint32_t* arrive = nullptr;
@@ -171,8 +171,8 @@ struct SweepStop {
 // sweep: `groups` workgroups of one wave, each with `lds_bytes` of LDS for its staged rows; all
 // of them must be resident at once (see pgs_own_setup).  Events ev0 / ev1, when given, are
 // recorded around both.  With the work list of the islands solved on their own, this step's
-// launch_pgs_local (with flow_init, in `cus` workgroups) has set up the inboxes and next visits
-// and left its largest islands to this launch when they fit.
+// launch_pgs_local (with flow_init) has set up the inboxes and next visits and left the islands
+// of the largest class to this launch.
 void launch_pgs_flow(const Bodies& B, const StepParams& sp, const SolverRows& R, uint32_t cap, const uint64_t* bmask,
                      uint32_t nsweeps, Counters* cnt, uint32_t spin_limit, uint32_t cus, uint32_t groups,
                      uint32_t lds_bytes, uint32_t tune, hipStream_t s, hipEvent_t ev0 = nullptr,

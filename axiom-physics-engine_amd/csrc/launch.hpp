@@ -144,11 +144,11 @@ struct Counters {
     uint32_t loc_res_bits; // the largest residual an island solved on its own ended with
     uint32_t loc_miss;     // 1: an island solved on its own stopped at the sweep cap above the tolerance
     uint32_t isl_n[ISLAND_CLASSES];  // islands of the work list per size class
-    uint32_t isl_wide;       // waves of 32 slots that the largest class would take in the register sweep
+    uint32_t isl_wide;       // pieces of 32 slots of the largest class's islands, and its largest island
+    uint32_t isl_most;
     uint32_t isl_wg_next;    // work taken from the workgroups' and from the waves' part of it,
     uint32_t isl_wave_next;  // beyond the first piece of each
     uint32_t loc_points;   // contact points of the islands solved on their own
-    uint32_t pad5;
     unsigned long long loc_point_sweeps;     // their contact points x the sweeps each island ran
     unsigned long long bundle_point_sweeps;  // the same for the islands of k_pgs_islands
     // ---- kept across steps

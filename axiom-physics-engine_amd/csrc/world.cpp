@@ -137,6 +137,7 @@ struct axm_world_s {
     uint64_t *prio = nullptr, *bmax0 = nullptr, *bmax1 = nullptr, *bmask = nullptr;
     uint32_t *ckey = nullptr, *ckey_alt = nullptr, *cval = nullptr, *cval_alt = nullptr, *csort_tmp = nullptr;
     uint2* isl_list = nullptr;  // the small islands' work lists (first slot, manifolds)
+    unsigned long long* isl_arrive = nullptr;  // arrival words of those in the register sweep
     const uint32_t* solve_order = nullptr;  // the sort output holding the last step's solve order
     uint32_t* col_off = nullptr;
     uint32_t* bdone = nullptr;
@@ -448,6 +449,7 @@ axm_status alloc_manifolds(axm_world_s* w, uint32_t cap) {
     w->mem.release(w->cval_alt);
     w->mem.release(w->csort_tmp);
     w->mem.release(w->isl_list);
+    w->mem.release(w->isl_arrive);
     AXM_TRY(w->mem.get(w->m_ab, cap));
     AXM_TRY(w->mem.get(w->m_np, cap));
     AXM_TRY(w->mem.get(w->c_pt, (size_t)cap * 4));
@@ -461,6 +463,7 @@ axm_status alloc_manifolds(axm_world_s* w, uint32_t cap) {
     AXM_TRY(w->mem.get(w->cval_alt, cap));
     AXM_TRY(w->mem.get(w->csort_tmp, radix_tmp_words(cap)));
     AXM_TRY(w->mem.get(w->isl_list, cap));
+    AXM_TRY(w->mem.get(w->isl_arrive, isl_arrive_words(cap)));
     if (hipMemset(w->csort_tmp, 0, 4 * radix_tmp_words(cap)) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
     w->cap_man = cap;
     if (w->rcap[w->cur] < cap) AXM_TRY(alloc_rows(w, w->cur, cap));
@@ -682,7 +685,7 @@ bool sweep_checks(const axm_world_s* w, bool colour_launches, SweepStop& st) {
     if (colour_launches || !(w->desc.residual_tol > 0.0f || w->desc.record_residual)) return false;
     st.bits = w->res_bits;
     st.arrive = w->res_bits + w->res_cap;
-    st.isl_arrive = reinterpret_cast<unsigned long long*>(w->res_bits + res_arrive(w->res_cap));
+    st.isl_arrive = w->isl_arrive;
     st.tol = w->desc.residual_tol > 0.0f ? w->desc.residual_tol : -1.0f;
     st.every = w->desc.record_residual ? 1u : std::max<uint32_t>(w->desc.residual_every, 1u);
     return true;
@@ -722,7 +725,7 @@ axm_status enqueue_step(axm_world_s* w, float dt, const StepOpts& o) {
             b1 = w->bprof_ev[1];
         }
         launch_pgs_local(w->B, sp, R, w->cnt, rc, w->solve_keys, w->isl_list, w->desc.residual_tol, max_it,
-                         (uint32_t)w->cu_count, s, w->bmask, flow_inited, b0, b1);
+                         (uint32_t)w->cu_count, s, w->bmask, flow_inited, w->isl_arrive, b0, b1);
     }
     const bool want_res = (o.flags & AXM_STEP_RESIDUAL) || w->desc.record_residual || tol_mode;
     const uint32_t every = std::max<uint32_t>(w->desc.residual_every, 1u);
@@ -1371,7 +1374,7 @@ axm_status axm_world_run(axm_world w, float dt, uint32_t iters, uint32_t steps, 
                 if (split)
                     launch_pgs_local(w->B, sp, w->R[c], w->cnt, w->rcap[c], w->solve_keys, w->isl_list,
                                      w->desc.residual_tol, nsw, (uint32_t)w->cu_count, w->stream, w->bmask, true,
-                                     w->bprof_ev[2 * c], w->bprof_ev[2 * c + 1]);
+                                     w->isl_arrive, w->bprof_ev[2 * c], w->bprof_ev[2 * c + 1]);
                 launch_pgs_flow(w->B, sp, w->R[c], w->rcap[c], w->bmask, nsw, w->cnt, SWEEP_SPIN_LIMIT_US,
                                 (uint32_t)w->cu_count, w->sweep_groups, w->sweep_lds, w->sweep_tune, w->stream, w->gprof_ev[2 * c],
                                 w->gprof_ev[2 * c + 1], checks ? stop : SweepStop{}, split ? w->isl_list : nullptr);

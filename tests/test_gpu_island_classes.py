@@ -1,7 +1,8 @@
 """The small islands' kernel at the edges of its size classes, through the C ABI: islands of at
 most 8 manifolds share waves by window, those up to 16, 32 and 64 take blocks of a wave's lanes,
-up to 256 a workgroup with two lanes per manifold, up to 4096 a workgroup with the rows in
-memory; above that the large islands' sweep takes over.
+up to 256 a workgroup with two lanes per manifold, up to 4096 the large islands' register sweep
+or, when they are many, a workgroup with the rows in memory; above that the large islands'
+sweep takes over.
 
 Bar: with a fixed sweep count the split into islands changes no result (islands share no dynamic
 body and every body sees the same visits in the same order), so positions, rotations, velocities
@@ -75,6 +76,8 @@ def _run(axm, b, split, sweeps, steps):
     [64, 65, 128, 255, 256, 257],
     [255, 257, 511, 512, 513, 1025],
     [4095, 4096, 4097],
+    [3900] * 18,  # the largest class in several rounds of the register sweep
+    [300] * 230,  # and one workgroup per island
 ])
 def test_island_classes_equal_the_joint_sweep(axm, gpu, sizes, boxes):
     b = _scene(axm, sizes, 17 + len(sizes), boxes)
