@@ -25,6 +25,7 @@
 
 #include "axiom/axm.h"
 #include "file_io.hpp"
+#include "k_bodies.hpp"
 #include "k_step.hpp"
 #include "mlp_impl.hpp"
 
@@ -91,6 +92,7 @@ struct axm_world_s {
     hipStream_t stream = nullptr;
     Alloc mem;
     uint32_t n = 0, cap_n = 0, cap_pairs = 0, cap_man = 0, n_worlds = 1;
+    uint32_t cap_first = 0;  // entries of B.world_first: world ids may have gaps
     float cell = 1.0f;
     int cu_count = 256;
     uint32_t colour_blocks = 256;
@@ -158,6 +160,14 @@ struct axm_world_s {
     Counters* cnt = nullptr;
     Counters* h_cnt = nullptr;
 
+    // body sets on their way to and from the host: device copies in the host's layout, and pinned
+    // memory the transfers go through (at most STAGE_BYTES)
+    uint8_t* dstage = nullptr;
+    size_t dstage_cap = 0;
+    uint8_t* hstage = nullptr;
+    size_t hstage_cap = 0;
+    hipEvent_t stage_ev[2] = {nullptr, nullptr};
+
     // kernel profiling
     bool prof_on = false;
     std::vector<hipEvent_t> prof_ev;
@@ -199,6 +209,9 @@ struct axm_world_s {
             if (e) (void)hipEventDestroy(e);
         mem.release_all();
         if (h_cnt) (void)hipHostFree(h_cnt);
+        if (hstage) (void)hipHostFree(hstage);
+        for (hipEvent_t e : stage_ev)
+            if (e) (void)hipEventDestroy(e);
         if (stream) (void)hipStreamDestroy(stream);
     }
 };
@@ -222,7 +235,6 @@ void free_bodies(axm_world_s* w) {
     w->mem.release(B.wake);
     w->mem.release(B.icnt);
     w->mem.release(B.world);
-    w->mem.release(B.world_first);
     w->mem.release(w->key);
     w->mem.release(w->key_alt);
     w->mem.release(w->val);
@@ -260,7 +272,6 @@ axm_status alloc_bodies(axm_world_s* w, uint32_t cap) {
     AXM_TRY(w->mem.get(B.wake, cap));
     AXM_TRY(w->mem.get(B.icnt, cap));
     AXM_TRY(w->mem.get(B.world, cap));
-    AXM_TRY(w->mem.get(B.world_first, cap + 1));
     AXM_TRY(w->mem.get(w->key, cap));
     AXM_TRY(w->mem.get(w->key_alt, cap));
     AXM_TRY(w->mem.get(w->val, cap));
@@ -1103,7 +1114,85 @@ struct HostBodies {
     std::vector<uint32_t> wake;
 };
 axm_status install_bodies(axm_world_s* w, uint32_t n, uint32_t nw, float cell, bool use_filter,
-                          const HostBodies& hb, bool keep_graphs = false);
+                          const HostBodies* hb, const BodyIn* in, bool keep_graphs);
+
+// Pinned memory a world keeps for its body transfers: large sets go through it in two halves,
+// one on the link while the host copies the other.  Pinned memory moves 57 GB/s here, pageable
+// memory 17 GB/s down and 29 GB/s up (and a small copy takes 36 us instead of 13), so a set is
+// bound by the host's own copy to or from the block.  Step and readback of 4096 worlds of 762
+// bodies: 41 ms with pageable copies and the conversion on the host, 21 ms so.
+constexpr size_t STAGE_BYTES = 8u << 20;
+
+// Device and pinned staging for `bytes` of a body set.
+axm_status ensure_stage(axm_world_s* w, size_t bytes) {
+    if (w->dstage_cap < bytes) {
+        w->mem.release(w->dstage);
+        w->dstage_cap = 0;
+        AXM_TRY(w->mem.get(w->dstage, bytes));
+        w->dstage_cap = bytes;
+    }
+    const size_t want = std::min(bytes, STAGE_BYTES);
+    if (w->hstage_cap < want) {
+        if (w->hstage) (void)hipHostFree(w->hstage);
+        w->hstage = nullptr;
+        w->hstage_cap = 0;
+        if (hipHostMalloc((void**)&w->hstage, want, hipHostMallocDefault) != hipSuccess) return AXM_BUFFER_ALLOCATION_FAILED;
+        w->hstage_cap = want;
+    }
+    for (hipEvent_t& e : w->stage_ev)
+        if (!e) AXM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    return AXM_SUCCESS;
+}
+
+// One host array's place in the staging.
+struct StagePart {
+    void* host;
+    size_t off, bytes;
+};
+// Copies the part of the staging range [lo, hi) between the arrays and `buf` (which holds it).
+void stage_copy(const StagePart* part, int parts, size_t lo, size_t hi, uint8_t* buf, bool out) {
+    for (int k = 0; k < parts; ++k) {
+        const size_t a = std::max(lo, part[k].off), b = std::min(hi, part[k].off + part[k].bytes);
+        if (a >= b) continue;
+        uint8_t* h = static_cast<uint8_t*>(part[k].host) + (a - part[k].off);
+        if (out) std::memcpy(h, buf + (a - lo), b - a);
+        else std::memcpy(buf + (a - lo), h, b - a);
+    }
+}
+// Moves `total` bytes of the staging to the arrays or from them, on the world's stream; on
+// return the arrays are free (upload) or filled (download).
+axm_status stage_move(axm_world_s* w, const StagePart* part, int parts, size_t total, bool out) {
+    hipStream_t s = w->stream;
+    const size_t piece = total <= w->hstage_cap ? total : w->hstage_cap / 2;
+    const size_t pieces = (total + piece - 1) / piece;
+    auto range = [&](size_t k, size_t& lo, size_t& hi) {
+        lo = k * piece;
+        hi = std::min(total, lo + piece);
+    };
+    for (size_t k = 0; k < pieces + (out ? 1 : 0); ++k) {
+        size_t lo, hi;
+        if (!out) {
+            range(k, lo, hi);
+            uint8_t* buf = w->hstage + (k & 1) * piece;
+            if (k >= 2) AXM_HIP(hipEventSynchronize(w->stage_ev[k & 1]));  // the piece before in this half
+            stage_copy(part, parts, lo, hi, buf, false);
+            AXM_HIP(hipMemcpyAsync(w->dstage + lo, buf, hi - lo, hipMemcpyHostToDevice, s));
+            AXM_HIP(hipEventRecord(w->stage_ev[k & 1], s));
+            continue;
+        }
+        if (k < pieces) {
+            range(k, lo, hi);
+            AXM_HIP(hipMemcpyAsync(w->hstage + (k & 1) * piece, w->dstage + lo, hi - lo, hipMemcpyDeviceToHost, s));
+            AXM_HIP(hipEventRecord(w->stage_ev[k & 1], s));
+        }
+        if (k > 0) {
+            range(k - 1, lo, hi);
+            AXM_HIP(hipEventSynchronize(w->stage_ev[(k - 1) & 1]));
+            stage_copy(part, parts, lo, hi, w->hstage + ((k - 1) & 1) * piece, true);
+        }
+    }
+    return AXM_SUCCESS;
+}
 
 axm_status axm_world_set_bodies(axm_world w, const axm_body_soa* b, uint32_t n) {
     if (!w || !b) return AXM_NULL_POINTER;
@@ -1112,81 +1201,58 @@ axm_status axm_world_set_bodies(axm_world w, const axm_body_soa* b, uint32_t n) 
         return AXM_NULL_POINTER;
     if (n >= (1u << 29)) return AXM_OUT_OF_RANGE;
     (void)hipSetDevice(w->desc.device);
-    std::vector<float4> x(n), q(n), v(n), av(n), ii(n), sh(n), mat(n);
-    std::vector<uint4> bfl(n);
-    std::vector<uint32_t> wd(n);
-    const axm_world_desc& D = w->desc;
+    BodyIn in{};
     float rmax = 0.0f;
     uint32_t nw = 0;
-    for (uint32_t i = 0; i < n; ++i) {
-        const float* p = b->pos + 3 * i;
-        const float* qq = b->quat + 4 * i;
-        const float* lv = b->lin_vel + 3 * i;
-        const float* aw = b->ang_vel + 3 * i;
-        const float* iv = b->inv_inertia + 3 * i;
-        const float* pr = b->shape_params + 3 * i;
-        const float im = b->inv_mass[i];
-        const uint32_t t = b->shape_type[i];
-        if (!finite3(p) || !finite3(lv) || !finite3(aw) || !finite3(iv) || !std::isfinite(im) || im < 0.0f ||
-            !std::isfinite(qq[0]) || !std::isfinite(qq[1]) || !std::isfinite(qq[2]) || !std::isfinite(qq[3]) ||
-            iv[0] < 0.0f || iv[1] < 0.0f || iv[2] < 0.0f)
-            return AXM_INVALID_RIGID_BODY;
-        const float ql = qq[0] * qq[0] + qq[1] * qq[1] + qq[2] * qq[2] + qq[3] * qq[3];
-        if (!(ql > 0.5f && ql < 1.5f)) return AXM_INVALID_RIGID_BODY;
-        if (t > AXM_SHAPE_CAPSULE || !finite3(pr)) return AXM_INVALID_SHAPE;
-        float br;
-        if (t == AXM_SHAPE_SPHERE) {
-            if (!(pr[0] > 0.0f)) return AXM_INVALID_SHAPE;
-            br = pr[0];
-        } else if (t == AXM_SHAPE_BOX) {
-            if (!(pr[0] > 0.0f && pr[1] > 0.0f && pr[2] > 0.0f)) return AXM_INVALID_SHAPE;
-            br = std::sqrt(pr[0] * pr[0] + pr[1] * pr[1] + pr[2] * pr[2]);
-        } else {
-            if (!(pr[0] > 0.0f && pr[1] >= 0.0f)) return AXM_INVALID_SHAPE;
-            br = pr[0] + pr[1];
+    if (n) {
+        // the arrays as they are, then the check's result
+        StagePart part[13];
+        int parts = 0;
+        size_t off = 0;
+        auto add = [&](const void* p, size_t words) -> size_t {
+            const size_t at = off;
+            part[parts++] = StagePart{const_cast<void*>(p), at, 4u * words * n};
+            off += (4u * words * n + 15u) / 16u * 16u;
+            return at;
+        };
+        const size_t pos = add(b->pos, 3), quat = add(b->quat, 4), lin = add(b->lin_vel, 3), ang = add(b->ang_vel, 3),
+                     mass = add(b->inv_mass, 1), inertia = add(b->inv_inertia, 3), type = add(b->shape_type, 1),
+                     params = add(b->shape_params, 3);
+        const size_t world = b->world ? add(b->world, 1) : 0, material = b->material ? add(b->material, 4) : 0,
+                     flags = b->flags ? add(b->flags, 1) : 0, filter = b->filter ? add(b->filter, 3) : 0;
+        BodyCheck check{~0ull, 0u, 0u};
+        const size_t at = off;
+        part[parts++] = StagePart{&check, at, sizeof(check)};
+        const size_t total = at + sizeof(check);
+        AXM_TRY(ensure_stage(w, total));
+        AXM_TRY(stage_move(w, part, parts, total, false));
+        auto f = [&](size_t o) { return reinterpret_cast<const float*>(w->dstage + o); };
+        auto u = [&](size_t o) { return reinterpret_cast<const uint32_t*>(w->dstage + o); };
+        in = BodyIn{f(pos), f(quat), f(lin), f(ang), f(mass), f(inertia), f(params), u(type),
+                    b->world ? u(world) : nullptr, b->material ? f(material) : nullptr, b->flags ? u(flags) : nullptr,
+                    b->filter ? u(filter) : nullptr};
+        BodyCheck* d_check = reinterpret_cast<BodyCheck*>(w->dstage + at);
+        launch_bodies_check(in, n, d_check, w->stream);
+        AXM_HIP(hipMemcpyAsync(w->hstage, d_check, sizeof(check), hipMemcpyDeviceToHost, w->stream));
+        AXM_HIP(hipStreamSynchronize(w->stream));
+        std::memcpy(&check, w->hstage, sizeof(check));
+        if (check.fault != ~0ull) {
+            const uint32_t fault = (uint32_t)check.fault;
+            return fault == BODY_BAD_SHAPE   ? AXM_INVALID_SHAPE
+                   : fault == BODY_BAD_WORLD ? AXM_INVALID_PARAMETER
+                                             : AXM_INVALID_RIGID_BODY;
         }
-        rmax = std::max(rmax, br);
-        const uint32_t wi = b->world ? b->world[i] : 0u;
-        if (i > 0 && wi < wd[i - 1]) return AXM_INVALID_PARAMETER;  // worlds must be contiguous
-        wd[i] = wi;
-        nw = std::max(nw, wi + 1);
-        const bool stat = im == 0.0f;
-        x[i] = make_float4(p[0], p[1], p[2], 0.0f);
-        q[i] = make_float4(qq[0], qq[1], qq[2], qq[3]);
-        v[i] = make_float4(lv[0], lv[1], lv[2], im);
-        av[i] = make_float4(aw[0], aw[1], aw[2], 0.0f);
-        ii[i] = stat ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : make_float4(iv[0], iv[1], iv[2], 0.0f);
-        uint32_t tb = t;
-        float tf;
-        std::memcpy(&tf, &tb, 4);
-        sh[i] = make_float4(pr[0], pr[1], pr[2], tf);
-        float mu = D.friction, e = D.restitution, ld = D.lin_damp, ad = D.ang_damp;
-        if (b->material) {
-            const float* mt = b->material + 4 * i;
-            if (!std::isfinite(mt[0]) || mt[0] < 0.0f || !std::isfinite(mt[1]) || mt[1] < 0.0f ||
-                !std::isfinite(mt[2]) || !std::isfinite(mt[3]))
-                return AXM_INVALID_RIGID_BODY;
-            mu = mt[0];
-            e = mt[1];
-            ld = mt[2];
-            ad = mt[3];
-        }
-        mat[i] = make_float4(mu, e, 1.0f - ld, 1.0f - ad);
-        const uint32_t fl = b->flags ? b->flags[i] : 0u;
-        if ((fl & BODY_KINEMATIC) && im != 0.0f) return AXM_INVALID_RIGID_BODY;  // kinematic bodies have no mass
-        bfl[i] = b->filter ? make_uint4(fl, b->filter[3 * i], b->filter[3 * i + 1], b->filter[3 * i + 2])
-                           : make_uint4(fl, 1u, 0xFFFFFFFFu, 0u);
+        std::memcpy(&rmax, &check.radius_bits, 4);
+        nw = check.worlds;
     }
     if (nw > (1u << 22)) return AXM_OUT_OF_RANGE;
-    std::vector<uint32_t> first(nw + 1, 0);
-    for (uint32_t i = n; i-- > 0;) first[wd[i]] = i;
     const float need = 2.0f * (rmax + w->desc.margin);
     float cell = w->desc.cell_size;
     if (cell == 0.0f) cell = need > 0.0f ? need : 1.0f;
     if (cell < need) return AXM_INVALID_PARAMETER;
-    HostBodies hb{std::move(x), std::move(q), std::move(v), std::move(av), std::move(ii), std::move(sh),
-                  std::move(mat), std::move(bfl), std::move(wd), std::move(first), {}, {}};
-    return install_bodies(w, n, std::max(nw, 1u), cell, b->filter != nullptr, hb);
+    // the captured steps hold the body count, the worlds, the cell and whether there are filters
+    const bool same = n == w->n && std::max(nw, 1u) == w->n_worlds && cell == w->cell && (b->filter != nullptr) == w->use_filter;
+    return install_bodies(w, n, std::max(nw, 1u), cell, b->filter != nullptr, nullptr, &in, same);
 }
 
 
@@ -1195,39 +1261,41 @@ axm_status axm_world_set_bodies(axm_world w, const axm_body_soa* b, uint32_t n) 
 // nothing they hold changes: description, body count, worlds, cell, filters) unless a buffer
 // has to grow.
 axm_status install_bodies(axm_world_s* w, uint32_t n, uint32_t nw, float cell, bool use_filter,
-                          const HostBodies& hb, bool keep_graphs) {
-    const std::vector<float4>&x = hb.x, &q = hb.q, &v = hb.v, &av = hb.av, &ii = hb.ii, &sh = hb.sh, &mat = hb.mat;
-    const std::vector<uint4>& bfl = hb.bfl;
-    const std::vector<uint32_t>&wd = hb.wd, &first = hb.first;
+                          const HostBodies* hb, const BodyIn* in, bool keep_graphs) {
     AXM_HIP(hipStreamSynchronize(w->stream));
     const bool grow = n > w->cap_n || (w->desc.max_pairs == 0 && w->cap_pairs < 8ull * n) ||
-                      (w->desc.max_manifolds == 0 && w->cap_man < 4ull * n) || w->rcap[1 - w->cur] < w->cap_man;
+                      (w->desc.max_manifolds == 0 && w->cap_man < 4ull * n) || w->rcap[1 - w->cur] < w->cap_man ||
+                      w->cap_first <= nw;
     if (!keep_graphs || grow) w->drop_graphs();
     if (n > w->cap_n) AXM_TRY(alloc_bodies(w, n));
+    if (w->cap_first <= nw) {
+        w->mem.release(w->B.world_first);
+        w->cap_first = 0;
+        AXM_TRY(w->mem.get(w->B.world_first, nw + 1));
+        w->cap_first = nw + 1;
+    }
     if (w->desc.max_pairs == 0 && w->cap_pairs < 8ull * n) AXM_TRY(alloc_pairs(w, 8 * n));
     if (w->desc.max_manifolds == 0 && w->cap_man < 4ull * n) AXM_TRY(alloc_manifolds(w, 4 * n));
     if (w->rcap[1 - w->cur] < w->cap_man) AXM_TRY(alloc_rows(w, 1 - w->cur, w->cap_man));
     hipStream_t s = w->stream;
-    if (n) {
-        AXM_HIP(hipMemcpyAsync(w->B.x, x.data(), 16ull * n, hipMemcpyHostToDevice, s));
-        AXM_HIP(hipMemcpyAsync(w->B.q, q.data(), 16ull * n, hipMemcpyHostToDevice, s));
-        AXM_HIP(hipMemcpyAsync(w->B.vel, v.data(), 16ull * n, hipMemcpyHostToDevice, s));
-        AXM_HIP(hipMemcpyAsync(w->B.angv, av.data(), 16ull * n, hipMemcpyHostToDevice, s));
-        AXM_HIP(hipMemcpyAsync(w->B.ii, ii.data(), 16ull * n, hipMemcpyHostToDevice, s));
-        AXM_HIP(hipMemcpyAsync(w->B.shape, sh.data(), 16ull * n, hipMemcpyHostToDevice, s));
-        AXM_HIP(hipMemcpyAsync(w->B.world, wd.data(), 4ull * n, hipMemcpyHostToDevice, s));
-        AXM_HIP(hipMemcpyAsync(w->B.mat, mat.data(), 16ull * n, hipMemcpyHostToDevice, s));
-        AXM_HIP(hipMemcpyAsync(w->B.bfl, bfl.data(), 16ull * n, hipMemcpyHostToDevice, s));
-        AXM_HIP(hipMemcpyAsync(w->B.world_first, first.data(), 4ull * first.size(), hipMemcpyHostToDevice, s));
-        if (hb.slp.size() == n && hb.wake.size() == n) {
-            AXM_HIP(hipMemcpyAsync(w->B.slp, hb.slp.data(), 8ull * n, hipMemcpyHostToDevice, s));
-            AXM_HIP(hipMemcpyAsync(w->B.wake, hb.wake.data(), 4ull * n, hipMemcpyHostToDevice, s));
-        } else {
-            // every body starts awake with no rest time and no island; no island has a wake request
-            const std::vector<uint2> slp(n, make_uint2(0u, LABEL_NONE));
-            AXM_HIP(hipMemcpyAsync(w->B.slp, slp.data(), 8ull * n, hipMemcpyHostToDevice, s));
-            AXM_HIP(hipMemsetAsync(w->B.wake, 0xFF, 4ull * n, s));
-        }
+    if (n && in) {
+        // a checked set in the staging
+        const axm_world_desc& D = w->desc;
+        AXM_HIP(hipMemsetAsync(w->B.world_first, 0, 4ull * (nw + 1), s));
+        launch_bodies_install(*in, n, w->B, make_float4(D.friction, D.restitution, D.lin_damp, D.ang_damp), s);
+    } else if (n) {
+        AXM_HIP(hipMemcpyAsync(w->B.x, hb->x.data(), 16ull * n, hipMemcpyHostToDevice, s));
+        AXM_HIP(hipMemcpyAsync(w->B.q, hb->q.data(), 16ull * n, hipMemcpyHostToDevice, s));
+        AXM_HIP(hipMemcpyAsync(w->B.vel, hb->v.data(), 16ull * n, hipMemcpyHostToDevice, s));
+        AXM_HIP(hipMemcpyAsync(w->B.angv, hb->av.data(), 16ull * n, hipMemcpyHostToDevice, s));
+        AXM_HIP(hipMemcpyAsync(w->B.ii, hb->ii.data(), 16ull * n, hipMemcpyHostToDevice, s));
+        AXM_HIP(hipMemcpyAsync(w->B.shape, hb->sh.data(), 16ull * n, hipMemcpyHostToDevice, s));
+        AXM_HIP(hipMemcpyAsync(w->B.world, hb->wd.data(), 4ull * n, hipMemcpyHostToDevice, s));
+        AXM_HIP(hipMemcpyAsync(w->B.mat, hb->mat.data(), 16ull * n, hipMemcpyHostToDevice, s));
+        AXM_HIP(hipMemcpyAsync(w->B.bfl, hb->bfl.data(), 16ull * n, hipMemcpyHostToDevice, s));
+        AXM_HIP(hipMemcpyAsync(w->B.world_first, hb->first.data(), 4ull * hb->first.size(), hipMemcpyHostToDevice, s));
+        AXM_HIP(hipMemcpyAsync(w->B.slp, hb->slp.data(), 8ull * n, hipMemcpyHostToDevice, s));
+        AXM_HIP(hipMemcpyAsync(w->B.wake, hb->wake.data(), 4ull * n, hipMemcpyHostToDevice, s));
     }
     AXM_HIP(hipMemsetAsync(w->cnt, 0, sizeof(Counters), s));
     // the tables' entry counts are zero now: empty the tables in full
@@ -1260,24 +1328,23 @@ axm_status axm_world_get_bodies(axm_world w, axm_body_soa* out) {
     if (!w || !out) return AXM_NULL_POINTER;
     (void)hipSetDevice(w->desc.device);
     const uint32_t n = w->n;
-    std::vector<float4> buf(n);
-    auto pull = [&](float4* src, float* dst, int comps) -> axm_status {
-        if (!dst || !n) return AXM_SUCCESS;
-        AXM_HIP(hipMemcpyAsync(buf.data(), src, 16ull * n, hipMemcpyDeviceToHost, w->stream));
-        AXM_HIP(hipStreamSynchronize(w->stream));
-        for (uint32_t i = 0; i < n; ++i) {
-            dst[comps * i] = buf[i].x;
-            dst[comps * i + 1] = buf[i].y;
-            dst[comps * i + 2] = buf[i].z;
-            if (comps == 4) dst[comps * i + 3] = buf[i].w;
-        }
-        return AXM_SUCCESS;
-    };
-    AXM_TRY(pull(w->B.x, out->pos, 3));
-    AXM_TRY(pull(w->B.q, out->quat, 4));
-    AXM_TRY(pull(w->B.vel, out->lin_vel, 3));
-    AXM_TRY(pull(w->B.angv, out->ang_vel, 3));
-    return AXM_SUCCESS;
+    // packed on the device into the caller's layout, then one transfer
+    StagePart part[4];
+    int parts = 0;
+    size_t total = 0;
+    size_t at[4];
+    float* const host[4] = {out->pos, out->quat, out->lin_vel, out->ang_vel};
+    for (int k = 0; k < 4; ++k) {
+        at[k] = total;
+        if (!host[k] || !n) continue;
+        part[parts++] = StagePart{host[k], total, (k == 1 ? 16ull : 12ull) * n};
+        total += ((k == 1 ? 16ull : 12ull) * n + 15u) / 16u * 16u;
+    }
+    if (!total) return AXM_SUCCESS;
+    AXM_TRY(ensure_stage(w, total));
+    auto f = [&](int k) { return host[k] ? reinterpret_cast<float*>(w->dstage + at[k]) : nullptr; };
+    launch_bodies_pack(w->B, n, f(0), f(1), f(2), f(3), w->stream);
+    return stage_move(w, part, parts, total, true);
 }
 
 axm_status axm_world_get_pre_solve_velocities(axm_world w, float* lin_vel, float* ang_vel) {
@@ -1973,7 +2040,7 @@ axm_status axm_world_load(axm_world w, const char* path) {
                       std::max(h.n_worlds, 1u) == w->n_worlds && h.cell == w->cell &&
                       (h.use_filter != 0) == w->use_filter;
     w->desc = d;
-    AXM_TRY(install_bodies(w, n, std::max(h.n_worlds, 1u), h.cell, h.use_filter != 0, hb, same));
+    AXM_TRY(install_bodies(w, n, std::max(h.n_worlds, 1u), h.cell, h.use_filter != 0, &hb, nullptr, same));
     hipStream_t s = w->stream;
     AXM_HIP(hipMemcpy(&w->cnt->steps_done, &h.steps_done, 4, hipMemcpyHostToDevice));
     if (mp) {
