@@ -63,7 +63,7 @@ uint64_t splitmix(uint64_t& s) {
 
 axm_status upload_params(axm_mlp_s* m, const float* p) {
     MLP_HIP(hipMemcpyAsync(m->prm, p, sizeof(float) * MLP_NPARAM, hipMemcpyHostToDevice, m->stream));
-    launch_mlp_cast(m->prm, m->w1, m->w2, m->w3, m->stream);
+    launch_mlp_cast(m->prm, m->weights(), m->stream);
     MLP_HIP(hipStreamSynchronize(m->stream));
     return AXM_SUCCESS;
 }
@@ -91,6 +91,7 @@ axm_status axm_mlp_create(int32_t device, axm_mlp* out) {
     if (st == AXM_SUCCESS) st = dalloc(m->grad, MLP_NPARAM);
     if (st == AXM_SUCCESS) st = dalloc(m->w1, (size_t)MLP_H * MLP_INP);
     if (st == AXM_SUCCESS) st = dalloc(m->w2, (size_t)MLP_H * MLP_H);
+    if (st == AXM_SUCCESS) st = dalloc(m->w2t, (size_t)MLP_H * MLP_H);
     if (st == AXM_SUCCESS) st = dalloc(m->w3, (size_t)MLP_OUTP * MLP_H);
     if (st == AXM_SUCCESS) st = dalloc(m->partial, mlp_grad_partial_floats(GRAD_BLOCKS));
     if (st == AXM_SUCCESS) st = dalloc(m->loss_partial, GRAD_BLOCKS);
@@ -117,8 +118,8 @@ axm_status axm_mlp_destroy(axm_mlp m) {
     (void)hipSetDevice(m->device);
     if (m->stream) (void)hipStreamSynchronize(m->stream);
     dfree(m->prm); dfree(m->m); dfree(m->v); dfree(m->grad);
-    dfree(m->w1); dfree(m->w2); dfree(m->w3);
-    dfree(m->partial); dfree(m->loss_partial); dfree(m->loss);
+    dfree(m->w1); dfree(m->w2); dfree(m->w2t); dfree(m->w3);
+    dfree(m->partial); dfree(m->loss_partial); dfree(m->loss); dfree(m->losses);
     dfree(m->X); dfree(m->Y);
     if (m->stream) (void)hipStreamDestroy(m->stream);
     delete m;
@@ -171,7 +172,7 @@ axm_status axm_mlp_forward(axm_mlp m, const float* X, uint32_t n, float* Y) {
     axm_status st = ensure_rows(m, n);
     if (st != AXM_SUCCESS) return st;
     MLP_HIP(hipMemcpyAsync(m->X, X, sizeof(float) * MLP_IN * (size_t)n, hipMemcpyHostToDevice, m->stream));
-    launch_mlp_forward(m->dev(), m->X, n, nullptr, 1, m->Y, 1024, m->stream);
+    launch_mlp_forward(m->dev(), m->X, n, nullptr, 1, m->Y, MLP_FWD_BLOCKS, m->stream);
     MLP_HIP(hipGetLastError());
     MLP_HIP(hipMemcpyAsync(Y, m->Y, sizeof(float) * MLP_OUT * (size_t)n, hipMemcpyDeviceToHost, m->stream));
     MLP_HIP(hipStreamSynchronize(m->stream));
@@ -186,7 +187,7 @@ axm_status axm_mlp_loss_grad(axm_mlp m, const float* X, const float* Y, uint32_t
     if (st != AXM_SUCCESS) return st;
     MLP_HIP(hipMemcpyAsync(m->X, X, sizeof(float) * MLP_IN * (size_t)n, hipMemcpyHostToDevice, m->stream));
     MLP_HIP(hipMemcpyAsync(m->Y, Y, sizeof(float) * MLP_OUT * (size_t)n, hipMemcpyHostToDevice, m->stream));
-    launch_mlp_grad(m->dev(), m->X, m->Y, n, m->partial, m->loss_partial, m->grad, m->loss, m->blocks, m->stream);
+    launch_mlp_grad(m->train(), m->X, m->Y, n, m->loss, nullptr, m->stream);
     MLP_HIP(hipGetLastError());
     if (grad) MLP_HIP(hipMemcpyAsync(grad, m->grad, sizeof(float) * MLP_NPARAM, hipMemcpyDeviceToHost, m->stream));
     if (loss) MLP_HIP(hipMemcpyAsync(loss, m->loss, sizeof(double), hipMemcpyDeviceToHost, m->stream));
@@ -203,8 +204,7 @@ axm_status axm_mlp_adam_step(axm_mlp m, const float* grad, float lr, float beta1
     m->adam_t += 1;
     const float c1 = 1.0f - std::pow(beta1, (float)m->adam_t);
     const float c2 = 1.0f - std::pow(beta2, (float)m->adam_t);
-    launch_mlp_adam(m->prm, m->m, m->v, m->grad, lr, beta1, beta2, eps, c1, c2, m->stream);
-    launch_mlp_cast(m->prm, m->w1, m->w2, m->w3, m->stream);
+    launch_mlp_adam(m->train(), MlpAdam{lr, beta1, beta2, eps, c1, c2}, m->stream);
     MLP_HIP(hipGetLastError());
     MLP_HIP(hipStreamSynchronize(m->stream));
     return AXM_SUCCESS;
@@ -220,24 +220,26 @@ axm_status axm_mlp_train(axm_mlp m, const float* X, const float* Y, uint32_t n, 
     MLP_HIP(hipMemcpyAsync(m->X, X, sizeof(float) * MLP_IN * (size_t)n, hipMemcpyHostToDevice, m->stream));
     MLP_HIP(hipMemcpyAsync(m->Y, Y, sizeof(float) * MLP_OUT * (size_t)n, hipMemcpyHostToDevice, m->stream));
     const uint32_t nb = (n + batch - 1) / batch;
-    double* losses = nullptr;
-    if (dalloc(losses, nb) != AXM_SUCCESS) return AXM_BUFFER_ALLOCATION_FAILED;
+    if (m->cap_losses < nb) {
+        MLP_HIP(hipStreamSynchronize(m->stream));
+        dfree(m->losses);
+        m->cap_losses = 0;
+        if (dalloc(m->losses, nb) != AXM_SUCCESS) return AXM_BUFFER_ALLOCATION_FAILED;
+        m->cap_losses = nb;
+    }
     std::vector<double> h(nb);
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     for (uint32_t e = 0; e < epochs && st == AXM_SUCCESS; ++e) {
         for (uint32_t b = 0; b < nb; ++b) {
             const uint32_t r0 = b * batch;
             const uint32_t rows = (n - r0) < batch ? (n - r0) : batch;
-            launch_mlp_grad(m->dev(), m->X + (size_t)r0 * MLP_IN, m->Y + (size_t)r0 * MLP_OUT, rows, m->partial,
-                            m->loss_partial, m->grad, losses + b, m->blocks, m->stream);
             m->adam_t += 1;
-            const float c1 = 1.0f - std::pow(b1, (float)m->adam_t);
-            const float c2 = 1.0f - std::pow(b2, (float)m->adam_t);
-            launch_mlp_adam(m->prm, m->m, m->v, m->grad, lr, b1, b2, eps, c1, c2, m->stream);
-            launch_mlp_cast(m->prm, m->w1, m->w2, m->w3, m->stream);
+            const MlpAdam adam{lr, b1, b2, eps, 1.0f - std::pow(b1, (float)m->adam_t), 1.0f - std::pow(b2, (float)m->adam_t)};
+            launch_mlp_grad(m->train(), m->X + (size_t)r0 * MLP_IN, m->Y + (size_t)r0 * MLP_OUT, rows, m->losses + b, &adam,
+                            m->stream);
         }
         if (hipGetLastError() != hipSuccess ||
-            hipMemcpyAsync(h.data(), losses, sizeof(double) * nb, hipMemcpyDeviceToHost, m->stream) != hipSuccess ||
+            hipMemcpyAsync(h.data(), m->losses, sizeof(double) * nb, hipMemcpyDeviceToHost, m->stream) != hipSuccess ||
             hipStreamSynchronize(m->stream) != hipSuccess) {
             st = AXM_GPU_OPERATION_FAILED;
             break;
@@ -251,7 +253,6 @@ axm_status axm_mlp_train(axm_mlp m, const float* X, const float* Y, uint32_t n, 
             epoch_loss[e] = (float)(s / n);
         }
     }
-    dfree(losses);
     return st;
 }
 

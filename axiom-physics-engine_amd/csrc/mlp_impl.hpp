@@ -13,6 +13,7 @@ struct axm_mlp_s {
     float* grad = nullptr;
     uint16_t* w1 = nullptr;   // bf16 weights used by the kernels
     uint16_t* w2 = nullptr;
+    uint16_t* w2t = nullptr;
     uint16_t* w3 = nullptr;
     float* partial = nullptr; // per-block gradient partials
     double* loss_partial = nullptr;
@@ -24,5 +25,10 @@ struct axm_mlp_s {
     float* Y = nullptr;
     uint32_t cap_rows = 0;
 
-    axm::MlpDev dev() const { return axm::MlpDev{prm, w1, w2, w3}; }
+    double* losses = nullptr; // per-batch losses of an epoch
+    uint32_t cap_losses = 0;
+
+    axm::MlpDev dev() const { return axm::MlpDev{prm, w1, w2, w2t, w3}; }
+    axm::MlpWeights weights() const { return axm::MlpWeights{w1, w2, w2t, w3}; }
+    axm::MlpTrain train() const { return axm::MlpTrain{prm, m, v, grad, partial, loss_partial, weights(), blocks}; }
 };

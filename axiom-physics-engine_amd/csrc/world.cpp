@@ -684,7 +684,7 @@ axm_status enqueue_pre(axm_world_s* w, const StepParams& sp, const StepOpts& o) 
                 w->bdone, w->cnt, w->want_feat ? w->feat : nullptr, X, s);
     if (w->mlp && w->desc.warm_start == AXM_WARM_MLP && !o.warm_in && w->feat) {
         launch_mlp_forward(w->mlp->dev(), w->feat, 4u * w->cap_man, &w->cnt->m_eff, 4u, w->ymlp,
-                           2u * (uint32_t)w->cu_count, s);
+                           (uint32_t)w->cu_count, s);
         launch_mlp_apply(R, w->cnt, rc, w->ymlp, sp, s);
     }
     return AXM_SUCCESS;
@@ -1024,7 +1024,6 @@ axm_status capture(axm_world_s* w, float dt, uint32_t iters, int parity, uint32_
     return AXM_SUCCESS;
 }
 
-bool finite3(const float* p) { return std::isfinite(p[0]) && std::isfinite(p[1]) && std::isfinite(p[2]); }
 
 }  // namespace
 
