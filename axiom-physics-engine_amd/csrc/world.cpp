@@ -28,6 +28,7 @@
 #include "k_bodies.hpp"
 #include "k_step.hpp"
 #include "mlp_impl.hpp"
+#include "staging.hpp"
 
 using namespace axm;
 
@@ -160,13 +161,7 @@ struct axm_world_s {
     Counters* cnt = nullptr;
     Counters* h_cnt = nullptr;
 
-    // body sets on their way to and from the host: device copies in the host's layout, and pinned
-    // memory the transfers go through (at most STAGE_BYTES)
-    uint8_t* dstage = nullptr;
-    size_t dstage_cap = 0;
-    uint8_t* hstage = nullptr;
-    size_t hstage_cap = 0;
-    hipEvent_t stage_ev[2] = {nullptr, nullptr};
+    Staging stage;  // body sets on their way to and from the host, in the host's layout
 
     // kernel profiling
     bool prof_on = false;
@@ -209,9 +204,7 @@ struct axm_world_s {
             if (e) (void)hipEventDestroy(e);
         mem.release_all();
         if (h_cnt) (void)hipHostFree(h_cnt);
-        if (hstage) (void)hipHostFree(hstage);
-        for (hipEvent_t e : stage_ev)
-            if (e) (void)hipEventDestroy(e);
+        stage.release();
         if (stream) (void)hipStreamDestroy(stream);
     }
 };
@@ -1115,84 +1108,6 @@ struct HostBodies {
 axm_status install_bodies(axm_world_s* w, uint32_t n, uint32_t nw, float cell, bool use_filter,
                           const HostBodies* hb, const BodyIn* in, bool keep_graphs);
 
-// Pinned memory a world keeps for its body transfers: large sets go through it in two halves,
-// one on the link while the host copies the other.  Pinned memory moves 57 GB/s here, pageable
-// memory 17 GB/s down and 29 GB/s up (and a small copy takes 36 us instead of 13), so a set is
-// bound by the host's own copy to or from the block.  Step and readback of 4096 worlds of 762
-// bodies: 41 ms with pageable copies and the conversion on the host, 21 ms so.
-constexpr size_t STAGE_BYTES = 8u << 20;
-
-// Device and pinned staging for `bytes` of a body set.
-axm_status ensure_stage(axm_world_s* w, size_t bytes) {
-    if (w->dstage_cap < bytes) {
-        w->mem.release(w->dstage);
-        w->dstage_cap = 0;
-        AXM_TRY(w->mem.get(w->dstage, bytes));
-        w->dstage_cap = bytes;
-    }
-    const size_t want = std::min(bytes, STAGE_BYTES);
-    if (w->hstage_cap < want) {
-        if (w->hstage) (void)hipHostFree(w->hstage);
-        w->hstage = nullptr;
-        w->hstage_cap = 0;
-        if (hipHostMalloc((void**)&w->hstage, want, hipHostMallocDefault) != hipSuccess) return AXM_BUFFER_ALLOCATION_FAILED;
-        w->hstage_cap = want;
-    }
-    for (hipEvent_t& e : w->stage_ev)
-        if (!e) AXM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    return AXM_SUCCESS;
-}
-
-// One host array's place in the staging.
-struct StagePart {
-    void* host;
-    size_t off, bytes;
-};
-// Copies the part of the staging range [lo, hi) between the arrays and `buf` (which holds it).
-void stage_copy(const StagePart* part, int parts, size_t lo, size_t hi, uint8_t* buf, bool out) {
-    for (int k = 0; k < parts; ++k) {
-        const size_t a = std::max(lo, part[k].off), b = std::min(hi, part[k].off + part[k].bytes);
-        if (a >= b) continue;
-        uint8_t* h = static_cast<uint8_t*>(part[k].host) + (a - part[k].off);
-        if (out) std::memcpy(h, buf + (a - lo), b - a);
-        else std::memcpy(buf + (a - lo), h, b - a);
-    }
-}
-// Moves `total` bytes of the staging to the arrays or from them, on the world's stream; on
-// return the arrays are free (upload) or filled (download).
-axm_status stage_move(axm_world_s* w, const StagePart* part, int parts, size_t total, bool out) {
-    hipStream_t s = w->stream;
-    const size_t piece = total <= w->hstage_cap ? total : w->hstage_cap / 2;
-    const size_t pieces = (total + piece - 1) / piece;
-    auto range = [&](size_t k, size_t& lo, size_t& hi) {
-        lo = k * piece;
-        hi = std::min(total, lo + piece);
-    };
-    for (size_t k = 0; k < pieces + (out ? 1 : 0); ++k) {
-        size_t lo, hi;
-        if (!out) {
-            range(k, lo, hi);
-            uint8_t* buf = w->hstage + (k & 1) * piece;
-            if (k >= 2) AXM_HIP(hipEventSynchronize(w->stage_ev[k & 1]));  // the piece before in this half
-            stage_copy(part, parts, lo, hi, buf, false);
-            AXM_HIP(hipMemcpyAsync(w->dstage + lo, buf, hi - lo, hipMemcpyHostToDevice, s));
-            AXM_HIP(hipEventRecord(w->stage_ev[k & 1], s));
-            continue;
-        }
-        if (k < pieces) {
-            range(k, lo, hi);
-            AXM_HIP(hipMemcpyAsync(w->hstage + (k & 1) * piece, w->dstage + lo, hi - lo, hipMemcpyDeviceToHost, s));
-            AXM_HIP(hipEventRecord(w->stage_ev[k & 1], s));
-        }
-        if (k > 0) {
-            range(k - 1, lo, hi);
-            AXM_HIP(hipEventSynchronize(w->stage_ev[(k - 1) & 1]));
-            stage_copy(part, parts, lo, hi, w->hstage + ((k - 1) & 1) * piece, true);
-        }
-    }
-    return AXM_SUCCESS;
-}
-
 axm_status axm_world_set_bodies(axm_world w, const axm_body_soa* b, uint32_t n) {
     if (!w || !b) return AXM_NULL_POINTER;
     if (n && (!b->pos || !b->quat || !b->lin_vel || !b->ang_vel || !b->inv_mass || !b->inv_inertia || !b->shape_type ||
@@ -1223,18 +1138,18 @@ axm_status axm_world_set_bodies(axm_world w, const axm_body_soa* b, uint32_t n) 
         const size_t at = off;
         part[parts++] = StagePart{&check, at, sizeof(check)};
         const size_t total = at + sizeof(check);
-        AXM_TRY(ensure_stage(w, total));
-        AXM_TRY(stage_move(w, part, parts, total, false));
-        auto f = [&](size_t o) { return reinterpret_cast<const float*>(w->dstage + o); };
-        auto u = [&](size_t o) { return reinterpret_cast<const uint32_t*>(w->dstage + o); };
+        AXM_TRY(w->stage.ensure(total));
+        AXM_HIP(w->stage.up(part, parts, total, w->stream));
+        auto f = [&](size_t o) { return reinterpret_cast<const float*>(w->stage.dev() + o); };
+        auto u = [&](size_t o) { return reinterpret_cast<const uint32_t*>(w->stage.dev() + o); };
         in = BodyIn{f(pos), f(quat), f(lin), f(ang), f(mass), f(inertia), f(params), u(type),
                     b->world ? u(world) : nullptr, b->material ? f(material) : nullptr, b->flags ? u(flags) : nullptr,
                     b->filter ? u(filter) : nullptr};
-        BodyCheck* d_check = reinterpret_cast<BodyCheck*>(w->dstage + at);
+        BodyCheck* d_check = reinterpret_cast<BodyCheck*>(w->stage.dev() + at);
         launch_bodies_check(in, n, d_check, w->stream);
-        AXM_HIP(hipMemcpyAsync(w->hstage, d_check, sizeof(check), hipMemcpyDeviceToHost, w->stream));
+        AXM_HIP(hipMemcpyAsync(w->stage.pinned(), d_check, sizeof(check), hipMemcpyDeviceToHost, w->stream));
         AXM_HIP(hipStreamSynchronize(w->stream));
-        std::memcpy(&check, w->hstage, sizeof(check));
+        std::memcpy(&check, w->stage.pinned(), sizeof(check));
         if (check.fault != ~0ull) {
             const uint32_t fault = (uint32_t)check.fault;
             return fault == BODY_BAD_SHAPE   ? AXM_INVALID_SHAPE
@@ -1327,7 +1242,9 @@ axm_status axm_world_get_bodies(axm_world w, axm_body_soa* out) {
     if (!w || !out) return AXM_NULL_POINTER;
     (void)hipSetDevice(w->desc.device);
     const uint32_t n = w->n;
-    // packed on the device into the caller's layout, then one transfer
+    // packed on the device into the caller's layout, then one transfer (step and readback of 4096
+    // worlds of 762 bodies: 21 ms; with pageable copies of the device's layout and the conversion
+    // on the host 41 ms)
     StagePart part[4];
     int parts = 0;
     size_t total = 0;
@@ -1340,10 +1257,11 @@ axm_status axm_world_get_bodies(axm_world w, axm_body_soa* out) {
         total += ((k == 1 ? 16ull : 12ull) * n + 15u) / 16u * 16u;
     }
     if (!total) return AXM_SUCCESS;
-    AXM_TRY(ensure_stage(w, total));
-    auto f = [&](int k) { return host[k] ? reinterpret_cast<float*>(w->dstage + at[k]) : nullptr; };
+    AXM_TRY(w->stage.ensure(total));
+    auto f = [&](int k) { return host[k] ? reinterpret_cast<float*>(w->stage.dev() + at[k]) : nullptr; };
     launch_bodies_pack(w->B, n, f(0), f(1), f(2), f(3), w->stream);
-    return stage_move(w, part, parts, total, true);
+    AXM_HIP(w->stage.down(part, parts, 0, total, w->stream));
+    return AXM_SUCCESS;
 }
 
 axm_status axm_world_get_pre_solve_velocities(axm_world w, float* lin_vel, float* ang_vel) {
