@@ -3959,6 +3959,77 @@ __global__ void __launch_bounds__(256) k_isl_union(Bodies B, const uint2* __rest
         }
     }
 }
+// The same by one workgroup with the parents in LDS, for worlds whose bodies fit: a step of a
+// walk is an LDS access instead of a coherent load from memory, which other workgroups'
+// links keep contended (19000 manifolds of 6000 bodies: 93 us, so 27; 1000 bodies: 11, so 5).
+// Above the limit the one workgroup could not hold them; 100000 bodies take 130 us by
+// k_isl_union.  The parents written back are the roots themselves.
+constexpr uint32_t UNION_LDS_BODIES = 36864u;
+constexpr int UNION_THREADS = 1024;
+__device__ __forceinline__ uint32_t lds_find(uint32_t* par, uint32_t x) {
+    auto ld = [par](uint32_t k) { return __hip_atomic_load(par + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
+    uint32_t cur = ld(x);
+    if (cur != x) {
+        uint32_t prev = x, next;
+        while (cur > (next = ld(cur))) {
+            __hip_atomic_store(par + prev, next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            prev = cur;
+            cur = next;
+        }
+    }
+    return cur;
+}
+__global__ void __launch_bounds__(UNION_THREADS) k_isl_union_lds(Bodies B, const uint2* __restrict__ m_ab, uint32_t cap,
+                                                                 uint32_t n, const Counters* __restrict__ cnt) {
+    extern __shared__ uint32_t par[];
+    if (cnt->sticky != 0u) return;
+    const uint32_t M = min(cap, cnt->m_eff);
+    const uint32_t stamp = cnt->steps_done + 1u;
+    for (uint32_t i = threadIdx.x; i < n; i += UNION_THREADS) par[i] = B.sv[i].w > 0.0f ? i : UNSET;
+    __syncthreads();
+    auto edges = [&](auto&& link) {
+        constexpr int U = 4;  // manifolds of a thread on the way at a time
+        for (uint32_t m0 = threadIdx.x; m0 < M; m0 += U * UNION_THREADS) {
+            uint2 e[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                e[u] = m0 + u * UNION_THREADS < M ? m_ab[m0 + u * UNION_THREADS] : make_uint2(0u, PLANE_BIT);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (!(e[u].y & PLANE_BIT)) link(e[u].x, e[u].y);
+        }
+    };
+    // each body's first link is to the smallest it touches, without a walk: most of the manifolds
+    // then find one root from both sides
+    edges([&](uint32_t a, uint32_t b) {
+        const bool da = par[a] != UNSET, db = par[b] != UNSET;  // never changes
+        if (da && db) {
+            atomicMin(par + max(a, b), min(a, b));
+        } else if (da || db) {
+            const uint32_t y = B.slp[da ? b : a].y;
+            if ((y & ASLEEP_BIT) && (y & LABEL_MASK) < n) B.wake[y & LABEL_MASK] = stamp;
+        }
+    });
+    __syncthreads();
+    edges([&](uint32_t a, uint32_t b) {
+        if (par[a] == UNSET || par[b] == UNSET) return;
+        uint32_t ra = lds_find(par, a), rb = lds_find(par, b);
+        while (ra != rb) {
+            const uint32_t hi = max(ra, rb), lo = min(ra, rb);
+            const uint32_t old = atomicCAS(par + hi, hi, lo);
+            if (old == hi) break;
+            ra = lds_find(par, old);
+            rb = lo;
+        }
+    });
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < n; i += UNION_THREADS)
+        if (par[i] != UNSET) B.upar[i] = lds_find(par, i);
+}
+int isl_union_setup() {
+    return hipFuncSetAttribute((const void*)k_isl_union_lds, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)(4u * UNION_LDS_BODIES)) == hipSuccess ? 1 : 0;
+}
 // Labels, rest times and each island's smallest rest time; counts islands and sleeping bodies.
 __global__ void __launch_bounds__(256) k_isl_label(Bodies B, StepParams sp, uint32_t n, Counters* cnt) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -4263,7 +4334,11 @@ void launch_integrate(const Bodies& B, const StepParams& sp, uint32_t n, Counter
 
 void launch_isl_union(const Bodies& B, uint32_t n, const uint2* m_ab, uint32_t cap_man, Counters* cnt,
                       hipStream_t s) {
-    if (n) hipLaunchKernelGGL(k_isl_union, grid_bounded(cap_man), dim3(256), 0, s, B, m_ab, cap_man, n, cnt);
+    if (n == 0u) return;
+    if (n <= UNION_LDS_BODIES)
+        hipLaunchKernelGGL(k_isl_union_lds, dim3(1), dim3(UNION_THREADS), 4u * n, s, B, m_ab, cap_man, n, cnt);
+    else
+        hipLaunchKernelGGL(k_isl_union, grid_bounded(cap_man), dim3(256), 0, s, B, m_ab, cap_man, n, cnt);
 }
 void launch_islands(const Bodies& B, const StepParams& sp, uint32_t n, Counters* cnt, hipStream_t s) {
     if (!n) return;

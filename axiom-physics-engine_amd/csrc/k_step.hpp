@@ -184,6 +184,7 @@ int pgs_flow_setup();
 int pgs_own_setup(uint32_t max_lds_bytes, uint32_t lds_bytes);
 // Allows the small islands' kernel its LDS (once per process); 0 on failure.
 int pgs_islands_setup();
+int isl_union_setup();
 void launch_pgs(const Bodies& B, const StepParams& sp, const SolverRows& R, uint32_t s0, uint32_t s1, uint32_t cap,
                 uint32_t first, hipStream_t s);
 void launch_residual(const Bodies& B, const StepParams& sp, const SolverRows& R, const Counters* cnt, uint32_t cap,

@@ -1050,7 +1050,7 @@ axm_status axm_world_create(const axm_world_desc* desc, axm_world* out) {
     w->max_lds = (uint32_t)std::min<size_t>(prop.sharedMemPerBlock, 160u * 1024u);
     w->sweep_lds = w->max_lds & ~16383u;
     const int own_per_cu = pgs_own_setup(w->max_lds, w->sweep_lds);
-    if (own_per_cu < 1 || pgs_flow_setup() < 1 || !pgs_islands_setup()) {
+    if (own_per_cu < 1 || pgs_flow_setup() < 1 || !pgs_islands_setup() || !isl_union_setup()) {
         delete w;
         return AXM_GPU_OPERATION_FAILED;
     }
