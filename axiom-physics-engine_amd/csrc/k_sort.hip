@@ -1,22 +1,18 @@
 // Device-wide exclusive scan and stable LSD radix sort for gfx950 (wave64).
 //
-// Radix sort: 8-bit digits, 256-thread workgroups over 4096-key tiles.
-//   pass = histogram (LDS atomics) -> exclusive scan of the digit-major
-//   histogram -> stable scatter.  Stability comes from ranking keys in index
-//   order: each wave finds the lanes sharing its digit with 8 ballots
-//   (a match-any over the digit bits), ranks itself by the population count of
-//   lower peer lanes, and per-wave digit counts are prefixed in LDS.
+// Radix sort: 8-bit digits, one launch for all passes (below).
 // Scan: one pass, tiles chained by decoupled look-back (below).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+#include <type_traits>
+
+#include "dev_islands.hpp"
 #include "launch.hpp"
 
 namespace axm {
 
-constexpr int RS_THREADS = 256;
-constexpr int RS_ITEMS = 4;  // keys per thread: small tiles, so that a 100k-key sort fills the GPU
-constexpr int RS_TILE = RS_THREADS * RS_ITEMS;
 constexpr int SC_THREADS = 256;
 constexpr int SC_ITEMS = 16;
 constexpr int SC_TILE = SC_THREADS * SC_ITEMS;
@@ -39,14 +35,14 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
 
 // Exclusive block scan (blockDim = 256 = 4 waves); returns the block total in `total`.
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t& total) {
-    __shared__ uint32_t s_w[RS_THREADS / 64];
+    __shared__ uint32_t s_w[SC_THREADS / 64];
     const uint32_t lane = lane_id(), wv = threadIdx.x >> 6;
     const uint32_t inc = wave_incl_scan(v);
     if (lane == 63) s_w[wv] = inc;
     __syncthreads();
     uint32_t base = 0, tot = 0;
 #pragma unroll
-    for (int w = 0; w < RS_THREADS / 64; ++w) {
+    for (int w = 0; w < SC_THREADS / 64; ++w) {
         const uint32_t x = s_w[w];
         if ((uint32_t)w < wv) base += x;
         tot += x;
@@ -238,32 +234,353 @@ void scan_exclusive(const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* tmp
 }
 
 // ---------------------------------------------------------------- radix sort
-template <class K> __device__ __forceinline__ uint32_t digit_of(K k, int shift) { return (uint32_t)(k >> shift) & 0xFFu; }
+// Stable LSD radix sort, 8-bit digits, every pass in one launch.  Workgroups of 16 waves take
+// tiles of 2048 or 4096 keys, a wave consecutive ones: it ranks 64 at a time in index order (the
+// lanes with one digit by a ballot per digit bit) on counters of its own in LDS, so a tile's
+// ranks take no barrier; the waves' counts are then prefixed.  As long as one workgroup can hold
+// the keys in registers (one_limit) it sorts alone, through LDS.  Beyond, each workgroup takes a
+// run of tiles; per pass it publishes its run's digit counts, the grid meets, it finds its places
+// from all counts, scatters, and the grid meets again.  The count may be read on the device:
+// workgroups without keys leave at once, so the grid is sized for the capacity at no cost.
+//
+// The grid that meets must be resident as a whole: at most RS_GROUPS workgroups, half of what the
+// chip holds, so that two worlds' sorts fit side by side.  200 and 1000 bodies: 14 us for the body
+// keys and 7 to 8 for the solve order (with launches per pass 47, and 23 to 47 in tiles of 256
+// threads whose ranks met at four barriers); 6000 bodies 27 and 30 (53 and 72); 100000 bodies 54
+// and 47 (65 and 117); the solve order of 1.7M manifolds 320 (889, its keys' own launch 35).
+constexpr int RS_THREADS = 1024, RS_WAVES = RS_THREADS / 64;
+constexpr uint32_t RS_GROUPS = 128, RS_HDR = 4;
 
-__device__ __forceinline__ uint32_t eff_count(uint32_t cap, const uint32_t* n_dev) {
-    if (!n_dev) return cap;
-    const uint32_t v = *n_dev;
-    return v < cap ? v : cap;
+// Sort keys read from memory.
+template <class K> struct KeysGiven {
+    using Key = K;
+    static constexpr int ITEMS = 4, ONE_ITEMS = 12;
+    uint32_t n;
+    int bits;
+    __device__ uint32_t count() const { return n; }
+    __device__ int key_bits() const { return bits; }
+    __device__ K key(const K* k, uint32_t i) const { return k[i]; }
+    __device__ uint32_t value(const uint32_t* v, uint32_t i) const { return v[i]; }
+    __device__ K order(K k) const { return k; }
+};
+// The solve order's keys, made from the colours and islands: the colour, or with the split
+// LOCAL_KEY | root << 8 | colour for a manifold of an island of at most ISLAND_LOCAL_MAX
+// manifolds; the value is the manifold's index.  A stable sort then gives the solve order: the
+// large islands' manifolds by colour, then the small islands one after another, each by colour
+// (manifold index last).  Digits are taken from the key without the colour and root bits that no
+// key of the step has (a pile of 6000 bodies: 19 bits, three passes instead of four).
+struct KeysSolve {
+    using Key = uint32_t;
+    static constexpr int ITEMS = 2, ONE_ITEMS = 4;
+    Bodies B;
+    const uint2* m_ab;
+    const uint32_t* col;
+    const Counters* cnt;
+    uint32_t cap, split;
+    int root_bits, colour_bits;  // colour_bits: set by the kernel from the step's colours
+    __device__ uint32_t count() const { return min(cap, cnt->m_eff); }
+    __device__ int key_bits() const { return split ? colour_bits + root_bits + 1 : colour_bits; }
+    __device__ uint32_t key(const uint32_t*, uint32_t m) const {
+        uint32_t k = col[m];
+        if (split) {
+            const uint32_t r = man_root(B, m_ab[m]);
+            if (r != UNSET && B.icnt[r] <= ISLAND_LOCAL_MAX) k |= LOCAL_KEY | (r << 8);
+        }
+        return k;
+    }
+    __device__ uint32_t value(const uint32_t*, uint32_t m) const { return m; }
+    __device__ uint32_t order(uint32_t k) const {
+        return (k & 0xFFu) | ((k & ~LOCAL_KEY) >> 8) << colour_bits |
+               (split ? (k >> 31) << (colour_bits + root_bits) : 0u);
+    }
+};
+
+// Barrier over the nb workgroups that take part (all resident): each wave's stores complete,
+// then one thread per workgroup arrives (agent-scope release) and waits for the last arrival
+// (agent-scope acquire); a bounded wait ORs STICKY_TIMEOUT into *err instead of hanging.
+// bar[0] counts arrivals and returns to 0; bar[1] is the generation.
+__device__ __forceinline__ void rs_sync(uint32_t* bar, uint32_t nb, uint32_t* err) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const uint32_t g = __hip_atomic_load(&bar[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint32_t arrived = __hip_atomic_fetch_add(&bar[0], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+        if (arrived == nb - 1) {
+            __hip_atomic_store(&bar[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_fetch_add(&bar[1], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        } else {
+            const uint64_t t0 = wall_clock64();
+            while (__hip_atomic_load(&bar[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == g) {
+                __builtin_amdgcn_s_sleep(1);
+                if (wall_clock64() - t0 > 200000000ull) {  // 2 s: report, do not hang
+                    if (err) atomicOr(err, STICKY_TIMEOUT);
+                    break;
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        }
+    }
+    __syncthreads();
 }
 
-// Per-tile digit counts, digit-major: hist[d * nt + tile] for the nt tiles that hold
-// keys (nt from the count read on the device; the grid is sized for the capacity).
-// The first workgroup writes 256 nt, the length of the scan that follows, to *len.
+// Most keys of a sort in one workgroup, and the LDS they pass through.  Given keys: 6000 take 27 us
+// alone and 37 in two workgroups.  Made keys are gathered through five arrays, which one CU does
+// slowly: 9144 take 88 us alone, 35 in five workgroups.
+template <class S> __host__ __device__ constexpr uint32_t one_limit() { return (uint32_t)RS_THREADS * S::ONE_ITEMS; }
+template <class S> constexpr uint32_t one_bytes(uint32_t n) {
+    return (uint32_t)sizeof(typename S::Key) * (n < one_limit<S>() ? n : one_limit<S>());
+}
+// Sorts into k0, v0.  Given keys start there, one tile per workgroup: the first pass may write over
+// them, its workgroups hold their keys in registers by then.
+template <class S>
+__global__ void __launch_bounds__(RS_THREADS) k_radix_sort(S src, typename S::Key* k0, uint32_t* v0,
+                                                           typename S::Key* k1, uint32_t* v1, uint32_t* tmp, uint32_t* err) {
+    using K = typename S::Key;
+    constexpr int ITEMS = S::ITEMS;
+    constexpr uint32_t TILE = RS_THREADS * ITEMS;
+    constexpr bool MADE = std::is_same<S, KeysSolve>::value;
+    __shared__ uint32_t s_wc[RS_WAVES][256], s_base[256], s_red[8][256], s_part[4];
+    extern __shared__ __align__(16) unsigned char s_stage[];
+    const uint32_t n = src.count();
+    const uint32_t nt = (n + TILE - 1u) / TILE;
+    // tiles of a workgroup, workgroups with keys
+    const bool one = n <= one_limit<S>();
+    const uint32_t run = one ? nt : (nt + gridDim.x - 1u) / gridDim.x;
+    const uint32_t ng = run ? (nt + run - 1u) / run : 0u;
+    const uint32_t g = blockIdx.x;
+    if (g >= ng) return;
+    if constexpr (MADE) {
+        src.colour_bits = 1;
+        while (src.colour_bits < 8 && src.cnt->max_colour > (1u << src.colour_bits)) ++src.colour_bits;
+    }
+    const int passes = (src.key_bits() + 7) / 8;
+    const uint32_t tid = threadIdx.x, lane = lane_id(), wv = tid >> 6;
+    const uint64_t lt = (1ull << lane) - 1ull;
+    uint32_t* const H = tmp + RS_HDR;
+    auto index = [&](uint32_t t, int it) { return t * TILE + wv * (64u * ITEMS) + (uint32_t)it * 64u + lane; };
+    auto digit = [&](K k, int p) { return (uint32_t)(src.order(k) >> (8 * p)) & 255u; };
+    // the rank of a key among its digit's in the wave's keys so far, on the wave's counters
+    uint32_t* const wc = s_wc[wv];
+    auto clear = [&]() {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) wc[64 * k + lane] = 0u;
+        __builtin_amdgcn_wave_barrier();
+    };
+    auto rank1 = [&](bool valid, uint32_t d) -> uint32_t {
+        uint64_t peers = __ballot(valid);
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+            const uint64_t bal = __ballot((d >> b) & 1u);
+            peers &= ((d >> b) & 1u) ? bal : ~bal;
+        }
+        const uint32_t r = (uint32_t)__popcll(peers & lt);
+        const uint32_t before = wc[d];
+        __builtin_amdgcn_wave_barrier();
+        if (valid && r == 0u) wc[d] = before + (uint32_t)__popcll(peers);
+        __builtin_amdgcn_wave_barrier();
+        return before + r;
+    };
+    // all waves ranked: their counts turned into the counts of the waves before; threads below 256
+    // return their digit's count
+    auto prefix = [&]() -> uint32_t {
+        __syncthreads();
+        uint32_t tot = 0;
+        if (tid < 256u) {
+#pragma unroll
+            for (int w = 0; w < RS_WAVES; ++w) {
+                const uint32_t c = s_wc[w][tid];
+                s_wc[w][tid] = tot;
+                tot += c;
+            }
+        }
+        return tot;
+    };
+    // s_base[d] = keys of smaller digits (c: the digit's count, threads below 256) + below
+    auto place = [&](uint32_t c, uint32_t below) {
+        const uint32_t inc = wave_incl_scan(tid < 256u ? c : 0u);
+        if (tid < 256u && lane == 63u) s_part[wv] = inc;
+        __syncthreads();
+        if (tid < 256u) {
+            uint32_t o = 0;
+            for (uint32_t w = 0; w < wv; ++w) o += s_part[w];
+            s_base[tid] = o + inc - c + below;
+        }
+        __syncthreads();
+    };
+    if (ng == 1u) {
+        // the keys in registers, a wave's consecutive
+        constexpr int ONE = S::ONE_ITEMS;
+        K key[ONE];
+        uint32_t val[ONE], rk[ONE];
+        const int items = (int)((n + RS_THREADS - 1u) / RS_THREADS);  // at most ONE: one_limit
+        const uint32_t first = wv * 64u * (uint32_t)items + lane;
+        auto valid = [&](int it) { return it < items && first + 64u * (uint32_t)it < n; };
+#pragma unroll
+        for (int it = 0; it < ONE; ++it) {
+            const uint32_t i = first + 64u * (uint32_t)it;
+            key[it] = valid(it) ? src.key(k0, i) : (K)0;
+            val[it] = valid(it) ? src.value(v0, i) : 0u;
+        }
+        for (int p = 0; p < passes; ++p) {
+            clear();
+#pragma unroll
+            for (int it = 0; it < ONE; ++it) {
+                rk[it] = 0u;
+                if (it < items) rk[it] = rank1(valid(it), digit(key[it], p));
+            }
+            place(prefix(), 0u);
+#pragma unroll
+            for (int it = 0; it < ONE; ++it) {
+                const uint32_t d = digit(key[it], p);
+                rk[it] += s_base[d] + s_wc[wv][d];
+            }
+            if (p + 1 == passes) {
+#pragma unroll
+                for (int it = 0; it < ONE; ++it)
+                    if (valid(it)) {
+                        k0[rk[it]] = key[it];
+                        v0[rk[it]] = val[it];
+                    }
+                return;
+            }
+            K* s_key = reinterpret_cast<K*>(s_stage);
+            uint32_t* s_val = reinterpret_cast<uint32_t*>(s_stage);
+#pragma unroll
+            for (int it = 0; it < ONE; ++it)
+                if (valid(it)) s_key[rk[it]] = key[it];
+            __syncthreads();
+#pragma unroll
+            for (int it = 0; it < ONE; ++it) key[it] = valid(it) ? s_key[first + 64u * (uint32_t)it] : (K)0;
+            __syncthreads();
+#pragma unroll
+            for (int it = 0; it < ONE; ++it)
+                if (valid(it)) s_val[rk[it]] = val[it];
+            __syncthreads();
+#pragma unroll
+            for (int it = 0; it < ONE; ++it) val[it] = valid(it) ? s_val[first + 64u * (uint32_t)it] : 0u;
+            __syncthreads();
+        }
+        return;
+    }
+    K key[ITEMS];
+    uint32_t val[ITEMS], rk[ITEMS];
+    auto rank = [&](uint32_t t, int p) -> uint32_t {
+        clear();
+#pragma unroll
+        for (int it = 0; it < ITEMS; ++it) rk[it] = rank1(index(t, it) < n, digit(key[it], p));
+        return prefix();
+    };
+    const uint32_t t0 = g * run, t1 = min(nt, t0 + run);
+    for (int p = 0; p < passes; ++p) {
+        const bool to1 = ((passes - 1 - p) & 1) != 0;
+        K* ko = to1 ? k1 : k0;
+        uint32_t* vo = to1 ? v1 : v0;
+        // the pass's keys: given ones start in k0, made ones where the first pass does not write
+        const bool from1 = p == 0 && !MADE ? false : !to1;
+        K* ki = from1 ? k1 : k0;
+        uint32_t* vi = from1 ? v1 : v0;
+        uint32_t mine = 0;  // the run's keys with this thread's digit
+        for (uint32_t t = t0; t < t1; ++t) {
+#pragma unroll
+            for (int it = 0; it < ITEMS; ++it) {
+                const uint32_t i = index(t, it);
+                if (p == 0) {
+                    key[it] = i < n ? src.key(ki, i) : (K)0;
+                    val[it] = i < n ? src.value(vi, i) : 0u;
+                    if (MADE && run > 1u && i < n) {
+                        ki[i] = key[it];
+                        vi[i] = val[it];
+                    }
+                } else {
+                    key[it] = i < n ? ki[i] : (K)0;
+                    val[it] = i < n ? vi[i] : 0u;
+                }
+            }
+            if (t != t0) __syncthreads();  // the counts of the tile before have been read
+            mine += rank(t, p);
+        }
+        if (tid < 256u) H[256u * g + tid] = mine;
+        rs_sync(tmp, ng, err);
+        // digit d's keys in all runs and in the runs before this one: four threads a digit
+        {
+            const uint32_t d = tid & 255u, q = tid >> 8;
+            uint32_t all = 0, below = 0;
+            for (uint32_t r = q; r < ng; r += 32u) {
+                uint32_t c[8];
+#pragma unroll
+                for (uint32_t u = 0; u < 8u; ++u) c[u] = r + 4u * u < ng ? H[256u * (r + 4u * u) + d] : 0u;
+#pragma unroll
+                for (uint32_t u = 0; u < 8u; ++u) {
+                    all += c[u];
+                    below += r + 4u * u < g ? c[u] : 0u;
+                }
+            }
+            s_red[q][d] = all;
+            s_red[4u + q][d] = below;
+        }
+        __syncthreads();
+        uint32_t all = 0, below = 0;
+        if (tid < 256u) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                all += s_red[q][tid];
+                below += s_red[4 + q][tid];
+            }
+        }
+        place(all, below);
+        for (uint32_t t = t0; t < t1; ++t) {
+            uint32_t tot = 0;
+            if (run > 1u) {
+#pragma unroll
+                for (int it = 0; it < ITEMS; ++it) {
+                    const uint32_t i = index(t, it);
+                    key[it] = i < n ? ki[i] : (K)0;
+                    val[it] = i < n ? vi[i] : 0u;
+                }
+                tot = rank(t, p);
+                __syncthreads();
+            }
+#pragma unroll
+            for (int it = 0; it < ITEMS; ++it) {
+                if (index(t, it) >= n) continue;
+                const uint32_t d = digit(key[it], p);
+                const uint32_t pos = s_base[d] + s_wc[wv][d] + rk[it];
+                if (pos < n) {
+                    ko[pos] = key[it];
+                    vo[pos] = val[it];
+                }
+            }
+            if (run > 1u) {
+                __syncthreads();
+                if (tid < 256u) s_base[tid] += tot;
+                __syncthreads();
+            }
+        }
+        if (p + 1 < passes) rs_sync(tmp, ng, err);
+    }
+}
+
+// ---------------------------------------------------------------- per-pass sort
+// More given keys than RS_GIVEN: three launches a pass (per-tile digit counts, their scan, the
+// scatter) in small tiles that fill the chip.  A grid that meets writes back and drops every
+// XCD's L2 at each meeting, once per workgroup: 1M keys of 30 bits take 257 us so, 106 us in
+// launches; 100000 keys 52 and 65 us.
+constexpr uint32_t RS_GIVEN = 131072u;
+constexpr int RP_THREADS = 256, RP_ITEMS = 4, RP_TILE = RP_THREADS * RP_ITEMS;
+template <class K> __device__ __forceinline__ uint32_t digit_of(K k, int shift) { return (uint32_t)(k >> shift) & 0xFFu; }
+
+// Per-tile digit counts, digit-major: hist[d * nt + tile] for the nt tiles.
 template <class K>
-__global__ void __launch_bounds__(RS_THREADS) k_rs_hist(const K* __restrict__ keys, uint32_t cap,
-                                                        const uint32_t* __restrict__ n_dev, int shift,
-                                                        uint32_t* __restrict__ hist, uint32_t* __restrict__ len) {
-    const uint32_t n = eff_count(cap, n_dev);
-    const uint32_t nt = (n + RS_TILE - 1) / RS_TILE;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *len = 256u * nt;
-    if (blockIdx.x >= nt) return;
+__global__ void __launch_bounds__(RP_THREADS) k_rs_hist(const K* __restrict__ keys, uint32_t n, int shift,
+                                                        uint32_t* __restrict__ hist) {
+    const uint32_t nt = (n + RP_TILE - 1) / RP_TILE;
     __shared__ uint32_t h[256];
     h[threadIdx.x] = 0;
     __syncthreads();
-    const uint32_t base = blockIdx.x * RS_TILE;
+    const uint32_t base = blockIdx.x * RP_TILE;
 #pragma unroll 4
-    for (int it = 0; it < RS_ITEMS; ++it) {
-        const uint32_t i = base + it * RS_THREADS + threadIdx.x;
+    for (int it = 0; it < RP_ITEMS; ++it) {
+        const uint32_t i = base + it * RP_THREADS + threadIdx.x;
         if (i < n) atomicAdd(&h[digit_of(keys[i], shift)], 1u);
     }
     __syncthreads();
@@ -271,21 +588,18 @@ __global__ void __launch_bounds__(RS_THREADS) k_rs_hist(const K* __restrict__ ke
 }
 
 template <class K>
-__global__ void __launch_bounds__(RS_THREADS) k_rs_scatter(const K* __restrict__ kin, const uint32_t* __restrict__ vin,
-                                                           K* __restrict__ kout, uint32_t* __restrict__ vout, uint32_t cap,
-                                                           const uint32_t* __restrict__ n_dev, int shift,
-                                                           const uint32_t* __restrict__ offs) {
-    const uint32_t n = eff_count(cap, n_dev);
-    if (blockIdx.x * RS_TILE >= n) return;
-    const uint32_t nt = (n + RS_TILE - 1) / RS_TILE;
+__global__ void __launch_bounds__(RP_THREADS) k_rs_scatter(const K* __restrict__ kin, const uint32_t* __restrict__ vin,
+                                                           K* __restrict__ kout, uint32_t* __restrict__ vout, uint32_t n,
+                                                           int shift, const uint32_t* __restrict__ offs) {
+    const uint32_t nt = (n + RP_TILE - 1) / RP_TILE;
     __shared__ uint32_t s_off[256];
-    __shared__ uint32_t s_wc[RS_THREADS / 64][256];
+    __shared__ uint32_t s_wc[RP_THREADS / 64][256];
     const uint32_t tid = threadIdx.x, lane = lane_id(), wv = tid >> 6;
     s_off[tid] = offs[(size_t)tid * nt + blockIdx.x];
     const uint64_t lt = (1ull << lane) - 1ull;
-    const uint32_t base = blockIdx.x * RS_TILE;
-    for (int it = 0; it < RS_ITEMS; ++it) {
-        const uint32_t i = base + it * RS_THREADS + tid;
+    const uint32_t base = blockIdx.x * RP_TILE;
+    for (int it = 0; it < RP_ITEMS; ++it) {
+        const uint32_t i = base + it * RP_THREADS + tid;
         const bool valid = i < n;
         K k = 0;
         uint32_t v = 0, d = 256u;
@@ -295,7 +609,7 @@ __global__ void __launch_bounds__(RS_THREADS) k_rs_scatter(const K* __restrict__
             d = digit_of(k, shift);
         }
 #pragma unroll
-        for (int w = 0; w < RS_THREADS / 64; ++w) s_wc[w][tid] = 0;
+        for (int w = 0; w < RP_THREADS / 64; ++w) s_wc[w][tid] = 0;
         // lanes with the same digit (9 bits so that invalid lanes, d = 256, form their own group)
         uint64_t peers = __ballot(1);
 #pragma unroll
@@ -315,7 +629,7 @@ __global__ void __launch_bounds__(RS_THREADS) k_rs_scatter(const K* __restrict__
         __syncthreads();
         uint32_t add = 0;
 #pragma unroll
-        for (int w = 0; w < RS_THREADS / 64; ++w) add += s_wc[w][tid];
+        for (int w = 0; w < RP_THREADS / 64; ++w) add += s_wc[w][tid];
         s_off[tid] += add;
         if (valid) {
             kout[pos] = k;
@@ -325,233 +639,40 @@ __global__ void __launch_bounds__(RS_THREADS) k_rs_scatter(const K* __restrict__
     }
 }
 
-// ---------------------------------------------------------------- cooperative sort
-// For a count read on the device (usually far below the capacity the grid would be
-// sized for), one launch of at most CO_GROUPS workgroups, all resident, runs every
-// pass with one grid barrier per pass instead of three launches per pass.  Per-tile
-// digit counts live in three rotating buffers (tile-major: [tile * 256 + digit]): pass
-// p reads its counts from H[p % 3]; its scatter adds each key's next digit at the key's
-// destination tile into H[(p + 1) % 3]; and it clears H[(p + 2) % 3], which pass p - 1
-// read and pass p + 1 adds into.  A prologue writes pass 0's counts and clears the
-// buffer pass 0 adds into.  Each workgroup finds its tiles' offsets from the counts
-// themselves (digit totals over all tiles, then the tiles below its own).
-constexpr uint32_t CO_GROUPS = 64, CO_HDR = 4;
-
-size_t coop_tmp_words(uint32_t n) {
-    const uint32_t nb = (n + RS_TILE - 1) / RS_TILE;
-    return CO_HDR + 3ull * 256u * (nb ? nb : 1u);
-}
-
-// Barrier over the grid (every workgroup resident): each wave's stores complete, then one
-// thread per workgroup arrives (agent-scope release) and waits for the last arrival
-// (agent-scope acquire); a bounded wait ORs STICKY_TIMEOUT into *err instead of hanging.
-// bar[0] counts arrivals and returns to 0; bar[1] is the generation.
-__device__ __forceinline__ void co_sync(uint32_t* bar, uint32_t* err) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const uint32_t g = __hip_atomic_load(&bar[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const uint32_t arrived = __hip_atomic_fetch_add(&bar[0], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        if (arrived == gridDim.x - 1) {
-            __hip_atomic_store(&bar[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_fetch_add(&bar[1], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        } else {
-            const uint64_t t0 = wall_clock64();
-            while (__hip_atomic_load(&bar[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == g) {
-                __builtin_amdgcn_s_sleep(2);
-                if (wall_clock64() - t0 > 200000000ull) {  // 2 s: report, do not hang
-                    if (err) atomicOr(err, STICKY_TIMEOUT);
-                    break;
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        }
-    }
-    __syncthreads();
-}
-
-// Sum of counts[t * 256 + d] over tiles t0 <= t < t1, eight loads in flight at a time.
-__device__ __forceinline__ uint32_t sum_tiles(const uint32_t* __restrict__ h, uint32_t t0, uint32_t t1, uint32_t d) {
-    uint32_t s = 0;
-    uint32_t t = t0;
-    for (; t + 8u <= t1; t += 8u) {
-        uint32_t a[8];
-#pragma unroll
-        for (uint32_t u = 0; u < 8u; ++u) a[u] = h[(size_t)(t + u) * 256u + d];
-#pragma unroll
-        for (uint32_t u = 0; u < 8u; ++u) s += a[u];
-    }
-    uint32_t a[8];
-#pragma unroll
-    for (uint32_t u = 0; u < 8u; ++u) a[u] = t + u < t1 ? h[(size_t)(t + u) * 256u + d] : 0u;
-#pragma unroll
-    for (uint32_t u = 0; u < 8u; ++u) s += a[u];
-    return s;
-}
-
-template <class K>
-__global__ void __launch_bounds__(RS_THREADS) k_rs_coop(K* __restrict__ k0, uint32_t* __restrict__ v0,
-                                                        K* __restrict__ k1, uint32_t* __restrict__ v1, uint32_t cap,
-                                                        const uint32_t* __restrict__ n_dev, int passes,
-                                                        uint32_t* __restrict__ tmp, uint32_t* __restrict__ err) {
-    __shared__ uint32_t s_off[256], s_cnt[256];
-    __shared__ uint32_t s_wc[RS_THREADS / 64][256];
-    const uint32_t n = eff_count(cap, n_dev);
-    const uint32_t nt = (n + RS_TILE - 1) / RS_TILE;
-    const uint32_t nbc = (cap + RS_TILE - 1) / RS_TILE;
-    uint32_t* bar = tmp;
-    uint32_t* const H0 = tmp + CO_HDR;
-    const size_t hsz = (size_t)256 * nbc;
-    const uint32_t tid = threadIdx.x, lane = lane_id(), wv = tid >> 6;
-    const uint64_t lt = (1ull << lane) - 1ull;
-    // prologue: pass 0's counts per tile, and the buffer pass 0 adds into cleared
-    for (uint32_t t = blockIdx.x; t < nt; t += gridDim.x) {
-        s_cnt[tid] = 0u;
-        __syncthreads();
-#pragma unroll
-        for (int it = 0; it < RS_ITEMS; ++it) {
-            const uint32_t i = t * RS_TILE + it * RS_THREADS + tid;
-            if (i < n) atomicAdd(&s_cnt[digit_of(k0[i], 0)], 1u);
-        }
-        __syncthreads();
-        H0[(size_t)t * 256u + tid] = s_cnt[tid];
-        H0[hsz + (size_t)t * 256u + tid] = 0u;
-        __syncthreads();
-    }
-    co_sync(bar, err);
-    K* ki = k0;
-    K* ko = k1;
-    uint32_t* vi = v0;
-    uint32_t* vo = v1;
-    for (int p = 0; p < passes; ++p) {
-        const uint32_t* Hp = H0 + hsz * (uint32_t)(p % 3);
-        uint32_t* Hn = H0 + hsz * (uint32_t)((p + 1) % 3);
-        uint32_t* Hz = H0 + hsz * (uint32_t)((p + 2) % 3);
-        const bool more = p + 1 < passes;
-        const int shift = 8 * p;
-        // digit tid's place among all keys: the counts of the lower digits over all tiles
-        // the first tile's keys and values are loaded before the counts, so that the two
-        // rounds of loads overlap
-        K kk[RS_ITEMS];
-        uint32_t vv[RS_ITEMS];
-        auto load_tile = [&](uint32_t t) {
-#pragma unroll
-            for (int it = 0; it < RS_ITEMS; ++it) {
-                const uint32_t i = t * RS_TILE + it * RS_THREADS + tid;
-                kk[it] = i < n ? ki[i] : (K)0;
-                vv[it] = i < n ? vi[i] : 0u;
-            }
-        };
-        if (blockIdx.x < nt) load_tile(blockIdx.x);
-        // up to 32 tiles: all of digit tid's counts in registers from one round of loads,
-        // which give the total and the count below each of this workgroup's tiles
-        const bool few = nt <= 32u;
-        uint32_t c32[32];
-#pragma unroll
-        for (uint32_t u = 0; u < 32u; ++u) c32[u] = few && u < nt ? Hp[(size_t)u * 256u + tid] : 0u;
-        uint32_t tot = 0;
-        if (few) {
-#pragma unroll
-            for (uint32_t u = 0; u < 32u; ++u) tot += c32[u];
-        } else {
-            tot = sum_tiles(Hp, 0u, nt, tid);
-        }
-        uint32_t all;
-        const uint32_t base = block_excl_scan(tot, all);
-        uint32_t below = 0;  // count of digit tid in the tiles before the current one
-        uint32_t tb = 0;
-        for (uint32_t t = blockIdx.x; t < nt; t += gridDim.x) {
-            if (t != blockIdx.x) load_tile(t);
-            if (few) {
-                below = 0;
-#pragma unroll
-                for (uint32_t u = 0; u < 32u; ++u) below += u < t ? c32[u] : 0u;
-            } else {
-                below += sum_tiles(Hp, tb, t, tid);
-                tb = t;
-            }
-            s_off[tid] = base + below;
-            if (more) Hz[(size_t)t * 256u + tid] = 0u;
-            // stable scatter, item by item in index order (as k_rs_scatter), adding each
-            // key's next digit at its destination tile
-#pragma unroll
-            for (int it = 0; it < RS_ITEMS; ++it) {
-                const uint32_t i = t * RS_TILE + it * RS_THREADS + tid;
-                const bool valid = i < n;
-                const K k = kk[it];
-                const uint32_t v = vv[it];
-                const uint32_t d = valid ? digit_of(k, shift) : 256u;
-#pragma unroll
-                for (int w = 0; w < RS_THREADS / 64; ++w) s_wc[w][tid] = 0;
-                uint64_t peers = __ballot(1);
-#pragma unroll
-                for (int b = 0; b < 9; ++b) {
-                    const uint64_t bal = __ballot((d >> b) & 1u);
-                    peers &= ((d >> b) & 1u) ? bal : ~bal;
-                }
-                const uint32_t rank = (uint32_t)__popcll(peers & lt);
-                __syncthreads();
-                if (valid && rank == 0) s_wc[wv][d] = (uint32_t)__popcll(peers);
-                __syncthreads();
-                uint32_t pos = 0;
-                if (valid) {
-                    pos = s_off[d] + rank;
-                    for (uint32_t w = 0; w < wv; ++w) pos += s_wc[w][d];
-                }
-                __syncthreads();
-                uint32_t add = 0;
-#pragma unroll
-                for (int w = 0; w < RS_THREADS / 64; ++w) add += s_wc[w][tid];
-                s_off[tid] += add;
-                if (valid && pos < n) {
-                    ko[pos] = k;
-                    vo[pos] = v;
-                    if (more) atomicAdd(&Hn[(size_t)(pos / RS_TILE) * 256u + digit_of(k, shift + 8)], 1u);
-                }
-            }
-            __syncthreads();
-        }
-        if (more) co_sync(bar, err);
-        K* tk = ki; ki = ko; ko = tk;
-        uint32_t* tv = vi; vi = vo; vo = tv;
-    }
-}
-
+// Scratch of the per-pass sort: the histogram with the scan's total, then the scan's scratch.
+static size_t hist_words(uint32_t nb) { return (size_t)256 * nb + 2; }
 size_t radix_tmp_words(uint32_t n) {
-    const uint32_t nb = (n + RS_TILE - 1) / RS_TILE;
-    const size_t split = (size_t)256 * nb + 2 + scan_tmp_words(256u * nb);
-    const size_t coop = coop_tmp_words(n);
-    return split > coop ? split : coop;
+    const uint32_t nb = (n + RP_TILE - 1) / RP_TILE;
+    return hist_words(nb) + scan_tmp_words(256u * nb);
 }
+size_t radix_meet_words() { return RS_HDR + 256u * RS_GROUPS; }
 
+template <class S> static uint32_t rs_groups(uint32_t n, uint32_t cus) {
+    return std::max(1u, std::min({(n - 1u) / (RS_THREADS * S::ITEMS) + 1u, RS_GROUPS, cus}));
+}
 template <class K>
 static int radix_sort_impl(K* keys, uint32_t* vals, K* keys_alt, uint32_t* vals_alt, uint32_t n, int end_bit,
-                           uint32_t* tmp, hipStream_t s, const uint32_t* n_dev, uint32_t* err) {
-    if (n == 0) return 0;
-    const uint32_t nb = (n + RS_TILE - 1) / RS_TILE;
-    if (n_dev) {
-        // the count is read on the device: one cooperative launch
-        const int passes = (end_bit + 7) / 8;
-        const uint32_t groups = nb < CO_GROUPS ? nb : CO_GROUPS;
-        hipLaunchKernelGGL(k_rs_coop<K>, dim3(groups), dim3(RS_THREADS), 0, s, keys, vals, keys_alt, vals_alt, n, n_dev,
-                           passes, tmp, err);
-        return passes & 1;
+                           uint32_t* tmp, uint32_t* meet, uint32_t cus, hipStream_t s, uint32_t* err) {
+    if (n == 0 || end_bit <= 0) return 0;
+    const uint32_t g = rs_groups<KeysGiven<K>>(n, cus);
+    if (n <= RS_GIVEN && (uint64_t)g * RS_THREADS * KeysGiven<K>::ITEMS >= n) {
+        const uint32_t lds = n <= one_limit<KeysGiven<K>>() ? one_bytes<KeysGiven<K>>(n) : 0u;
+        hipLaunchKernelGGL(k_radix_sort<KeysGiven<K>>, dim3(g), dim3(RS_THREADS), lds, s, KeysGiven<K>{n, end_bit}, keys, vals,
+                           keys_alt, vals_alt, meet, err);
+        return 0;
     }
-    uint32_t* hist = tmp;
-    uint32_t* offs = tmp;  // scanned in place
-    // the histogram length in use (256 x tiles with keys); the word before it takes the
-    // scan's total (out[len])
-    uint32_t* len = tmp + (size_t)256 * nb + 1;
-    uint32_t* scan_tmp = tmp + (size_t)256 * nb + 2;  // 8-byte aligned for the scan's status words
+    const uint32_t nb = (n + RP_TILE - 1) / RP_TILE;
+    uint32_t* hist = tmp;  // scanned in place
+    uint32_t* scan_tmp = tmp + hist_words(nb);  // 8-byte aligned for the scan's status words
     K* ki = keys;
     K* ko = keys_alt;
     uint32_t* vi = vals;
     uint32_t* vo = vals_alt;
     int passes = 0;
     for (int shift = 0; shift < end_bit; shift += 8) {
-        hipLaunchKernelGGL(k_rs_hist<K>, dim3(nb), dim3(RS_THREADS), 0, s, ki, n, n_dev, shift, hist, len);
-        scan_exclusive(hist, offs, 256u * nb, scan_tmp, s, nullptr, len, false, err);
-        hipLaunchKernelGGL(k_rs_scatter<K>, dim3(nb), dim3(RS_THREADS), 0, s, ki, vi, ko, vo, n, n_dev, shift, offs);
+        hipLaunchKernelGGL(k_rs_hist<K>, dim3(nb), dim3(RP_THREADS), 0, s, ki, n, shift, hist);
+        scan_exclusive(hist, hist, 256u * nb, scan_tmp, s, nullptr, nullptr, false, err);
+        hipLaunchKernelGGL(k_rs_scatter<K>, dim3(nb), dim3(RP_THREADS), 0, s, ki, vi, ko, vo, n, shift, hist);
         K* tk = ki; ki = ko; ko = tk;
         uint32_t* tv = vi; vi = vo; vo = tv;
         ++passes;
@@ -560,13 +681,33 @@ static int radix_sort_impl(K* keys, uint32_t* vals, K* keys_alt, uint32_t* vals_
 }
 
 int radix_sort_u64(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt, uint32_t n, int end_bit,
-                   uint32_t* tmp, hipStream_t s, const uint32_t* n_dev, uint32_t* err) {
-    return radix_sort_impl<uint64_t>(keys, vals, keys_alt, vals_alt, n, end_bit, tmp, s, n_dev, err);
+                   uint32_t* tmp, uint32_t* meet, uint32_t cus, hipStream_t s, uint32_t* err) {
+    return radix_sort_impl<uint64_t>(keys, vals, keys_alt, vals_alt, n, end_bit, tmp, meet, cus, s, err);
 }
 
 int radix_sort_u32(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt, uint32_t n, int end_bit,
-                   uint32_t* tmp, hipStream_t s, const uint32_t* n_dev, uint32_t* err) {
-    return radix_sort_impl<uint32_t>(keys, vals, keys_alt, vals_alt, n, end_bit, tmp, s, n_dev, err);
+                   uint32_t* tmp, uint32_t* meet, uint32_t cus, hipStream_t s, uint32_t* err) {
+    return radix_sort_impl<uint32_t>(keys, vals, keys_alt, vals_alt, n, end_bit, tmp, meet, cus, s, err);
+}
+
+int radix_setup() {
+    auto allow = [](const void* f, uint32_t bytes) {
+        return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) == hipSuccess;
+    };
+    return allow((const void*)k_radix_sort<KeysGiven<uint32_t>>, one_bytes<KeysGiven<uint32_t>>(~0u)) &&
+                   allow((const void*)k_radix_sort<KeysGiven<uint64_t>>, one_bytes<KeysGiven<uint64_t>>(~0u)) &&
+                   allow((const void*)k_radix_sort<KeysSolve>, one_bytes<KeysSolve>(~0u))
+               ? 1 : 0;
+}
+
+void sort_solve_order(const Bodies& B, const uint2* m_ab, const uint32_t* col, uint32_t cap, uint32_t split, int root_bits,
+                      uint32_t* key, uint32_t* val, uint32_t* key_alt, uint32_t* val_alt, uint32_t* meet, uint32_t cus,
+                      Counters* cnt, hipStream_t s) {
+    if (cap == 0) return;
+    KeysSolve src{B, m_ab, col, cnt, cap, split, root_bits, 8};
+    hipLaunchKernelGGL(k_radix_sort<KeysSolve>, dim3(rs_groups<KeysSolve>(cap, cus)), dim3(RS_THREADS),
+                       one_bytes<KeysSolve>(cap), s, src, key, val, key_alt,
+                       val_alt, meet, &cnt->sticky);
 }
 
 }  // namespace axm

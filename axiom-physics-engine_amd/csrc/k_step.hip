@@ -19,6 +19,7 @@
 // solve-order arrays, so a wave of 64 manifolds of one colour reads 64
 // consecutive 16-byte rows.
 #include "dev_geom.hpp"
+#include "dev_islands.hpp"
 #include "k_mlp.hpp"
 #include "k_step.hpp"
 
@@ -845,40 +846,6 @@ __device__ __forceinline__ bool prev_find(const PrevCache& c, uint64_t k, uint32
     return false;
 }
 
-// Union-find over body indices.  Every link points from a larger root to a smaller one
-// (compare-and-swap on the root), so the root of a finished component is its smallest
-// body index whatever the order of the links (lock-free union-find with path halving:
-// Jaiganesh & Burtscher 2018, ECL-CC).  The parents are shared between workgroups, so
-// they move through agent-scope atomics.
-__device__ __forceinline__ uint32_t uf_load(uint32_t* p, uint32_t x) {
-    return __hip_atomic_load(p + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ uint32_t uf_find(uint32_t* par, uint32_t x) {
-    uint32_t cur = uf_load(par, x);
-    if (cur != x) {
-        uint32_t prev = x, next;
-        while (cur > (next = uf_load(par, cur))) {
-            __hip_atomic_store(par + prev, next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            prev = cur;
-            cur = next;
-        }
-    }
-    return cur;
-}
-// Root of x in the finished forest (after the union kernel, which no later kernel of the
-// step changes): the union's coherent loads, without its path-halving stores (in one giant
-// island every walk ends on the same root word, which stores would keep contended).
-__device__ __forceinline__ uint32_t uf_root(uint32_t* par, uint32_t x) {
-    uint32_t p;
-    while ((p = uf_load(par, x)) != x) x = p;
-    return x;
-}
-// Island (union-find root) of a manifold: that of its dynamic body, UNSET with none.
-__device__ __forceinline__ uint32_t man_root(const Bodies& B, uint2 ab) {
-    const bool plane = (ab.y & PLANE_BIT) != 0u;
-    const uint32_t d = B.sv[ab.x].w > 0.0f ? ab.x : (!plane && B.sv[ab.y].w > 0.0f ? ab.y : UNSET);
-    return d == UNSET ? UNSET : uf_root(B.upar, d);
-}
 // Per-island atomics of a wave: the lanes whose island is that of the first lane taking
 // part combine their values into one atomic made by that lane; the others make their own.
 // In one giant island a wave makes one atomic instead of 64 on the same word.
@@ -1115,25 +1082,6 @@ __global__ void __launch_bounds__(256) k_colour(Bodies B, const uint2* __restric
     }
 }
 
-// Colour sort input: values = manifold index, keys = colour, or with the island split
-// LOCAL_KEY | root << 8 | colour for a manifold of an island of at most ISLAND_LOCAL_MAX
-// manifolds.  A stable sort then gives the solve order: the large islands' manifolds by
-// colour, then the small islands one after another, each by colour (manifold index last).
-__global__ void __launch_bounds__(256) k_col_sort_input(Bodies B, const uint2* __restrict__ m_ab,
-                                                        const uint32_t* __restrict__ col, uint32_t cap,
-                                                        uint32_t* __restrict__ key, uint32_t* __restrict__ val,
-                                                        const Counters* __restrict__ cnt, uint32_t split) {
-    const uint32_t M = min(cap, cnt->m_eff);
-    for (uint32_t m = blockIdx.x * blockDim.x + threadIdx.x; m < M; m += gridDim.x * blockDim.x) {
-        uint32_t k = col[m];
-        if (split) {
-            const uint32_t r = man_root(B, m_ab[m]);
-            if (r != UNSET && B.icnt[r] <= ISLAND_LOCAL_MAX) k |= LOCAL_KEY | (r << 8);
-        }
-        key[m] = k;
-        val[m] = m;
-    }
-}
 // Size classes of the islands of more than ISLAND_LANE_MAX manifolds (k_pgs_islands solves
 // the largest first): 0 above 256 manifolds, 1 above 64, 2 above 32, 3 above 16, 4 the rest.
 // Their work list entries (first slot, manifolds) lie in one region per class, each as long as
@@ -4212,10 +4160,6 @@ void launch_colour(const Bodies& B, const uint2* m_ab, uint32_t cap_man, uint32_
                        65000u, SMALL);
     hipLaunchKernelGGL(k_colour, dim3(blocks), dim3(256), 0, s, B, m_ab, col, prio, bmax0, bmax1, bmask, list, bar,
                        cnt, 65000u, SMALL);
-}
-void launch_col_sort_input(const Bodies& B, const uint2* m_ab, const uint32_t* col, uint32_t cap, uint32_t* key,
-                           uint32_t* val, const Counters* cnt, uint32_t split, hipStream_t s) {
-    hipLaunchKernelGGL(k_col_sort_input, grid_bounded(cap), dim3(256), 0, s, B, m_ab, col, cap, key, val, cnt, split);
 }
 void launch_pgs_local(const Bodies& B, const StepParams& sp, const SolverRows& R, Counters* cnt, uint32_t cap,
                       const uint32_t* skey, uint2* list, float tol, uint32_t max_sweeps, uint32_t groups,

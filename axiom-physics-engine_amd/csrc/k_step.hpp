@@ -104,9 +104,6 @@ int colour_blocks_per_cu();
 void launch_colour(const Bodies& B, const uint2* m_ab, uint32_t cap_man, uint32_t* col, uint64_t* prio,
                    uint64_t* bmax0, uint64_t* bmax1, uint64_t* bmask, uint32_t* bdeg, uint32_t* list, GridBar* bar,
                    Counters* cnt, uint32_t blocks, const PrevCacheArgs& prev, uint32_t split, hipStream_t s);
-void launch_col_sort_input(const Bodies& B, const uint2* m_ab, const uint32_t* col, uint32_t cap, uint32_t* key,
-                           uint32_t* val, const Counters* cnt, uint32_t split,
-                           hipStream_t s);
 // The islands solved on their own (after the row preparation, which built their work list),
 // in `groups` workgroups (one per CU): tol > 0 stops each at its own residual.  bmask holds
 // the colouring's per-body colour masks.  With flow_init, the same launch also sets up the

@@ -203,13 +203,23 @@ size_t scan_tmp_words(uint32_t n);
 void scan_exclusive(const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* tmp, hipStream_t s,
                     uint32_t* total_out = nullptr, const uint32_t* n_dev = nullptr, bool flags = false,
                     uint32_t* err = nullptr);
+// Stable sort of n keys below 2^end_bit with their values, in one launch of at most `cus`
+// workgroups or several.  tmp (radix_tmp_words) and meet (radix_meet_words) start zeroed and are
+// left ready for the next call; tmp is zeroed anew before a call with another n.  Returns 1 when
+// the sorted result lives in the *_alt buffers.
 size_t radix_tmp_words(uint32_t n);
-// Returns 1 when the sorted result lives in the *_alt buffers.  `n` is the
-// capacity the grid is sized for; with n_dev the element count is read on the
-// device (min(*n_dev, n)), so the launch needs no host synchronisation.
+size_t radix_meet_words();
+// Allows the sorts their LDS (once per process); 0 on failure.
+int radix_setup();
 int radix_sort_u64(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt, uint32_t n, int end_bit,
-                   uint32_t* tmp, hipStream_t s, const uint32_t* n_dev = nullptr, uint32_t* err = nullptr);
+                   uint32_t* tmp, uint32_t* meet, uint32_t cus, hipStream_t s, uint32_t* err = nullptr);
 int radix_sort_u32(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt, uint32_t n, int end_bit,
-                   uint32_t* tmp, hipStream_t s, const uint32_t* n_dev = nullptr, uint32_t* err = nullptr);
+                   uint32_t* tmp, uint32_t* meet, uint32_t cus, hipStream_t s, uint32_t* err = nullptr);
+// The solve order: the step's manifolds (at most cap, counted on the device) sorted by colour
+// and, with the split, the small islands' after the others, island by island; keys in key,
+// manifold indices in val.  root_bits: bits of a body index.
+void sort_solve_order(const Bodies& B, const uint2* m_ab, const uint32_t* col, uint32_t cap, uint32_t split, int root_bits,
+                      uint32_t* key, uint32_t* val, uint32_t* key_alt, uint32_t* val_alt, uint32_t* meet, uint32_t cus,
+                      Counters* cnt, hipStream_t s);
 
 }  // namespace axm

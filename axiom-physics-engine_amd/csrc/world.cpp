@@ -138,7 +138,8 @@ struct axm_world_s {
     uint32_t* col = nullptr;
     uint32_t* clist = nullptr;  // colouring: the manifolds not kept from the previous step
     uint64_t *prio = nullptr, *bmax0 = nullptr, *bmax1 = nullptr, *bmask = nullptr;
-    uint32_t *ckey = nullptr, *ckey_alt = nullptr, *cval = nullptr, *cval_alt = nullptr, *csort_tmp = nullptr;
+    uint32_t *ckey = nullptr, *ckey_alt = nullptr, *cval = nullptr, *cval_alt = nullptr;
+    uint32_t* sort_meet = nullptr;  // the one-launch sorts' meeting words and digit counts
     uint2* isl_list = nullptr;  // the small islands' work lists (first slot, manifolds)
     unsigned long long* isl_arrive = nullptr;  // arrival words of those in the register sweep
     const uint32_t* solve_order = nullptr;  // the sort output holding the last step's solve order
@@ -451,7 +452,6 @@ axm_status alloc_manifolds(axm_world_s* w, uint32_t cap) {
     w->mem.release(w->ckey_alt);
     w->mem.release(w->cval);
     w->mem.release(w->cval_alt);
-    w->mem.release(w->csort_tmp);
     w->mem.release(w->isl_list);
     w->mem.release(w->isl_arrive);
     AXM_TRY(w->mem.get(w->m_ab, cap));
@@ -465,10 +465,8 @@ axm_status alloc_manifolds(axm_world_s* w, uint32_t cap) {
     AXM_TRY(w->mem.get(w->ckey_alt, cap));
     AXM_TRY(w->mem.get(w->cval, cap));
     AXM_TRY(w->mem.get(w->cval_alt, cap));
-    AXM_TRY(w->mem.get(w->csort_tmp, radix_tmp_words(cap)));
     AXM_TRY(w->mem.get(w->isl_list, cap));
     AXM_TRY(w->mem.get(w->isl_arrive, isl_arrive_words(cap)));
-    if (hipMemset(w->csort_tmp, 0, 4 * radix_tmp_words(cap)) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
     w->cap_man = cap;
     if (w->rcap[w->cur] < cap) AXM_TRY(alloc_rows(w, w->cur, cap));
     if (w->rcap[1 - w->cur] > 0 && w->rcap[1 - w->cur] < cap) AXM_TRY(grow_rows_keep(w, 1 - w->cur, cap));
@@ -575,12 +573,14 @@ void enqueue_broad(axm_world_s* w, const StepParams& sp) {
     SortedKeys skey;
     int alt;
     if (k32) {
-        alt = radix_sort_u32(key32, w->val, key32_alt, w->val_alt, n, 30, w->sort_tmp, s, nullptr, &w->cnt->sticky);
+        alt = radix_sort_u32(key32, w->val, key32_alt, w->val_alt, n, 30, w->sort_tmp, w->sort_meet,
+                             (uint32_t)w->cu_count, s,
+                             &w->cnt->sticky);
         skey.k32 = alt ? key32_alt : key32;
     } else {
         const int end_bit = 30 + bits_for(w->n_worlds > 1 ? w->n_worlds - 1 : 0);
-        alt = radix_sort_u64(w->key, w->val, w->key_alt, w->val_alt, n, end_bit, w->sort_tmp, s, nullptr,
-                             &w->cnt->sticky);
+        alt = radix_sort_u64(w->key, w->val, w->key_alt, w->val_alt, n, end_bit, w->sort_tmp,
+                             w->sort_meet, (uint32_t)w->cu_count, s, &w->cnt->sticky);
         skey.k64 = alt ? w->key_alt : w->key;
     }
     const uint32_t* sval = alt ? w->val_alt : w->val;
@@ -650,12 +650,10 @@ axm_status enqueue_pre(axm_world_s* w, const StepParams& sp, const StepOpts& o) 
     const uint32_t split = island_split(w);
     launch_colour(w->B, w->m_ab, w->cap_man, w->col, w->prio, w->bmax0, w->bmax1, w->bmask, w->bdone, w->clist,
                   w->bar, w->cnt, w->colour_blocks, pca, split, s);
-    launch_col_sort_input(w->B, w->m_ab, w->col, w->cap_man, w->ckey, w->cval, w->cnt, split, s);
-    radix_sort_u32(w->ckey, w->cval, w->ckey_alt, w->cval_alt, w->cap_man, split ? 32 : 8, w->csort_tmp, s,
-                   &w->cnt->m_eff, &w->cnt->sticky);
-    // an odd number of 8-bit passes leaves the result in the alternate buffers
-    const uint32_t* scol = split ? w->ckey : w->ckey_alt;
-    const uint32_t* order = split ? w->cval : w->cval_alt;
+    sort_solve_order(w->B, w->m_ab, w->col, w->cap_man, split, bits_for(n ? n - 1 : 0), w->ckey, w->cval, w->ckey_alt, w->cval_alt,
+                     w->sort_meet, (uint32_t)w->cu_count, w->cnt, s);
+    const uint32_t* scol = w->ckey;
+    const uint32_t* order = w->cval;
     w->solve_order = order;
     w->solve_keys = scol;
     // ---- solver
@@ -1050,7 +1048,7 @@ axm_status axm_world_create(const axm_world_desc* desc, axm_world* out) {
     w->max_lds = (uint32_t)std::min<size_t>(prop.sharedMemPerBlock, 160u * 1024u);
     w->sweep_lds = w->max_lds & ~16383u;
     const int own_per_cu = pgs_own_setup(w->max_lds, w->sweep_lds);
-    if (own_per_cu < 1 || pgs_flow_setup() < 1 || !pgs_islands_setup() || !isl_union_setup()) {
+    if (own_per_cu < 1 || pgs_flow_setup() < 1 || !pgs_islands_setup() || !isl_union_setup() || !radix_setup()) {
         delete w;
         return AXM_GPU_OPERATION_FAILED;
     }
@@ -1066,6 +1064,7 @@ axm_status axm_world_create(const axm_world_desc* desc, axm_world* out) {
     axm_status st = w->mem.get(w->cnt, 1);
     if (st == AXM_SUCCESS) st = w->mem.get(w->bar, 1);
     if (st == AXM_SUCCESS) st = w->mem.get(w->pkinds, 32);
+    if (st == AXM_SUCCESS) st = w->mem.get(w->sort_meet, radix_meet_words());
     if (st == AXM_SUCCESS) st = w->mem.get(w->col_off, MAX_SORT_COLOURS + 2);
     if (st == AXM_SUCCESS) st = alloc_bodies(w, std::max<uint32_t>(desc->max_bodies, 16u));
     // explicit capacities are honoured as given; 0 means "sized from the body count"
@@ -1073,7 +1072,8 @@ axm_status axm_world_create(const axm_world_desc* desc, axm_world* out) {
     if (st == AXM_SUCCESS) st = alloc_manifolds(w, desc->max_manifolds ? desc->max_manifolds : 1024u);
     if (st == AXM_SUCCESS && w->rcap[1 - w->cur] < w->cap_man) st = alloc_rows(w, 1 - w->cur, w->cap_man);
     if (st == AXM_SUCCESS && (hipMemset(w->cnt, 0, sizeof(Counters)) != hipSuccess ||
-                              hipMemset(w->bar, 0, sizeof(GridBar)) != hipSuccess))
+                              hipMemset(w->bar, 0, sizeof(GridBar)) != hipSuccess ||
+                              hipMemset(w->sort_meet, 0, 4 * radix_meet_words()) != hipSuccess))
         st = AXM_GPU_OPERATION_FAILED;
     if (st != AXM_SUCCESS) {
         delete w;
@@ -1212,6 +1212,8 @@ axm_status install_bodies(axm_world_s* w, uint32_t n, uint32_t nw, float cell, b
         AXM_HIP(hipMemcpyAsync(w->B.wake, hb->wake.data(), 4ull * n, hipMemcpyHostToDevice, s));
     }
     AXM_HIP(hipMemsetAsync(w->cnt, 0, sizeof(Counters), s));
+    // the body sort's scratch lies by the body count
+    if (n != w->n) AXM_HIP(hipMemsetAsync(w->sort_tmp, 0, 4 * radix_tmp_words(w->cap_n), s));
     // the tables' entry counts are zero now: empty the tables in full
     for (int set = 0; set < 2; ++set)
         if (w->pc_key[set]) AXM_HIP(hipMemsetAsync(w->pc_key[set], 0xFF, 8ull * (w->pc_mask[set] + 1), s));
