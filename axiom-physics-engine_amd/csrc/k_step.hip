@@ -1082,7 +1082,7 @@ __global__ void __launch_bounds__(256) k_colour(Bodies B, const uint2* __restric
     }
 }
 
-// Size classes of the islands of more than ISLAND_LANE_MAX manifolds (k_pgs_islands solves
+// Size classes of the islands of more than ISLAND_LANE_MAX manifolds (islands_part solves
 // the largest first): 0 above 256 manifolds, 1 above 64, 2 above 32, 3 above 16, 4 the rest.
 // Their work list entries (first slot, manifolds) lie in one region per class, each as long as
 // the manifold capacity allows islands of its class.
@@ -1804,8 +1804,7 @@ __device__ __forceinline__ uint32_t next_colour(unsigned long long mk, uint32_t 
 // Before a launch, per slot of [s0, s1): the next visit of each dynamic body, and the inbox
 // words: a body's first visit (rank 0) gets the body's solver velocity with version 0, every
 // other inbox a version no visit waits for.  The rows exist only when this step's preparation
-// ran.  (Thread gid of gsz; also run by the small islands' kernel, k_pgs_islands, whose own
-// bodies and slots are disjoint from these.)
+// ran.  (Thread gid of gsz.)
 __device__ __forceinline__ void flow_init_part(const Bodies& B, const SolverRows& R, const uint64_t* __restrict__ bmask,
                                                uint32_t s0, uint32_t s1, uint32_t gid, uint32_t gsz) {
     for (uint32_t s = s0 + gid; s < s1; s += gsz) {
@@ -1840,12 +1839,7 @@ __device__ __forceinline__ void flow_init_part(const Bodies& B, const SolverRows
     q[3] = make_uint4((uint32_t)ob[2], (uint32_t)(ob[2] >> 32), (uint32_t)ob[3], (uint32_t)(ob[3] >> 32));
     }
 }
-__global__ void __launch_bounds__(256) k_flow_init(Bodies B, SolverRows R, const uint64_t* __restrict__ bmask,
-                                                   const Counters* __restrict__ cnt) {
-    if (cnt->sticky != 0u) return;
-    flow_init_part(B, R, bmask, 0u, cnt->m_glob, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
-}
-// Launch shape of the register sweep (k_pgs_flow).
+// Launch shape of the register sweep (flow_part).
 constexpr uint32_t FLOW_THREADS = 512, FLOW_WAVES = FLOW_THREADS / 64u;
 constexpr uint32_t FLOW_WAVE_SLOTS = 32;
 // Pieces of 32 slots of the islands of the largest class that the register sweep takes on G
@@ -1859,6 +1853,19 @@ __device__ __forceinline__ uint32_t wide_pieces(const Counters* cnt, uint32_t G)
     if (cnt->max_colour > 64u) return 0u;
     const bool fits = nl <= G * FLOW_WAVES && nl + w <= G * FLOW_WAVES;
     return fits || (uint64_t)cnt->isl_most * 50u > (uint64_t)w * FLOW_WAVE_SLOTS ? w : 0u;
+}
+// The large islands' slots and, when the register sweep takes them, those of the islands of the
+// largest class, whose arrival words start from zero.  G: the workgroups of the solve launch.
+__global__ void __launch_bounds__(256) k_flow_init(Bodies B, SolverRows R, const uint64_t* __restrict__ bmask,
+                                                   const Counters* __restrict__ cnt, const uint2* __restrict__ list,
+                                                   unsigned long long* __restrict__ isl_arrive, uint32_t G) {
+    if (cnt->sticky != 0u) return;
+    flow_init_part(B, R, bmask, 0u, cnt->m_glob, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
+    if (!list || wide_pieces(cnt, G) == 0u) return;
+    for (uint32_t i = blockIdx.x; i < cnt->isl_n[0]; i += gridDim.x) {
+        flow_init_part(B, R, bmask, list[i].x, list[i].x + list[i].y, threadIdx.x, blockDim.x);
+        if (threadIdx.x < 2u) isl_arrive[(size_t)i * ISL_ARRIVE_WORDS + threadIdx.x * (ISL_ARRIVE_WORDS / 2u)] = 0ull;
+    }
 }
 // Residual of one contact point: the largest velocity-space change (impulse change
 // times the row's effective mass inverse) that one more visit would make along the
@@ -1980,7 +1987,7 @@ __global__ void __launch_bounds__(OWN_WAVE) k_pgs_own(Bodies B, StepParams sp, S
         return;
     }
     if (cnt->sticky != 0u || nsweeps == 0u) return;
-    if (M > 0u && M <= flow_slots) return;  // k_pgs_flow ran them
+    if (M > 0u && M <= flow_slots) return;  // flow_part ran them
     if (M == 0u && cnt->m_eff > 0u) {
         // every island was solved on its own: no sweep of the large ones runs
         if (blockIdx.x == 0 && lane == 0 && stop.bits) {
@@ -2498,7 +2505,7 @@ __device__ __forceinline__ void block_max_sum(uint32_t& mx, uint32_t& sum, uint3
 // stays on chip: rows and impulses in registers (a lane visits the same slot in every sweep),
 // body velocities in LDS.  Velocities and impulses go back to memory once per island.  Above
 // 256 manifolds a CU no longer holds the rows (240 B per point): those islands run across CUs in
-// the large islands' register sweep (k_pgs_flow), or, when there are too many (wide_pieces), here
+// the large islands' register sweep (flow_part), or, when there are too many (wide_pieces), here
 // with the rows read at each visit.
 //
 // Work is taken largest first, so that the long solves start early and the short ones fill
@@ -3298,34 +3305,33 @@ __device__ __forceinline__ void memory_island(const Bodies& B, const StepParams&
     if (t == 0u) acc.add(it, res, tol_mode && !(res <= tol), pts);
 }
 
-__global__ void __launch_bounds__(ISL_THREADS, 2)
-k_pgs_islands(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap, const uint2* __restrict__ list,
-              const uint32_t* __restrict__ skey, float tol, uint32_t max_sweeps, const uint64_t* __restrict__ bmask,
-              uint32_t flow_init, unsigned long long* __restrict__ isl_arrive) {
-    extern __shared__ __align__(16) unsigned char isl_lds[];
-    if (cnt->sticky != 0u) return;
+// wide: the register sweep takes the islands of the largest class.  The workgroups below `late`
+// have swept large islands first: the others share the work out among themselves at the start,
+// they take what is left.
+__device__ __forceinline__ void islands_part(const Bodies& B, const StepParams& sp, const SolverRows& R, Counters* cnt,
+                                             uint32_t cap, const uint2* __restrict__ list,
+                                             const uint32_t* __restrict__ skey, float tol, uint32_t max_sweeps,
+                                             const uint64_t* __restrict__ bmask, bool wide, uint32_t late,
+                                             unsigned char* isl_lds) {
     const uint32_t t = threadIdx.x, lane = t & 63u;
+    const uint32_t first = gridDim.x - late;  // workgroups that start with the islands
+    const bool is_late = blockIdx.x < late;
     // the row preparation records no first visits when there are more colours than mask bits
     const bool masks = cnt->max_colour <= 64u;
-    // with flow_init, the sweep launch that follows is prepared here: the large islands (as
-    // k_flow_init) and, when it takes them, the islands of the largest class
-    const bool wide = flow_init != 0u && wide_pieces(cnt, gridDim.x) != 0u;
-    if (flow_init) {
-        const uint32_t gid = blockIdx.x * blockDim.x + t, gsz = gridDim.x * blockDim.x;
-        flow_init_part(B, R, bmask, 0u, cnt->m_glob, gid, gsz);
-        if (wide)
-            for (uint32_t i = blockIdx.x; i < cnt->isl_n[0]; i += gridDim.x) {
-                flow_init_part(B, R, bmask, list[i].x, list[i].x + list[i].y, t, blockDim.x);
-                if (t < 2u) isl_arrive[(size_t)i * ISL_ARRIVE_WORDS + t * (ISL_ARRIVE_WORDS / 2u)] = 0ull;
-            }
-    }
     IslandAcc acc = {0u, 0u, 0u, 0u, 0ull};
     GroupLds& G = *reinterpret_cast<GroupLds*>(isl_lds);
     const uint32_t n0 = wide ? 0u : cnt->isl_n[0], n1 = cnt->isl_n[1], n2 = cnt->isl_n[2], n3 = cnt->isl_n[3], n4 = cnt->isl_n[4];
 
     // ---- islands of one workgroup each (without masks: every island of the list)
     const uint32_t n_wg = masks ? n0 + n1 : n0 + n1 + n2 + n3 + n4;
-    for (uint32_t w = blockIdx.x; w < n_wg;) {
+    uint32_t w0 = blockIdx.x - late;
+    if (is_late) {
+        if (t == 0u) G.next = first + (n_wg ? atomicAdd(&cnt->isl_wg_next, 1u) : 0u);
+        __syncthreads();
+        w0 = G.next;
+        __syncthreads();
+    }
+    for (uint32_t w = w0; w < n_wg;) {
         uint32_t c = 0, i = w;
         if (i >= n0) c = 1u, i -= n0;
         if (c == 1u && i >= n1) c = 2u, i -= n1;
@@ -3335,7 +3341,7 @@ k_pgs_islands(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap
         if (!masks) memory_island(B, sp, R, cap, tol, max_sweeps, skey, G.red, e, acc);
         else if (c == 0u) stream_island(B, sp.keep, R, cap, tol, max_sweeps, bmask, skey, isl_lds, e, acc);
         else pair_island(B, sp.keep, R, cap, tol, max_sweeps, bmask, skey, isl_lds, e, acc);
-        if (t == 0u) G.next = gridDim.x + atomicAdd(&cnt->isl_wg_next, 1u);
+        if (t == 0u) G.next = first + atomicAdd(&cnt->isl_wg_next, 1u);
         __syncthreads();
         w = G.next;
         __syncthreads();
@@ -3348,8 +3354,14 @@ k_pgs_islands(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap
     const uint32_t n64 = masks ? n2 : 0u, n32 = masks ? (n3 + 1u) / 2u : 0u, n16 = masks ? (n4 + 3u) / 4u : 0u;
     const uint32_t n_win = M > M0 ? (M - M0 + BUNDLE_SLOTS - 1u) / BUNDLE_SLOTS : 0u;
     const uint32_t n_wave = n64 + n32 + n16 + n_win;
-    const uint32_t waves = gridDim.x * ISL_WAVES;
-    for (uint32_t w = blockIdx.x + gridDim.x * (t >> 6); w < n_wave;) {
+    const uint32_t waves = first * ISL_WAVES;
+    uint32_t v0 = blockIdx.x - late + first * (t >> 6);
+    if (is_late) {
+        uint32_t nx = 0;
+        if (lane == 0u) nx = atomicAdd(&cnt->isl_wave_next, 1u);
+        v0 = waves + (uint32_t)__shfl((int)nx, 0, 64);
+    }
+    for (uint32_t w = v0; w < n_wave;) {
         // the next piece is asked for before this one is worked on
         uint32_t nx = 0;
         if (lane == 0u) nx = atomicAdd(&cnt->isl_wave_next, 1u);
@@ -3390,10 +3402,6 @@ k_pgs_islands(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap
     }
     island_flush(cnt, acc);
 }
-int pgs_islands_setup() {
-    return hipFuncSetAttribute((const void*)k_pgs_islands, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)ISL_LDS_BYTES) == hipSuccess ? 1 : 0;
-}
 
 // ---------------------------------------------------------------- large islands in registers
 // The large islands' sweeps when every slot has two lanes of the GPU to itself (FLOW_SLOTS
@@ -3427,23 +3435,27 @@ __device__ __forceinline__ u32x4_t flow_quad(const uint64_t* inbox, uint32_t byt
     // aux: sc0 | sc1, as vin_quad
     return __builtin_amdgcn_raw_buffer_load_b128(rs, (int)byte, 0, 1 | 16);
 }
+//
+// M: the slots of the large islands, wide: the pieces of the others, G: the workgroups that take
+// part (this one does).
+struct FlowLds {
+    uint32_t arrived, above, max;
+};
 template <bool CHECKS>
-__global__ void __launch_bounds__(FLOW_THREADS, 2)
-k_pgs_flow(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap, uint32_t nsweeps, uint32_t spin_limit,
-           const uint64_t* __restrict__ bmask, const uint2* __restrict__ list, SweepStop stop) {
-    __shared__ uint32_t s_arrived, s_above, s_max;
-    const uint32_t G = gridDim.x, C = G * FLOW_WAVES;
-    if (cnt->max_colour > 64u || cnt->sticky != 0u || nsweeps == 0u) return;
-    const uint32_t M = cnt->m_glob <= C * FLOW_WAVE_SLOTS ? cnt->m_glob : 0u;  // more: k_pgs_own
+__device__ __forceinline__ void flow_part(const Bodies& B, const StepParams& sp, const SolverRows& R, Counters* cnt,
+                                          uint32_t cap, uint32_t nsweeps, uint32_t spin_limit,
+                                          const uint64_t* __restrict__ bmask, const uint2* __restrict__ list,
+                                          const SweepStop& stop, uint32_t M, uint32_t wide, uint32_t G, FlowLds& L) {
+    uint32_t &s_arrived = L.arrived, &s_above = L.above, &s_max = L.max;
+    const uint32_t C = G * FLOW_WAVES;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     // Piece v is slots 32 v on of the large islands, or, from piece nl on, 32 slots of an island
     // of the work list.  Wave w works on pieces w, w + C, ... in turn (C: the waves of the grid;
     // the large islands are in the first round).  An island's pieces wait only for each other,
     // and every wave comes to them through pieces of earlier islands, so none waits for ever.
     // Neighbouring waves (the same colour) lie on different CUs.
-    const uint32_t nl = (M + FLOW_WAVE_SLOTS - 1u) / FLOW_WAVE_SLOTS, nw = nl + (list ? wide_pieces(cnt, G) : 0u);
+    const uint32_t nl = (M + FLOW_WAVE_SLOTS - 1u) / FLOW_WAVE_SLOTS, nw = nl + wide;
     const uint32_t wid = wave * G + blockIdx.x;
-    if (blockIdx.x >= nw) return;  // the whole workgroup has nothing
     const uint32_t wg_waves = blockIdx.x < nl ? (nl - blockIdx.x + G - 1u) / G : 0u;  // with slots of the large islands
     if (threadIdx.x == 0u) s_arrived = s_above = s_max = 0u;
     __syncthreads();
@@ -3757,9 +3769,57 @@ k_pgs_flow(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap, u
     }
     }
 }
-int pgs_flow_setup() {
+// Both: the large islands by the first workgroups, the others by the rest, and by the first
+// when they are done (parts: 1 the large islands, 2 the others, 3 both at once).  Neither fills
+// the chip for its whole length: the sweeps of the large islands are one chain, and the others end
+// in a tail of the slowest.  One after the other and at once: 100000 bodies (20 sweeps, 21k slots
+// in large islands and 55k in others) 585 -> 471 us, 256 worlds at 1e-4 2050 -> 1170.
+template <bool CHECKS>
+__global__ void __launch_bounds__(FLOW_THREADS, 2)
+k_pgs_solve(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap, uint32_t nsweeps, uint32_t spin_limit,
+            const uint64_t* __restrict__ bmask, const uint2* __restrict__ list, const uint32_t* __restrict__ skey,
+            float tol, uint32_t parts, uint32_t wide_on, SweepStop stop) {
+    static_assert(FLOW_THREADS == ISL_THREADS, "one launch shape");
+    extern __shared__ __align__(16) unsigned char isl_lds[];
+    if (cnt->sticky != 0u || nsweeps == 0u) return;
+    const uint32_t G = gridDim.x;
+    const uint32_t wide = list && wide_on ? wide_pieces(cnt, G) : 0u;
+    uint32_t flows = 0;  // workgroups that sweep the large islands
+    if ((parts & 1u) && cnt->max_colour <= 64u) {
+        const uint32_t M = cnt->m_glob <= G * FLOW_WAVES * FLOW_WAVE_SLOTS ? cnt->m_glob : 0u;  // more: k_pgs_own
+        const uint32_t nw = (M + FLOW_WAVE_SLOTS - 1u) / FLOW_WAVE_SLOTS + wide;
+        // as thinly as the chip allows (a visit's wave holds up the others of its SIMD: 19.1k slots
+        // on 75 workgroups take 24 us per sweep, on 256 21), but with a workgroup left for every 490
+        // slots of the other islands, which take about as long then (a slot costs a workgroup 42
+        // ns per sweep, a sweep of the large islands is 20 us)
+        const uint32_t other = min(cnt->m_eff, cap) - min(min(cnt->m_eff, cap), M + wide * FLOW_WAVE_SLOTS);
+        const uint32_t least = (nw + FLOW_WAVES - 1u) / FLOW_WAVES;
+        flows = min(min(G, nw), max(least, G - min(G, (parts & 2u) ? (other + 489u) / 490u : 0u)));
+        if (blockIdx.x < flows)
+            flow_part<CHECKS>(B, sp, R, cnt, cap, nsweeps, spin_limit, bmask, list, stop, M, wide, flows,
+                              *reinterpret_cast<FlowLds*>(isl_lds));
+    }
+    if (!(parts & 2u)) return;
+    if (blockIdx.x < flows) {
+        // every wave is done with its pieces; a sweep that gave up ends the launch here
+        uint32_t* bad = reinterpret_cast<uint32_t*>(isl_lds);
+        __syncthreads();
+        if (threadIdx.x == 0u) *bad = __hip_atomic_load(&cnt->sticky, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (*bad != 0u) return;
+        __syncthreads();
+    }
+    islands_part(B, sp, R, cnt, cap, list, skey, tol, nsweeps, bmask, wide != 0u, flows, isl_lds);
+}
+// Allows the solve launch its LDS and returns how many of its workgroups fit on one CU (0 on error).
+int pgs_solve_setup() {
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_pgs_flow<true>, FLOW_THREADS, 0) != hipSuccess) return 0;
+    if (hipFuncSetAttribute((const void*)k_pgs_solve<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)ISL_LDS_BYTES) != hipSuccess ||
+        hipFuncSetAttribute((const void*)k_pgs_solve<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)ISL_LDS_BYTES) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_pgs_solve<true>, FLOW_THREADS, ISL_LDS_BYTES) != hipSuccess)
+        return 0;
     return nb;
 }
 
@@ -4161,16 +4221,6 @@ void launch_colour(const Bodies& B, const uint2* m_ab, uint32_t cap_man, uint32_
     hipLaunchKernelGGL(k_colour, dim3(blocks), dim3(256), 0, s, B, m_ab, col, prio, bmax0, bmax1, bmask, list, bar,
                        cnt, 65000u, SMALL);
 }
-void launch_pgs_local(const Bodies& B, const StepParams& sp, const SolverRows& R, Counters* cnt, uint32_t cap,
-                      const uint32_t* skey, uint2* list, float tol, uint32_t max_sweeps, uint32_t groups,
-                      hipStream_t s, const uint64_t* bmask, bool flow_init, unsigned long long* isl_arrive,
-                      hipEvent_t ev0, hipEvent_t ev1) {
-    if (max_sweeps == 0u) return;
-    if (ev0) (void)hipEventRecord(ev0, s);
-    hipLaunchKernelGGL(k_pgs_islands, dim3(groups), dim3(ISL_THREADS), ISL_LDS_BYTES, s, B, sp, R, cnt, cap, list, skey,
-                       tol, max_sweeps, bmask, flow_init ? 1u : 0u, isl_arrive);
-    if (ev1) (void)hipEventRecord(ev1, s);
-}
 void launch_prep(const Bodies& B, const StepParams& sp, const uint32_t* order, uint32_t cap, const uint2* m_ab,
                  const uint32_t* m_np, const float4* c_pt, const float4* c_nf, const SolverRows& R,
                  const PrevCacheArgs& pca, const float4* warm_in, const uint32_t* col, const uint64_t* bmask,
@@ -4224,22 +4274,26 @@ int pgs_own_setup(uint32_t max_lds_bytes, uint32_t lds_bytes) {
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_pgs_own, OWN_WAVE, lds_bytes) != hipSuccess) return 0;
     return nb;
 }
-void launch_pgs_flow(const Bodies& B, const StepParams& sp, const SolverRows& R, uint32_t cap, const uint64_t* bmask,
-                     uint32_t nsweeps, Counters* cnt, uint32_t spin_limit, uint32_t cus, uint32_t groups,
-                     uint32_t lds_bytes, uint32_t tune, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1,
-                     const SweepStop& stop, const uint2* list) {
+void launch_flow_init(const Bodies& B, const SolverRows& R, uint32_t cap, const uint64_t* bmask, const Counters* cnt,
+                      const uint2* list, unsigned long long* isl_arrive, uint32_t cus, hipStream_t s) {
+    hipLaunchKernelGGL(k_flow_init, grid_bounded(cap), dim3(256), 0, s, B, R, bmask, cnt, list, isl_arrive, cus);
+}
+void launch_pgs_solve(const Bodies& B, const StepParams& sp, const SolverRows& R, uint32_t cap, const uint64_t* bmask,
+                      uint32_t nsweeps, Counters* cnt, uint32_t spin_limit, uint32_t cus, const uint32_t* skey,
+                      const uint2* list, float tol, uint32_t parts, bool wide, const OwnShape& own, const SweepStop& stop,
+                      hipStream_t s, hipEvent_t ev0, hipEvent_t ev1) {
     if (!nsweeps) return;
-    if (!list) hipLaunchKernelGGL(k_flow_init, grid_bounded(cap), dim3(256), 0, s, B, R, bmask, cnt);
     if (ev0) (void)hipEventRecord(ev0, s);
     if (stop.bits)
-        hipLaunchKernelGGL(k_pgs_flow<true>, dim3(cus), dim3(FLOW_THREADS), 0, s, B, sp, R, cnt, cap, nsweeps,
-                           spin_limit, bmask, list, stop);
+        hipLaunchKernelGGL(k_pgs_solve<true>, dim3(cus), dim3(FLOW_THREADS), ISL_LDS_BYTES, s, B, sp, R, cnt, cap, nsweeps,
+                           spin_limit, bmask, list, skey, tol, parts, wide ? 1u : 0u, stop);
     else
-        hipLaunchKernelGGL(k_pgs_flow<false>, dim3(cus), dim3(FLOW_THREADS), 0, s, B, sp, R, cnt, cap, nsweeps,
-                           spin_limit, bmask, list, stop);
-    hipLaunchKernelGGL(k_pgs_own, dim3(groups ? groups : 1u), dim3(OWN_WAVE), lds_bytes, s, B, sp, R, cnt, cap, nsweeps,
-                       cus * FLOW_WAVES * FLOW_WAVE_SLOTS, lds_bytes / (uint32_t)sizeof(float4), spin_limit, tune, bmask,
-                       stop);
+        hipLaunchKernelGGL(k_pgs_solve<false>, dim3(cus), dim3(FLOW_THREADS), ISL_LDS_BYTES, s, B, sp, R, cnt, cap, nsweeps,
+                           spin_limit, bmask, list, skey, tol, parts, wide ? 1u : 0u, stop);
+    if (parts & SOLVE_LARGE)
+        hipLaunchKernelGGL(k_pgs_own, dim3(own.groups ? own.groups : 1u), dim3(OWN_WAVE), own.lds_bytes, s, B, sp, R, cnt,
+                           cap, nsweeps, cus * FLOW_WAVES * FLOW_WAVE_SLOTS, own.lds_bytes / (uint32_t)sizeof(float4),
+                           spin_limit, own.tune, bmask, stop);
     if (ev1) (void)hipEventRecord(ev1, s);
 }
 void launch_pgs(const Bodies& B, const StepParams& sp, const SolverRows& R, uint32_t s0, uint32_t s1, uint32_t cap,

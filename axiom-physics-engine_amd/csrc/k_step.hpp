@@ -104,15 +104,6 @@ int colour_blocks_per_cu();
 void launch_colour(const Bodies& B, const uint2* m_ab, uint32_t cap_man, uint32_t* col, uint64_t* prio,
                    uint64_t* bmax0, uint64_t* bmax1, uint64_t* bmask, uint32_t* bdeg, uint32_t* list, GridBar* bar,
                    Counters* cnt, uint32_t blocks, const PrevCacheArgs& prev, uint32_t split, hipStream_t s);
-// The islands solved on their own (after the row preparation, which built their work list),
-// in `groups` workgroups (one per CU): tol > 0 stops each at its own residual.  bmask holds
-// the colouring's per-body colour masks.  With flow_init, the same launch also sets up the
-// launch_pgs_flow that follows, which then solves the list's largest class too (isl_arrive: its
-// arrival words).  Events ev0 / ev1, when given, are recorded around it.
-void launch_pgs_local(const Bodies& B, const StepParams& sp, const SolverRows& R, Counters* cnt, uint32_t cap,
-                      const uint32_t* skey, uint2* list, float tol, uint32_t max_sweeps, uint32_t groups,
-                      hipStream_t s, const uint64_t* bmask, bool flow_init, unsigned long long* isl_arrive,
-                      hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
 // Work the row preparation launch also does for the launches after it, each in a loop of
 // its own over the grid: the colour offsets of the sorted keys skey (col_off[c] = first
 // position whose key has colour >= c, c = 0..K, and m_glob = col_off[K], when col_off is
@@ -163,24 +154,34 @@ struct SweepStop {
     float tol = -1.0f;
     uint32_t every = 1;
 };
-// The large islands' sweeps.  Up to cus x 256 slots run with one slot per pair of lanes (`cus`
-// workgroups of 512 threads, all resident at once, see pgs_flow_setup); more in the staged
-// sweep: `groups` workgroups of one wave, each with `lds_bytes` of LDS for its staged rows; all
-// of them must be resident at once (see pgs_own_setup).  Events ev0 / ev1, when given, are
-// recorded around both.  With the work list of the islands solved on their own, this step's
-// launch_pgs_local (with flow_init) has set up the inboxes and next visits and left the islands
-// of the largest class to this launch.
-void launch_pgs_flow(const Bodies& B, const StepParams& sp, const SolverRows& R, uint32_t cap, const uint64_t* bmask,
-                     uint32_t nsweeps, Counters* cnt, uint32_t spin_limit, uint32_t cus, uint32_t groups,
-                     uint32_t lds_bytes, uint32_t tune, hipStream_t s, hipEvent_t ev0 = nullptr,
-                     hipEvent_t ev1 = nullptr, const SweepStop& stop = SweepStop{}, const uint2* list = nullptr);
-// Workgroups of the register sweep that fit on one CU (0 on error).
-int pgs_flow_setup();
+// Prepares the large islands' sweeps (after the row preparation): inboxes and next visits, with
+// the work list also those of the islands of its largest class that the solve launch of `cus`
+// workgroups will take (isl_arrive: their arrival words).
+void launch_flow_init(const Bodies& B, const SolverRows& R, uint32_t cap, const uint64_t* bmask, const Counters* cnt,
+                      const uint2* list, unsigned long long* isl_arrive, uint32_t cus, hipStream_t s);
+// Shape of the staged sweep: `groups` workgroups of one wave, each with `lds_bytes` of LDS for
+// its staged rows; all of them must be resident at once (see pgs_own_setup).
+struct OwnShape {
+    uint32_t groups, lds_bytes, tune;
+};
+// The solver's sweeps, in `cus` workgroups of 512 threads, all resident at once (see
+// pgs_solve_setup).  SOLVE_LARGE: the large islands; up to cus x 256 slots run with one slot per
+// pair of lanes, more in the staged sweep.  SOLVE_LIST: the islands of the work list and the small
+// ones, which tol > 0 stops each at its own residual.  With `wide` the register sweep takes the
+// islands of the list's largest class when that is faster (launch_flow_init has prepared them);
+// parts in launches of their own name the same.  bmask holds the colouring's per-body colour
+// masks.  Events ev0 / ev1, when given, are recorded around the launch.
+constexpr uint32_t SOLVE_LARGE = 1u, SOLVE_LIST = 2u;
+void launch_pgs_solve(const Bodies& B, const StepParams& sp, const SolverRows& R, uint32_t cap, const uint64_t* bmask,
+                      uint32_t nsweeps, Counters* cnt, uint32_t spin_limit, uint32_t cus, const uint32_t* skey,
+                      const uint2* list, float tol, uint32_t parts, bool wide, const OwnShape& own, const SweepStop& stop,
+                      hipStream_t s, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr);
+// Allows the solve launch its LDS; its workgroups that fit on one CU (0 on error).
+int pgs_solve_setup();
 // Raises the sweep kernel's dynamic-LDS limit to max_lds_bytes and returns how many of
 // its workgroups with lds_bytes each fit on one CU (0 on error).
 int pgs_own_setup(uint32_t max_lds_bytes, uint32_t lds_bytes);
-// Allows the small islands' kernel its LDS (once per process); 0 on failure.
-int pgs_islands_setup();
+// Allows the islands' union its LDS; 0 on failure.
 int isl_union_setup();
 void launch_pgs(const Bodies& B, const StepParams& sp, const SolverRows& R, uint32_t s0, uint32_t s1, uint32_t cap,
                 uint32_t first, hipStream_t s);

@@ -150,7 +150,7 @@ struct Counters {
     uint32_t isl_wave_next;  // beyond the first piece of each
     uint32_t loc_points;   // contact points of the islands solved on their own
     unsigned long long loc_point_sweeps;     // their contact points x the sweeps each island ran
-    unsigned long long bundle_point_sweeps;  // the same for the islands of k_pgs_islands
+    unsigned long long bundle_point_sweeps;  // the same for the islands of islands_part
     // ---- kept across steps
     uint32_t sticky;       // STICKY_* bits; while set the integration is skipped (state untouched)
     uint32_t steps_done;   // steps whose integration ran

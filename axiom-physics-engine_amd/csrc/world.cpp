@@ -716,19 +716,28 @@ axm_status enqueue_step(axm_world_s* w, float dt, const StepOpts& o) {
     w->last_iters_dev = dev_checks;
     std::vector<uint32_t> off;
     if (pre) AXM_TRY(enqueue_pre(w, sp, o));
-    // the islands solved on their own run first; their launch also sets up the large
-    // islands' sweep launch (its inboxes and next visits)
-    const bool flow_inited = sweep && island_split(w) && !o.colour_launches;
-    if (sweep && island_split(w)) {
+    // the islands solved on their own run beside the large ones' sweeps, in the same launch; in one
+    // of their own when the sweeps are launched per colour, or timed
+    const bool split = island_split(w) != 0u;
+    const uint2* list = split && !o.colour_launches ? w->isl_list : nullptr;
+    const OwnShape own{w->sweep_groups, w->sweep_lds, w->sweep_tune};
+    const bool apart = split && (o.colour_launches || (w->prof_on && !o.capture));
+    auto init = [&]() {
+        launch_flow_init(w->B, R, rc, w->bmask, w->cnt, list, w->isl_arrive, (uint32_t)w->cu_count, s);
+    };
+    if (sweep && list) init();
+    if (sweep && apart) {
         hipEvent_t b0 = nullptr, b1 = nullptr;
         if (w->prof_on && !o.capture) {
             AXM_TRY(bundle_events(w, 0));
             b0 = w->bprof_ev[0];
             b1 = w->bprof_ev[1];
         }
-        launch_pgs_local(w->B, sp, R, w->cnt, rc, w->solve_keys, w->isl_list, w->desc.residual_tol, max_it,
-                         (uint32_t)w->cu_count, s, w->bmask, flow_inited, w->isl_arrive, b0, b1);
+        launch_pgs_solve(w->B, sp, R, rc, w->bmask, max_it, w->cnt, SWEEP_SPIN_LIMIT_US, (uint32_t)w->cu_count,
+                         w->solve_keys, w->isl_list, w->desc.residual_tol, SOLVE_LIST, list != nullptr, own, SweepStop{}, s,
+                         b0, b1);
     }
+    const uint32_t parts = SOLVE_LARGE | (split && !apart ? SOLVE_LIST : 0u);
     const bool want_res = (o.flags & AXM_STEP_RESIDUAL) || w->desc.record_residual || tol_mode;
     const uint32_t every = std::max<uint32_t>(w->desc.residual_every, 1u);
     uint32_t it = sweep ? 0u : max_it;
@@ -747,9 +756,9 @@ axm_status enqueue_step(axm_world_s* w, float dt, const StepOpts& o) {
         hipEvent_t e0, e1;
         AXM_TRY(prof_event(w, nev, o.capture, e0));
         AXM_TRY(prof_event(w, nev, o.capture, e1));
-        launch_pgs_flow(w->B, sp, R, rc, w->bmask, max_it, w->cnt, SWEEP_SPIN_LIMIT_US, (uint32_t)w->cu_count,
-                        w->sweep_groups, w->sweep_lds, w->sweep_tune, s, e0, e1, stop,
-                        flow_inited ? w->isl_list : nullptr);
+        if (!list) init();
+        launch_pgs_solve(w->B, sp, R, rc, w->bmask, max_it, w->cnt, SWEEP_SPIN_LIMIT_US, (uint32_t)w->cu_count,
+                         w->solve_keys, list, w->desc.residual_tol, parts, true, own, stop, s, e0, e1);
         it = max_it;  // at most; the count the launch ran is read back with the counters
     }
     bool all_local = false;
@@ -775,9 +784,9 @@ axm_status enqueue_step(axm_world_s* w, float dt, const StepOpts& o) {
             AXM_TRY(prof_event(w, nev, o.capture, e0));
             AXM_TRY(prof_event(w, nev, o.capture, e1));
             // (one segment: the host checks a residual between segments in the per-colour launches only)
-            launch_pgs_flow(w->B, sp, R, rc, w->bmask, seg, w->cnt, SWEEP_SPIN_LIMIT_US, (uint32_t)w->cu_count,
-                            w->sweep_groups, w->sweep_lds, w->sweep_tune, s, e0, e1, SweepStop{},
-                            flow_inited ? w->isl_list : nullptr);
+            if (!list) init();
+            launch_pgs_solve(w->B, sp, R, rc, w->bmask, seg, w->cnt, SWEEP_SPIN_LIMIT_US, (uint32_t)w->cu_count,
+                             w->solve_keys, list, w->desc.residual_tol, parts, true, own, SweepStop{}, s, e0, e1);
         }
         it += seg;
         const bool last = it == max_it;
@@ -1048,7 +1057,7 @@ axm_status axm_world_create(const axm_world_desc* desc, axm_world* out) {
     w->max_lds = (uint32_t)std::min<size_t>(prop.sharedMemPerBlock, 160u * 1024u);
     w->sweep_lds = w->max_lds & ~16383u;
     const int own_per_cu = pgs_own_setup(w->max_lds, w->sweep_lds);
-    if (own_per_cu < 1 || pgs_flow_setup() < 1 || !pgs_islands_setup() || !isl_union_setup() || !radix_setup()) {
+    if (own_per_cu < 1 || pgs_solve_setup() < 1 || !isl_union_setup() || !radix_setup()) {
         delete w;
         return AXM_GPU_OPERATION_FAILED;
     }
@@ -1357,13 +1366,18 @@ axm_status axm_world_run(axm_world w, float dt, uint32_t iters, uint32_t steps, 
                 const bool checks = sweep_checks(w, false, stop);
                 const uint32_t nsw = w->desc.residual_tol > 0.0f ? std::max<uint32_t>(w->desc.max_iterations, 1u)
                                                                  : iters;
+                // timed apart
+                const uint2* list = split ? w->isl_list : nullptr;
+                const OwnShape own{w->sweep_groups, w->sweep_lds, w->sweep_tune};
+                launch_flow_init(w->B, w->R[c], w->rcap[c], w->bmask, w->cnt, list, w->isl_arrive, (uint32_t)w->cu_count,
+                                 w->stream);
                 if (split)
-                    launch_pgs_local(w->B, sp, w->R[c], w->cnt, w->rcap[c], w->solve_keys, w->isl_list,
-                                     w->desc.residual_tol, nsw, (uint32_t)w->cu_count, w->stream, w->bmask, true,
-                                     w->isl_arrive, w->bprof_ev[2 * c], w->bprof_ev[2 * c + 1]);
-                launch_pgs_flow(w->B, sp, w->R[c], w->rcap[c], w->bmask, nsw, w->cnt, SWEEP_SPIN_LIMIT_US,
-                                (uint32_t)w->cu_count, w->sweep_groups, w->sweep_lds, w->sweep_tune, w->stream, w->gprof_ev[2 * c],
-                                w->gprof_ev[2 * c + 1], checks ? stop : SweepStop{}, split ? w->isl_list : nullptr);
+                    launch_pgs_solve(w->B, sp, w->R[c], w->rcap[c], w->bmask, nsw, w->cnt, SWEEP_SPIN_LIMIT_US,
+                                     (uint32_t)w->cu_count, w->solve_keys, list, w->desc.residual_tol, SOLVE_LIST, true, own,
+                                     SweepStop{}, w->stream, w->bprof_ev[2 * c], w->bprof_ev[2 * c + 1]);
+                launch_pgs_solve(w->B, sp, w->R[c], w->rcap[c], w->bmask, nsw, w->cnt, SWEEP_SPIN_LIMIT_US,
+                                 (uint32_t)w->cu_count, w->solve_keys, list, w->desc.residual_tol, SOLVE_LARGE, true, own,
+                                 checks ? stop : SweepStop{}, w->stream, w->gprof_ev[2 * c], w->gprof_ev[2 * c + 1]);
                 AXM_HIP(hipGraphLaunch(w->gpost[c], w->stream));
             } else {
                 AXM_HIP(hipGraphLaunch(w->gexec[c], w->stream));

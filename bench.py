@@ -12,9 +12,9 @@ The scene runs its 120 steps: 10 warm-up steps, then 110 timed steps replayed
 from hipGraphs.
 
 Prints one JSON line: body-steps/s at the tolerance and the fraction of steps
-that reached it, the roofline of the dominant kernel (the persistent sweep
-kernel k_pgs_own: 240 B per contact point per sweep, divided by its event-timed
-launch durations) and of the whole step (304 N + 104 P + 304 C + 12 R C +
+that reached it, the roofline of the dominant part of the solver's sweeps (240 B
+per contact point per sweep, divided by the event-timed durations of its
+launches) and of the whole step (304 N + 104 P + 304 C + 12 R C +
 240 I C bytes per step), the energy drift of one step against an FP64 CPU
 re-solve of the same manifolds, and the CPU oracle on the same workload (one
 thread and all host cores).  Further sections: the dense 100k-body pile at its
@@ -239,14 +239,14 @@ def headline(args):
     value = bodies.n * args.steps / elapsed
     steps_done = max(int(tot.steps), 1)
     mean_sweeps = tot.sweeps / steps_done
-    # the sweep kernels, 240 B per contact point per sweep each: the kernel of the small
+    # the sweeps (timed apart), 240 B per contact point per sweep each: those of the small
     # islands solved on their own (their points x the sweeps each island ran) and the persistent
     # sweep of the large islands (the rest); the roofline line is the one with more time
-    kern = {"k_pgs_own": (B_SWEEP * float(tot.contact_sweeps - tot.local_contact_sweeps), prof.pgs_ms * 1e-3,
-                          int(prof.pgs_launches))}
+    kern = {"k_pgs_solve (large islands)": (B_SWEEP * float(tot.contact_sweeps - tot.local_contact_sweeps),
+                                            prof.pgs_ms * 1e-3, int(prof.pgs_launches))}
     if prof.bundle_launches:
-        kern["k_pgs_islands"] = (B_SWEEP * float(prof.bundle_point_sweeps), prof.bundle_ms * 1e-3,
-                                int(prof.bundle_launches))
+        kern["k_pgs_solve (other islands)"] = (B_SWEEP * float(prof.bundle_point_sweeps), prof.bundle_ms * 1e-3,
+                                               int(prof.bundle_launches))
 
     def roof_of(name):
         nbytes, secs, n = kern[name]
