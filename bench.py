@@ -169,7 +169,8 @@ def committed_traffic(kernel, cfg, n, args):
     """HBM bytes per launch of `kernel` from the committed counter runs (FETCH_SIZE and WRITE_SIZE,
     each scaled by what it reads for a plain copy of known size), when they were taken on this
     exact workload; None otherwise."""
-    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles", "%s_scene%d_traffic.json" % (kernel, cfg))
+    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles",
+                        "%s_scene%d_traffic.json" % (kernel.split(" ")[0], cfg))
     try:
         with open(path) as f:
             t = json.load(f)
