@@ -280,8 +280,8 @@ axm_status alloc_bodies(axm_world_s* w, uint32_t cap) {
     AXM_TRY(w->mem.get(w->ct.bits, TB / 32u));
     w->ct.bmask = TB - 1;
     AXM_TRY(w->mem.get(w->ct.mlist, cap));
-    AXM_TRY(w->mem.get(w->ct.cstart, cap + 1));
-    AXM_TRY(w->mem.get(w->ct.crank, cap));
+    AXM_TRY(w->mem.get(w->ct.cstart, (size_t)cap + 1));
+    AXM_TRY(w->mem.get(w->ct.crank, (size_t)cap + 1));  // scanned in place: the total follows
     AXM_TRY(w->mem.get(w->pair_cnt, (size_t)BP_PARTS * cap));
     AXM_TRY(w->mem.get(w->pair_off, (size_t)BP_PARTS * cap + 1));
     AXM_TRY(w->mem.get(w->scan_tmp, scan_tmp_words(BP_PARTS * cap)));

@@ -52,3 +52,13 @@ def test_sorts(axm, gpu, sizes):
     for k, n in enumerate(sizes):
         _check(axm, w, n, k)
     w.close()
+
+
+def test_sort_arrays_end_at_a_page(axm, gpu):
+    """524288 bodies: the arrays of a word per body are whole pages, so a word written past one of
+    them (the total of the cell ranks' scan was) would be in a page of something else or of nothing."""
+    d = axm.default_desc()
+    d.gravity[0] = d.gravity[1] = d.gravity[2] = 0.0
+    w = axm.World(d)
+    _check(axm, w, 524288, 4)
+    w.close()
