@@ -562,88 +562,125 @@ __global__ void __launch_bounds__(RS_THREADS) k_radix_sort(S src, typename S::Ke
 
 // ---------------------------------------------------------------- per-pass sort
 // More given keys than RS_GIVEN: three launches a pass (per-tile digit counts, their scan, the
-// scatter) in small tiles that fill the chip.  A grid that meets writes back and drops every
-// XCD's L2 at each meeting, once per workgroup: 1M keys of 30 bits take 257 us so, 106 us in
-// launches; 100000 keys 52 and 65 us.
+// scatter).  A grid that meets writes back and drops every XCD's L2 at each meeting, once per
+// workgroup: 1M keys of 30 bits take 257 us so, 100000 52.  Digits of up to ten bits, so 30 bits
+// take three passes.  The scatter is bound by its write requests (1M random keys are 2M of them
+// a pass when each lane writes its own): a tile goes through LDS into digit order first and then
+// out in runs.  1M keys of 30 bits: 79 us (8-bit digits, tiles of 1024 keys written by lane: 106;
+// ten bits written by lane: 91); 600000 68 (83), 300000 65 (72), 140000 60 (65).
 constexpr uint32_t RS_GIVEN = 131072u;
-constexpr int RP_THREADS = 256, RP_ITEMS = 4, RP_TILE = RP_THREADS * RP_ITEMS;
-template <class K> __device__ __forceinline__ uint32_t digit_of(K k, int shift) { return (uint32_t)(k >> shift) & 0xFFu; }
+constexpr int RP_THREADS = 1024, RP_ITEMS = 4, RP_TILE = RP_THREADS * RP_ITEMS;
+constexpr int RP_BITS = 10, RP_DIGITS = 1 << RP_BITS;
 
-// Per-tile digit counts, digit-major: hist[d * nt + tile] for the nt tiles.
+// Per-tile digit counts, digit-major: hist[d * tiles + tile].
 template <class K>
-__global__ void __launch_bounds__(RP_THREADS) k_rs_hist(const K* __restrict__ keys, uint32_t n, int shift,
+__global__ void __launch_bounds__(RP_THREADS) k_rs_hist(const K* __restrict__ keys, uint32_t n, int shift, uint32_t mask,
                                                         uint32_t* __restrict__ hist) {
-    const uint32_t nt = (n + RP_TILE - 1) / RP_TILE;
-    __shared__ uint32_t h[256];
+    __shared__ uint32_t h[RP_DIGITS];
     h[threadIdx.x] = 0;
     __syncthreads();
     const uint32_t base = blockIdx.x * RP_TILE;
-#pragma unroll 4
+#pragma unroll
     for (int it = 0; it < RP_ITEMS; ++it) {
         const uint32_t i = base + it * RP_THREADS + threadIdx.x;
-        if (i < n) atomicAdd(&h[digit_of(keys[i], shift)], 1u);
+        if (i < n) atomicAdd(&h[(uint32_t)(keys[i] >> shift) & mask], 1u);
     }
     __syncthreads();
-    hist[(size_t)threadIdx.x * nt + blockIdx.x] = h[threadIdx.x];
+    hist[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = h[threadIdx.x];
 }
 
 template <class K>
 __global__ void __launch_bounds__(RP_THREADS) k_rs_scatter(const K* __restrict__ kin, const uint32_t* __restrict__ vin,
                                                            K* __restrict__ kout, uint32_t* __restrict__ vout, uint32_t n,
-                                                           int shift, const uint32_t* __restrict__ offs) {
-    const uint32_t nt = (n + RP_TILE - 1) / RP_TILE;
-    __shared__ uint32_t s_off[256];
-    __shared__ uint32_t s_wc[RP_THREADS / 64][256];
+                                                           int shift, uint32_t mask, const uint32_t* __restrict__ offs) {
+    constexpr int WAVES = RP_THREADS / 64;
+    // the waves' digit counts (at most a tile: 16 bits), then the tile's keys in digit order
+    __shared__ __align__(8) unsigned char s_mem[2 * WAVES * RP_DIGITS];
+    static_assert(sizeof(K) * RP_TILE <= sizeof(s_mem), "keys lie where the counts were");
+    __shared__ uint32_t s_val[RP_TILE], s_start[RP_DIGITS], s_delta[RP_DIGITS], s_w[WAVES];
+    uint16_t* const s_wc = reinterpret_cast<uint16_t*>(s_mem);
+    K* const s_key = reinterpret_cast<K*>(s_mem);
     const uint32_t tid = threadIdx.x, lane = lane_id(), wv = tid >> 6;
-    s_off[tid] = offs[(size_t)tid * nt + blockIdx.x];
+    const uint32_t off = offs[(size_t)tid * gridDim.x + blockIdx.x];  // this thread's digit
+    const uint32_t base = blockIdx.x * RP_TILE, first = base + wv * (64u * RP_ITEMS) + lane;
     const uint64_t lt = (1ull << lane) - 1ull;
-    const uint32_t base = blockIdx.x * RP_TILE;
+    K k[RP_ITEMS];
+    uint32_t v[RP_ITEMS], rk[RP_ITEMS];
+#pragma unroll
     for (int it = 0; it < RP_ITEMS; ++it) {
-        const uint32_t i = base + it * RP_THREADS + tid;
-        const bool valid = i < n;
-        K k = 0;
-        uint32_t v = 0, d = 256u;
-        if (valid) {
-            k = kin[i];
-            v = vin[i];
-            d = digit_of(k, shift);
-        }
+        const uint32_t i = first + 64u * it;
+        k[it] = i < n ? kin[i] : (K)0;
+        v[it] = i < n ? vin[i] : 0u;
+    }
+    uint16_t* const wc = s_wc + wv * RP_DIGITS;
 #pragma unroll
-        for (int w = 0; w < RP_THREADS / 64; ++w) s_wc[w][tid] = 0;
-        // lanes with the same digit (9 bits so that invalid lanes, d = 256, form their own group)
-        uint64_t peers = __ballot(1);
+    for (int q = 0; q < RP_DIGITS / 64; ++q) wc[64 * q + lane] = 0u;
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int b = 0; b < 9; ++b) {
+    for (int it = 0; it < RP_ITEMS; ++it) {
+        const bool valid = first + 64u * it < n;
+        const uint32_t d = (uint32_t)(k[it] >> shift) & mask;
+        uint64_t peers = __ballot(valid);
+#pragma unroll
+        for (int b = 0; b < RP_BITS; ++b) {
             const uint64_t bal = __ballot((d >> b) & 1u);
             peers &= ((d >> b) & 1u) ? bal : ~bal;
         }
-        const uint32_t rank = (uint32_t)__popcll(peers & lt);
-        __syncthreads();
-        if (valid && rank == 0) s_wc[wv][d] = (uint32_t)__popcll(peers);
-        __syncthreads();
-        uint32_t pos = 0;
-        if (valid) {
-            pos = s_off[d] + rank;
-            for (uint32_t w = 0; w < wv; ++w) pos += s_wc[w][d];
-        }
-        __syncthreads();
-        uint32_t add = 0;
+        const uint32_t r = (uint32_t)__popcll(peers & lt);
+        const uint32_t before = wc[d];
+        __builtin_amdgcn_wave_barrier();
+        if (valid && r == 0u) wc[d] = (uint16_t)(before + (uint32_t)__popcll(peers));
+        __builtin_amdgcn_wave_barrier();
+        rk[it] = before + r;
+    }
+    __syncthreads();
+    // the waves' counts of a digit turned into the counts of the waves before, the digits' starts
+    uint32_t tot = 0;
 #pragma unroll
-        for (int w = 0; w < RP_THREADS / 64; ++w) add += s_wc[w][tid];
-        s_off[tid] += add;
-        if (valid) {
-            kout[pos] = k;
-            vout[pos] = v;
-        }
-        __syncthreads();
+    for (int w = 0; w < WAVES; ++w) {
+        const uint32_t c = s_wc[w * RP_DIGITS + tid];
+        s_wc[w * RP_DIGITS + tid] = (uint16_t)tot;
+        tot += c;
+    }
+    const uint32_t inc = wave_incl_scan(tot);
+    if (lane == 63u) s_w[wv] = inc;
+    __syncthreads();
+    uint32_t start = inc - tot;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) start += (uint32_t)w < wv ? s_w[w] : 0u;
+    s_start[tid] = start;
+    s_delta[tid] = off - start;
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < RP_ITEMS; ++it) {
+        const uint32_t d = (uint32_t)(k[it] >> shift) & mask;
+        rk[it] += s_start[d] + wc[d];
+    }
+    __syncthreads();  // the counts are read: keys take their place
+#pragma unroll
+    for (int it = 0; it < RP_ITEMS; ++it) {
+        if (first + 64u * it >= n) continue;
+        s_key[rk[it]] = k[it];
+        s_val[rk[it]] = v[it];
+    }
+    __syncthreads();
+    const uint32_t m = n - base < (uint32_t)RP_TILE ? n - base : (uint32_t)RP_TILE;
+#pragma unroll
+    for (int it = 0; it < RP_ITEMS; ++it) {
+        const uint32_t j = (uint32_t)it * RP_THREADS + tid;
+        if (j >= m) continue;
+        const K key = s_key[j];
+        const uint32_t pos = s_delta[(uint32_t)(key >> shift) & mask] + j;
+        kout[pos] = key;
+        vout[pos] = s_val[j];
     }
 }
 
 // Scratch of the per-pass sort: the histogram with the scan's total, then the scan's scratch.
-static size_t hist_words(uint32_t nb) { return (size_t)256 * nb + 2; }
+static size_t hist_words(uint32_t nb) { return (size_t)RP_DIGITS * nb + 2; }
 size_t radix_tmp_words(uint32_t n) {
     const uint32_t nb = (n + RP_TILE - 1) / RP_TILE;
-    return hist_words(nb) + scan_tmp_words(256u * nb);
+    return hist_words(nb) + scan_tmp_words(RP_DIGITS * nb);
 }
 size_t radix_meet_words() { return RS_HDR + 256u * RS_GROUPS; }
 
@@ -664,15 +701,18 @@ static int radix_sort_impl(K* keys, uint32_t* vals, K* keys_alt, uint32_t* vals_
     const uint32_t nb = (n + RP_TILE - 1) / RP_TILE;
     uint32_t* hist = tmp;  // scanned in place
     uint32_t* scan_tmp = tmp + hist_words(nb);  // 8-byte aligned for the scan's status words
+    // the fewest passes, their digits as narrow as they can be
+    const int np = (end_bit + RP_BITS - 1) / RP_BITS, bits = (end_bit + np - 1) / np;
+    const uint32_t mask = (1u << bits) - 1u;
     K* ki = keys;
     K* ko = keys_alt;
     uint32_t* vi = vals;
     uint32_t* vo = vals_alt;
     int passes = 0;
-    for (int shift = 0; shift < end_bit; shift += 8) {
-        hipLaunchKernelGGL(k_rs_hist<K>, dim3(nb), dim3(RP_THREADS), 0, s, ki, n, shift, hist);
-        scan_exclusive(hist, hist, 256u * nb, scan_tmp, s, nullptr, nullptr, false, err);
-        hipLaunchKernelGGL(k_rs_scatter<K>, dim3(nb), dim3(RP_THREADS), 0, s, ki, vi, ko, vo, n, shift, hist);
+    for (int shift = 0; shift < end_bit; shift += bits) {
+        hipLaunchKernelGGL(k_rs_hist<K>, dim3(nb), dim3(RP_THREADS), 0, s, ki, n, shift, mask, hist);
+        scan_exclusive(hist, hist, RP_DIGITS * nb, scan_tmp, s, nullptr, nullptr, false, err);
+        hipLaunchKernelGGL(k_rs_scatter<K>, dim3(nb), dim3(RP_THREADS), 0, s, ki, vi, ko, vo, n, shift, mask, hist);
         K* tk = ki; ki = ko; ko = tk;
         uint32_t* tv = vi; vi = vo; vo = tv;
         ++passes;

@@ -24,8 +24,10 @@ def _towers(axm, n, s):
     return b
 
 
-def _check(axm, w, n, s):
+def _check(axm, w, n, s, worlds=1):
     b = _towers(axm, n, s)
+    if worlds > 1:
+        b.world[:] = np.arange(n) * worlds // n
     w.set_bodies(b)
     st = w.step(DT, 2)
     assert st.overflow == 0
@@ -61,4 +63,15 @@ def test_sort_arrays_end_at_a_page(axm, gpu):
     d.gravity[0] = d.gravity[1] = d.gravity[2] = 0.0
     w = axm.World(d)
     _check(axm, w, 524288, 4)
+    w.close()
+
+
+@pytest.mark.parametrize("n, worlds", [(131072, 1), (131073, 1), (135168, 1), (140001, 1), (131073, 2), (139264, 700)])
+def test_sort_by_passes(axm, gpu, n, worlds):
+    """Either side of the count above which bodies are sorted pass by pass: a last tile of one key, whole
+    tiles, and keys with the world above the cell (31 and 40 bits, in four passes)."""
+    d = axm.default_desc()
+    d.gravity[0] = d.gravity[1] = d.gravity[2] = 0.0
+    w = axm.World(d)
+    _check(axm, w, n, 5, worlds)
     w.close()
