@@ -18,7 +18,7 @@ using namespace axm;
 // Staging of axm_collide_pairs_noalloc: the inputs, outputs and per-pair status of at
 // most NOALLOC_MAX_PAIRS pairs, one region of 32-bit words per field (each region holds
 // that field for every pair slot: NOALLOC_MAX_PAIRS x width words).  One copy per
-// device, held until the process ends; every call on a device shares it.
+// device, held until the process ends; the calls on a device take turns on it.
 constexpr uint32_t NOALLOC_MAX_PAIRS = 16384;
 // region offsets, in words per pair slot: ta 1, pa 3, xa 3, qa 4, tb 1, pb 3, xb 3, qb 4 (inputs),
 // npts 1, pos 12, normal 12, depth 4, feature 4, status 1 (outputs), queue of deep pairs 1; the
@@ -274,6 +274,9 @@ const uint32_t NO_PAIRS = 0u;
 constexpr int NOALLOC_MAX_DEVICES = 64;
 std::mutex g_scratch_mu;
 uint32_t* g_scratch_ptr[NOALLOC_MAX_DEVICES] = {};
+// per device: held by a call from its first upload to its last read.  Two calls at once would share
+// the queue's length and append past the queue.
+std::mutex g_scratch_use[NOALLOC_MAX_DEVICES];
 
 // The device address of `scratch` on `device`, looked up once per device with that device
 // current (each device holds its own copy at its own address; the host-side name of the
@@ -355,6 +358,7 @@ axm_status axm_collide_pairs_noalloc(int32_t device, uint32_t n, const uint32_t*
     if (hipSetDevice(device) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
     uint32_t* base = scratch_on(device);
     if (!base) return AXM_GPU_OPERATION_FAILED;
+    std::lock_guard<std::mutex> turn(g_scratch_use[device]);
     // region r starts at base + r * NOALLOC_MAX_PAIRS
     auto reg = [&](uint32_t r) { return base + (size_t)r * NOALLOC_MAX_PAIRS; };
     struct Up {

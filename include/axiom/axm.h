@@ -323,9 +323,8 @@ axm_status axm_collide_pairs(int32_t device, uint32_t n, const uint32_t* type_a,
  * copies of the inputs, the outputs and the per-pair status staged in a fixed buffer the
  * library holds on each device until the process ends (3.5 MiB: at most 16384 pairs per
  * call; more returns OutOfRange).  It calls no hipMalloc / hipFree, for callers that
- * cannot allocate (tight stepping loops, harnesses that forbid device allocation).  Calls
- * that overlap on one device share the buffer and race: serialise them.  No counterpart in
- * the reference. */
+ * cannot allocate (tight stepping loops, harnesses that forbid device allocation).  Calls on
+ * one device take turns on the buffer.  No counterpart in the reference. */
 axm_status axm_collide_pairs_noalloc(int32_t device, uint32_t n, const uint32_t* type_a, const float* prm_a,
                                      const float* pos_a, const float* quat_a, const uint32_t* type_b,
                                      const float* prm_b, const float* pos_b, const float* quat_b, float margin,
