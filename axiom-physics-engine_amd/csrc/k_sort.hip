@@ -244,7 +244,8 @@ void scan_exclusive(const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* tmp
 // workgroups without keys leave at once, so the grid is sized for the capacity at no cost.
 //
 // The grid that meets must be resident as a whole: at most RS_GROUPS workgroups, half of what the
-// chip holds, so that two worlds' sorts fit side by side.  200 and 1000 bodies: 14 us for the body
+// chip holds (the steps of a device's worlds take turns, so no other grid that meets runs beside
+// it).  200 and 1000 bodies: 14 us for the body
 // keys and 7 to 8 for the solve order (with launches per pass 47, and 23 to 47 in tiles of 256
 // threads whose ranks met at four barriers); 6000 bodies 27 and 30 (53 and 72); 100000 bodies 54
 // and 47 (65 and 117); the solve order of 1.7M manifolds 320 (889, its keys' own launch 35).

@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "axiom/axm.h"
+#include "device_turn.hpp"
 #include "file_io.hpp"
 #include "k_bodies.hpp"
 #include "k_step.hpp"
@@ -91,6 +92,7 @@ struct Alloc {
 struct axm_world_s {
     axm_world_desc desc{};
     hipStream_t stream = nullptr;
+    hipEvent_t turn_ev = nullptr;  // where another world's stream ended when this one took its turn
     Alloc mem;
     uint32_t n = 0, cap_n = 0, cap_pairs = 0, cap_man = 0, n_worlds = 1;
     uint32_t cap_first = 0;  // entries of B.world_first: world ids may have gaps
@@ -196,7 +198,11 @@ struct axm_world_s {
                 }
     }
     ~axm_world_s() {
-        if (stream) (void)hipStreamSynchronize(stream);
+        if (stream) {
+            (void)hipStreamSynchronize(stream);
+            DeviceTurn::of(desc.device).idle(stream);
+        }
+        if (turn_ev) (void)hipEventDestroy(turn_ev);
         drop_graphs();
         for (hipEvent_t e : prof_ev) (void)hipEventDestroy(e);
         for (hipEvent_t e : gprof_ev)
@@ -510,6 +516,12 @@ StepParams make_params(const axm_world_s* w, float dt) {
 axm_status read_counters(axm_world_s* w) {
     AXM_HIP(hipMemcpyAsync(w->h_cnt, w->cnt, sizeof(Counters), hipMemcpyDeviceToHost, w->stream));
     AXM_HIP(hipStreamSynchronize(w->stream));
+    return AXM_SUCCESS;
+}
+// The same with the world's turn on the device over: nothing of it runs any more.
+axm_status end_turn(axm_world_s* w) {
+    AXM_TRY(read_counters(w));
+    DeviceTurn::of(w->desc.device).idle(w->stream);
     return AXM_SUCCESS;
 }
 
@@ -937,12 +949,17 @@ axm_status step_sync(axm_world_s* w, float dt, StepOpts o, axm_step_stats* st) {
             if (e) (void)hipEventDestroy(e);
     };
     for (int attempt = 0;; ++attempt) {
-        const axm_status es = enqueue_step(w, dt, o);
+        axm_status es;
+        {
+            const Turn turn(w->desc.device, w->stream, w->turn_ev);
+            es = turn.status();
+            if (es == AXM_SUCCESS) es = enqueue_step(w, dt, o);
+        }
         if (es != AXM_SUCCESS) {
             free_ev();
             return es;
         }
-        AXM_TRY(read_counters(w));
+        AXM_TRY(end_turn(w));
         if (w->last_iters_dev) w->last_iters = w->h_cnt->sweeps_run;
         if (w->h_cnt->sticky == 0u) break;
         fill_stats(w, S);
@@ -1042,7 +1059,7 @@ axm_status axm_world_create(const axm_world_desc* desc, axm_world* out) {
     if (desc->cell_size < 0.0f || !std::isfinite(desc->cell_size)) return AXM_INVALID_PARAMETER;
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return AXM_GPU_OPERATION_FAILED;
-    if (desc->device < 0 || desc->device >= ndev) return AXM_INVALID_PARAMETER;
+    if (desc->device < 0 || desc->device >= ndev || desc->device >= DeviceTurn::DEVICES) return AXM_INVALID_PARAMETER;
     if (hipSetDevice(desc->device) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
     axm_world_s* w = new (std::nothrow) axm_world_s;
     if (!w) return AXM_OUT_OF_MEMORY;
@@ -1062,7 +1079,8 @@ axm_status axm_world_create(const axm_world_desc* desc, axm_world* out) {
         return AXM_GPU_OPERATION_FAILED;
     }
     w->sweep_groups = (uint32_t)w->cu_count;
-    if (hipStreamCreateWithFlags(&w->stream, hipStreamNonBlocking) != hipSuccess) {
+    if (hipStreamCreateWithFlags(&w->stream, hipStreamNonBlocking) != hipSuccess ||
+        hipEventCreateWithFlags(&w->turn_ev, hipEventDisableTiming) != hipSuccess) {
         delete w;
         return AXM_GPU_OPERATION_FAILED;
     }
@@ -1313,7 +1331,7 @@ axm_status axm_world_run(axm_world w, float dt, uint32_t iters, uint32_t steps, 
     }
     AXM_TRY(ensure_res(w, iters));
     // run totals at the start, for the strict status of the whole run
-    AXM_TRY(read_counters(w));
+    AXM_TRY(end_turn(w));
     const uint32_t acc0_steps = w->h_cnt->acc_steps, acc0_reached = w->h_cnt->acc_reached;
     const uint32_t acc0_gjk = w->h_cnt->acc_gjk_fail, acc0_epa = w->h_cnt->acc_epa_fail;
     uint32_t done = 0;
@@ -1360,27 +1378,31 @@ axm_status axm_world_run(axm_world w, float dt, uint32_t iters, uint32_t steps, 
         int prev = -1;
         for (uint32_t k = 0; k < todo; ++k) {
             const int c = w->cur;
-            if (w->prof_on) {
-                AXM_HIP(hipGraphLaunch(w->gpre[c], w->stream));
-                SweepStop stop;
-                const bool checks = sweep_checks(w, false, stop);
-                const uint32_t nsw = w->desc.residual_tol > 0.0f ? std::max<uint32_t>(w->desc.max_iterations, 1u)
-                                                                 : iters;
-                // timed apart
-                const uint2* list = split ? w->isl_list : nullptr;
-                const OwnShape own{w->sweep_groups, w->sweep_lds, w->sweep_tune};
-                launch_flow_init(w->B, w->R[c], w->rcap[c], w->bmask, w->cnt, list, w->isl_arrive, (uint32_t)w->cu_count,
-                                 w->stream);
-                if (split)
+            {
+                const Turn turn(w->desc.device, w->stream, w->turn_ev);
+                AXM_TRY(turn.status());
+                if (w->prof_on) {
+                    AXM_HIP(hipGraphLaunch(w->gpre[c], w->stream));
+                    SweepStop stop;
+                    const bool checks = sweep_checks(w, false, stop);
+                    const uint32_t nsw = w->desc.residual_tol > 0.0f ? std::max<uint32_t>(w->desc.max_iterations, 1u)
+                                                                     : iters;
+                    // timed apart
+                    const uint2* list = split ? w->isl_list : nullptr;
+                    const OwnShape own{w->sweep_groups, w->sweep_lds, w->sweep_tune};
+                    launch_flow_init(w->B, w->R[c], w->rcap[c], w->bmask, w->cnt, list, w->isl_arrive, (uint32_t)w->cu_count,
+                                     w->stream);
+                    if (split)
+                        launch_pgs_solve(w->B, sp, w->R[c], w->rcap[c], w->bmask, nsw, w->cnt, SWEEP_SPIN_LIMIT_US,
+                                         (uint32_t)w->cu_count, w->solve_keys, list, w->desc.residual_tol, SOLVE_LIST, true, own,
+                                         SweepStop{}, w->stream, w->bprof_ev[2 * c], w->bprof_ev[2 * c + 1]);
                     launch_pgs_solve(w->B, sp, w->R[c], w->rcap[c], w->bmask, nsw, w->cnt, SWEEP_SPIN_LIMIT_US,
-                                     (uint32_t)w->cu_count, w->solve_keys, list, w->desc.residual_tol, SOLVE_LIST, true, own,
-                                     SweepStop{}, w->stream, w->bprof_ev[2 * c], w->bprof_ev[2 * c + 1]);
-                launch_pgs_solve(w->B, sp, w->R[c], w->rcap[c], w->bmask, nsw, w->cnt, SWEEP_SPIN_LIMIT_US,
-                                 (uint32_t)w->cu_count, w->solve_keys, list, w->desc.residual_tol, SOLVE_LARGE, true, own,
-                                 checks ? stop : SweepStop{}, w->stream, w->gprof_ev[2 * c], w->gprof_ev[2 * c + 1]);
-                AXM_HIP(hipGraphLaunch(w->gpost[c], w->stream));
-            } else {
-                AXM_HIP(hipGraphLaunch(w->gexec[c], w->stream));
+                                     (uint32_t)w->cu_count, w->solve_keys, list, w->desc.residual_tol, SOLVE_LARGE, true, own,
+                                     checks ? stop : SweepStop{}, w->stream, w->gprof_ev[2 * c], w->gprof_ev[2 * c + 1]);
+                    AXM_HIP(hipGraphLaunch(w->gpost[c], w->stream));
+                } else {
+                    AXM_HIP(hipGraphLaunch(w->gexec[c], w->stream));
+                }
             }
             if (w->prof_on && prev >= 0) {
                 float e = 0.0f;
@@ -1395,7 +1417,7 @@ axm_status axm_world_run(axm_world w, float dt, uint32_t iters, uint32_t steps, 
             prev = w->cur;
             w->cur = 1 - w->cur;
         }
-        AXM_TRY(read_counters(w));
+        AXM_TRY(end_turn(w));
         if (w->prof_on && prev >= 0) {
             float e = 0.0f;
             AXM_HIP(hipEventElapsedTime(&e, w->gprof_ev[2 * prev], w->gprof_ev[2 * prev + 1]));
@@ -1528,9 +1550,13 @@ axm_status axm_broadphase(axm_world w, uint32_t* count) {
     (void)hipSetDevice(w->desc.device);
     const StepParams sp = make_params(w, 1.0f / 120.0f);
     for (int attempt = 0; attempt < 3; ++attempt) {
-        launch_counters_begin(w->cnt, w->pkinds, w->stream);
-        if (w->n) enqueue_broad(w, sp);
-        AXM_TRY(read_counters(w));
+        {
+            const Turn turn(w->desc.device, w->stream, w->turn_ev);
+            AXM_TRY(turn.status());
+            launch_counters_begin(w->cnt, w->pkinds, w->stream);
+            if (w->n) enqueue_broad(w, sp);
+        }
+        AXM_TRY(end_turn(w));
         if (!(w->h_cnt->sticky & STICKY_PAIRS)) break;
         if (!w->desc.auto_grow) return AXM_OUT_OF_RANGE;
         const uint64_t P = w->h_cnt->pairs;
@@ -1549,12 +1575,16 @@ axm_status axm_collide(axm_world w, uint32_t* manifold_count) {
     (void)hipSetDevice(w->desc.device);
     const StepParams sp = make_params(w, 1.0f / 120.0f);
     for (int attempt = 0; attempt < 4; ++attempt) {
-        launch_counters_begin(w->cnt, w->pkinds, w->stream);
-        if (w->n) {
-            enqueue_broad(w, sp);
-            enqueue_narrow(w, sp);
+        {
+            const Turn turn(w->desc.device, w->stream, w->turn_ev);
+            AXM_TRY(turn.status());
+            launch_counters_begin(w->cnt, w->pkinds, w->stream);
+            if (w->n) {
+                enqueue_broad(w, sp);
+                enqueue_narrow(w, sp);
+            }
         }
-        AXM_TRY(read_counters(w));
+        AXM_TRY(end_turn(w));
         const uint32_t st = w->h_cnt->sticky;
         if (!(st & (STICKY_PAIRS | STICKY_MANIFOLDS))) break;
         if (!w->desc.auto_grow) return AXM_OUT_OF_RANGE;

@@ -21,6 +21,8 @@
  *     (src/debug/physics_debug_draw.cpp:111-115).
  *   - Host pointers are borrowed for the duration of a call.  Calls on one
  *     handle are not thread-safe; each handle owns its own HIP stream.
+ *     Worlds may be used from several threads, one world by one thread at a
+ *     time: the steps of worlds on one device run one after the other there.
  *     Steps run asynchronously until axm_world_sync or an axm_*_get_* call.
  */
 #ifndef AXIOM_AXM_H
