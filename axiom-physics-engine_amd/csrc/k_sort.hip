@@ -250,7 +250,7 @@ void scan_exclusive(const uint32_t* in, uint32_t* out, uint32_t n, uint32_t* tmp
 // threads whose ranks met at four barriers); 6000 bodies 27 and 30 (53 and 72); 100000 bodies 54
 // and 47 (65 and 117); the solve order of 1.7M manifolds 320 (889, its keys' own launch 35).
 constexpr int RS_THREADS = 1024, RS_WAVES = RS_THREADS / 64;
-constexpr uint32_t RS_GROUPS = 128, RS_HDR = 4;
+constexpr uint32_t RS_GROUPS = 128, RS_HDR = SORT_MEET_WORDS;
 
 // Sort keys read from memory.
 template <class K> struct KeysGiven {

@@ -43,8 +43,11 @@ template <class T> __device__ __forceinline__ T spread_sum(const Counters* cnt, 
 
 constexpr uint32_t PAIR_KINDS = 16;  // narrowphase test kinds (pair_kind)
 // The per-step counters back to zero (the threads of one workgroup).
-__device__ __forceinline__ void counters_reset(Counters* cnt, uint32_t* __restrict__ kinds) {
+__device__ __forceinline__ void counters_reset(Counters* cnt, uint32_t* __restrict__ kinds, const Meeting& meet) {
     uint32_t* w = reinterpret_cast<uint32_t*>(cnt);
+    constexpr uint32_t BAR_WORDS = sizeof(GridBar) / sizeof(uint32_t);
+    if (threadIdx.x < BAR_WORDS) reinterpret_cast<uint32_t*>(meet.colour)[threadIdx.x] = 0u;
+    else if (threadIdx.x - BAR_WORDS < SORT_MEET_WORDS) meet.sort[threadIdx.x - BAR_WORDS] = 0u;
     if (threadIdx.x < COUNTERS_RESET_WORDS) w[threadIdx.x] = 0u;
     for (uint32_t k = threadIdx.x; k < SPREAD; k += blockDim.x) {
         cnt->sp[k].islands = 0u;
@@ -61,11 +64,11 @@ __global__ void __launch_bounds__(256) k_begin(Bodies B, StepParams sp, uint32_t
                                                uint32_t* __restrict__ key32, uint32_t* __restrict__ val, uint64_t* __restrict__ bmax0,
                                                uint64_t* __restrict__ bmax1, uint64_t* __restrict__ bmask,
                                                uint32_t* __restrict__ bdeg, Counters* __restrict__ cnt,
-                                               uint32_t* __restrict__ kinds, CellTable ct) {
+                                               uint32_t* __restrict__ kinds, Meeting meet, CellTable ct) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     // the step's counters start from zero (the kernels that count run after this launch;
     // steps_done, read below, is kept across steps)
-    if (blockIdx.x == 0) counters_reset(cnt, kinds);
+    if (blockIdx.x == 0) counters_reset(cnt, kinds, meet);
     // with the Morton bitmap: the words the last step set go back to zero (several bodies
     // may name one word: all write zero); the cell table sets this step's after the sort
     if (ct.mbits && i < ct.mlist_n) {
@@ -3886,8 +3889,10 @@ __global__ void __launch_bounds__(256) k_cache_rehash(const uint64_t* __restrict
 
 
 
-// Clears the per-step part of the control block.
-__global__ void k_counters_begin(Counters* cnt, uint32_t* __restrict__ kinds) { counters_reset(cnt, kinds); }
+// Clears the per-step part of the control block and the meeting words.
+__global__ void k_counters_begin(Counters* cnt, uint32_t* __restrict__ kinds, Meeting meet) {
+    counters_reset(cnt, kinds, meet);
+}
 
 // Integration is skipped while any sticky error is set, so an overflowing step
 // leaves the state exactly as it was.
@@ -4105,19 +4110,19 @@ static inline dim3 grid_bounded(uint32_t cap, uint32_t max_groups = 1024u) {
 }
 
 
-void launch_counters_begin(Counters* cnt, uint32_t* kinds, hipStream_t s) {
-    hipLaunchKernelGGL(k_counters_begin, dim3(1), dim3(64), 0, s, cnt, kinds);
+void launch_counters_begin(Counters* cnt, uint32_t* kinds, const Meeting& meet, hipStream_t s) {
+    hipLaunchKernelGGL(k_counters_begin, dim3(1), dim3(64), 0, s, cnt, kinds, meet);
 }
 void launch_begin(const Bodies& B, const StepParams& sp, uint32_t n, uint64_t* key, uint32_t* key32, uint32_t* val,
                   uint64_t* bmax0,
                   uint64_t* bmax1, uint64_t* bmask, uint32_t* bdeg, Counters* cnt, uint32_t* kinds,
-                  const CellTable& ct, hipStream_t s) {
+                  const Meeting& meet, const CellTable& ct, hipStream_t s) {
     const uint32_t m = std::max(n, ct.mbits ? ct.mlist_n : 0u);
     if (m)
         hipLaunchKernelGGL(k_begin, grid_for(m), dim3(256), 0, s, B, sp, n, key, key32, val, bmax0, bmax1, bmask, bdeg,
-                           cnt, kinds, ct);
+                           cnt, kinds, meet, ct);
     else
-        launch_counters_begin(cnt, kinds, s);
+        launch_counters_begin(cnt, kinds, meet, s);
 }
 void launch_fill_u64(uint64_t* p, uint64_t v, uint32_t n, hipStream_t s) {
     if (n) hipLaunchKernelGGL(k_fill_u64, grid_for(n), dim3(256), 0, s, p, v, n);

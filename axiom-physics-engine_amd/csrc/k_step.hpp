@@ -42,8 +42,9 @@ struct PrevCacheArgs {
     uint32_t valid;
 };
 
-// Clears the per-step counters and, when given, the 32 pair-kind counters.
-void launch_counters_begin(Counters* cnt, uint32_t* kinds, hipStream_t s);
+// Clears the per-step counters, the step's meeting words and, when given, the 32 pair-kind
+// counters.
+void launch_counters_begin(Counters* cnt, uint32_t* kinds, const Meeting& meet, hipStream_t s);
 // Start of a step: velocities, world inertia, AABBs, cell keys; clears the
 // colouring's per-body words.
 // The sorted cell keys of the broadphase: 32-bit in the Morton rank mode (one world, where
@@ -53,12 +54,12 @@ struct SortedKeys {
     const uint32_t* k32 = nullptr;
     __host__ __device__ uint64_t operator[](uint32_t s) const { return k32 ? (uint64_t)k32[s] : k64[s]; }
 };
-// Also resets the step's counters (as launch_counters_begin).  The keys go to key32 (the
+// Also resets the step's counters and meeting words (as launch_counters_begin).  The keys go to key32 (the
 // Morton code) with the Morton bitmap, else to key.
 void launch_begin(const Bodies& B, const StepParams& sp, uint32_t n, uint64_t* key, uint32_t* key32, uint32_t* val,
                   uint64_t* bmax0,
                   uint64_t* bmax1, uint64_t* bmask, uint32_t* bdeg, Counters* cnt, uint32_t* kinds,
-                  const CellTable& ct, hipStream_t s);
+                  const Meeting& meet, const CellTable& ct, hipStream_t s);
 // Islands of the step, after the narrowphase: union-find over the manifolds between awake
 // dynamic bodies (root = smallest body index), and wake requests for sleeping islands an
 // awake body touched.

@@ -193,6 +193,14 @@ struct GridBar {
     uint32_t pad[2];
 };
 
+// The words the step's grids meet at.  Every step sets them to zero in its first launch: a
+// wait that gave up in an earlier one left them between two meetings.
+struct Meeting {
+    GridBar* colour;  // the colouring's
+    uint32_t* sort;   // the sorts' (the first SORT_MEET_WORDS of radix_meet_words)
+};
+constexpr uint32_t SORT_MEET_WORDS = 4;
+
 // k_sort.hip
 size_t scan_tmp_words(uint32_t n);
 // out[0..n] = exclusive prefix sums, out[n] = total (also written to *total_out when given).

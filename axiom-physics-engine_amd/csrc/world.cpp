@@ -581,7 +581,7 @@ void enqueue_broad(axm_world_s* w, const StepParams& sp) {
     uint32_t* key32 = reinterpret_cast<uint32_t*>(w->key);
     uint32_t* key32_alt = reinterpret_cast<uint32_t*>(w->key_alt);
     launch_begin(w->B, sp, n, w->key, k32 ? key32 : nullptr, w->val, w->bmax0, w->bmax1, w->bmask, w->bdone, w->cnt,
-                 w->pkinds, w->ct, s);
+                 w->pkinds, Meeting{w->bar, w->sort_meet}, w->ct, s);
     SortedKeys skey;
     int alt;
     if (k32) {
@@ -1553,7 +1553,7 @@ axm_status axm_broadphase(axm_world w, uint32_t* count) {
         {
             const Turn turn(w->desc.device, w->stream, w->turn_ev);
             AXM_TRY(turn.status());
-            launch_counters_begin(w->cnt, w->pkinds, w->stream);
+            launch_counters_begin(w->cnt, w->pkinds, Meeting{w->bar, w->sort_meet}, w->stream);
             if (w->n) enqueue_broad(w, sp);
         }
         AXM_TRY(end_turn(w));
@@ -1578,7 +1578,7 @@ axm_status axm_collide(axm_world w, uint32_t* manifold_count) {
         {
             const Turn turn(w->desc.device, w->stream, w->turn_ev);
             AXM_TRY(turn.status());
-            launch_counters_begin(w->cnt, w->pkinds, w->stream);
+            launch_counters_begin(w->cnt, w->pkinds, Meeting{w->bar, w->sort_meet}, w->stream);
             if (w->n) {
                 enqueue_broad(w, sp);
                 enqueue_narrow(w, sp);
