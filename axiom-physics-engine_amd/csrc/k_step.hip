@@ -1842,21 +1842,6 @@ __device__ __forceinline__ void flow_init_part(const Bodies& B, const SolverRows
     q[3] = make_uint4((uint32_t)ob[2], (uint32_t)(ob[2] >> 32), (uint32_t)ob[3], (uint32_t)(ob[3] >> 32));
     }
 }
-// Launch shape of the register sweep (flow_part).
-constexpr uint32_t FLOW_THREADS = 512, FLOW_WAVES = FLOW_THREADS / 64u;
-constexpr uint32_t FLOW_WAVE_SLOTS = 32;
-// Pieces of 32 slots of the islands of the largest class that the register sweep takes on G
-// workgroups: all of them, or none, when one workgroup per island (stream_island) is faster.
-// A sweep costs the register sweep its chain of visits (15 us at ten colours) while everything
-// fits its waves, and about 0.5 ns per slot beyond (160k slots: 80 us); one workgroup takes
-// about 25 ns per slot of its island, all islands at once on as many CUs (44 us for 1880 slots,
-// 100 us for 3950).
-__device__ __forceinline__ uint32_t wide_pieces(const Counters* cnt, uint32_t G) {
-    const uint32_t nl = (cnt->m_glob + FLOW_WAVE_SLOTS - 1u) / FLOW_WAVE_SLOTS, w = cnt->isl_wide;
-    if (cnt->max_colour > 64u) return 0u;
-    const bool fits = nl <= G * FLOW_WAVES && nl + w <= G * FLOW_WAVES;
-    return fits || (uint64_t)cnt->isl_most * 50u > (uint64_t)w * FLOW_WAVE_SLOTS ? w : 0u;
-}
 // The large islands' slots and, when the register sweep takes them, those of the islands of the
 // largest class, whose arrival words start from zero.  G: the workgroups of the solve launch.
 __global__ void __launch_bounds__(256) k_flow_init(Bodies B, SolverRows R, const uint64_t* __restrict__ bmask,
@@ -3434,7 +3419,7 @@ __device__ __forceinline__ void islands_part(const Bodies& B, const StepParams& 
 // sleep, a tight loop, two polls in flight) gains nothing or loses.
 __device__ __forceinline__ u32x4_t flow_quad(const uint64_t* inbox, uint32_t byte) {
     const __amdgpu_buffer_rsrc_t rs =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint64_t*>(inbox), 0, 0x7FFFFFFF, 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint64_t*>(inbox), 0, FLOW_INBOX_BYTES, 0x00020000);
     // aux: sc0 | sc1, as vin_quad
     return __builtin_amdgcn_raw_buffer_load_b128(rs, (int)byte, 0, 1 | 16);
 }
@@ -3638,7 +3623,7 @@ __device__ __forceinline__ void flow_part(const Bodies& B, const StepParams& sp,
                     uint64_t o[4];
                     vpack4(X.v, X.w, ver + rank + 1u, o);
                     const __amdgpu_buffer_rsrc_t rs =
-                        __builtin_amdgcn_make_buffer_rsrc(R.inbox, 0, 0x7FFFFFFF, 0x00020000);
+                        __builtin_amdgcn_make_buffer_rsrc(R.inbox, 0, FLOW_INBOX_BYTES, 0x00020000);
                     const u32x4_t q0 = {(uint32_t)o[0], (uint32_t)(o[0] >> 32), (uint32_t)o[1], (uint32_t)(o[1] >> 32)};
                     const u32x4_t q1 = {(uint32_t)o[2], (uint32_t)(o[2] >> 32), (uint32_t)o[3], (uint32_t)(o[3] >> 32)};
                     // aux: sc1, as vin_store

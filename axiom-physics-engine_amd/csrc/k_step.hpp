@@ -155,6 +155,25 @@ struct SweepStop {
     float tol = -1.0f;
     uint32_t every = 1;
 };
+// Launch shape of the register sweep (flow_part).
+constexpr uint32_t FLOW_THREADS = 512, FLOW_WAVES = FLOW_THREADS / 64u;
+constexpr uint32_t FLOW_WAVE_SLOTS = 32;
+// It reaches the inboxes by 32-bit byte offsets into a buffer of this many bytes.
+constexpr uint32_t FLOW_INBOX_BYTES = 0x7FFFFFFFu;
+// Pieces of 32 slots of the islands of the largest class that the register sweep takes on G
+// workgroups: all of them, or none, when one workgroup per island (stream_island) is faster.
+// A sweep costs the register sweep its chain of visits (15 us at ten colours) while everything
+// fits its waves, and about 0.5 ns per slot beyond (160k slots: 80 us); one workgroup takes
+// about 25 ns per slot of its island, all islands at once on as many CUs (44 us for 1880 slots,
+// 100 us for 3950).  None, too, when a step has more manifolds than its inboxes' offsets reach
+// (33 million): these islands' slots come after the large ones', anywhere up to the last.
+inline __host__ __device__ uint32_t wide_pieces(const Counters* cnt, uint32_t G) {
+    const uint32_t nl = (cnt->m_glob + FLOW_WAVE_SLOTS - 1u) / FLOW_WAVE_SLOTS, w = cnt->isl_wide;
+    if (cnt->max_colour > 64u) return 0u;
+    if ((uint64_t)cnt->m_eff * INBOX_WORDS * 8u > FLOW_INBOX_BYTES) return 0u;
+    const bool fits = nl <= G * FLOW_WAVES && nl + w <= G * FLOW_WAVES;
+    return fits || (uint64_t)cnt->isl_most * 50u > (uint64_t)w * FLOW_WAVE_SLOTS ? w : 0u;
+}
 // Prepares the large islands' sweeps (after the row preparation): inboxes and next visits, with
 // the work list also those of the islands of its largest class that the solve launch of `cus`
 // workgroups will take (isl_arrive: their arrival words).
