@@ -3540,7 +3540,30 @@ __device__ __forceinline__ void flow_part(const Bodies& B, const StepParams& sp,
     uint32_t decided = 0;                  // the last check point known not to stop
     uint32_t stop_at = UNSET;
     uint32_t spins = 0;
-    const uint64_t t_start = wall_clock64(), t_limit = (uint64_t)spin_limit * 100ull;  // wall clock: 100 MHz
+    // The wait gives up after spin_limit without progress, its own or (a wave may wait for those that
+    // still work on earlier pieces) any other wave's: a wave that got on since it last looked stores
+    // the clock, one that did not looks whether another has.
+    uint64_t t_last = wall_clock64();
+    const uint64_t t_limit = (uint64_t)spin_limit * 100ull;  // wall clock: 100 MHz
+    uint32_t beat = 0;
+    bool moved = false;
+    auto stalled = [&]() -> bool {
+        const uint64_t now = wall_clock64();
+        if (moved) {
+            moved = false;
+            t_last = now;
+            if (lane == 0u)
+                __hip_atomic_store(&cnt->flow_beat, (uint32_t)now, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return false;
+        }
+        const uint32_t b = __hip_atomic_load(&cnt->flow_beat, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (b != beat) {
+            beat = b;
+            t_last = now;
+            return false;
+        }
+        return now - t_last > t_limit;
+    };
     bool failed = false;
     // Whether all have arrived at check point c; then whether one is above the tolerance.  The
     // large islands count in words of their own per check point, an island in two words for
@@ -3700,11 +3723,12 @@ __device__ __forceinline__ void flow_part(const Bodies& B, const StepParams& sp,
         }
         if (got != 0ull) {
             if (__ballot(live) == 0ull) break;
+            moved = true;
             continue;
         }
         __builtin_amdgcn_s_sleep(1);
         if ((++spins & 255u) == 0u) {
-            if (wall_clock64() - t_start > t_limit) {
+            if (stalled()) {
                 if (lane == 0u) atomicOr(err, STICKY_TIMEOUT);
                 failed = true;
                 break;
@@ -3721,8 +3745,9 @@ __device__ __forceinline__ void flow_part(const Bodies& B, const StepParams& sp,
         bool hit = stop_at != UNSET;
         if (!hit) {
             bool above = true, all = false;
+            t_last = wall_clock64();
             while (!(all = arrivals(nsweeps, above))) {
-                if (wall_clock64() - t_start > t_limit) break;
+                if ((++spins & 255u) == 0u && stalled()) break;
                 __builtin_amdgcn_s_sleep(1);
             }
             if (!all) {

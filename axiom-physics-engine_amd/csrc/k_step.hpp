@@ -190,7 +190,9 @@ struct OwnShape {
 // ones, which tol > 0 stops each at its own residual.  With `wide` the register sweep takes the
 // islands of the list's largest class when that is faster (launch_flow_init has prepared them);
 // parts in launches of their own name the same.  bmask holds the colouring's per-body colour
-// masks.  Events ev0 / ev1, when given, are recorded around the launch.
+// masks.  spin_limit: microseconds after which a wait gives up, in the register sweep those without
+// progress of any wave, in the staged sweep those from its start.  Events ev0 / ev1, when given, are
+// recorded around the launch.
 constexpr uint32_t SOLVE_LARGE = 1u, SOLVE_LIST = 2u;
 void launch_pgs_solve(const Bodies& B, const StepParams& sp, const SolverRows& R, uint32_t cap, const uint64_t* bmask,
                       uint32_t nsweeps, Counters* cnt, uint32_t spin_limit, uint32_t cus, const uint32_t* skey,

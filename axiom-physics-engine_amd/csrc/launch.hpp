@@ -149,6 +149,8 @@ struct Counters {
     uint32_t isl_wg_next;    // work taken from the workgroups' and from the waves' part of it,
     uint32_t isl_wave_next;  // beyond the first piece of each
     uint32_t loc_points;   // contact points of the islands solved on their own
+    uint32_t flow_beat;    // clock of the register sweep's last report of progress by some wave
+    uint32_t pad;
     unsigned long long loc_point_sweeps;     // their contact points x the sweeps each island ran
     unsigned long long bundle_point_sweeps;  // the same for the islands of islands_part
     // ---- kept across steps
@@ -175,7 +177,7 @@ template <class T> inline T spread_total(const Counters& c, T SpreadRow::*f) {
     for (uint32_t k = 0; k < SPREAD; ++k) s += c.sp[k].*f;
     return s;
 }
-constexpr uint32_t COUNTERS_RESET_WORDS = 32;  // words of the first block (cleared per step)
+constexpr uint32_t COUNTERS_RESET_WORDS = 34;  // words of the first block (cleared per step)
 static_assert(offsetof(Counters, sticky) == 4 * COUNTERS_RESET_WORDS, "per-step block ends at sticky");
 enum : uint32_t {
     STICKY_PAIRS = 1u,        // pair capacity exceeded
