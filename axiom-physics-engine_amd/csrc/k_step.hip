@@ -3699,6 +3699,8 @@ __device__ __forceinline__ void flow_part(const Bodies& B, const StepParams& sp,
                         if (n == wg_waves - 1u) {
                             const uint32_t mx = s_max, ab = s_above;
                             s_max = s_above = s_arrived = 0u;
+                            // a wave that sees this arrival finds the words cleared
+                            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
                             atomicMax(stop.bits + next - 1u, mx);
                             __hip_atomic_fetch_add(
                                 stop.arrive + ((size_t)(next - 1u) * CHECK_ROWS + blockIdx.x % CHECK_ROWS) * CHECK_ROW_WORDS,
@@ -3717,6 +3719,7 @@ __device__ __forceinline__ void flow_part(const Bodies& B, const StepParams& sp,
                         stop_at = c;
                         break;
                     }
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");  // the arrival words in LDS
                     decided = c;
                 }
             }
