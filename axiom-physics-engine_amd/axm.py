@@ -480,8 +480,9 @@ class World:
         _check(self._L.axm_world_set_sweep_config(self._h, groups, lds_kib, policy), "axm_world_set_sweep_config")
 
     def autotune(self, dt, iters, steps=5):
-        """Picks the fastest sweep launch shape on this world (advances it by a few steps per
-        candidate); returns (groups, lds_kib, policy, sweep_ms)."""
+        """Picks the fastest launch shape of the staged sweep on this world (advances it by a few steps
+        per candidate; keeps its shape where that sweep does not run); returns (groups, lds_kib,
+        policy, sweep_ms)."""
         c = SweepConfig()
         _check(self._L.axm_world_autotune(self._h, dt, iters, steps, C.byref(c)), "axm_world_autotune")
         return c.groups, c.lds_kib, c.policy, c.sweep_ms

@@ -1963,7 +1963,7 @@ constexpr uint32_t OWN_SLOTS = 16;  // slots per lane with a staged record
 // run in chunks of stop.every with a residual check after each chunk (every wave of
 // the grid meets at one arrival count per check).
 __global__ void __launch_bounds__(OWN_WAVE) k_pgs_own(Bodies B, StepParams sp, SolverRows R, Counters* cnt,
-                                                      uint32_t cap, uint32_t nsweeps, uint32_t flow_slots,
+                                                      uint32_t cap, uint32_t nsweeps, uint32_t flow_max,
                                                       uint32_t lds_f4, uint32_t spin_limit, uint32_t tune,
                                                       const uint64_t* __restrict__ bmask, SweepStop stop) {
     extern __shared__ float4 own_lds[];
@@ -1975,7 +1975,7 @@ __global__ void __launch_bounds__(OWN_WAVE) k_pgs_own(Bodies B, StepParams sp, S
         return;
     }
     if (cnt->sticky != 0u || nsweeps == 0u) return;
-    if (M > 0u && M <= flow_slots) return;  // flow_part ran them
+    if (M > 0u && M <= flow_max) return;  // flow_part ran them
     if (M == 0u && cnt->m_eff > 0u) {
         // every island was solved on its own: no sweep of the large ones runs
         if (blockIdx.x == 0 && lane == 0 && stop.bits) {
@@ -3802,7 +3802,7 @@ k_pgs_solve(Bodies B, StepParams sp, SolverRows R, Counters* cnt, uint32_t cap, 
     const uint32_t wide = list && wide_on ? wide_pieces(cnt, G) : 0u;
     uint32_t flows = 0;  // workgroups that sweep the large islands
     if ((parts & 1u) && cnt->max_colour <= 64u) {
-        const uint32_t M = cnt->m_glob <= G * FLOW_WAVES * FLOW_WAVE_SLOTS ? cnt->m_glob : 0u;  // more: k_pgs_own
+        const uint32_t M = cnt->m_glob <= flow_slots(G) ? cnt->m_glob : 0u;  // more: k_pgs_own
         const uint32_t nw = (M + FLOW_WAVE_SLOTS - 1u) / FLOW_WAVE_SLOTS + wide;
         // as thinly as the chip allows (a visit's wave holds up the others of its SIMD: 19.1k slots
         // on 75 workgroups take 24 us per sweep, on 256 21), but with a workgroup left for every 490
@@ -4310,7 +4310,7 @@ void launch_pgs_solve(const Bodies& B, const StepParams& sp, const SolverRows& R
                            spin_limit, bmask, list, skey, tol, parts, wide ? 1u : 0u, stop);
     if (parts & SOLVE_LARGE)
         hipLaunchKernelGGL(k_pgs_own, dim3(own.groups ? own.groups : 1u), dim3(OWN_WAVE), own.lds_bytes, s, B, sp, R, cnt,
-                           cap, nsweeps, cus * FLOW_WAVES * FLOW_WAVE_SLOTS, own.lds_bytes / (uint32_t)sizeof(float4),
+                           cap, nsweeps, flow_slots(cus), own.lds_bytes / (uint32_t)sizeof(float4),
                            spin_limit, own.tune, bmask, stop);
     if (ev1) (void)hipEventRecord(ev1, s);
 }

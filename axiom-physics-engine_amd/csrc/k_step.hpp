@@ -158,6 +158,8 @@ struct SweepStop {
 // Launch shape of the register sweep (flow_part).
 constexpr uint32_t FLOW_THREADS = 512, FLOW_WAVES = FLOW_THREADS / 64u;
 constexpr uint32_t FLOW_WAVE_SLOTS = 32;
+// Most slots of large islands that it takes on G workgroups; the staged sweep takes more.
+inline __host__ __device__ uint32_t flow_slots(uint32_t G) { return G * FLOW_WAVES * FLOW_WAVE_SLOTS; }
 // It reaches the inboxes by 32-bit byte offsets into a buffer of this many bytes.
 constexpr uint32_t FLOW_INBOX_BYTES = 0x7FFFFFFFu;
 // Pieces of 32 slots of the islands of the largest class that the register sweep takes on G

@@ -1766,8 +1766,10 @@ axm_status axm_world_autotune(axm_world w, float dt, uint32_t iters, uint32_t st
     }
     if (cands.empty()) return AXM_GPU_OPERATION_FAILED;
     const bool was_on = w->prof_on;
-    double best = 1e300;
-    Cand pick = cands[0];
+    const uint32_t groups0 = w->sweep_groups, lds0 = w->sweep_lds, policy0 = w->sweep_tune;
+    double best = 1e300, least = 1e300;
+    Cand pick{groups0, lds0 / 1024u, policy0};
+    bool staged = true;  // the staged sweep ran with every candidate
     for (const Cand& c : cands) {
         AXM_TRY(axm_world_set_sweep_config(w, c.groups, c.lds_kib, c.policy));
         AXM_TRY(axm_world_run(w, dt, iters, 1, 1, nullptr));  // capture outside the timing
@@ -1777,10 +1779,19 @@ axm_status axm_world_autotune(axm_world w, float dt, uint32_t iters, uint32_t st
         axm_kernel_profile p{};
         AXM_TRY(axm_world_profile(w, 0, &p));
         const double ms = p.pgs_launches ? p.pgs_ms / (double)p.pgs_launches : 1e300;
+        // only it has this shape: up to flow_slots slots the register sweep ran instead
+        AXM_TRY(read_counters(w));
+        staged = staged && w->h_cnt->m_glob > flow_slots((uint32_t)w->cu_count);
+        least = std::min(least, ms);
         if (ms < best) {
             best = ms;
             pick = c;
         }
+    }
+    if (!staged) {
+        // nothing to choose between: the shape stays as it was
+        pick = Cand{groups0, lds0 / 1024u, policy0};
+        best = least;
     }
     AXM_TRY(axm_world_set_sweep_config(w, pick.groups, pick.lds_kib, pick.policy));
     w->prof_on = was_on;

@@ -266,7 +266,10 @@ axm_status axm_world_load(axm_world w, const char* path);
  * (optional) receives the accumulated profile, which is then reset. */
 axm_status axm_world_profile(axm_world w, int enable, axm_kernel_profile* out);
 
-/* Launch shape of the persistent sweep kernel: workgroups of one wave (0: one per CU;
+/* Launch shape of the staged sweep kernel, which sweeps the large islands (with
+ * island_solve those of more than 4096 manifolds, else all) when they have more than 256
+ * manifolds per CU together (65536); up to there, and for the islands solved on their own,
+ * the sweep has no shape to set.  Workgroups of one wave (0: one per CU;
  * at most what can be resident at once), KiB of LDS per workgroup for the staged
  * Jacobian rows and impulses of its slots (0: the device maximum, up to 160), and
  * policy bits (bit 1, default on: poll one 16-byte hint before loading the
@@ -280,9 +283,10 @@ typedef struct axm_sweep_config {
     uint32_t groups, lds_kib, policy;
     double sweep_ms; /* its average sweep-kernel time over the trial steps */
 } axm_sweep_config;
-/* Autotuner of the persistent sweep: times `steps` graph-replayed steps (after one
+/* Autotuner of the staged sweep: times `steps` graph-replayed steps (after one
  * untimed capture step) for each candidate launch shape (one, two and four
- * workgroups per CU, LDS split between them), keeps the fastest and reports it.
+ * workgroups per CU, LDS split between them), keeps the fastest and reports it.  Where
+ * the staged sweep does not run (see above) it keeps and reports the world's shape.
  * The world advances by (steps + 1) x candidates steps; results do not depend on the
  * shape (no reference counterpart: the batched-world tuning hook). */
 axm_status axm_world_autotune(axm_world w, float dt, uint32_t iters, uint32_t steps, axm_sweep_config* out);
