@@ -183,6 +183,19 @@ def committed_traffic(kernel, cfg, n, args):
     return {"bytes_per_launch": t["bytes_per_launch"], "source": "profiles/" + os.path.basename(path)}
 
 
+def sweep_launches(tot, prof):
+    """(bytes, seconds, launches) of the two launches the sweeps are timed in, 240 B per contact point
+    and sweep each: the islands each solved by a workgroup or a wave (their points x the sweeps each
+    ran), and the rest: the large islands, and those of 257 to 4096 manifolds that the large islands'
+    sweep takes along."""
+    kern = {"k_pgs_solve (large islands)": (B_SWEEP * float(tot.contact_sweeps - prof.bundle_point_sweeps),
+                                            prof.pgs_ms * 1e-3, int(prof.pgs_launches))}
+    if prof.bundle_launches:
+        kern["k_pgs_solve (other islands)"] = (B_SWEEP * float(prof.bundle_point_sweeps), prof.bundle_ms * 1e-3,
+                                               int(prof.bundle_launches))
+    return kern
+
+
 def headline(args):
     cfg = args.config
     bodies, desc = axm.scene(cfg, SEED_BASE + 1000 * cfg, args.bodies, args.worlds)
@@ -240,14 +253,7 @@ def headline(args):
     value = bodies.n * args.steps / elapsed
     steps_done = max(int(tot.steps), 1)
     mean_sweeps = tot.sweeps / steps_done
-    # the sweeps (timed apart), 240 B per contact point per sweep each: those of the small
-    # islands solved on their own (their points x the sweeps each island ran) and the persistent
-    # sweep of the large islands (the rest); the roofline line is the one with more time
-    kern = {"k_pgs_solve (large islands)": (B_SWEEP * float(tot.contact_sweeps - tot.local_contact_sweeps),
-                                            prof.pgs_ms * 1e-3, int(prof.pgs_launches))}
-    if prof.bundle_launches:
-        kern["k_pgs_solve (other islands)"] = (B_SWEEP * float(prof.bundle_point_sweeps), prof.bundle_ms * 1e-3,
-                                               int(prof.bundle_launches))
+    kern = sweep_launches(tot, prof)  # the roofline line is the one with more time
 
     def roof_of(name):
         nbytes, secs, n = kern[name]

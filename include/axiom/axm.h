@@ -175,15 +175,17 @@ typedef struct axm_step_stats {
     uint32_t sleeping;      /* PhysicsWorldStats::sleepingBodies */
 } axm_step_stats;
 
-/* Kernel-level timing of the solver sweep kernel, accumulated over steps run
- * with profiling enabled (HIP events around every launch on the world's stream). */
+/* Kernel-level timing of the solver's sweeps, accumulated over steps run with profiling
+ * enabled (HIP events around every launch on the world's stream).  The sweeps then run in
+ * two launches: the islands that a workgroup or a wave solves on its own (bundle_*), and
+ * the large islands with those of 257 to 4096 manifolds that their sweep takes along. */
 typedef struct axm_kernel_profile {
     uint64_t steps;
     uint64_t pgs_launches;
     double pgs_ms;        /* summed kernel durations */
-    double pgs_bytes;     /* summed algorithmic bytes of those launches */
+    double pgs_bytes;     /* algorithmic bytes of the steps' sweeps: all rows x the step's sweeps */
     uint64_t sweeps;
-    /* the kernel of the islands solved on their own (island_solve) */
+    /* the launch of the islands solved by a workgroup or a wave each (island_solve) */
     uint64_t bundle_launches;
     double bundle_ms;     /* summed kernel durations */
     uint64_t bundle_point_sweeps; /* contact points x sweeps of its islands (240 B each) */
