@@ -40,7 +40,7 @@ struct PairIn {
     const float* qb;
 };
 
-__device__ Shp shape_at(const uint32_t* t, const float* p, const float* x, const float* q, uint32_t i) {
+__device__ __forceinline__ Shp shape_at(const uint32_t* t, const float* p, const float* x, const float* q, uint32_t i) {
     Shp s;
     s.type = t[i];
     s.prm = f3{p[3 * i], p[3 * i + 1], p[3 * i + 2]};
@@ -69,7 +69,9 @@ __device__ __forceinline__ void queue_deep(const DeepQueue& Q, bool deep, uint32
     if (deep) Q.list[base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = i;
 }
 
-__device__ void store_pair(const PairOut& out, uint32_t i, const Man& m, int st) {
+// Inlined: called, it has the manifold and its own arguments in scratch memory (1000 pairs of boxes
+// 28 us, inlined 21; spheres 8 and 4).
+__device__ __forceinline__ void store_pair(const PairOut& out, uint32_t i, const Man& m, int st) {
     out.npts[i] = m.np;
     out.status[i] = st;
 #pragma unroll
@@ -93,7 +95,7 @@ __device__ void store_pair(const PairOut& out, uint32_t i, const Man& m, int st)
 // the caller's order ran every test of its wave in turn (and the expansions of deep pairs in
 // scratch memory).  The chain of one test bounds a small batch, so tiles are 64 pairs while every
 // wave has a SIMD of its own (16384 pairs: 1024 waves) and grow with the batch to fill the lanes.
-// 16384 mixed pairs: 25 us, and 25 us for their deep pairs; together they took 317.
+// 16384 mixed pairs: 27 us, and 29 us for their deep pairs; together they took 317.
 constexpr uint32_t PAIR_TILE_MIN = 64u, PAIR_TILE_MAX = 1024u, PAIR_TILES = 256u;
 constexpr uint32_t PAIR_GROUPS = 4u;
 __device__ __forceinline__ uint32_t pair_group(uint32_t ta, uint32_t tb) {
@@ -139,6 +141,7 @@ __global__ void __launch_bounds__(64) k_collide_pairs(PairIn in, uint32_t n, uin
         queue_deep(Q, deep, i);
     }
 }
+__global__ void k_queue_clear(uint32_t* count) { *count = 0u; }
 // The deep box-capsule pairs, one wave each.
 __global__ void __launch_bounds__(64) k_collide_deep(PairIn in, PairOut out, DeepQueue Q) {
     __shared__ EpaWork W;
@@ -198,11 +201,13 @@ __global__ void __launch_bounds__(64) k_epa_pairs(PairIn in, float* out, int32_t
 // Waves of an expansion kernel: two on a SIMD are all that its registers leave room for; they
 // stride over the queue.
 uint32_t deep_waves(uint32_t n) { return std::min<uint32_t>(n, 2048u); }
-void launch_collide(const PairIn& in, uint32_t n, float margin, const PairOut& out, const DeepQueue& Q, hipStream_t s) {
+// deep: some pair may be queued (any_deep).
+void launch_collide(const PairIn& in, uint32_t n, float margin, const PairOut& out, const DeepQueue& Q, bool deep,
+                    hipStream_t s) {
     uint32_t tile = PAIR_TILE_MIN;
     while (tile < PAIR_TILE_MAX && (uint64_t)tile * PAIR_TILES < n) tile *= 2u;
     hipLaunchKernelGGL(k_collide_pairs, dim3((n - 1u) / tile + 1u, PAIR_GROUPS), dim3(64), 0, s, in, n, tile, margin, out, Q);
-    hipLaunchKernelGGL(k_collide_deep, dim3(deep_waves(n)), dim3(64), 0, s, in, out, Q);
+    if (deep) hipLaunchKernelGGL(k_collide_deep, dim3(deep_waves(n)), dim3(64), 0, s, in, out, Q);
 }
 
 // What a batched call holds while it runs: staging for its arrays and a stream.  A process keeps
@@ -300,6 +305,13 @@ bool valid_types(uint32_t n, const uint32_t* ta, const uint32_t* tb, bool allow_
     return true;
 }
 
+// Whether a pair may go through the queue of deep pairs: a box with a capsule.
+bool any_deep(uint32_t n, const uint32_t* ta, const uint32_t* tb) {
+    for (uint32_t i = 0; i < n; ++i)
+        if ((ta[i] == SHAPE_BOX && tb[i] == SHAPE_CAPSULE) || (ta[i] == SHAPE_CAPSULE && tb[i] == SHAPE_BOX)) return true;
+    return false;
+}
+
 }  // namespace
 
 extern "C" {
@@ -335,7 +347,7 @@ axm_status axm_collide_pairs(int32_t device, uint32_t n, const uint32_t* type_a,
     const PairIn in{u32(d + ta), f32(d + pa), f32(d + xa), f32(d + qa), u32(d + tb), f32(d + pb), f32(d + xb), f32(d + qb)};
     const PairOut out{u32(o + d_np), f32(o + d_pos), f32(o + d_n), f32(o + d_d), u32(o + d_f),
                       reinterpret_cast<int32_t*>(o + d_s)};
-    launch_collide(in, n, margin, out, DeepQueue{u32(o + down.total), u32(d + qn)}, s);
+    launch_collide(in, n, margin, out, DeepQueue{u32(o + down.total), u32(d + qn)}, any_deep(n, type_a, type_b), s);
     if (hipGetLastError() != hipSuccess ||
         c->stage.down(down.part, down.parts, up.total, down.total, s) != hipSuccess)
         return AXM_GPU_OPERATION_FAILED;
@@ -368,7 +380,11 @@ axm_status axm_collide_pairs_noalloc(int32_t device, uint32_t n, const uint32_t*
     };
     const Up ups[] = {{NA_TA, type_a, 4ull * n}, {NA_PA, prm_a, 12ull * n}, {NA_XA, pos_a, 12ull * n},
                       {NA_QA, quat_a, 16ull * n}, {NA_TB, type_b, 4ull * n}, {NA_PB, prm_b, 12ull * n},
-                      {NA_XB, pos_b, 12ull * n}, {NA_QB, quat_b, 16ull * n}, {NA_WORDS, &NO_PAIRS, 4ull}};
+                      {NA_XB, pos_b, 12ull * n}, {NA_QB, quat_b, 16ull * n}};
+    // cleared by a launch, which the uploads do not wait for: a ninth upload took 13 us of a small call's
+    // 205, this and the queue's launch 5, and neither is made when no pair can be deep
+    const bool deep = any_deep(n, type_a, type_b);
+    if (deep) hipLaunchKernelGGL(k_queue_clear, dim3(1), dim3(1), 0, 0, reg(NA_WORDS));
     for (const Up& u : ups)
         if (hipMemcpy(reg(u.r), u.h, u.bytes, hipMemcpyHostToDevice) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
     PairIn in;
@@ -384,7 +400,7 @@ axm_status axm_collide_pairs_noalloc(int32_t device, uint32_t n, const uint32_t*
     // so nothing left by an earlier call is read back
     const PairOut out{reg(NA_NP), reinterpret_cast<float*>(reg(NA_POS)), reinterpret_cast<float*>(reg(NA_NRM)),
                       reinterpret_cast<float*>(reg(NA_DEP)), reg(NA_FID), reinterpret_cast<int32_t*>(reg(NA_ST))};
-    launch_collide(in, n, margin, out, DeepQueue{reg(NA_QUEUE), reg(NA_WORDS)}, 0);
+    launch_collide(in, n, margin, out, DeepQueue{reg(NA_QUEUE), reg(NA_WORDS)}, deep, 0);
     if (hipDeviceSynchronize() != hipSuccess) return AXM_GPU_OPERATION_FAILED;
     if (hipMemcpy(npts, reg(NA_NP), 4ull * n, hipMemcpyDeviceToHost) != hipSuccess ||
         hipMemcpy(pos, reg(NA_POS), 48ull * n, hipMemcpyDeviceToHost) != hipSuccess ||
