@@ -1,6 +1,7 @@
 // Device-wide exclusive scan and stable LSD radix sort for gfx950 (wave64).
 //
-// Radix sort: 8-bit digits, one launch for all passes (below).
+// Radix sort: digits of 8 bits with every pass in one launch, or, for more than 131072 keys read
+// from memory, of up to 10 bits in three launches a pass (below).
 // Scan: one pass, tiles chained by decoupled look-back (below).
 #include <hip/hip_runtime.h>
 #include <stdint.h>

@@ -4,14 +4,15 @@
 // examples/profiling_example.cpp:132-165, with semi-implicit Euler from
 // examples/body_inspector_example.cpp:48-60):
 //   k_begin            gravity/damping -> solver velocities, world inverse inertia, AABB, cell key
-//   radix sort         (key, body) stable, 8-bit digits
+//   radix sort         (key, body) stable
 //   k_cell_table       hash of cell -> (first sorted index, count)
 //   k_pair_count/emit  27-neighbour grid scan, inclusive AABB test, j > i; exclusive scan between
 //   k_narrow(+_epa)    primitive narrowphase -> <= 4 points per pair (staged per pair)
 //   k_compact          pairs with points -> manifolds (pair order, exclusive scan of the flags)
 //   k_col_*            Jones-Plassmann colouring with first-fit colours
 //   k_prep             per-point rows + warm start (previous-step impulses keyed by (a, b, feature))
-//   k_pgs              one colour of one sequential-impulse sweep
+//   k_pgs_solve        all sweeps of all islands (k_pgs_own: very large ones; k_pgs: one colour of
+//                      one sweep)
 //   k_residual         velocity-space fixed-point residual
 //   k_integrate        x += v dt, q += dt/2 (w,0) q, normalise
 // Every body-parallel kernel is one thread per body; every manifold-parallel
@@ -3392,14 +3393,15 @@ __device__ __forceinline__ void islands_part(const Bodies& B, const StepParams& 
 }
 
 // ---------------------------------------------------------------- large islands in registers
-// The large islands' sweeps when every slot has two lanes of the GPU to itself (FLOW_SLOTS
+// The large islands' sweeps when every slot has two lanes of the GPU to itself (flow_slots
 // slots at most; k_pgs_own takes more): the even lane of a pair holds body a's side of the
 // slot's rows, the odd lane body b's (half_jvel), with the impulses, in registers for the whole
 // solve.  Visits pass velocities on through the inboxes as in k_pgs_own; with one slot per pair
 // a wave's lanes wait for nothing but their own bodies, and a visit reads only the 32 bytes of
 // its inbox side from memory.  What binds is the chain of dependent visits: a handoff (store,
 // poll) of about 0.5 us and three row updates of 22 instructions per point.  Slots are dealt
-// out thinly (spw per wave, as few as M allows) so that a visit holds up few others.
+// out 32 to a wave, over as many workgroups as are free (k_pgs_solve), so that a visit holds up
+// few others.
 //
 // Residual checks run one sweep behind: after s sweeps (a check point) a slot's residual needs
 // its bodies' velocities after the sweep, which their first visits of the next sweep have in

@@ -108,8 +108,7 @@ void launch_colour(const Bodies& B, const uint2* m_ab, uint32_t cap_man, uint32_
 // Work the row preparation launch also does for the launches after it, each in a loop of
 // its own over the grid: the colour offsets of the sorted keys skey (col_off[c] = first
 // position whose key has colour >= c, c = 0..K, and m_glob = col_off[K], when col_off is
-// set), the small islands' work list from the same keys (when list is set;
-// launch_pgs_local then builds none), clearing zero_n words (the sweep's residual words),
+// set), the small islands' work list from the same keys (when list is set), clearing zero_n words (the sweep's residual words),
 // and emptying the (a, b) -> slot table of row set cset (the entries its last build
 // recorded, at the positions cpos holds; when ckey is set, the table's build is then made
 // without clearing it).  More than max_k colours fail the step (STICKY_COLOURS).
@@ -141,7 +140,7 @@ void launch_mlp_apply(const SolverRows& R, const Counters* cnt, uint32_t cap, co
 // arrays start the step at zero.  bits == nullptr means no checks.
 constexpr uint32_t CHECK_ROWS = 8, CHECK_ROW_WORDS = 32;
 // The islands swept in the same launch count their arrivals in two 64-bit words each, 64 bytes
-// apart, ISL_ARRIVE_WORDS per island of the work list's largest class (launch_pgs_local clears
+// apart, ISL_ARRIVE_WORDS per island of the work list's largest class (launch_flow_init clears
 // them): isl_arrive_words for a manifold capacity.
 constexpr uint32_t ISL_ARRIVE_WORDS = 16;
 inline size_t isl_arrive_words(uint32_t cap_man) { return (size_t)ISL_ARRIVE_WORDS * (cap_man / 257u + 1u); }

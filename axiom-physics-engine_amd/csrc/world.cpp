@@ -126,7 +126,7 @@ struct axm_world_s {
     axm_mlp_s* mlp = nullptr;
     float last_dt = 0.0f;
 
-    // persistent sweep launch shape: workgroups (one wave each, all resident at
+    // staged sweep (k_pgs_own) launch shape: workgroups (one wave each, all resident at
     // once), LDS per workgroup for the staged rows of its slots, and the policy
     // (bit 1 poll a 16-byte hint before the full load, bit 2 adaptive back-off,
     // bits 4-6 poll back-off).
@@ -559,7 +559,7 @@ axm_status prof_mark(axm_world_s* w, size_t& nev, bool capturing) {
 // A step is enqueued in three phases so that a profiled graph replay can launch
 // the sweep kernel eagerly between two captured graphs, bracketed by events.
 enum : uint32_t { PH_PRE = 1u, PH_SWEEP = 2u, PH_POST = 4u, PH_ALL = 7u };
-constexpr uint32_t SWEEP_SPIN_LIMIT_US = 2000000u;  // bounded dependency wait of the sweep kernel
+constexpr uint32_t SWEEP_SPIN_LIMIT_US = 2000000u;  // bounded dependency waits of the sweeps
 
 struct StepOpts {
     uint32_t iters = 10;
@@ -706,8 +706,8 @@ bool sweep_checks(const axm_world_s* w, bool colour_launches, SweepStop& st) {
 }
 
 // Enqueues one step.  Synchronises only for per-colour sweep launches (with a
-// residual tolerance they check it on the host); the persistent sweep checks the
-// residual itself, so a step with a tolerance enqueues without synchronising.
+// residual tolerance they check it on the host); the other sweeps check the
+// residual themselves, so a step with a tolerance enqueues without synchronising.
 axm_status enqueue_step(axm_world_s* w, float dt, const StepOpts& o) {
     // every kernel below sizes its grid and row strides by the current set's capacity
     if (w->rcap[w->cur] < w->cap_man || w->rcap[1 - w->cur] < w->cap_man) return AXM_GPU_INVALID_OPERATION;
@@ -973,8 +973,8 @@ axm_status step_sync(axm_world_s* w, float dt, StepOpts o, axm_step_stats* st) {
     fill_stats(w, S);
     const bool want_res = (o.flags & AXM_STEP_RESIDUAL) || w->desc.record_residual || w->desc.residual_tol > 0.0f;
     w->h_res.clear();
-    // the islands solved on their own are finished before the large ones' sweeps: every
-    // entry of the history reports the larger of the two residuals
+    // the islands solved on their own report only the residual they ended with: every entry
+    // of the history is the larger of that and the large ones' residual
     float loc_res;
     std::memcpy(&loc_res, &w->h_cnt->loc_res_bits, 4);
     if (want_res && w->last_iters) {
