@@ -201,7 +201,7 @@ __global__ void __launch_bounds__(64) k_epa_pairs(PairIn in, float* out, int32_t
 // Waves of an expansion kernel: two on a SIMD are all that its registers leave room for; they
 // stride over the queue.
 uint32_t deep_waves(uint32_t n) { return std::min<uint32_t>(n, 2048u); }
-// deep: some pair may be queued (any_deep).
+// deep: some pair may be queued.
 void launch_collide(const PairIn& in, uint32_t n, float margin, const PairOut& out, const DeepQueue& Q, bool deep,
                     hipStream_t s) {
     uint32_t tile = PAIR_TILE_MIN;
@@ -297,19 +297,18 @@ uint32_t* scratch_on(int32_t device) {
     return g_scratch_ptr[device];
 }
 
-bool valid_types(uint32_t n, const uint32_t* ta, const uint32_t* tb, bool allow_plane_b) {
+// Whether the types are allowed; sets *deep when a pair may go through the queue of deep pairs (a box
+// with a capsule).
+bool valid_types(uint32_t n, const uint32_t* ta, const uint32_t* tb, bool allow_plane_b, bool* deep = nullptr) {
+    bool any = false;
     for (uint32_t i = 0; i < n; ++i) {
-        if (ta[i] > AXM_SHAPE_CAPSULE) return false;
-        if (tb[i] > (allow_plane_b ? (uint32_t)AXM_SHAPE_PLANE : (uint32_t)AXM_SHAPE_CAPSULE)) return false;
+        const uint32_t a = ta[i], b = tb[i];
+        if (a > AXM_SHAPE_CAPSULE) return false;
+        if (b > (allow_plane_b ? (uint32_t)AXM_SHAPE_PLANE : (uint32_t)AXM_SHAPE_CAPSULE)) return false;
+        any |= (a == SHAPE_BOX && b == SHAPE_CAPSULE) || (a == SHAPE_CAPSULE && b == SHAPE_BOX);
     }
+    if (deep) *deep = any;
     return true;
-}
-
-// Whether a pair may go through the queue of deep pairs: a box with a capsule.
-bool any_deep(uint32_t n, const uint32_t* ta, const uint32_t* tb) {
-    for (uint32_t i = 0; i < n; ++i)
-        if ((ta[i] == SHAPE_BOX && tb[i] == SHAPE_CAPSULE) || (ta[i] == SHAPE_CAPSULE && tb[i] == SHAPE_BOX)) return true;
-    return false;
 }
 
 }  // namespace
@@ -324,7 +323,8 @@ axm_status axm_collide_pairs(int32_t device, uint32_t n, const uint32_t* type_a,
     if (!type_a || !prm_a || !pos_a || !quat_a || !type_b || !prm_b || !pos_b || !quat_b || !npts || !pos || !normal ||
         !depth || !feature)
         return AXM_NULL_POINTER;
-    if (!valid_types(n, type_a, type_b, true)) return AXM_INVALID_SHAPE;
+    bool deep;
+    if (!valid_types(n, type_a, type_b, true, &deep)) return AXM_INVALID_SHAPE;
     PairLayout up, down;
     const size_t N = n;
     const size_t ta = up.add(type_a, N), pa = up.add(prm_a, 3 * N), xa = up.add(pos_a, 3 * N), qa = up.add(quat_a, 4 * N),
@@ -347,7 +347,7 @@ axm_status axm_collide_pairs(int32_t device, uint32_t n, const uint32_t* type_a,
     const PairIn in{u32(d + ta), f32(d + pa), f32(d + xa), f32(d + qa), u32(d + tb), f32(d + pb), f32(d + xb), f32(d + qb)};
     const PairOut out{u32(o + d_np), f32(o + d_pos), f32(o + d_n), f32(o + d_d), u32(o + d_f),
                       reinterpret_cast<int32_t*>(o + d_s)};
-    launch_collide(in, n, margin, out, DeepQueue{u32(o + down.total), u32(d + qn)}, any_deep(n, type_a, type_b), s);
+    launch_collide(in, n, margin, out, DeepQueue{u32(o + down.total), u32(d + qn)}, deep, s);
     if (hipGetLastError() != hipSuccess ||
         c->stage.down(down.part, down.parts, up.total, down.total, s) != hipSuccess)
         return AXM_GPU_OPERATION_FAILED;
@@ -366,7 +366,8 @@ axm_status axm_collide_pairs_noalloc(int32_t device, uint32_t n, const uint32_t*
         !depth || !feature)
         return AXM_NULL_POINTER;
     if (n > NOALLOC_MAX_PAIRS) return AXM_OUT_OF_RANGE;
-    if (!valid_types(n, type_a, type_b, true)) return AXM_INVALID_SHAPE;
+    bool deep;
+    if (!valid_types(n, type_a, type_b, true, &deep)) return AXM_INVALID_SHAPE;
     if (hipSetDevice(device) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
     uint32_t* base = scratch_on(device);
     if (!base) return AXM_GPU_OPERATION_FAILED;
@@ -383,7 +384,6 @@ axm_status axm_collide_pairs_noalloc(int32_t device, uint32_t n, const uint32_t*
                       {NA_XB, pos_b, 12ull * n}, {NA_QB, quat_b, 16ull * n}};
     // cleared by a launch, which the uploads do not wait for: a ninth upload took 13 us of a small call's
     // 205, this and the queue's launch 5, and neither is made when no pair can be deep
-    const bool deep = any_deep(n, type_a, type_b);
     if (deep) hipLaunchKernelGGL(k_queue_clear, dim3(1), dim3(1), 0, 0, reg(NA_WORDS));
     for (const Up& u : ups)
         if (hipMemcpy(reg(u.r), u.h, u.bytes, hipMemcpyHostToDevice) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
@@ -401,7 +401,7 @@ axm_status axm_collide_pairs_noalloc(int32_t device, uint32_t n, const uint32_t*
     const PairOut out{reg(NA_NP), reinterpret_cast<float*>(reg(NA_POS)), reinterpret_cast<float*>(reg(NA_NRM)),
                       reinterpret_cast<float*>(reg(NA_DEP)), reg(NA_FID), reinterpret_cast<int32_t*>(reg(NA_ST))};
     launch_collide(in, n, margin, out, DeepQueue{reg(NA_QUEUE), reg(NA_WORDS)}, deep, 0);
-    if (hipDeviceSynchronize() != hipSuccess) return AXM_GPU_OPERATION_FAILED;
+    if (hipStreamSynchronize(0) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
     if (hipMemcpy(npts, reg(NA_NP), 4ull * n, hipMemcpyDeviceToHost) != hipSuccess ||
         hipMemcpy(pos, reg(NA_POS), 48ull * n, hipMemcpyDeviceToHost) != hipSuccess ||
         hipMemcpy(normal, reg(NA_NRM), 48ull * n, hipMemcpyDeviceToHost) != hipSuccess ||
