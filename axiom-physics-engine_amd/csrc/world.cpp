@@ -276,6 +276,9 @@ axm_status alloc_bodies(axm_world_s* w, uint32_t cap) {
     AXM_TRY(w->mem.get(w->key_alt, cap));
     AXM_TRY(w->mem.get(w->val, cap));
     AXM_TRY(w->mem.get(w->val_alt, cap));
+    // a body sort whose meeting gives up leaves what was in its buffers among the sorted bodies, and the
+    // broadphase after it gathers by them (the step fails later): body indices from the start
+    if (hipMemset(w->val_alt, 0, 4ull * cap) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
     AXM_TRY(w->mem.get(w->sort_tmp, radix_tmp_words(cap)));
     // the scans' look-back scratch must start zeroed (each scan leaves it zeroed)
     if (hipMemset(w->sort_tmp, 0, 4 * radix_tmp_words(cap)) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
