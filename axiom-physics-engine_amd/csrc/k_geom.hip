@@ -300,15 +300,15 @@ uint32_t* scratch_on(int32_t device) {
 // Whether the types are allowed; sets *deep when a pair may go through the queue of deep pairs (a box
 // with a capsule).
 bool valid_types(uint32_t n, const uint32_t* ta, const uint32_t* tb, bool allow_plane_b, bool* deep = nullptr) {
-    bool any = false;
+    const uint32_t top_b = allow_plane_b ? (uint32_t)AXM_SHAPE_PLANE : (uint32_t)AXM_SHAPE_CAPSULE;
+    uint32_t bad = 0, any = 0;  // no branch in the loop: the compiler takes several pairs at a time
     for (uint32_t i = 0; i < n; ++i) {
         const uint32_t a = ta[i], b = tb[i];
-        if (a > AXM_SHAPE_CAPSULE) return false;
-        if (b > (allow_plane_b ? (uint32_t)AXM_SHAPE_PLANE : (uint32_t)AXM_SHAPE_CAPSULE)) return false;
-        any |= (a == SHAPE_BOX && b == SHAPE_CAPSULE) || (a == SHAPE_CAPSULE && b == SHAPE_BOX);
+        bad |= (uint32_t)(a > (uint32_t)AXM_SHAPE_CAPSULE) | (uint32_t)(b > top_b);
+        any |= (uint32_t)(a + b == SHAPE_BOX + SHAPE_CAPSULE) & (uint32_t)(b - SHAPE_BOX <= SHAPE_CAPSULE - SHAPE_BOX);
     }
-    if (deep) *deep = any;
-    return true;
+    if (deep) *deep = any != 0u;
+    return bad == 0u;
 }
 
 }  // namespace
