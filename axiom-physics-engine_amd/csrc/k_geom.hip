@@ -10,6 +10,7 @@
 
 #include "axiom/axm.h"
 #include "dev_geom.hpp"
+#include "host_copy.hpp"
 #include "staging.hpp"
 
 using namespace axm;
@@ -386,7 +387,7 @@ axm_status axm_collide_pairs_noalloc(int32_t device, uint32_t n, const uint32_t*
     // 205, this and the queue's launch 5, and neither is made when no pair can be deep
     if (deep) hipLaunchKernelGGL(k_queue_clear, dim3(1), dim3(1), 0, 0, reg(NA_WORDS));
     for (const Up& u : ups)
-        if (hipMemcpy(reg(u.r), u.h, u.bytes, hipMemcpyHostToDevice) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
+        if (copy_sync(reg(u.r), u.h, u.bytes, hipMemcpyHostToDevice) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
     PairIn in;
     in.ta = reg(NA_TA);
     in.pa = reinterpret_cast<const float*>(reg(NA_PA));
@@ -402,18 +403,18 @@ axm_status axm_collide_pairs_noalloc(int32_t device, uint32_t n, const uint32_t*
                       reinterpret_cast<float*>(reg(NA_DEP)), reg(NA_FID), reinterpret_cast<int32_t*>(reg(NA_ST))};
     launch_collide(in, n, margin, out, DeepQueue{reg(NA_QUEUE), reg(NA_WORDS)}, deep, 0);
     if (hipStreamSynchronize(0) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
-    if (hipMemcpy(npts, reg(NA_NP), 4ull * n, hipMemcpyDeviceToHost) != hipSuccess ||
-        hipMemcpy(pos, reg(NA_POS), 48ull * n, hipMemcpyDeviceToHost) != hipSuccess ||
-        hipMemcpy(normal, reg(NA_NRM), 48ull * n, hipMemcpyDeviceToHost) != hipSuccess ||
-        hipMemcpy(depth, reg(NA_DEP), 16ull * n, hipMemcpyDeviceToHost) != hipSuccess ||
-        hipMemcpy(feature, reg(NA_FID), 16ull * n, hipMemcpyDeviceToHost) != hipSuccess)
+    if (copy_sync(npts, reg(NA_NP), 4ull * n, hipMemcpyDeviceToHost) != hipSuccess ||
+        copy_sync(pos, reg(NA_POS), 48ull * n, hipMemcpyDeviceToHost) != hipSuccess ||
+        copy_sync(normal, reg(NA_NRM), 48ull * n, hipMemcpyDeviceToHost) != hipSuccess ||
+        copy_sync(depth, reg(NA_DEP), 16ull * n, hipMemcpyDeviceToHost) != hipSuccess ||
+        copy_sync(feature, reg(NA_FID), 16ull * n, hipMemcpyDeviceToHost) != hipSuccess)
         return AXM_GPU_OPERATION_FAILED;
     // the first failing pair's status, as axm_collide_pairs reports it; read 4096 at a time
     // into a fixed host buffer
     int32_t st[4096];
     for (uint32_t i0 = 0; i0 < n; i0 += 4096) {
         const uint32_t c = std::min<uint32_t>(4096u, n - i0);
-        if (hipMemcpy(st, reg(NA_ST) + i0, 4ull * c, hipMemcpyDeviceToHost) != hipSuccess)
+        if (copy_sync(st, reg(NA_ST) + i0, 4ull * c, hipMemcpyDeviceToHost) != hipSuccess)
             return AXM_GPU_OPERATION_FAILED;
         for (uint32_t i = 0; i < c; ++i)
             if (st[i] != GEOM_OK) return st[i];

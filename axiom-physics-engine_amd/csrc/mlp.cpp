@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "file_io.hpp"
+#include "host_copy.hpp"
 #include "mlp_impl.hpp"
 
 using namespace axm;
@@ -99,8 +100,8 @@ axm_status axm_mlp_create(int32_t device, axm_mlp* out) {
     if (st == AXM_SUCCESS) {
         m->blocks = GRAD_BLOCKS;
         std::vector<float> zero(MLP_NPARAM, 0.0f);
-        if (hipMemcpy(m->m, zero.data(), sizeof(float) * MLP_NPARAM, hipMemcpyHostToDevice) != hipSuccess ||
-            hipMemcpy(m->v, zero.data(), sizeof(float) * MLP_NPARAM, hipMemcpyHostToDevice) != hipSuccess)
+        if (copy_sync(m->m, zero.data(), sizeof(float) * MLP_NPARAM, hipMemcpyHostToDevice) != hipSuccess ||
+            copy_sync(m->v, zero.data(), sizeof(float) * MLP_NPARAM, hipMemcpyHostToDevice) != hipSuccess)
             st = AXM_GPU_OPERATION_FAILED;
         else
             st = upload_params(m, zero.data());
@@ -144,8 +145,8 @@ axm_status axm_mlp_init(axm_mlp m, uint64_t seed) {
     fill(MLP_OFF_W3, MLP_OUT * MLP_H, MLP_H);
     m->adam_t = 0;
     std::vector<float> zero(MLP_NPARAM, 0.0f);
-    MLP_HIP(hipMemcpy(m->m, zero.data(), sizeof(float) * MLP_NPARAM, hipMemcpyHostToDevice));
-    MLP_HIP(hipMemcpy(m->v, zero.data(), sizeof(float) * MLP_NPARAM, hipMemcpyHostToDevice));
+    MLP_HIP(copy_sync(m->m, zero.data(), sizeof(float) * MLP_NPARAM, hipMemcpyHostToDevice));
+    MLP_HIP(copy_sync(m->v, zero.data(), sizeof(float) * MLP_NPARAM, hipMemcpyHostToDevice));
     return upload_params(m, p.data());
 }
 

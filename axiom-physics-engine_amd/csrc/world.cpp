@@ -26,6 +26,7 @@
 #include "axiom/axm.h"
 #include "device_turn.hpp"
 #include "file_io.hpp"
+#include "host_copy.hpp"
 #include "k_bodies.hpp"
 #include "k_step.hpp"
 #include "mlp_impl.hpp"
@@ -278,10 +279,10 @@ axm_status alloc_bodies(axm_world_s* w, uint32_t cap) {
     AXM_TRY(w->mem.get(w->val_alt, cap));
     // a body sort whose meeting gives up leaves what was in its buffers among the sorted bodies, and the
     // broadphase after it gathers by them (the step fails later): body indices from the start
-    if (hipMemset(w->val_alt, 0, 4ull * cap) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
+    if (fill_sync(w->val_alt, 0, 4ull * cap) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
     AXM_TRY(w->mem.get(w->sort_tmp, radix_tmp_words(cap)));
     // the scans' look-back scratch must start zeroed (each scan leaves it zeroed)
-    if (hipMemset(w->sort_tmp, 0, 4 * radix_tmp_words(cap)) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
+    if (fill_sync(w->sort_tmp, 0, 4 * radix_tmp_words(cap)) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
     const uint32_t T = pow2_at_least(2ull * cap + 16);
     AXM_TRY(w->mem.get(w->ct.ent, T));
     w->ct.mask = T - 1;
@@ -294,7 +295,7 @@ axm_status alloc_bodies(axm_world_s* w, uint32_t cap) {
     AXM_TRY(w->mem.get(w->pair_cnt, (size_t)BP_PARTS * cap));
     AXM_TRY(w->mem.get(w->pair_off, (size_t)BP_PARTS * cap + 1));
     AXM_TRY(w->mem.get(w->scan_tmp, scan_tmp_words(BP_PARTS * cap)));
-    if (hipMemset(w->scan_tmp, 0, 4 * scan_tmp_words(BP_PARTS * cap)) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
+    if (fill_sync(w->scan_tmp, 0, 4 * scan_tmp_words(BP_PARTS * cap)) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
     AXM_TRY(w->mem.get(w->bmax0, cap));
     AXM_TRY(w->mem.get(w->bmax1, cap));
     AXM_TRY(w->mem.get(w->bmask, cap));
@@ -324,7 +325,7 @@ axm_status alloc_pairs(axm_world_s* w, uint32_t cap) {
     AXM_TRY(w->mem.get(w->p_pt, (size_t)cap * 4));
     AXM_TRY(w->mem.get(w->p_nf, (size_t)cap * 4));
     AXM_TRY(w->mem.get(w->pscan_tmp, scan_tmp_words(cap)));
-    if (hipMemset(w->pscan_tmp, 0, 4 * scan_tmp_words(cap)) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
+    if (fill_sync(w->pscan_tmp, 0, 4 * scan_tmp_words(cap)) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
     w->cap_pairs = cap;
     return AXM_SUCCESS;
 }
@@ -359,9 +360,9 @@ axm_status alloc_rows(axm_world_s* w, int set, uint32_t cap) {
     AXM_TRY(w->mem.get(w->pc_slot[set], T));
     AXM_TRY(w->mem.get(w->pc_pos[set], cap));
     // an empty table: no warm-start hit until a step has filled it
-    if (hipMemset(w->pc_key[set], 0xFF, 8ull * T) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
-    if (w->cnt && hipMemset(&w->cnt->cache_m[set], 0, 4) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
-    if (hipMemset(w->np_slot[set], 0, 4ull * cap) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
+    if (fill_sync(w->pc_key[set], 0xFF, 8ull * T) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
+    if (w->cnt && fill_sync(&w->cnt->cache_m[set], 0, 4) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
+    if (fill_sync(w->np_slot[set], 0, 4ull * cap) != hipSuccess) return AXM_GPU_OPERATION_FAILED;
     w->pc_mask[set] = T - 1;
     w->rcap[set] = cap;
     return AXM_SUCCESS;
@@ -982,7 +983,7 @@ axm_status step_sync(axm_world_s* w, float dt, StepOpts o, axm_step_stats* st) {
     std::memcpy(&loc_res, &w->h_cnt->loc_res_bits, 4);
     if (want_res && w->last_iters) {
         std::vector<uint32_t> bits(w->last_iters);
-        AXM_HIP(hipMemcpy(bits.data(), w->res_bits, 4ull * w->last_iters, hipMemcpyDeviceToHost));
+        AXM_HIP(copy_sync(bits.data(), w->res_bits, 4ull * w->last_iters, hipMemcpyDeviceToHost));
         for (uint32_t k = 0; k < w->last_iters; ++k) {
             float f;
             std::memcpy(&f, &bits[k], 4);
@@ -1022,10 +1023,12 @@ axm_status capture(axm_world_s* w, float dt, uint32_t iters, int parity, uint32_
     o.iters = iters;
     o.capture = true;
     o.phases = phases;
+    std::unique_lock<std::shared_mutex> alone(capture_lock());
     AXM_HIP(hipStreamBeginCapture(w->stream, hipStreamCaptureModeThreadLocal));
     const axm_status st = enqueue_step(w, dt, o);
     hipGraph_t g = nullptr;
     const hipError_t ee = hipStreamEndCapture(w->stream, &g);
+    alone.unlock();
     w->cur = saved_cur;
     w->prev_valid = saved_prev;
     w->have_step = saved_step;
@@ -1101,9 +1104,9 @@ axm_status axm_world_create(const axm_world_desc* desc, axm_world* out) {
     if (st == AXM_SUCCESS) st = alloc_pairs(w, desc->max_pairs ? desc->max_pairs : 1024u);
     if (st == AXM_SUCCESS) st = alloc_manifolds(w, desc->max_manifolds ? desc->max_manifolds : 1024u);
     if (st == AXM_SUCCESS && w->rcap[1 - w->cur] < w->cap_man) st = alloc_rows(w, 1 - w->cur, w->cap_man);
-    if (st == AXM_SUCCESS && (hipMemset(w->cnt, 0, sizeof(Counters)) != hipSuccess ||
-                              hipMemset(w->bar, 0, sizeof(GridBar)) != hipSuccess ||
-                              hipMemset(w->sort_meet, 0, 4 * radix_meet_words()) != hipSuccess))
+    if (st == AXM_SUCCESS && (fill_sync(w->cnt, 0, sizeof(Counters)) != hipSuccess ||
+                              fill_sync(w->bar, 0, sizeof(GridBar)) != hipSuccess ||
+                              fill_sync(w->sort_meet, 0, 4 * radix_meet_words()) != hipSuccess))
         st = AXM_GPU_OPERATION_FAILED;
     if (st != AXM_SUCCESS) {
         delete w;
@@ -1302,8 +1305,8 @@ axm_status axm_world_get_pre_solve_velocities(axm_world w, float* lin_vel, float
     (void)hipSetDevice(w->desc.device);
     const uint32_t n = w->n;
     std::vector<float4> v(n), a(n);
-    AXM_HIP(hipMemcpy(v.data(), w->pre_v, 16ull * n, hipMemcpyDeviceToHost));
-    AXM_HIP(hipMemcpy(a.data(), w->pre_w, 16ull * n, hipMemcpyDeviceToHost));
+    AXM_HIP(copy_sync(v.data(), w->pre_v, 16ull * n, hipMemcpyDeviceToHost));
+    AXM_HIP(copy_sync(a.data(), w->pre_w, 16ull * n, hipMemcpyDeviceToHost));
     for (uint32_t i = 0; i < n; ++i) {
         if (lin_vel) { lin_vel[3 * i] = v[i].x; lin_vel[3 * i + 1] = v[i].y; lin_vel[3 * i + 2] = v[i].z; }
         if (ang_vel) { ang_vel[3 * i] = a[i].x; ang_vel[3 * i + 1] = a[i].y; ang_vel[3 * i + 2] = a[i].z; }
@@ -1617,8 +1620,8 @@ axm_status axm_world_get_pairs(axm_world w, uint32_t* a, uint32_t* b, uint32_t c
     *count = P;
     if (cap < P) return AXM_OUT_OF_RANGE;
     if (P) {
-        if (a) AXM_HIP(hipMemcpy(a, w->pa, 4ull * P, hipMemcpyDeviceToHost));
-        if (b) AXM_HIP(hipMemcpy(b, w->pb, 4ull * P, hipMemcpyDeviceToHost));
+        if (a) AXM_HIP(copy_sync(a, w->pa, 4ull * P, hipMemcpyDeviceToHost));
+        if (b) AXM_HIP(copy_sync(b, w->pb, 4ull * P, hipMemcpyDeviceToHost));
     }
     return AXM_SUCCESS;
 }
@@ -1636,10 +1639,10 @@ axm_status axm_world_get_manifolds(axm_world w, uint32_t* a, uint32_t* b, uint32
     std::vector<uint2> ab(M);
     std::vector<uint32_t> np(M);
     std::vector<float4> pt((size_t)M * 4), nf((size_t)M * 4);
-    AXM_HIP(hipMemcpy(ab.data(), w->m_ab, 8ull * M, hipMemcpyDeviceToHost));
-    AXM_HIP(hipMemcpy(np.data(), w->m_np, 4ull * M, hipMemcpyDeviceToHost));
-    AXM_HIP(hipMemcpy(pt.data(), w->c_pt, 64ull * M, hipMemcpyDeviceToHost));
-    AXM_HIP(hipMemcpy(nf.data(), w->c_nf, 64ull * M, hipMemcpyDeviceToHost));
+    AXM_HIP(copy_sync(ab.data(), w->m_ab, 8ull * M, hipMemcpyDeviceToHost));
+    AXM_HIP(copy_sync(np.data(), w->m_np, 4ull * M, hipMemcpyDeviceToHost));
+    AXM_HIP(copy_sync(pt.data(), w->c_pt, 64ull * M, hipMemcpyDeviceToHost));
+    AXM_HIP(copy_sync(nf.data(), w->c_nf, 64ull * M, hipMemcpyDeviceToHost));
     for (uint32_t m = 0; m < M; ++m) {
         if (a) a[m] = ab[m].x;
         if (b) b[m] = ab[m].y;
@@ -1671,9 +1674,9 @@ axm_status axm_world_get_colours(axm_world w, uint32_t* colour, uint32_t* solve_
     if (num_colours) *num_colours = w->h_cnt->max_colour;
     if (cap < M) return AXM_OUT_OF_RANGE;
     if (M) {
-        if (colour) AXM_HIP(hipMemcpy(colour, w->col, 4ull * M, hipMemcpyDeviceToHost));
+        if (colour) AXM_HIP(copy_sync(colour, w->col, 4ull * M, hipMemcpyDeviceToHost));
         if (solve_order && w->solve_order)
-            AXM_HIP(hipMemcpy(solve_order, w->solve_order, 4ull * M, hipMemcpyDeviceToHost));
+            AXM_HIP(copy_sync(solve_order, w->solve_order, 4ull * M, hipMemcpyDeviceToHost));
     }
     return AXM_SUCCESS;
 }
@@ -1691,11 +1694,11 @@ axm_status axm_world_get_impulses(axm_world w, float* initial, float* final_, ui
     const SolverRows& R = w->R[set];
     const uint32_t rc = w->rcap[set];
     std::vector<uint4> hdr(M);
-    AXM_HIP(hipMemcpy(hdr.data(), R.hdr, 16ull * M, hipMemcpyDeviceToHost));
+    AXM_HIP(copy_sync(hdr.data(), R.hdr, 16ull * M, hipMemcpyDeviceToHost));
     std::vector<float4> l(M), l0(M);
     for (uint32_t k = 0; k < 4; ++k) {
-        AXM_HIP(hipMemcpy(l.data(), R.lam + (size_t)k * rc, 16ull * M, hipMemcpyDeviceToHost));
-        AXM_HIP(hipMemcpy(l0.data(), R.lam0 + (size_t)k * rc, 16ull * M, hipMemcpyDeviceToHost));
+        AXM_HIP(copy_sync(l.data(), R.lam + (size_t)k * rc, 16ull * M, hipMemcpyDeviceToHost));
+        AXM_HIP(copy_sync(l0.data(), R.lam0 + (size_t)k * rc, 16ull * M, hipMemcpyDeviceToHost));
         for (uint32_t s = 0; s < M; ++s) {
             const uint32_t m = hdr[s].w;
             const bool on = k < hdr[s].z;
@@ -1720,11 +1723,11 @@ axm_status axm_world_get_friction_bounds(axm_world w, float* bound, uint32_t cap
     const SolverRows& R = w->R[set];
     const uint32_t rc = w->rcap[set];
     std::vector<uint4> hdr(M);
-    AXM_HIP(hipMemcpy(hdr.data(), R.hdr, 16ull * M, hipMemcpyDeviceToHost));
+    AXM_HIP(copy_sync(hdr.data(), R.hdr, 16ull * M, hipMemcpyDeviceToHost));
     std::vector<float4> row(M);
     for (uint32_t k = 0; k < 4; ++k) {
         // row 8 of point k (t1's inverse-inertia row) carries the bound in .w
-        AXM_HIP(hipMemcpy(row.data(), R.J + ((size_t)k * JROWS + 8) * rc, 16ull * M, hipMemcpyDeviceToHost));
+        AXM_HIP(copy_sync(row.data(), R.J + ((size_t)k * JROWS + 8) * rc, 16ull * M, hipMemcpyDeviceToHost));
         for (uint32_t s = 0; s < M; ++s) bound[(size_t)hdr[s].w * 4 + k] = k < hdr[s].z ? row[s].w : 0.0f;
     }
     return AXM_SUCCESS;
@@ -1849,14 +1852,14 @@ axm_status axm_world_get_features(axm_world w, float* X, float* Y, uint32_t cap,
     const SolverRows& R = w->R[set];
     const uint32_t rc = w->rcap[set];
     std::vector<uint4> hdr(M);
-    AXM_HIP(hipMemcpy(hdr.data(), R.hdr, 16ull * M, hipMemcpyDeviceToHost));
+    AXM_HIP(copy_sync(hdr.data(), R.hdr, 16ull * M, hipMemcpyDeviceToHost));
     std::vector<float> f((size_t)M * 4 * MLP_IN);
-    AXM_HIP(hipMemcpy(f.data(), w->feat, sizeof(float) * f.size(), hipMemcpyDeviceToHost));
+    AXM_HIP(copy_sync(f.data(), w->feat, sizeof(float) * f.size(), hipMemcpyDeviceToHost));
     std::vector<float4> l(M), r0(M);
     const float gdt = MLP_G_REF * w->last_dt;
     for (uint32_t k = 0; k < 4; ++k) {
-        AXM_HIP(hipMemcpy(l.data(), R.lam + (size_t)k * rc, 16ull * M, hipMemcpyDeviceToHost));
-        AXM_HIP(hipMemcpy(r0.data(), R.J + (size_t)k * JROWS * rc, 16ull * M, hipMemcpyDeviceToHost));  // (n, mN)
+        AXM_HIP(copy_sync(l.data(), R.lam + (size_t)k * rc, 16ull * M, hipMemcpyDeviceToHost));
+        AXM_HIP(copy_sync(r0.data(), R.J + (size_t)k * JROWS * rc, 16ull * M, hipMemcpyDeviceToHost));  // (n, mN)
         for (uint32_t s = 0; s < M; ++s) {
             const uint32_t m = hdr[s].w;
             const bool on = k < hdr[s].z;
@@ -2019,7 +2022,7 @@ axm_status axm_world_load(axm_world w, const char* path) {
     w->desc = d;
     AXM_TRY(install_bodies(w, n, std::max(h.n_worlds, 1u), h.cell, h.use_filter != 0, &hb, nullptr, same));
     hipStream_t s = w->stream;
-    AXM_HIP(hipMemcpy(&w->cnt->steps_done, &h.steps_done, 4, hipMemcpyHostToDevice));
+    AXM_HIP(copy_sync(&w->cnt->steps_done, &h.steps_done, 4, hipMemcpyHostToDevice));
     if (mp) {
         // the previous step's cache in the set the next step reads, and its lookup table
         const int pv = 1 - w->cur;

@@ -111,7 +111,8 @@ typedef struct axm_world_desc {
     uint32_t max_manifolds;
     uint32_t auto_grow;    /* 1: grow pair/manifold buffers on overflow instead of failing */
     float residual_tol;    /* > 0: stop sweeping once the residual <= tol (checked every residual_every sweeps,
-                              inside the sweep launch; stats.iterations reports the sweeps run) */
+                              by islands solved on their own after each of theirs, inside the sweep
+                              launch; stats.iterations reports the sweeps run) */
     uint32_t residual_every;
     uint32_t max_iterations; /* cap when residual_tol > 0 */
     int32_t device;        /* HIP device ordinal */
